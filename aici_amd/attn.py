@@ -11,8 +11,7 @@ import numpy as np
 import torch
 
 from . import kernels
-from ._lib import call
-from .kernels import _desc, _stream
+from .kernels import _native
 from .paged import BatchInfo
 
 
@@ -84,30 +83,24 @@ def varlen_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, batch_info: B
         if batch_info.multi_block_tables is None:
             raise ValueError("paged_prefill needs batch_info.multi_block_tables (slots must follow the blocks in order)")
         has_m, has_p = batch_info.q_multi > 0, batch_info.q_multi < T
-        call("hipattn_varlen_attn_paged", _desc(q, "q"), _desc(k, "k"), _desc(v, "v"), _desc(key_cache, "key_cache"),
-             _desc(value_cache, "value_cache"), None if cached else _desc(batch_info.slot_mapping, "slot_mapping"),
-             _desc(batch_info.multi_block_tables, "multi_block_tables") if has_m else None,
-             _desc(batch_info.seqlens_q, "seqlens_q") if has_m else None,
-             _desc(batch_info.multi_context_lens, "multi_context_lens") if has_m else None, int(batch_info.q_multi),
-             int(batch_info.max_seqlen_q), int(batch_info.max_seqlen_k),
-             _desc(batch_info.paged_block_tables, "paged_block_tables") if has_p else None,
-             _desc(batch_info.paged_context_lens, "paged_context_lens") if has_p else None,
-             int(batch_info.paged_block_size), int(batch_info.paged_max_context_len), float(softmax_scale),
-             _desc(y, "y"), _stream(q))
+        _native.varlen_attn_paged(q, k, v, key_cache, value_cache, None if cached else batch_info.slot_mapping,
+                                  batch_info.multi_block_tables if has_m else None,
+                                  batch_info.seqlens_q if has_m else None,
+                                  batch_info.multi_context_lens if has_m else None, batch_info.q_multi,
+                                  batch_info.max_seqlen_q, batch_info.max_seqlen_k,
+                                  batch_info.paged_block_tables if has_p else None,
+                                  batch_info.paged_context_lens if has_p else None,
+                                  batch_info.paged_block_size, batch_info.paged_max_context_len, softmax_scale, y)
         return y.reshape(T, Hq * d)
     G = batch_info.gather_mapping.numel()
     gk = torch.empty((G, Hkv, d), dtype=q.dtype, device=q.device) if G else None
     gv = torch.empty_like(gk) if G else None
     has_multi = batch_info.q_multi > 0
     has_paged = batch_info.q_multi < T
-    call("hipattn_varlen_attn", _desc(q, "q"), _desc(k, "k"), _desc(v, "v"), _desc(key_cache, "key_cache"),
-         _desc(value_cache, "value_cache"), None if cached else _desc(batch_info.slot_mapping, "slot_mapping"),
-         _desc(batch_info.gather_mapping, "gather_mapping") if has_multi else None,
-         _desc(batch_info.seqlens_q, "seqlens_q") if has_multi else None,
-         _desc(batch_info.seqlens_k, "seqlens_k") if has_multi else None, int(batch_info.q_multi),
-         int(batch_info.max_seqlen_q), int(batch_info.max_seqlen_k),
-         _desc(batch_info.paged_block_tables, "paged_block_tables") if has_paged else None,
-         _desc(batch_info.paged_context_lens, "paged_context_lens") if has_paged else None,
-         int(batch_info.paged_block_size), int(batch_info.paged_max_context_len), float(softmax_scale),
-         _desc(gk, "gather_k"), _desc(gv, "gather_v"), _desc(y, "y"), _stream(q))
+    _native.varlen_attn(q, k, v, key_cache, value_cache, None if cached else batch_info.slot_mapping,
+                        batch_info.gather_mapping if has_multi else None, batch_info.seqlens_q if has_multi else None,
+                        batch_info.seqlens_k if has_multi else None, batch_info.q_multi, batch_info.max_seqlen_q,
+                        batch_info.max_seqlen_k, batch_info.paged_block_tables if has_paged else None,
+                        batch_info.paged_context_lens if has_paged else None, batch_info.paged_block_size,
+                        batch_info.paged_max_context_len, softmax_scale, gk, gv, y)
     return y.reshape(T, Hq * d)

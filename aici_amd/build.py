@@ -1,5 +1,6 @@
 """Builds libhipattn.so (the HIP kernels + C ABI) and libmembench.so (the benchmark's memory-system
-yardsticks, csrc/bench/) for gfx950 with hipcc.
+yardsticks, csrc/bench/) for gfx950 with hipcc, and _native.so (the CPython binding of the hot entry
+points, csrc/bind/) with g++.
 
     python -m aici_amd.build [--force] [-j N]
 
@@ -12,9 +13,11 @@ from __future__ import annotations
 
 import argparse
 import concurrent.futures
+import importlib.util
 import os
 import subprocess
 import sys
+import sysconfig
 import time
 from pathlib import Path
 
@@ -24,6 +27,8 @@ OBJ = CSRC / "build"
 LIB = PKG / "libhipattn.so"
 BENCH_SRC = CSRC / "bench" / "membench.hip"
 BENCH_LIB = PKG / "libmembench.so"
+BIND_SRC = CSRC / "bind" / "native.cpp"
+BIND_LIB = PKG / "_native.so"
 
 # -packed-fp32-ops: keep hipcc from forming packed FP32 instructions; the
 # host pass does not know the feature and says so, which is harmless.
@@ -56,6 +61,21 @@ def _compile(src: Path, force: bool, hdr_mtime: float) -> tuple[str, float, str]
     return src.name, time.time() - t0, msgs
 
 
+def _build_binding(force: bool, verbose: bool) -> None:
+    """_native.so: needs Python.h and torch's DLPack header, links libhipattn.so beside it."""
+    if not force and BIND_LIB.exists() and BIND_LIB.stat().st_mtime >= max(
+            BIND_SRC.stat().st_mtime, (PKG.parent / "include" / "hipattn.h").stat().st_mtime):
+        return
+    torch_dir = Path(importlib.util.find_spec("torch").origin).parent
+    r = subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", str(BIND_SRC), "-o", str(BIND_LIB),
+                        f"-I{sysconfig.get_paths()['include']}", f"-I{torch_dir / 'include'}", f"-L{PKG}",
+                        "-l:libhipattn.so", "-Wl,-rpath,$ORIGIN"], capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on {BIND_SRC.name}:\n{r.stdout}{r.stderr}")
+    if verbose:
+        print(f"[build] linked {BIND_LIB}", flush=True)
+
+
 def build(force: bool = False, jobs: int | None = None, verbose: bool = True) -> Path:
     OBJ.mkdir(parents=True, exist_ok=True)
     jobs = jobs or min(8, os.cpu_count() or 4)
@@ -74,6 +94,7 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = True) ->
             raise RuntimeError(f"link failed:\n{r.stdout}{r.stderr}")
         if verbose:
             print(f"[build] linked {LIB}", flush=True)
+    _build_binding(force, verbose)
     if force or not BENCH_LIB.exists() or BENCH_LIB.stat().st_mtime < BENCH_SRC.stat().st_mtime:
         r = subprocess.run(["hipcc", "-shared", "-fPIC", "-O3", "-std=c++17", "--offload-arch=gfx950", str(BENCH_SRC),
                             "-o", str(BENCH_LIB)], capture_output=True, text=True)

@@ -17,6 +17,11 @@ import torch
 from . import _lib
 from ._lib import HipAttnError, Tensor, call
 
+try:
+    from . import _native  # the hot entry points, bound without ctypes (csrc/bind/native.cpp)
+except ImportError as e:
+    raise ImportError("aici_amd/_native.so is missing or was built for another torch: run `python -m aici_amd.build`") from e
+
 _DTYPES = {
     torch.float32: _lib.F32,
     torch.float16: _lib.F16,
@@ -64,10 +69,8 @@ def flash_attn_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, seqlens
     lse = None
     if return_lse:
         lse = torch.empty((seqlens_q.numel() - 1, q.size(1), max_seqlen_q), dtype=torch.float32, device=q.device)
-    call("hipattn_mha_varlen_fwd", _desc(q, "q"), _desc(k, "k"), _desc(v, "v"), _desc(seqlens_q, "seqlens_q"),
-         _desc(seqlens_k, "seqlens_k"), _desc(seqused_k, "seqused_k"), int(max_seqlen_q), int(max_seqlen_k), 0.0,
-         float(softmax_scale), False, bool(causal), int(window[0]), int(window[1]), _desc(out, "out"),
-         _desc(lse, "lse"), _stream(q))
+    _native.mha_varlen_fwd(q, k, v, seqlens_q, seqlens_k, seqused_k, max_seqlen_q, max_seqlen_k, 0.0, softmax_scale,
+                           False, causal, window[0], window[1], out, lse)
     return (out, lse) if return_lse else out
 
 
@@ -87,10 +90,8 @@ def flash_attn_varlen_paged(q: torch.Tensor, key_cache: torch.Tensor, value_cach
     if return_lse:
         lse = torch.empty((context_lens.numel(), q.size(1), max(int(max_seqlen_q), 1)), dtype=torch.float32,
                           device=q.device)
-    call("hipattn_mha_varlen_fwd_paged", _desc(q, "q"), _desc(key_cache, "key_cache"), _desc(value_cache, "value_cache"),
-         _desc(block_tables, "block_tables"), _desc(seqlens_q, "cu_seqlens_q"), _desc(context_lens, "context_lens"),
-         int(max_seqlen_q), int(max_seqlen_k), float(softmax_scale), bool(causal), _desc(out, "out"), _desc(lse, "lse"),
-         _stream(q))
+    _native.mha_varlen_fwd_paged(q, key_cache, value_cache, block_tables, seqlens_q, context_lens, max_seqlen_q,
+                                 max_seqlen_k, softmax_scale, causal, out, lse)
     return (out, lse) if return_lse else out
 
 
@@ -98,10 +99,8 @@ def paged_attention_v1(out: torch.Tensor, query: torch.Tensor, key_cache: torch.
                        num_kv_heads: int, scale: float, block_tables: torch.Tensor, context_lens: torch.Tensor,
                        block_size: int, max_context_len: int, alibi_slopes: Optional[torch.Tensor] = None) -> None:
     """lib.rs:356-391."""
-    call("hipattn_paged_attention_v1", _desc(out, "out"), _desc(query, "query"), _desc(key_cache, "key_cache"),
-         _desc(value_cache, "value_cache"), int(num_kv_heads), float(scale), _desc(block_tables, "block_tables"),
-         _desc(context_lens, "context_lens"), int(block_size), int(max_context_len), _desc(alibi_slopes, "alibi"),
-         _stream(query))
+    _native.paged_attention_v1(out, query, key_cache, value_cache, num_kv_heads, scale, block_tables, context_lens,
+                               block_size, max_context_len, alibi_slopes)
 
 
 def paged_attention_workspace_size(num_seqs: int, num_heads: int, num_kv_heads: int, head_size: int, block_size: int,
@@ -131,10 +130,8 @@ def paged_attention_v1_static(out: torch.Tensor, query: torch.Tensor, key_cache:
                               context_lens: torch.Tensor, block_size: int, max_context_len: int,
                               alibi_slopes: Optional[torch.Tensor] = None) -> None:
     """paged_attention_v1 on the library's built-in scratch array: allocates nothing."""
-    call("hipattn_paged_attention_v1_static", _desc(out, "out"), _desc(query, "query"), _desc(key_cache, "key_cache"),
-         _desc(value_cache, "value_cache"), int(num_kv_heads), float(scale), _desc(block_tables, "block_tables"),
-         _desc(context_lens, "context_lens"), int(block_size), int(max_context_len), _desc(alibi_slopes, "alibi"),
-         _stream(query))
+    _native.paged_attention_v1_static(out, query, key_cache, value_cache, num_kv_heads, scale, block_tables,
+                                      context_lens, block_size, max_context_len, alibi_slopes)
 
 
 def init() -> None:
@@ -158,28 +155,22 @@ def paged_attention_v2(out: torch.Tensor, exp_sums: torch.Tensor, max_logits: to
                        scale: float, block_tables: torch.Tensor, context_lens: torch.Tensor, block_size: int,
                        max_context_len: int, alibi_slopes: Optional[torch.Tensor] = None) -> None:
     """lib.rs:122-137 (declared there, no safe wrapper in the reference)."""
-    call("hipattn_paged_attention_v2", _desc(out, "out"), _desc(exp_sums, "exp_sums"),
-         _desc(max_logits, "max_logits"), _desc(tmp_out, "tmp_out"), _desc(query, "query"),
-         _desc(key_cache, "key_cache"), _desc(value_cache, "value_cache"), int(num_kv_heads), float(scale),
-         _desc(block_tables, "block_tables"), _desc(context_lens, "context_lens"), int(block_size),
-         int(max_context_len), _desc(alibi_slopes, "alibi"), _stream(query))
+    _native.paged_attention_v2(out, exp_sums, max_logits, tmp_out, query, key_cache, value_cache, num_kv_heads, scale,
+                               block_tables, context_lens, block_size, max_context_len, alibi_slopes)
 
 
 # --------------------------------------------------------------------------- cache movement
 
 def reshape_and_cache(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor,
                       slot_mapping: torch.Tensor) -> None:
-    """lib.rs:192-213; like the reference wrapper, the slots are widened to int64."""
-    slot_mapping = slot_mapping.to(torch.int64)
-    call("hipattn_reshape_and_cache", _desc(key, "key"), _desc(value, "value"), _desc(key_cache, "key_cache"),
-         _desc(value_cache, "value_cache"), _desc(slot_mapping, "slot_mapping"), _stream(key))
+    """lib.rs:192-213.  The reference's wrapper widens the slots to int64; the kernels read either width."""
+    _native.reshape_and_cache(key, value, key_cache, value_cache, slot_mapping)
 
 
 def gather_cached_kv(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor,
                      slot_mapping: torch.Tensor) -> None:
     """lib.rs:215-234."""
-    call("hipattn_gather_cached_kv", _desc(key, "key"), _desc(value, "value"), _desc(key_cache, "key_cache"),
-         _desc(value_cache, "value_cache"), _desc(slot_mapping, "slot_mapping"), _stream(key))
+    _native.gather_cached_kv(key, value, key_cache, value_cache, slot_mapping)
 
 
 def copy_blocks(key_caches: List[torch.Tensor], value_caches: List[torch.Tensor],
@@ -221,8 +212,7 @@ def swap_blocks(src: torch.Tensor, dst: torch.Tensor, block_mapping: Dict[int, i
 def rotary_embedding(positions: torch.Tensor, query: torch.Tensor, key: torch.Tensor, head_size: int,
                      cos_sin_cache: torch.Tensor, is_neox: bool) -> None:
     """lib.rs:333-354; query/key [T, H*d] are rotated in place."""
-    call("hipattn_rotary_embedding", _desc(positions, "positions"), _desc(query, "query"), _desc(key, "key"),
-         int(head_size), _desc(cos_sin_cache, "cos_sin_cache"), bool(is_neox), _stream(query))
+    _native.rotary_embedding(positions, query, key, head_size, cos_sin_cache, is_neox)
 
 
 def rotary_embedding_and_cache(positions: torch.Tensor, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
@@ -230,20 +220,16 @@ def rotary_embedding_and_cache(positions: torch.Tensor, query: torch.Tensor, key
                                value_cache: torch.Tensor, slot_mapping: torch.Tensor) -> None:
     """rotary_embedding (llm/mod.rs:88-114) and reshape_and_cache (mod.rs:147-164) of a step's new tokens in
     one launch: query/key [T, H*d] rotated in place, rotated keys and value [T, Hkv, d] written to the cache."""
-    call("hipattn_rotary_embedding_and_cache", _desc(positions, "positions"), _desc(query, "query"),
-         _desc(key, "key"), _desc(value, "value"), int(head_size), _desc(cos_sin_cache, "cos_sin_cache"),
-         bool(is_neox), _desc(key_cache, "key_cache"), _desc(value_cache, "value_cache"),
-         _desc(slot_mapping, "slot_mapping"), _stream(query))
+    _native.rotary_embedding_and_cache(positions, query, key, value, head_size, cos_sin_cache, is_neox, key_cache,
+                                       value_cache, slot_mapping)
 
 
 def rms_norm(out: torch.Tensor, input: torch.Tensor, weight: torch.Tensor, epsilon: float) -> None:
-    call("hipattn_rms_norm", _desc(out, "out"), _desc(input, "input"), _desc(weight, "weight"), float(epsilon),
-         _stream(input))
+    _native.rms_norm(out, input, weight, epsilon)
 
 
 def fused_add_rms_norm(input: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, epsilon: float) -> None:
-    call("hipattn_fused_add_rms_norm", _desc(input, "input"), _desc(residual, "residual"), _desc(weight, "weight"),
-         float(epsilon), _stream(input))
+    _native.fused_add_rms_norm(input, residual, weight, epsilon)
 
 
 LINEAR_MAX_ROWS = 128
@@ -263,8 +249,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     it for the rows of a generation step (llm/mod.rs:401-416; llama.rs:81-83, 96, 135-143, 210)."""
     if out is None:
         out = torch.empty((x.size(0), weight.size(0)), dtype=x.dtype, device=x.device)
-    call("hipattn_linear", _desc(out, "out"), _desc(x, "x"), _desc(weight, "weight"), _desc(bias, "bias"),
-         _desc(residual, "residual"), _desc(workspace, "workspace"), _stream(x))
+    _native.linear(out, x, weight, bias, residual, workspace)
     return out
 
 
@@ -275,9 +260,7 @@ def linear_rms_norm(x: torch.Tensor, weight: torch.Tensor, norm_weight: torch.Te
     the same bits as `linear` followed by `rms_norm`."""
     out = torch.empty((x.size(0), weight.size(0)), dtype=x.dtype, device=x.device)
     normed = torch.empty_like(out)
-    call("hipattn_linear_rms_norm", _desc(out, "out"), _desc(normed, "norm_out"), _desc(x, "x"), _desc(weight, "weight"),
-         _desc(bias, "bias"), _desc(residual, "residual"), _desc(norm_weight, "norm_weight"), float(epsilon),
-         _desc(workspace, "workspace"), _stream(x))
+    _native.linear_rms_norm(out, normed, x, weight, bias, residual, norm_weight, epsilon, workspace)
     return out, normed
 
 
@@ -294,15 +277,15 @@ def linear_workspace_size(x: torch.Tensor, weight: torch.Tensor) -> int:
 
 
 def silu_and_mul(out: torch.Tensor, input: torch.Tensor) -> None:
-    call("hipattn_silu_and_mul", _desc(out, "out"), _desc(input, "input"), _stream(input))
+    _native.silu_and_mul(out, input)
 
 
 def gelu_new(out: torch.Tensor, input: torch.Tensor) -> None:
-    call("hipattn_gelu_new", _desc(out, "out"), _desc(input, "input"), _stream(input))
+    _native.gelu_new(out, input)
 
 
 def gelu_fast(out: torch.Tensor, input: torch.Tensor) -> None:
-    call("hipattn_gelu_fast", _desc(out, "out"), _desc(input, "input"), _stream(input))
+    _native.gelu_fast(out, input)
 
 
 def bias_argmax(logits: torch.Tensor, bias: Optional[torch.Tensor] = None, mask: Optional[torch.Tensor] = None,
@@ -313,8 +296,7 @@ def bias_argmax(logits: torch.Tensor, bias: Optional[torch.Tensor] = None, mask:
     S = logits.size(0)
     tokens = torch.empty((S,), dtype=torch.int32, device=logits.device)
     best = torch.empty((S,), dtype=torch.float32, device=logits.device) if return_logits else None
-    call("hipattn_bias_argmax", _desc(logits, "logits"), _desc(bias, "bias"), _desc(mask, "mask"),
-         _desc(bias_rows, "bias_rows"), _desc(tokens, "out_tokens"), _desc(best, "out_logits"), _stream(logits))
+    _native.bias_argmax(logits, bias, mask, bias_rows, tokens, best)
     return (tokens, best) if return_logits else tokens
 
 
@@ -326,9 +308,7 @@ def bias_sample(logits: torch.Tensor, temperature: torch.Tensor, top_p: torch.Te
     the caller's random numbers (one per row).  Returns int32 [S]."""
     S = logits.size(0)
     tokens = torch.empty((S,), dtype=torch.int32, device=logits.device)
-    call("hipattn_bias_sample", _desc(logits, "logits"), _desc(bias, "bias"), _desc(mask, "mask"),
-         _desc(bias_rows, "bias_rows"), _desc(temperature, "temperature"), _desc(top_p, "top_p"),
-         _desc(uniforms, "uniforms"), _desc(tokens, "out_tokens"), _stream(logits))
+    _native.bias_sample(logits, bias, mask, bias_rows, temperature, top_p, uniforms, tokens)
     return tokens
 
 

@@ -1,0 +1,44 @@
+"""The CPython binding of the hot entry points (csrc/bind/native.cpp) and the one-copy upload of a batch."""
+import pytest
+import torch
+
+from aici_amd import _lib, _native, paged
+
+
+def test_arguments_are_checked_before_the_call():
+    x = torch.zeros((2, 16), dtype=torch.bfloat16)
+    with pytest.raises(_lib.HipAttnError, match="out: expected a GPU tensor, got one on cpu"):
+        _native.silu_and_mul(x, x)
+    with pytest.raises(_lib.HipAttnError, match="input: unsupported dtype torch.bool"):
+        _native.gelu_new(None, x.bool())
+    with pytest.raises(TypeError, match="weight: expected a torch.Tensor or None, got int"):
+        _native.rms_norm(None, None, 3, 1e-5)
+    with pytest.raises(TypeError, match="takes 4 arguments"):
+        _native.rms_norm(x)
+    with pytest.raises(_lib.HipAttnError, match="hipattn_reshape_and_cache: .*NULL"):
+        _native.reshape_and_cache(None, None, None, None, None)
+
+
+def _batch(lens):
+    alloc = paged.BlockAllocator(16, 256)
+    b = paged.BatchInfoBuilder(16, 4096, 1)
+    for sid, (n, computed) in enumerate(lens, start=1):
+        alloc.alloc_seq(sid, n)
+        b.sched_out(alloc, sid, list(range(n)), computed)
+    return b.finish()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens", [[(1, 0)], [(37, 0), (5, 4), (100, 99)], [(64, 17)], [(3, 2), (300, 299)]])
+def test_batch_upload_keeps_every_array(device, lens):
+    host = _batch(lens)
+    for _ in range(3):  # the staging buffer is reused
+        dev = host.to(device)
+        for name, want in host.__dict__.items():
+            got = getattr(dev, name)
+            if isinstance(want, torch.Tensor):
+                assert got.is_cuda and got.dtype == want.dtype and got.shape == want.shape
+                assert got.data_ptr() % 16 == 0 or got.numel() == 0
+                assert torch.equal(got.cpu(), want), name
+            else:
+                assert got == want
