@@ -60,6 +60,13 @@ __device__ __forceinline__ T sub_t(T a, T b) {
   return from_float<T>(to_float(a) - to_float(b));
 }
 
+// x * sigmoid(x), rounded once (activation_kernels.cu:15-18).
+template <typename T>
+__device__ __forceinline__ T silu_t(T x) {
+  const float f = to_float(x);
+  return from_float<T>(f / (1.0f + expf(-f)));
+}
+
 // A 16-byte load of data that a kernel reads once: with the non-temporal hint the line is not kept in the
 // caches at the expense of data that is used again (or, in a purely streaming kernel, of the lines still on
 // their way).  HA_NT_STREAM = 0 builds the plain load, for comparison.

@@ -184,12 +184,6 @@ __global__ __launch_bounds__(1024) void rms_norm_vec8_kernel(T *__restrict__ out
 // Activations (activation_kernels.cu:15-115).
 // ---------------------------------------------------------------------------
 template <typename T>
-__device__ __forceinline__ T silu_t(T x) {
-  const float f = to_float(x);
-  return from_float<T>(f / (1.0f + expf(-f)));
-}
-
-template <typename T>
 __global__ __launch_bounds__(1024) void silu_and_mul_kernel(T *__restrict__ out, const T *__restrict__ in, int d) {
   const int64_t row = blockIdx.x;
   for (int i = threadIdx.x; i < d; i += blockDim.x) {

@@ -3,41 +3,51 @@
 // `linear_no_bias`, llm/mod.rs:401-407; phi.rs:70-71, 99, 116-117 through `linear`, mod.rs:409-416), where every
 // element of W is used once per row of x and the time goes into reading W from HBM exactly once.
 //
-// Shape of the kernel: a workgroup of four (or eight) wavefronts owns 128 (64 .. 256) rows of W and a range of k; a
-// wavefront owns 32 (or 16) of those rows.  Per 32 values of k a wavefront loads its pieces of W straight from
-// global memory into the A operand of v_mfma_f32_16x16x32 (lane l: row l % 16, the 8 values of k at 8 (l / 16): 64
-// contiguous bytes per row and instruction, plain loads; the pieces of four to eight steps are in flight per wavefront, asked
-// for two steps at a time) and multiplies them with the eight 16-row tiles of x, which the workgroup keeps in LDS
-// in operand order (a lane's 16 bytes at its lane index: read without bank conflicts, one step ahead of the
-// MFMAs that use them), three stages of 64 values of k, one barrier per stage.  Rows of x reach LDS through
-// registers, asked for as far ahead as the pieces of W: a wavefront's loads complete in order, so anything closer
-// would drain the pieces of W at every stage.  The accumulators hold y transposed: lane l has rows 4 (l / 16) .. + 3
-// of its 16 rows of W -- four consecutive outputs of one row of y.
+// Both kernels copy W and x global -> LDS (global_load_lds_dwordx4, no registers) into a ring of stages of 64 values
+// of k: an instruction brings 128 whole bytes of eight rows, its runs of 16 bytes swizzled by the row's low bits so that the
+// operands of v_mfma_f32_16x16x32 are read from LDS without bank conflicts.  What bounds them is how many whole
+// cache lines are on their way: the same loop with W loaded straight into the operands (16 rows x 64 bytes per instruction, so
+// every line asked for twice, and both copies of it held in the 32 KB L1) reached 5.1 TB/s on a 28672 x 4096 weight and one row of x,
+// 4.0 with sixteen; this form 6.0 and 5.5 (library GEMM: 3.9 / 3.9).
 //
-// When W has too few rows to occupy the device, the range of k is split between workgroups; each leaves its sums
-// in fp32 in operand order, and a second launch adds them up in a fixed order (no atomics: the same bits on every
-// run), then bias, rounding and residual as in the one-launch form.
+//   linear_stream_kernel, up to 16 rows of x: a wavefront owns 16 (or 64) rows of W and keeps a private ring, its own copy of
+//   the rows of x in it, so nothing waits for anything but the wavefront's own copies; wavefronts that share rows of W
+//   take different ranges of k and meet once, in LDS, at the end.
+//   linear_tile_kernel, 17 to 128 rows: the copies of x are shared by the workgroup (one barrier per stage); ranges of k
+//   go to workgroups of their own, which leave fp32 sums for a second launch to add up.
 //
-// Rounding points: fp32 accumulation over k (in the order the splits dictate), + bias in fp32, rounded to T -- what
-// a library GEMM with a bias epilogue does; then, if a residual is given, T(y + residual): the separate addition
-// of llama.rs:166, 173, rounded again.
+// The ranges of k are a function of the weight's shape alone, every range is summed front to back and the ranges are
+// added up first to last: a row gets the same bits whichever kernel, launch shape and company it is computed in, and
+// on every run (no atomics).
+//
+// Microseconds (bf16, copies of W in turns so that no cache holds it; library GEMM -> here):
+//                       1 row          16 rows        32 rows        64 rows        128 rows
+//   4096 x 4096         22.8 -> 7.7    20.8 -> 8.2    21.1 -> 11.3   21.1 -> 12.2   24.2 -> 16.1
+//   6144 x 4096         20.8 -> 10.9   19.8 -> 12.7   19.8 -> 14.5   19.6 -> 16.6   25.3 -> 21.3
+//   4096 x 14336        25.6 -> 19.2   25.8 -> 22.7   30.8 -> 24.9   38.9 -> 27.0   75.3 -> 31.4
+//   28672 x 4096        58.8 -> 40.1   59.8 -> 43.7   51.2 -> 43.0   51.4 -> 47.2   53.9 -> 53.1
+//     + silu_and_mul    62.9 -> 41.7   64.2 -> 44.0   56.8 -> 43.1   57.9 -> 49.7   61.0 -> 54.8
+//   128256 x 4096       183 -> 166     186 -> 166     196 -> 186     208 -> 211     232 -> 248
+// (one row of 28672 x 4096 is 5.9 TB/s; what bounds the many-row end is the LDS: 128 rows of x are read from it by every
+// wavefront, eight times the bytes of W, and a workgroup has the compute unit to itself, its start and end open.)
+//
+// Rounding points: fp32 accumulation over k, + bias in fp32, rounded to T -- what a library GEMM with a bias epilogue
+// does; then, if a residual is given, T(y + residual): the separate addition of llama.rs:166, 173, rounded again.
 #include "common.h"
 #include "device_types.h"
 #include "workspace.h"
+
+// The copies set M0, and say so; the compiler reports that it is a reserved register.
+#pragma clang diagnostic ignored "-Winline-asm"
 
 namespace hipattn {
 namespace {
 
 constexpr int kLinMaxRows = 128;  // rows of x
 constexpr int kLinMT = 8;         // 16-row tiles of x
-constexpr int kLinStepK = 32;     // values of k per MFMA
-constexpr int kLinChunkSteps = 2;
-constexpr int kLinChunkK = kLinStepK * kLinChunkSteps;
-constexpr int kLinGroupK = 256;  // the inner dimension goes to the splits in pieces of this size: kLinGroupSteps steps
-constexpr int kLinStages = 3;
-constexpr int kLinBunch = 2;  // steps whose pieces of W are asked for together
-constexpr int kLinGroupSteps = 8;  // the host hands out the inner dimension in groups of this many steps
-constexpr int kLinStageUnits = kLinChunkSteps * kLinMT * 64;  // 16-byte units per stage
+constexpr int kLinStageK = 64;    // values of k per stage: 128 bytes of a row
+constexpr int kLinStreamRows = 16;
+constexpr int kLinMaxRanges = 8;  // ranges of k that the library itself chooses
 
 struct LinearParams {
   const void *x, *w, *bias, *residual;
@@ -46,7 +56,9 @@ struct LinearParams {
   int M, N, K;
   int mtiles;  // ceil(M / 16)
   int64_t ldx, ldw, ldr, ldo;
-  int splits, steps_per_split, total_steps;
+  int splits, stages_per_split, total_stages;  // ranges of k
+  // silu_and_mul behind the layer: W holds `half` gate rows and then as many up rows, the output has `half` columns
+  int half;
   // with an RMS norm behind the layer: the sums go to the workspace as rows ([range][128 rows][N] fp32), and the
   // launch that adds them up also normalises the finished row
   int row_sums;
@@ -71,17 +83,6 @@ struct LinMfma<bf16_t> {
   }
 };
 
-// A piece of W: a plain load.  The two 64-byte halves of a cache line are asked for by two instructions, and with
-// the read-once hint the line may be gone before the second one arrives (measured: 10 % slower on the shapes of a
-// decode step).
-__device__ __forceinline__ uint4 load_w(const void *p) { return *static_cast<const uint4 *>(p); }
-
-template <typename To, typename From>
-__device__ __forceinline__ To lin_cast(From v) {
-  static_assert(sizeof(To) == sizeof(From), "size");
-  return __builtin_bit_cast(To, v);
-}
-
 // v[r] = the fp32 sum for y[m][n + r], r = 0..3: bias, rounding, residual, one 8-byte store.
 template <typename T>
 __device__ __forceinline__ void linear_finish(const LinearParams &p, f32x4_t v, int m, int n) {
@@ -103,184 +104,322 @@ __device__ __forceinline__ void linear_finish(const LinearParams &p, f32x4_t v, 
   *reinterpret_cast<vec4 *>(static_cast<T *>(p.out) + (int64_t)m * p.ldo + n) = o;
 }
 
-// WAVES: wavefronts per workgroup (4 or 8).  NT: 16-row tiles of W per wavefront.  DEPTH: steps for which a wavefront has its pieces of W in flight (and the
-// unrolling of the main loop); DEPTH / 2 stages of x are in flight in registers beside them.
-template <typename T, int NT, int DEPTH, int WAVES>
-__global__ __launch_bounds__(WAVES * 64, 2) void skinny_linear_kernel(const LinearParams p) {
+// The same for a gated layer: gate and up sums of y[m][n + r], each rounded, then the arithmetic of silu_and_mul.
+template <typename T>
+__device__ __forceinline__ void linear_finish_gated(const LinearParams &p, f32x4_t gate, f32x4_t up, int m, int n) {
+  typedef T vec4 __attribute__((ext_vector_type(4)));
+  if (m >= p.M || n >= p.half) return;
+  vec4 o;
+#pragma unroll
+  for (int r = 0; r < 4; r++) o[r] = mul_t<T>(silu_t<T>(from_float<T>(gate[r])), from_float<T>(up[r]));
+  *reinterpret_cast<vec4 *>(static_cast<T *>(p.out) + (int64_t)m * p.ldo + n) = o;
+}
+
+template <int N>
+__device__ __forceinline__ void wait_copies() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+template <typename P>
+__device__ __forceinline__ const P *uniform_base(const P *ptr) {
+  const uint64_t v = reinterpret_cast<uint64_t>(ptr);
+  return reinterpret_cast<const P *>(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) << 32) |
+                                     (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v));
+}
+
+// What a copy instruction brings of a stage: 128 bytes of each of eight rows (first .. first + 7; rows past `last` repeat
+// it, and what is made of them is never stored).  One scalar base for the eight rows, a 32-bit offset per lane.
+struct CopySource {
+  const char *base;
+  uint32_t off;
+};
+template <typename T>
+__device__ __forceinline__ CopySource copy_source(const void *rows, int64_t ld, int first, int last, int stage0) {
+  const int lane = threadIdx.x & 63, r = lane >> 3, q = (lane & 7) ^ r;  // run q of row r goes to this lane's place
+  const int b = min(first, last);
+  CopySource s;
+  s.base = uniform_base(reinterpret_cast<const char *>(static_cast<const T *>(rows) + b * ld + (int64_t)stage0 * kLinStageK));
+  s.off = (uint32_t)min(first + r, last) - (uint32_t)b;
+  s.off = s.off * (uint32_t)(ld * 2) + q * 16;
+  return s;
+}
+
+// 64 lanes x 16 bytes of stage st, global -> LDS: lane l's bytes go to lds + 16 l.  ONCE: with the read-once hint.
+template <bool ONCE>
+__device__ __forceinline__ void copy_1k(uint32_t lds, const CopySource &s, int st) {
+  const char *base = s.base + (int64_t)st * (kLinStageK * 2);
+  if (ONCE)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(s.off), "s"(base) : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(s.off), "s"(base) : "memory", "m0");
+}
+
+__device__ __forceinline__ uint32_t lds_address(const void *p) {
+  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char *)p);
+}
+
+// A stage's rows lie 128 bytes apart; run q (16 bytes) of row r is kept at place q ^ (r & 7).
+__device__ __forceinline__ const uint4 *staged_run(const char *rows, int r, int q) {
+  return reinterpret_cast<const uint4 *>(rows + r * (kLinStageK * 2) + ((q ^ (r & 7)) * 16));
+}
+
+// Up to 16 rows of x.  WAVES wavefronts; each owns 16 NT rows of W.  GATED: odd wavefronts take the up rows that
+// belong to the gate rows of the wavefront before them.
+template <typename T, int NT, int S, int WAVES, bool GATED>
+__global__ __launch_bounds__(WAVES * 64) void linear_stream_kernel(const LinearParams p) {
   using vec8 = typename Vec8<T>::type;
-  constexpr int kLinDepth = DEPTH, kLinXAhead = DEPTH / kLinChunkSteps;
-  static_assert(kLinGroupSteps % DEPTH == 0 && DEPTH % kLinChunkSteps == 0, "depth");
-  __shared__ uint4 xs[kLinStages * kLinStageUnits];
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int kParts = GATED ? 2 : 1;
+  constexpr int kCopiesW = 2 * NT, kCopiesX = 2, kCopies = kCopiesW + kCopiesX;  // of 1 KB: eight rows each
+  constexpr int kStageBytes = kCopies * 1024;
+  static_assert(NT == 1 || !GATED, "gated: one tile per wavefront");
+  __shared__ __align__(1024) char ring[WAVES * S * kStageBytes];
+  // NT > 1 is for weights of so many rows that k is not cut
+  __shared__ f32x4_t sums[NT == 1 ? kParts * kLinMaxRanges * 64 : 1];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, kg = lane >> 4;
-  const int n_wave = (blockIdx.x * WAVES + wave) * 16 * NT;
-  const int split = blockIdx.y;
-  const int step0 = split * p.steps_per_split;
-  const int nsteps = min(p.steps_per_split, p.total_steps - step0);
-  const int nchunks = nsteps / kLinChunkSteps;
-  const int64_t k_first = (int64_t)step0 * kLinStepK;
+  // wavefronts per tile of 16 NT rows, and the ranges of k each of them takes, one after the other
+  const int per_tile = min(p.splits, WAVES / kParts);
+  const int ranges = p.splits / per_tile;
+  const int part = GATED ? wave & 1 : 0;
+  const int tile = (wave / kParts) / per_tile, first_range = ((wave / kParts) % per_tile) * ranges;
+  const int tiles = WAVES / kParts / per_tile;
+  const int n_tile = (blockIdx.x * tiles + tile) * 16 * NT;
+  const int n_end = GATED ? p.half : p.N;
+  const int stage0 = first_range * p.stages_per_split;
+  const int nst = max(0, min(ranges * p.stages_per_split, p.total_stages - stage0));
 
-  // This lane's rows of W (rows past the end repeat the last one; their sums are never stored).
-  const T *wrow[NT];
+  CopySource wsrc[kCopiesW], xsrc[kCopiesX];
 #pragma unroll
-  for (int t = 0; t < NT; t++) {
-    const int n = min(n_wave + t * 16 + col, p.N - 1);
-    wrow[t] = static_cast<const T *>(p.w) + (int64_t)n * p.ldw + k_first + 8 * kg;
-  }
-  // The 16-byte units of x that this thread copies per stage: of the sixteen fragments (step * 8 + row tile) a
-  // wavefront takes every WAVES-th, starting at its own number.
-  constexpr int kUnits = kLinChunkSteps * kLinMT / WAVES;
-  const T *xsrc[kUnits];
+  for (int i = 0; i < kCopiesW; i++)
+    wsrc[i] = copy_source<T>(p.w, p.ldw, part * p.half + n_tile + i * 8, part * p.half + n_end - 1, stage0);
 #pragma unroll
-  for (int i = 0; i < kUnits; i++) {
-    const int f = wave + WAVES * i;
-    const int m = min((f % kLinMT) * 16 + col, p.M - 1);
-    xsrc[i] = static_cast<const T *>(p.x) + (int64_t)m * p.ldx + k_first + (f / kLinMT) * kLinStepK + 8 * kg;
-  }
-  // Rows of x travel through registers into LDS, several stages' worth in flight (a stage's rows are asked for
-  // kLinXAhead stages before they are written to LDS): the loads of a wavefront complete in order, so waiting for a
-  // stage's rows also waits for every piece of W asked for before them, and only this distance leaves the pieces
-  // of the last kLinDepth steps in flight.
-  struct XRows {
-    uint4 u[kUnits];
+  for (int i = 0; i < kCopiesX; i++) xsrc[i] = copy_source<T>(p.x, p.ldx, i * 8, p.M - 1, stage0);
+  const char *mine = ring + wave * S * kStageBytes;
+  const uint32_t mine_lds = lds_address(ring) + wave * S * kStageBytes;
+  auto ask = [&](int slot, int st) {
+    const uint32_t at = mine_lds + slot * kStageBytes;
+#pragma unroll
+    for (int i = 0; i < kCopiesX; i++) copy_1k<false>(at + (kCopiesW + i) * 1024, xsrc[i], st);
+#pragma unroll
+    for (int i = 0; i < kCopiesW; i++) copy_1k<true>(at + i * 1024, wsrc[i], st);
   };
-  auto load_x = [&](int chunk) {
-    const int64_t k = (int64_t)chunk * kLinChunkK;
-    XRows r;
+  f32x4_t acc[NT];
 #pragma unroll
-    for (int i = 0; i < kUnits; i++) r.u[i] = *reinterpret_cast<const uint4 *>(xsrc[i] + k);
-    return r;
-  };
-  auto store_x = [&](int chunk, const XRows &r) {
-    uint4 *st = xs + (chunk % kLinStages) * kLinStageUnits + wave * 64 + lane;
-#pragma unroll
-    for (int i = 0; i < kUnits; i++) st[WAVES * i * 64] = r.u[i];
-  };
+  for (int t = 0; t < NT; t++) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const bool meet = GATED || p.splits > 1;
+  f32x4_t *range_sums = sums + ((tile * kParts + part) * p.splits + first_range) * 64 + lane;
+  int left = p.stages_per_split, range = 0;  // of the range in hand
 
-  f32x4_t acc[NT][kLinMT];
 #pragma unroll
-  for (int t = 0; t < NT; t++)
+  for (int j = 0; j < S; j++)
+    if (j < nst) ask(j, j);
+  for (int base = 0; base < nst; base += S) {
 #pragma unroll
-    for (int mt = 0; mt < kLinMT; mt++) acc[t][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  // The main loop runs in groups of kLinDepth steps (four stages) with nothing conditional inside: the host
-  // hands every split a whole number of groups, loads past a split's end are clamped to its last step and
-  // stage (their data is never used), and a stage written past the end is one that nobody reads any more.
-  uint4 wq[kLinDepth][NT];
-  XRows xq[kLinXAhead];
-  const XRows x_first = load_x(0);
+    for (int j = 0; j < S; j++) {
+      const int st = base + j;
+      if (st < nst) {
+        // S stages are on their way, this one first; near the end fewer, and the wait is for all of them
+        if (st + S - 1 < nst)
+          wait_copies<(S - 1) * kCopies>();
+        else
+          wait_copies<0>();
+        const char *stage = mine + j * kStageBytes;
+        uint4 wf[2][NT], xf[2];
 #pragma unroll
-  for (int j = 0; j < kLinDepth; j++)
+        for (int s = 0; s < 2; s++) {
 #pragma unroll
-    for (int t = 0; t < NT; t++) wq[j][t] = load_w(wrow[t] + (int64_t)j * kLinStepK);
+          for (int t = 0; t < NT; t++) wf[s][t] = *staged_run(stage, t * 16 + col, 4 * s + kg);
+          xf[s] = *staged_run(stage + kCopiesW * 1024, col, 4 * s + kg);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage is in registers: its place can be filled again
+        if (st + S < nst) ask(j, st + S);
 #pragma unroll
-  for (int i = 1; i <= kLinXAhead; i++) xq[i % kLinXAhead] = load_x(min(i, nchunks - 1));
-  __builtin_amdgcn_sched_barrier(0);  // every load above is on its way before the first wait
-  store_x(0, x_first);
-  __syncthreads();
-
-  // The tiles of x for a step are read from LDS one step ahead, all eight before the MFMAs of the step in hand:
-  // with the reads next to their uses a wavefront spends most of a step waiting for LDS.
-  uint4 bq[2][kLinMT];
+        for (int s = 0; s < 2; s++)
 #pragma unroll
-  for (int mt = 0; mt < kLinMT; mt++) bq[0][mt] = xs[mt * 64 + lane];
-
-  for (int base = 0; base < nsteps; base += kLinDepth) {
-#pragma unroll
-    for (int j = 0; j < kLinDepth; j++) {
-      const int step = base + j;
-      const int c = step >> 1;
-      if ((j & 1) == 0) {
-        // Start of a stage: the next stage's rows go into LDS, the stage four further on is asked for, and one
-        // barrier both publishes the former and retires the reads of the stage that is written next time.
-        const int slot = (j / 2 + 1) % kLinXAhead;  // known at compile time once the loop is unrolled
-        store_x(c + 1, xq[slot]);
-        xq[slot] = load_x(min(c + 1 + kLinXAhead, nchunks - 1));
-        __syncthreads();
-      }
-      {
-        const int cn = (step + 1) >> 1;  // past the end: a stage whose contents no longer matter
-        const uint4 *st = xs + (cn % kLinStages) * kLinStageUnits + ((j + 1) & 1) * kLinMT * 64 + lane;
-#pragma unroll
-        for (int mt = 0; mt < kLinMT; mt++) bq[(j + 1) & 1][mt] = st[mt * 64];
-      }
-      __builtin_amdgcn_sched_barrier(0);  // the reads go out in front of the MFMAs, not behind them
-      vec8 a[NT];
-#pragma unroll
-      for (int t = 0; t < NT; t++) a[t] = lin_cast<vec8>(wq[j][t]);
-#pragma unroll
-      for (int mt = 0; mt < kLinMT; mt++) {
-        const vec8 b = lin_cast<vec8>(bq[j & 1][mt]);
-#pragma unroll
-        for (int t = 0; t < NT; t++) acc[t][mt] = LinMfma<T>::run(a[t], b, acc[t][mt]);
-      }
-      // The pieces of W are asked for in bunches of kLinBunch steps (consecutive 64-byte runs of every row go out
-      // together: DRAM pages are still open for the second run), each into the slots that have just been used.
-      if ((j % kLinBunch) == kLinBunch - 1) {
-#pragma unroll
-        for (int jj = j - (kLinBunch - 1); jj <= j; jj++) {
-          const int ahead = min(base + jj + kLinDepth, nsteps - 1);
-#pragma unroll
-          for (int t = 0; t < NT; t++) wq[jj][t] = load_w(wrow[t] + (int64_t)ahead * kLinStepK);
+          for (int t = 0; t < NT; t++)
+            acc[t] = LinMfma<T>::run(bit_cast<vec8>(wf[s][t]), bit_cast<vec8>(xf[s]), acc[t]);
+        if (NT == 1 && ranges > 1 && --left == 0) {
+          range_sums[range++ * 64] = acc[0];
+          acc[0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          left = p.stages_per_split;
         }
       }
-      // Steps stay apart: nothing of a later step is moved in front of this one's MFMAs.
-      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if (!meet) {
+#pragma unroll
+    for (int t = 0; t < NT; t++) linear_finish<T>(p, acc[t], col, n_tile + t * 16 + 4 * kg);
+    return;
+  }
+  if constexpr (NT == 1) {
+    for (; range < ranges; range++) {  // what is left of the last range; ranges past the end of k are zero
+      range_sums[range * 64] = acc[0];
+      acc[0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    __syncthreads();
+    if (wave < tiles) {
+      const int n = (blockIdx.x * tiles + wave) * 16 + 4 * kg;
+      f32x4_t total[kParts];
+#pragma unroll
+      for (int q = 0; q < kParts; q++) {
+        const f32x4_t *src = sums + (wave * kParts + q) * p.splits * 64 + lane;
+        total[q] = src[0];
+        for (int i = 1; i < p.splits; i++) {
+          const f32x4_t v = src[i * 64];
+#pragma unroll
+          for (int r = 0; r < 4; r++) total[q][r] += v[r];
+        }
+      }
+      if constexpr (GATED)
+        linear_finish_gated<T>(p, total[0], total[1], col, n);
+      else
+        linear_finish<T>(p, total[0], col, n);
+    }
+  }
+}
+
+// Up to 16 MT rows of x: a workgroup owns 16 WAVES rows of W over one range of k.  GATED: the second half of the
+// wavefronts takes the up rows that belong to the gate rows of the first.
+template <typename T, int MT, int S, int WAVES, bool GATED>
+__global__ __launch_bounds__(WAVES * 64) void linear_tile_kernel(const LinearParams p) {
+  using vec8 = typename Vec8<T>::type;
+  // The read-once hint on W (stream kernel: always) measured 3 to 8 % faster here as well, except on the short ranges that the
+  // 64-row workgroups serve with many rows of x (4096 x 4096, 128 rows: 15.6 us without, 17.0 with).
+  constexpr bool kOnce = MT == 2 || WAVES == 8;
+  constexpr int kCopiesW = 2;                           // of 1 KB per stage: this wavefront's rows of W
+  constexpr int kAllX = 2 * MT, kCopiesX = (kAllX + WAVES - 1) / WAVES;  // all copies of x, this wavefront's share
+  constexpr int kCopies = kCopiesW + kCopiesX;
+  constexpr int kStageBytes = (kCopiesW * WAVES + kAllX) * 1024;
+  constexpr int kCols = WAVES * 16;
+  constexpr int kPitch = kCols + 4;  // floats per row of finished sums in LDS
+  static_assert(S * kStageBytes >= MT * 16 * kPitch * 4, "the sums reuse the ring");
+  __shared__ __align__(1024) char ring[S * kStageBytes];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, kg = lane >> 4;
+  const int part = GATED ? wave / (WAVES / 2) : 0;
+  const int n_end = GATED ? p.half : p.N;
+  const int n_group = blockIdx.x * (GATED ? kCols / 2 : kCols);
+  const int n_tile = n_group + (GATED ? wave % (WAVES / 2) : wave) * 16;  // within the part
+  const int split = blockIdx.y;
+  const int stage0 = split * p.stages_per_split;
+  const int nst = max(0, min(p.stages_per_split, p.total_stages - stage0));
+
+  CopySource wsrc[kCopiesW], xsrc[kCopiesX];
+#pragma unroll
+  for (int i = 0; i < kCopiesW; i++)
+    wsrc[i] = copy_source<T>(p.w, p.ldw, part * p.half + n_tile + i * 8, part * p.half + n_end - 1, stage0);
+  // Where the copies of x do not divide evenly some are made twice (the same bytes to the same place): every wavefront
+  // counts the same number of copies per stage.
+#pragma unroll
+  for (int i = 0; i < kCopiesX; i++) xsrc[i] = copy_source<T>(p.x, p.ldx, ((wave + i * WAVES) % kAllX) * 8, p.M - 1, stage0);
+  const uint32_t ring_lds = lds_address(ring);
+  auto ask = [&](int slot, int st) {
+    const uint32_t at = ring_lds + slot * kStageBytes;
+#pragma unroll
+    for (int i = 0; i < kCopiesX; i++)
+      copy_1k<false>(at + (kCopiesW * WAVES + (wave + i * WAVES) % kAllX) * 1024, xsrc[i], st);
+#pragma unroll
+    for (int i = 0; i < kCopiesW; i++) copy_1k<kOnce>(at + (wave * kCopiesW + i) * 1024, wsrc[i], st);
+  };
+  f32x4_t acc[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++) acc[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < S - 1; j++)
+    if (j < nst) ask(j, j);
+  for (int base = 0; base < nst; base += S) {
+#pragma unroll
+    for (int j = 0; j < S; j++) {
+      const int st = base + j;
+      if (st < nst) {
+        // This wavefront's copies of the stage have landed, and behind the barrier everybody's; the barrier also says
+        // that the stage before has been read, so its place takes the copies of the stage S - 1 further on.
+        if (st + S - 2 < nst)
+          wait_copies<(S - 2) * kCopies>();
+        else
+          wait_copies<0>();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (st + S - 1 < nst) ask((j + S - 1) % S, st + S - 1);
+        const char *stage = ring + j * kStageBytes;
+        const char *wrows = stage + wave * kCopiesW * 1024, *xrows = stage + kCopiesW * WAVES * 1024;
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          const uint4 wf = *staged_run(wrows, col, 4 * s + kg);
+          uint4 xf[MT];
+#pragma unroll
+          for (int mt = 0; mt < MT; mt++) xf[mt] = *staged_run(xrows, mt * 16 + col, 4 * s + kg);
+#pragma unroll
+          for (int mt = 0; mt < MT; mt++) acc[mt] = LinMfma<T>::run(bit_cast<vec8>(wf), bit_cast<vec8>(xf[mt]), acc[mt]);
+        }
+      }
     }
   }
 
   if (p.row_sums) {
     // rows of fp32 sums, one 16-byte piece per lane and tile (four lanes make 64 contiguous bytes of a row)
+    const int n = n_tile + 4 * kg;
+    if (n < p.N) {
 #pragma unroll
-    for (int t = 0; t < NT; t++) {
-      const int n = n_wave + t * 16 + 4 * kg;
-      if (n < p.N) {
-#pragma unroll
-        for (int mt = 0; mt < kLinMT; mt++)
-          if (mt < p.mtiles)
-            *reinterpret_cast<f32x4_t *>(p.partial + ((int64_t)split * kLinMaxRows + mt * 16 + col) * p.N + n) = acc[t][mt];
-      }
+      for (int mt = 0; mt < MT; mt++)
+        if (mt < p.mtiles)
+          *reinterpret_cast<f32x4_t *>(p.partial + ((int64_t)split * kLinMaxRows + mt * 16 + col) * p.N + n) = acc[mt];
     }
-  } else if (p.splits == 1) {
+  } else if (p.splits > 1) {
+    if (n_tile < n_end) {
+      const int nt = (part * p.half + n_tile) / 16;
+      f32x4_t *dst = reinterpret_cast<f32x4_t *>(p.partial) + ((int64_t)(split * (p.N / 16) + nt) * kLinMT) * 64 + lane;
 #pragma unroll
-    for (int t = 0; t < NT; t++)
-#pragma unroll
-      for (int mt = 0; mt < kLinMT; mt++)
-        if (mt < p.mtiles) linear_finish<T>(p, acc[t][mt], mt * 16 + col, n_wave + t * 16 + 4 * kg);
+      for (int mt = 0; mt < MT; mt++)
+        if (mt < p.mtiles) dst[mt * 64] = acc[mt];
+    }
   } else {
-    const int ntiles = (p.N + 15) / 16;
+    // Turned through LDS so that the stores are whole stretches of a row (kCols outputs): straight from the accumulators
+    // they are 32 bytes per row and instruction, which cost 25 of 240 us on a 128256 x 4096 weight with 128 rows.
+    float *tile = reinterpret_cast<float *>(ring);
+    __syncthreads();
 #pragma unroll
-    for (int t = 0; t < NT; t++) {
-      const int nt = n_wave / 16 + t;
-      if (nt < ntiles) {
-        f32x4_t *dst = reinterpret_cast<f32x4_t *>(p.partial) + ((int64_t)(split * ntiles + nt) * kLinMT) * 64 + lane;
-#pragma unroll
-        for (int mt = 0; mt < kLinMT; mt++)
-          if (mt < p.mtiles) dst[mt * 64] = acc[t][mt];
-      }
+    for (int mt = 0; mt < MT; mt++)
+      *reinterpret_cast<f32x4_t *>(tile + (mt * 16 + col) * kPitch + wave * 16 + 4 * kg) = acc[mt];
+    __syncthreads();
+    constexpr int kQuads = (GATED ? kCols / 2 : kCols) / 4;
+    for (int i = tid; i < p.M * kQuads; i += WAVES * 64) {
+      const int m = i / kQuads, c = (i % kQuads) * 4;
+      const f32x4_t v = *reinterpret_cast<const f32x4_t *>(tile + m * kPitch + c);
+      if constexpr (GATED)
+        linear_finish_gated<T>(p, v, *reinterpret_cast<const f32x4_t *>(tile + m * kPitch + kCols / 2 + c), m, n_group + c);
+      else
+        linear_finish<T>(p, v, m, n_group + c);
     }
   }
 }
 
-// Adds up the splits' sums, split 0 first, and finishes the tile: one thread per (16 rows of W, row tile, lane).
-template <typename T>
-__global__ __launch_bounds__(256) void skinny_linear_reduce_kernel(const LinearParams p) {
-  const int ntiles = (p.N + 15) / 16;
+// Adds up the ranges' sums, the first range first, and finishes the tile: one thread per (16 rows of W, row tile, lane).
+template <typename T, bool GATED>
+__global__ __launch_bounds__(256) void linear_reduce_kernel(const LinearParams p) {
+  const int ntiles = p.N / 16;
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int lane = (int)(idx & 63);
   const int mt = (int)((idx >> 6) % p.mtiles);
   const int64_t nt = (idx >> 6) / p.mtiles;
-  if (nt >= ntiles) return;
-  const f32x4_t *src = reinterpret_cast<const f32x4_t *>(p.partial) + (nt * kLinMT + mt) * 64 + lane;
+  if (nt >= (GATED ? p.half / 16 : ntiles)) return;
   const int64_t stride = (int64_t)ntiles * kLinMT * 64;
-  f32x4_t s = src[0];
-  for (int i = 1; i < p.splits; i++) {
-    const f32x4_t v = src[i * stride];
+  auto add_up = [&](int64_t tile) {
+    const f32x4_t *src = reinterpret_cast<const f32x4_t *>(p.partial) + (tile * kLinMT + mt) * 64 + lane;
+    f32x4_t s = src[0];
+    for (int i = 1; i < p.splits; i++) {
+      const f32x4_t v = src[i * stride];
 #pragma unroll
-    for (int r = 0; r < 4; r++) s[r] += v[r];
-  }
-  linear_finish<T>(p, s, mt * 16 + (lane & 15), (int)nt * 16 + 4 * (lane >> 4));
+      for (int r = 0; r < 4; r++) s[r] += v[r];
+    }
+    return s;
+  };
+  const int m = mt * 16 + (lane & 15), n = (int)nt * 16 + 4 * (lane >> 4);
+  if constexpr (GATED)
+    linear_finish_gated<T>(p, add_up(nt), add_up(nt + p.half / 16), m, n);
+  else
+    linear_finish<T>(p, add_up(nt), m, n);
 }
 
 // Adds up the ranges' sums of one row of y, finishes the row (bias, rounding, residual: as linear_finish) and
@@ -289,7 +428,7 @@ __global__ __launch_bounds__(256) void skinny_linear_reduce_kernel(const LinearP
 // order of its additions are those of the stand-alone kernel (rms_norm_vec8_kernel: the same thread owns the same
 // eight columns, the same block_sum), so the two routes give the same bits.
 template <typename T>
-__global__ __launch_bounds__(1024) void skinny_linear_reduce_norm_kernel(const LinearParams p) {
+__global__ __launch_bounds__(1024) void linear_reduce_norm_kernel(const LinearParams p) {
   __shared__ float smem[17];
   const int row = blockIdx.x;
   const int i = threadIdx.x * 8;
@@ -347,58 +486,92 @@ __global__ __launch_bounds__(1024) void skinny_linear_reduce_norm_kernel(const L
 }
 
 struct LinearPlan {
-  int waves;   // wavefronts per workgroup
-  int nt;      // 16-row tiles of W per wavefront
-  int splits;  // ranges of k
-  int steps_per_split;
+  bool stream;  // the few-rows kernel
+  int waves;    // tile kernel: wavefronts per workgroup
+  int splits;   // ranges of k
+  int stages_per_split;
   size_t partial_bytes;
 };
 
+// The ranges of k depend on the weight alone (see above).  At least 1024 wavefronts' worth of (16 rows, range) pairs, four per
+// compute unit, and no range longer than 2048 once k is cut at all: 4096 x 4096 and 6144 x 4096 four, 4096 x 14336
+// eight, weights of 16384 rows and more none.
 LinearPlan plan_linear(int M, int N, int K) {
-  (void)M;
   const Tuning &tn = tuning();
   LinearPlan pl;
-  pl.nt = tn.linear_tiles > 0 ? tn.linear_tiles : 2;
-  pl.waves = tn.linear_waves > 0 ? tn.linear_waves : 4;
-  const int rows_per_wg = pl.waves * 16 * pl.nt;
-  const int n_wgs = (N + rows_per_wg - 1) / rows_per_wg;
-  const int groups = K / kLinGroupK;
-  // One workgroup per compute unit is what measured best on the shapes of a decode step (4096 x 4096 and
-  // 4096 x 14336: eight ranges of k; 6144 x 4096: four).
-  int splits = tn.linear_splits > 0 ? tn.linear_splits : (256 + n_wgs / 2) / n_wgs;
-  if (splits < 1) splits = 1;
-  if (splits > groups) splits = groups;
-  if (splits > 32) splits = 32;
-  const int per = (groups + splits - 1) / splits;
-  pl.splits = (groups + per - 1) / per;
-  pl.steps_per_split = per * (kLinGroupK / kLinStepK);
-  pl.partial_bytes = pl.splits > 1 ? (size_t)pl.splits * ((N + 15) / 16) * kLinMT * 64 * sizeof(f32x4_t) : 0;
+  const int stages = K / kLinStageK;
+  int splits = 1;
+  while (splits < kLinMaxRanges && (int64_t)N * splits < 16384) splits *= 2;
+  while (splits > 1 && splits < kLinMaxRanges && K / splits > 2048) splits *= 2;
+  while (splits > stages) splits /= 2;
+  pl.stream = M <= kLinStreamRows;
+  if (tn.linear_splits > 0) splits = tn.linear_splits < stages ? tn.linear_splits : stages;
+  if (tn.linear_splits > 0 || tn.linear_waves > 0 || tn.linear_tiles > 0) pl.stream = false;
+  pl.splits = splits;
+  pl.stages_per_split = (stages + splits - 1) / splits;
+  // Workgroups of 64 rows while the device holds all of them at once, one per compute unit, or where 32 rows of x leave the copies of x
+  // cheap (28672 x 4096, 32 rows: 43.5 us against 46.3; 64 rows: 49.5 against 47.3); else of 128 rows.
+  pl.waves = ((int64_t)((N + 63) / 64) * splits <= 256 || (splits == 1 && M <= 32)) ? 4 : 8;
+  if (tn.linear_tiles > 0) pl.waves = 4 * tn.linear_tiles;
+  if (tn.linear_waves > 0) pl.waves = tn.linear_waves;
+  pl.partial_bytes = pl.splits > 1 && !pl.stream ? (size_t)pl.splits * (N / 16) * kLinMT * 64 * sizeof(f32x4_t) : 0;
   return pl;
 }
 
-template <typename T>
-void launch_linear(const LinearParams &p, const LinearPlan &pl, hipStream_t stream) {
-  const int rows_per_wg = pl.waves * 16 * pl.nt;
-  const dim3 grid((p.N + rows_per_wg - 1) / rows_per_wg, pl.splits);
-  const dim3 block(pl.waves * 64);
-  if (pl.nt == 2 && pl.waves == 8)
-    hipLaunchKernelGGL((skinny_linear_kernel<T, 2, 4, 8>), grid, block, 0, stream, p);
-  else if (pl.nt == 2)
-    hipLaunchKernelGGL((skinny_linear_kernel<T, 2, 4, 4>), grid, block, 0, stream, p);
-  else if (pl.waves == 8)
-    hipLaunchKernelGGL((skinny_linear_kernel<T, 1, 8, 8>), grid, block, 0, stream, p);
+// Stages of the ring: what fits half of the 160 KB of LDS (two workgroups per compute unit), or all of it where a stage takes more
+// than 24 KB.
+template <int MT, int WAVES>
+constexpr int ring_stages() {
+  constexpr int kb = 2 * WAVES + 2 * MT;
+  constexpr int s = (kb <= 24 ? 80 : 160) / kb;
+  return s > 6 ? 6 : s;
+}
+
+template <typename T, int MT, bool GATED>
+void launch_tile(const LinearParams &p, const LinearPlan &pl, hipStream_t stream) {
+  const int n = GATED ? p.half : p.N, per_wg = pl.waves * 16 / (GATED ? 2 : 1);
+  const dim3 grid((n + per_wg - 1) / per_wg, pl.splits), block(pl.waves * 64);
+  if (pl.waves == 8)
+    hipLaunchKernelGGL((linear_tile_kernel<T, MT, ring_stages<MT, 8>(), 8, GATED>), grid, block, 0, stream, p);
   else
-    hipLaunchKernelGGL((skinny_linear_kernel<T, 1, 8, 4>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((linear_tile_kernel<T, MT, ring_stages<MT, 4>(), 4, GATED>), grid, block, 0, stream, p);
+}
+
+template <typename T, bool GATED>
+void launch_linear(const LinearParams &p, const LinearPlan &pl, hipStream_t stream) {
+  if (pl.stream) {
+    if (!GATED && p.splits == 1 && p.N >= 65536) {
+      // A vocabulary's rows: 512 per workgroup, so that one round of workgroups covers the device (128256 x 4096, 16 rows: 161
+      // us against 182 with 64 rows per workgroup).
+      if constexpr (!GATED)
+        hipLaunchKernelGGL((linear_stream_kernel<T, 4, 2, 8, false>), dim3((p.N + 511) / 512), dim3(512), 0, stream, p);
+    } else {
+      const int parts = GATED ? 2 : 1, n = GATED ? p.half : p.N;
+      const int per_tile = p.splits < 4 / parts ? p.splits : 4 / parts;
+      const int rows = 16 * (4 / parts / per_tile);
+      hipLaunchKernelGGL((linear_stream_kernel<T, 1, 3, 4, GATED>), dim3((n + rows - 1) / rows), dim3(256), 0, stream, p);
+    }
+    check_launch("linear (few rows)");
+    return;
+  }
+  if (p.M <= 32)
+    launch_tile<T, 2, GATED>(p, pl, stream);
+  else if (p.M <= 64)
+    launch_tile<T, 4, GATED>(p, pl, stream);
+  else if (p.M <= 96)
+    launch_tile<T, 6, GATED>(p, pl, stream);
+  else
+    launch_tile<T, 8, GATED>(p, pl, stream);
   check_launch("linear");
   if (p.row_sums) {
     int threads = (int)(((p.N / 8 + 63) / 64) * 64);
     if (threads > 1024) threads = 1024;  // (the entry point bounds N)
-    hipLaunchKernelGGL((skinny_linear_reduce_norm_kernel<T>), dim3((unsigned)p.M), dim3((unsigned)threads), 0, stream, p);
+    hipLaunchKernelGGL((linear_reduce_norm_kernel<T>), dim3((unsigned)p.M), dim3((unsigned)threads), 0, stream, p);
     check_launch("linear (sum of the ranges + rms_norm)");
   } else if (pl.splits > 1) {
-    const int64_t threads = (int64_t)((p.N + 15) / 16) * p.mtiles * 64;
-    hipLaunchKernelGGL((skinny_linear_reduce_kernel<T>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, p);
-    check_launch("linear (sum of the splits)");
+    const int64_t threads = (int64_t)((GATED ? p.half : p.N) / 16) * p.mtiles * 64;
+    hipLaunchKernelGGL((linear_reduce_kernel<T, GATED>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, p);
+    check_launch("linear (sum of the ranges)");
   }
 }
 
@@ -409,7 +582,7 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_tensor *weight, const hipattn_tensor *bias,
                  const hipattn_tensor *residual, const hipattn_tensor *workspace, void *stream_arg, int64_t *ws_query,
                  hipattn_tensor *norm_out = nullptr, const hipattn_tensor *norm_weight = nullptr, float eps = 0.f,
-                 bool ws_query_with_norm = false) {
+                 bool ws_query_with_norm = false, bool gated = false) {
   check_tensor(x, "x", 2);
   check_tensor(weight, "weight", 2);
   const int dt = x->dtype;
@@ -419,22 +592,24 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
   HA_CHECK(weight->sizes[1] == K, "linear: weight has %lld columns, x has %lld", (long long)weight->sizes[1], (long long)K);
   HA_CHECK(M <= kLinMaxRows, "linear: %lld rows of x; this kernel takes at most %d (use a library GEMM beyond that)",
            (long long)M, kLinMaxRows);
-  HA_CHECK(K > 0 && K % kLinGroupK == 0, "linear: the inner size %lld must be a positive multiple of %d", (long long)K,
-           kLinGroupK);
+  HA_CHECK(K > 0 && K % 256 == 0, "linear: the inner size %lld must be a positive multiple of %d", (long long)K, 256);
   HA_CHECK(N % 16 == 0, "linear: the number of rows of weight (%lld) must be a multiple of 16", (long long)N);
   HA_CHECK(N < (1 << 24) && K < (1 << 24), "linear: sizes out of range");
+  HA_CHECK(!gated || N % 32 == 0, "linear_silu_and_mul: gate and up rows (%lld together) must be multiples of 16 each", (long long)N);
   LinearPlan pl = plan_linear((int)M, (int)N, (int)K);
+  const int64_t outputs = gated ? N / 2 : N;
   const bool with_norm = norm_out != nullptr || ws_query_with_norm;
-  // rows of sums for the norm: [range][128 rows][N] fp32 -- the size the tiles of sums take as well
-  if (with_norm) pl.partial_bytes = (size_t)pl.splits * kLinMaxRows * (size_t)N * sizeof(float);
+  // rows of sums for the norm: [range][128 rows][N] fp32 -- the size the tiles of sums take as well.  (The few-rows kernel leaves
+  // finished rows: a launch of rms_norm normalises them.)
+  if (with_norm && !pl.stream) pl.partial_bytes = (size_t)pl.splits * kLinMaxRows * (size_t)N * sizeof(float);
   if (ws_query != nullptr) {
     *ws_query = (int64_t)pl.partial_bytes;
     return;
   }
   check_tensor(out, "out", 2);
   HA_CHECK(out->dtype == dt, "linear: out is %s, x is %s", dtype_name(out->dtype), dtype_name(dt));
-  HA_CHECK(out->sizes[0] == M && out->sizes[1] == N, "linear: out is [%lld, %lld], expected [%lld, %lld]",
-           (long long)out->sizes[0], (long long)out->sizes[1], (long long)M, (long long)N);
+  HA_CHECK(out->sizes[0] == M && out->sizes[1] == outputs, "linear: out is [%lld, %lld], expected [%lld, %lld]",
+           (long long)out->sizes[0], (long long)out->sizes[1], (long long)M, (long long)outputs);
   if (M == 0 || N == 0) return;
   check_data(x, "x");
   check_data(weight, "weight");
@@ -445,6 +620,10 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
            "linear: rows of x and weight must start on 16-byte boundaries");
   HA_CHECK(out->strides[0] % 4 == 0 && (reinterpret_cast<uintptr_t>(out->data) & 7) == 0,
            "linear: rows of out must start on 8-byte boundaries");
+
+  // offsets between eight rows are 32 bits
+  HA_CHECK(weight->strides[0] >= 0 && weight->strides[0] < (1 << 28) && x->strides[0] >= 0 && x->strides[0] < (1 << 28),
+           "linear: row strides %lld / %lld of x / weight out of range", (long long)x->strides[0], (long long)weight->strides[0]);
 
   LinearParams p{};
   p.x = x->data;
@@ -492,17 +671,18 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
                  aligned16(norm_weight->data) && (bias == nullptr || aligned16(bias->data)) &&
                  (residual == nullptr || (residual->strides[0] % 8 == 0 && aligned16(residual->data))),
              "linear_rms_norm: rows of out, norm_out and residual, and bias and norm_weight, must start on 16-byte boundaries");
-    p.row_sums = 1;
+    p.row_sums = pl.stream ? 0 : 1;
     p.norm_w = norm_weight->data;
     p.norm_out = norm_out->data;
     p.ldn = norm_out->strides[0];
     p.eps = eps;
   }
   p.splits = pl.splits;
-  p.steps_per_split = pl.steps_per_split;
-  p.total_steps = (int)(K / kLinStepK);
+  p.stages_per_split = pl.stages_per_split;
+  p.total_stages = (int)(K / kLinStageK);
+  p.half = gated ? (int)(N / 2) : 0;
   hipStream_t stream = resolve_stream(stream_arg);
-  if (pl.splits > 1 || with_norm) {
+  if (pl.partial_bytes > 0) {
     if (workspace != nullptr) {
       check_tensor(workspace, "workspace", 1);
       HA_CHECK(workspace->dtype == HIPATTN_U8 && workspace->strides[0] == 1, "linear: workspace must be contiguous u8");
@@ -516,9 +696,17 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
     }
   }
   if (dt == HIPATTN_BF16)
-    launch_linear<bf16_t>(p, pl, stream);
+    gated ? launch_linear<bf16_t, true>(p, pl, stream) : launch_linear<bf16_t, false>(p, pl, stream);
   else
-    launch_linear<half_t>(p, pl, stream);
+    gated ? launch_linear<half_t, true>(p, pl, stream) : launch_linear<half_t, false>(p, pl, stream);
+  if (norm_out != nullptr && pl.stream) {
+    char *err = hipattn_rms_norm(norm_out, out, norm_weight, eps, stream_arg);
+    if (err != nullptr) {
+      const std::string msg(err);
+      free(err);
+      fail("%s", msg.c_str());
+    }
+  }
 }
 
 }  // namespace
@@ -530,6 +718,11 @@ extern "C" char *hipattn_linear(hipattn_tensor *out, const hipattn_tensor *x, co
                                 const hipattn_tensor *bias, const hipattn_tensor *residual,
                                 const hipattn_tensor *workspace, void *stream) {
   HA_PROTECT(linear_impl(out, x, weight, bias, residual, workspace, stream, nullptr));
+}
+
+extern "C" char *hipattn_linear_silu_and_mul(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_tensor *weight,
+                                             const hipattn_tensor *workspace, void *stream) {
+  HA_PROTECT(linear_impl(out, x, weight, nullptr, nullptr, workspace, stream, nullptr, nullptr, nullptr, 0.f, false, true));
 }
 
 extern "C" char *hipattn_linear_workspace_size(const hipattn_tensor *x, const hipattn_tensor *weight, int64_t *bytes) {

@@ -32,8 +32,8 @@ struct Tuning {
   int cache_move_lds;      // -1: the library chooses; 0: never the LDS-transposing kernels
   int prefill_wg_heads;      // eight-wavefront prefill: query heads of one kv group per workgroup, at most (0: the library chooses -- up to four; 1: one)
   int prefill_rescale_log2;  // prefill: a row's reference maximum moves when outgrown by more than 2^this (0..16, default 8)
-  int linear_tiles;          // linear: 16-row tiles of the weight per wavefront (0: the library chooses; 1 or 2)
-  int linear_waves;          // linear: wavefronts per workgroup (0: the library chooses; 4 or 8)
+  int linear_tiles;          // linear: 64-row tiles of the weight per workgroup (0: the library chooses; 1 or 2)
+  int linear_waves;          // linear: wavefronts per workgroup, 16 rows of the weight each (0: the library chooses; 4 or 8)
   int linear_splits;         // linear: ranges of the inner dimension (0: the library chooses; else 1..32)
 };
 const Tuning &tuning();

@@ -253,6 +253,14 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     return out
 
 
+def linear_silu_and_mul(x: torch.Tensor, weight: torch.Tensor, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """silu_and_mul(x @ weight.T) for at most 128 rows of x, weight [2 n, K] with the gate rows first (llama.rs:135-142):
+    the bits of `linear` followed by `silu_and_mul`, without the [M, 2 n] product in memory."""
+    out = torch.empty((x.size(0), weight.size(0) // 2), dtype=x.dtype, device=x.device)
+    _native.linear_silu_and_mul(out, x, weight, workspace)
+    return out
+
+
 def linear_rms_norm(x: torch.Tensor, weight: torch.Tensor, norm_weight: torch.Tensor, epsilon: float,
                     bias: Optional[torch.Tensor] = None, residual: Optional[torch.Tensor] = None,
                     workspace: Optional[torch.Tensor] = None):

@@ -319,6 +319,13 @@ char *hipattn_linear_workspace_size(const hipattn_tensor *x,
                                     const hipattn_tensor *weight,
                                     int64_t *bytes);
 
+/* hipattn_linear with silu_and_mul behind it (llama.rs:135-142): weight [2 n, K] holds the gate rows and then
+ * the up rows, out [M, n] = silu_and_mul(x . weight^T), the bits of the two calls; the [M, 2 n] product is not
+ * written to memory.  Workspace: hipattn_linear_workspace_size of the same x and weight. */
+char *hipattn_linear_silu_and_mul(hipattn_tensor *out, const hipattn_tensor *x,
+                                  const hipattn_tensor *weight,
+                                  const hipattn_tensor *workspace, void *stream);
+
 /* hipattn_linear followed by the RMS norm of the finished rows, in the launch
  * that adds up the ranges of the inner dimension: out = x . weight^T (+ bias)
  * (+ residual) as above, norm_out = rms_norm(out, norm_weight, epsilon) with the
@@ -489,8 +496,8 @@ char *hipattn_shutdown(void);
  * prefill_rescale_log2 (0..16, default 8: the prefill
  * kernels move a row's reference maximum only when the row outgrows it by
  * more than 2^value; 0 follows the row maximum exactly, as the reference
- * does), linear_tiles (0 library's choice, 1 / 2: 16 / 32 rows of the weight
- * per wavefront of hipattn_linear), linear_splits (0 library's choice, else
+ * does), linear_tiles (0 library's choice, 1 / 2: workgroups of 64 /
+ * 128 rows of the weight in hipattn_linear), linear_splits (0 library's choice, else
  * the number of ranges the inner dimension is cut into, at most 32).  Every
  * setting computes the same results -- prefill_rescale_log2 and linear_splits
  * up to rounding.  Not

@@ -205,3 +205,37 @@ def test_refusals(device):
     assert not K.linear_takes(t(129, 256), t(64, 256)) and not K.linear_takes(t(8, 320), t(64, 320))
     assert K.linear_takes(t(8, 256), t(64, 256))
     assert K.linear(t(0, 256), t(64, 256)).shape == (0, 64)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,kd", [(16, 256), (2560, 2560), (4096, 1024), (1376, 4352), (14336, 512), (8208, 256)])
+def test_linear_silu_and_mul_gives_the_bits_of_the_two_calls(device, n, kd, dtype):
+    """Every kernel of the layer (16 rows of x and fewer; up to 32, 64, 96, 128) at its edges, weights whose inner size is
+    cut into one to eight ranges, one with a last range that is shorter, and rows that do not fill a workgroup."""
+    x, w, _ = operands(128, 2 * n, kd, dtype, seed=n + kd)
+    xd, wd = x.to(device), w.to(device)
+    for m in (1, 15, 16, 17, 32, 33, 64, 65, 96, 97, 128):
+        both = K.linear(xd[:m], wd)
+        want = torch.empty((m, n), dtype=dtype, device=device)
+        K.silu_and_mul(want, both)
+        assert torch.equal(K.linear_silu_and_mul(xd[:m], wd), want), m
+        if m == 17:
+            check(both, x[:m], w)
+        # a row's bits do not depend on the kernel its company selects
+        assert torch.equal(both[:1], K.linear(xd[:1], wd)), m
+    for waves in (4, 8):
+        K.tuning_set("linear_waves", waves)
+        for splits in (1, 3):
+            K.tuning_set("linear_splits", splits)
+            both = K.linear(xd[:50], wd)
+            want = torch.empty((50, n), dtype=dtype, device=device)
+            K.silu_and_mul(want, both)
+            assert torch.equal(K.linear_silu_and_mul(xd[:50], wd), want)
+
+
+@pytest.mark.parametrize("m", [1, 16, 33, 128])
+def test_vocabulary_rows(device, m):
+    """Weights of 65536 rows and more: a workgroup of 512 rows, the last one partly empty."""
+    x, w, _ = operands(m, 65536 + 80, 256, torch.bfloat16, seed=m)
+    y = K.linear(x.to(device), w.to(device))
+    check(y, x, w)
