@@ -287,6 +287,33 @@ def test_bias_sample_equal_values_and_distribution(device):
             assert (cum[t - 1] if t else 0.0) - 1e-4 <= float(u[i]) <= cum[t] + 1e-4, (top_p, i, t, int(want[i]))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V,share", [(128256, 0.05), (128256, 1.0), (50003, 0.0005), (1001, 0.5), (7, 1.0)])
+def test_bias_sample_counts_equal_logits_to_the_same_tokens(device, dtype, V, share):
+    """16-bit logits under allow-bits are sampled by counting equal values, float32 ones are not: the same values give
+    the same token either way, whatever their range -- ordinary logits, all below zero, equal ones, ones too small or too
+    far below the largest to be counted, NaN and infinities among them -- at every nucleus and uniform number."""
+    g = torch.Generator().manual_seed(V)
+    n = torch.randn((10, V), generator=g)
+    kinds = torch.stack([n[0] * 2.5, n[1] * 0.5 - 30, n[2] * 0, n[3].round(), n[4] * 1e-3, n[5] * 40, n[6] * 1e-6,
+                         n[7] * 3, n[8] * 3, torch.where(n[9] > 1.5, n[9], n[9] * 1e-4)])
+    if V > 100:
+        kinds[7, 33:] = torch.where(n[7, 33:].abs() < 0.05, torch.tensor(float("nan")), kinds[7, 33:])
+        kinds[8, 20:] = torch.where(n[8, 20:] < -1, torch.tensor(float("-inf")), kinds[8, 20:])
+    rows = kinds.repeat_interleave(12, 0).to(dtype)
+    S = rows.size(0)
+    allowed = torch.rand((S, V), generator=g) < share
+    allowed[:, V // 2] = True
+    packed = torch.from_numpy(np.stack([aici.pack_allowed(a) for a in allowed.numpy()])).to(device)
+    temperature = torch.tensor([0.8, 0.3, 1.5, 20.0]).repeat(S // 4).to(device)
+    top_p = torch.tensor([0.9, 0.5, 1.0, 0.95, 1e-4, 0.9999]).repeat_interleave(2).repeat(S // 12).to(device)
+    u = torch.rand((S,), generator=g)
+    u[::7], u[3::11] = 0.0, 0.99999994
+    got = K.bias_sample(rows.to(device), temperature, top_p, u.to(device), mask=packed)
+    want = K.bias_sample(rows.float().to(device), temperature, top_p, u.to(device), mask=packed)
+    assert torch.equal(got, want), torch.nonzero(got != want).flatten().tolist()
+
+
 def test_bias_sample_corner_rows(device):
     """Rows outside what the reference defines still give a defined, allowed token: an infinite logit (its first
     holder), uniform numbers outside [0, 1) (the first / the last token with weight), an infinite temperature
