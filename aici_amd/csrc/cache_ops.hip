@@ -215,71 +215,88 @@ __global__ __launch_bounds__(256) void cache_move_run8_kernel(
   }
 }
 
-// Coalesced on both sides (2-byte elements, head size a multiple of 8; the last group of a head has fewer
-// than 8 chunks when it is not a multiple of 64, and the lanes beyond them sit out).  The input is token-major,
-// the cache chunk-major, so some side of a direct copy always touches 16-byte pieces 256 bytes apart.
-// Here a wavefront moves one (8 tokens) x (8 chunks = 64 head elements) tile of one head through a
-// private LDS slab: it reads the source in the source's order (128-byte runs), transposes in LDS, and
-// writes the destination in the destination's order -- K as 128-byte runs [chunk][8 tokens], V as the 8
-// tokens (16 bytes) of each of the tile's 64 head elements.  16 tokens per workgroup as in the kernel
-// above; groups that are not a run of 8 slots take its per-token path, and a workgroup whose 16 tokens
-// fill one whole block moves 16-token tiles, whose cache side is whole rows ([chunk][16 tokens] = 256
-// bytes of K, [16 tokens] = 32 bytes of each V element, 1 KiB contiguous per instruction).
+// Coalesced on both sides (2-byte elements, head size a multiple of 8, blocks of a multiple of 16 tokens; the last group of a head
+// has fewer than 8 chunks when it is not a multiple of 64, and the lanes beyond them sit out).  The input is
+// token-major, the cache chunk-major, so some side of a direct copy always touches 16-byte pieces 256 bytes apart.
+// Here a wavefront moves a tile of 16 tokens x 8 chunks (64 head elements) of one head through a private LDS
+// slab: it reads the source in the source's order, transposes in LDS, and writes the destination in the
+// destination's order -- whole rows of the cache ([chunk][16 tokens] = 256 bytes of K, [16 tokens] = 32 bytes of
+// each V element, 1 KiB contiguous per instruction), whole 128-byte runs of a token.
+//
+// A tile is 16 consecutive tokens that fill 16 consecutive slots from a multiple of 16 on.  The sequences of a batch lie
+// end to end, so tiles start at any token: a wavefront takes the tile that starts among its 16 tokens, wherever it ends, and the
+// tokens of its own that belong to no tile (ends of sequences, decode rows) one by one, eight at a time.  Tiles cut at
+// multiples of 16 of the token index (as before) fit the first sequence of a ragged batch only.
+//
+// us, before -> now (fp16): 1375 tokens of 4 sequences x 32 heads x 128 27 -> 9.3, 40012 tokens of 32 sequences x 2 heads x 64 34.7 -> 11.0,
+// 32768 tokens of 8 sequences x 8 heads x 128 44 -> 43.5.
 template <typename Slot, bool SCATTER, bool FULL_GROUPS>
 __global__ __launch_bounds__(256) void cache_move_tile_kernel(
     uint16_t *__restrict__ key, uint16_t *__restrict__ value, uint16_t *__restrict__ key_cache,
     uint16_t *__restrict__ value_cache, const Slot *__restrict__ slot_mapping, int64_t num_tokens,
     int64_t key_tok_stride, int64_t key_head_stride, int64_t val_tok_stride,
-    int64_t val_head_stride, CacheGeom g) {
+    int64_t val_head_stride, CacheGeom g, int items_per_wave, int waves_per_group) {
   typedef uint16_t E;
   constexpr int X = 8;
   constexpr int KP = 72;  // K slab row pitch in elements: 8 chunks + 16 bytes, keeps the transposed 16-byte reads apart
   constexpr int VP = 64;  // V slab row pitch: the 2-byte column accesses of a wavefront fall in one row
   __shared__ __attribute__((aligned(16))) E slab[4][16 * KP + 16 * VP];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   E *ks = slab[wave], *vs = slab[wave] + 16 * KP;
-  const int64_t wg_t0 = (int64_t)blockIdx.x * 16;
+  const int64_t w = (int64_t)blockIdx.x * 4 + wave;
+  const int64_t t0 = w / waves_per_group * 16;
+  if (t0 >= num_tokens) return;
   const int chunks_per_head = g.head_size / X;
   const int groups_per_head = (chunks_per_head + 7) / 8;  // the last group of a head may hold fewer than 8 chunks
-  const int items_per_half = g.num_heads * groups_per_head;
-  int64_t run_slot[2];
-#pragma unroll
-  for (int half = 0; half < 2; half++) {
-    const int64_t t0 = wg_t0 + 8 * half;
-    run_slot[half] = -1;
-    if (t0 + 8 <= num_tokens) {
-      const int64_t slot0 = (int64_t)slot_mapping[t0];
-      bool run = slot0 >= 0 && slot0 % 8 == 0 && slot0 / g.block_size < g.num_blocks;
-      if (run) {
-#pragma unroll
-        for (int i = 1; i < 8; i++) run = run && (int64_t)slot_mapping[t0 + i] == slot0 + i;
-      }
-      if (run) run_slot[half] = slot0;
-    }
-  }
+  const int item0 = (int)(w % waves_per_group) * items_per_wave;
+  const int item1 = min(item0 + items_per_wave, g.num_heads * groups_per_head);
+
+  // Lanes 0 .. 31 look at tokens t0 .. t0 + 31: a tile that starts among the first 16 ends among them.
+  const int64_t t = t0 + (lane & 31);
+  int64_t slot = t < num_tokens ? (int64_t)slot_mapping[t] : -1;
+  if (slot >= 0 && slot / g.block_size >= g.num_blocks) slot = -1;  // never outside the cache
+  const bool follows = t > 0 && t < num_tokens && slot > 0 && slot % 16 != 0 && (int64_t)slot_mapping[t - 1] == slot - 1;
+  const unsigned starts = (unsigned)__ballot(!follows), valid = (unsigned)__ballot(slot >= 0);
+  const unsigned own_starts = starts & 0xffffu;
+  if (own_starts == 0) return;  // all 16 belong to the tile of the wavefront before
+  // no other start among the 15 tokens behind it: all of them follow one another within the row of 16 slots
+  const bool is_tile = lane < 16 && !follows && slot >= 0 && slot % 16 == 0 && ((starts >> (lane + 1)) & 0x7fffu) == 0;
+  const unsigned tile = (unsigned)__ballot(is_tile);  // at most one
+  const unsigned later = starts & 0xffff0000u;
+  unsigned owned = ~0u << __builtin_ctz(own_starts);
+  if (later != 0) owned &= (1u << __builtin_ctz(later)) - 1u;
+  unsigned rest = owned & valid;
+  const int tile_at = tile != 0 ? __builtin_ctz(tile) : 0;
+  if (tile != 0) rest &= ~(0xffffu << tile_at);
+  const int64_t tile_slot = ((int64_t)__builtin_amdgcn_readlane((int)(slot >> 32), tile_at) << 32) |
+                            (unsigned)__builtin_amdgcn_readlane((int)slot, tile_at);
   const int hi = lane >> 3, lo = lane & 7;
-  // A workgroup whose 16 tokens fill one whole block: a tile is then 16 tokens deep and every access to
-  // the cache covers whole rows -- K as 256-byte [chunk][16 tokens] rows, V as the 32-byte [16 tokens]
-  // rows of 32 consecutive head elements, 1 KiB contiguous either way.
-  if (g.block_size == 16 && run_slot[0] >= 0 && run_slot[0] % 16 == 0 && run_slot[1] == run_slot[0] + 8) {
-    const int64_t blk = run_slot[0] / 16;
-    for (int item = wave; item < items_per_half; item += 4) {
-      const int h = item / groups_per_head, cg = item % groups_per_head;
-      const int nc = FULL_GROUPS ? 8 : min(8, chunks_per_head - 8 * cg);  // chunks in this group
-      E *kc_base = key_cache + blk * g.k_block_stride + h * g.k_head_stride;
-      E *vc_base = value_cache + blk * g.v_block_stride + h * g.v_head_stride;
-      const int tok = lane & 15, c4 = lane >> 4;
-      const int th = lane & 1;  // which 8 tokens of a V row
+  const int tok = lane & 15, c4 = lane >> 4;
+  const int th = lane & 1;  // which 8 tokens of a V row
+
+  for (int item = item0; item < item1; item++) {
+    const int h = item / groups_per_head, cg = item % groups_per_head;
+    const int nc = FULL_GROUPS ? 8 : min(8, chunks_per_head - 8 * cg);  // chunks in this group
+    if (tile != 0) {
+      const int64_t blk = tile_slot / g.block_size, off = tile_slot % g.block_size;
+      E *kc_base = key_cache + blk * g.k_block_stride + h * g.k_head_stride + ((int64_t)cg * 8 * g.block_size + off) * X;
+      E *vc_base = value_cache + blk * g.v_block_stride + h * g.v_head_stride + (int64_t)cg * 64 * g.block_size + off;
+      E *k_tok = key + (t0 + tile_at + hi) * key_tok_stride + h * key_head_stride + (cg * 8 + lo) * X;
+      E *v_tok = value + (t0 + tile_at + hi) * val_tok_stride + h * val_head_stride + (cg * 8 + lo) * X;
       if (SCATTER) {
+        uint4 kk[2], vv[2];
 #pragma unroll
-        for (int half = 0; half < 2; half++) {  // tokens hi and hi + 8, chunk lo
-          const E *k_tok = key + (wg_t0 + 8 * half + hi) * key_tok_stride + h * key_head_stride + (cg * 8 + lo) * X;
-          const E *v_tok = value + (wg_t0 + 8 * half + hi) * val_tok_stride + h * val_head_stride + (cg * 8 + lo) * X;
+        for (int half = 0; half < 2; half++)  // tokens hi and hi + 8, chunk lo
           if (lo < nc) {
-            *reinterpret_cast<uint4 *>(ks + (8 * half + hi) * KP + lo * X) = *reinterpret_cast<const uint4 *>(k_tok);
-            *reinterpret_cast<uint4 *>(vs + (8 * half + hi) * VP + lo * X) = *reinterpret_cast<const uint4 *>(v_tok);
+            kk[half] = *reinterpret_cast<const uint4 *>(k_tok + 8 * half * key_tok_stride);
+            vv[half] = *reinterpret_cast<const uint4 *>(v_tok + 8 * half * val_tok_stride);
           }
-        }
+#pragma unroll
+        for (int half = 0; half < 2; half++)
+          if (lo < nc) {
+            *reinterpret_cast<uint4 *>(ks + (8 * half + hi) * KP + lo * X) = kk[half];
+            *reinterpret_cast<uint4 *>(vs + (8 * half + hi) * VP + lo * X) = vv[half];
+          }
         __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the slab is private to this wavefront
 #pragma unroll
         for (int i = 0; i < 2; i++) {  // chunk rows 4i + c4: 4 rows x 256 bytes per instruction
@@ -287,7 +304,7 @@ __global__ __launch_bounds__(256) void cache_move_tile_kernel(
           if (c < nc)
             // (the cache is not read again before a later step: stored with the written-once hint, 47.8 -> 44.1 us
             // for 32768 tokens x 8 kv heads x 128)
-            store16_once(kc_base + ((int64_t)(cg * 8 + c) * 16 + tok) * X, *reinterpret_cast<const uint4 *>(ks + tok * KP + c * X));
+            store16_once(kc_base + ((int64_t)c * g.block_size + tok) * X, *reinterpret_cast<const uint4 *>(ks + tok * KP + c * X));
         }
 #pragma unroll
         for (int i = 0; i < 2; i++) {  // head elements 32i + lane / 2: 32 rows x 32 bytes per instruction
@@ -295,104 +312,55 @@ __global__ __launch_bounds__(256) void cache_move_tile_kernel(
           uint4 o;
           E *oe = reinterpret_cast<E *>(&o);
 #pragma unroll
-          for (int t = 0; t < 8; t++) oe[t] = vs[(8 * th + t) * VP + e];
-          if (e < nc * X) store16_once(vc_base + (int64_t)(cg * 64 + e) * 16 + 8 * th, o);
+          for (int k = 0; k < 8; k++) oe[k] = vs[(8 * th + k) * VP + e];
+          if (e < nc * X) store16_once(vc_base + (int64_t)e * g.block_size + 8 * th, o);
         }
       } else {
+        uint4 kk[2], vv[2];
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-          const int c = 4 * i + c4;
-          if (c < nc)
-            *reinterpret_cast<uint4 *>(ks + tok * KP + c * X) = load16_once(kc_base + ((int64_t)(cg * 8 + c) * 16 + tok) * X);
-          const int e = 32 * i + (lane >> 1);
+          const int c = 4 * i + c4, e = 32 * i + (lane >> 1);
+          if (c < nc) kk[i] = load16_once(kc_base + ((int64_t)c * g.block_size + tok) * X);
+          if (e < nc * X) vv[i] = load16_once(vc_base + (int64_t)e * g.block_size + 8 * th);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          const int c = 4 * i + c4, e = 32 * i + (lane >> 1);
+          if (c < nc) *reinterpret_cast<uint4 *>(ks + tok * KP + c * X) = kk[i];
           if (e < nc * X) {
-            const uint4 vin = load16_once(vc_base + (int64_t)(cg * 64 + e) * 16 + 8 * th);
-            const E *ve = reinterpret_cast<const E *>(&vin);
+            const E *ve = reinterpret_cast<const E *>(&vv[i]);
 #pragma unroll
-            for (int t = 0; t < 8; t++) vs[(8 * th + t) * VP + e] = ve[t];
+            for (int k = 0; k < 8; k++) vs[(8 * th + k) * VP + e] = ve[k];
           }
         }
         __builtin_amdgcn_s_waitcnt(0xc07f);
 #pragma unroll
-        for (int half = 0; half < 2; half++) {
-          E *k_tok = key + (wg_t0 + 8 * half + hi) * key_tok_stride + h * key_head_stride + (cg * 8 + lo) * X;
-          E *v_tok = value + (wg_t0 + 8 * half + hi) * val_tok_stride + h * val_head_stride + (cg * 8 + lo) * X;
+        for (int half = 0; half < 2; half++)
           if (lo < nc) {
-            *reinterpret_cast<uint4 *>(k_tok) = *reinterpret_cast<const uint4 *>(ks + (8 * half + hi) * KP + lo * X);
-            *reinterpret_cast<uint4 *>(v_tok) = *reinterpret_cast<const uint4 *>(vs + (8 * half + hi) * VP + lo * X);
+            *reinterpret_cast<uint4 *>(k_tok + 8 * half * key_tok_stride) =
+                *reinterpret_cast<const uint4 *>(ks + (8 * half + hi) * KP + lo * X);
+            *reinterpret_cast<uint4 *>(v_tok + 8 * half * val_tok_stride) =
+                *reinterpret_cast<const uint4 *>(vs + (8 * half + hi) * VP + lo * X);
           }
-        }
       }
       __builtin_amdgcn_s_waitcnt(0xc07f);  // slab reads done before the next item overwrites it
     }
-    return;
-  }
-  for (int item = wave; item < 2 * items_per_half; item += 4) {  // uniform per wavefront
-    const int half = item / items_per_half;
-    const int rem = item % items_per_half;
-    const int h = rem / groups_per_head, cg = rem % groups_per_head;
-    const int64_t t0 = wg_t0 + 8 * half;
-    const int64_t slot0 = half == 0 ? run_slot[0] : run_slot[1];
-    if (slot0 >= 0) {
-      const int64_t blk = slot0 / g.block_size;
-      const int off0 = (int)(slot0 % g.block_size);
-      E *kc_base = key_cache + blk * g.k_block_stride + h * g.k_head_stride;
-      E *vc_base = value_cache + blk * g.v_block_stride + h * g.v_head_stride;
-      // token-major side: lane (token hi, chunk lo); cache side: lane (chunk hi, token lo) for K,
-      // lane (chunk hi, element lo) for V
-      E *k_tok = key + (t0 + hi) * key_tok_stride + h * key_head_stride + (cg * 8 + lo) * X;
-      E *v_tok = value + (t0 + hi) * val_tok_stride + h * val_head_stride + (cg * 8 + lo) * X;
-      E *k_cache = kc_base + ((int64_t)(cg * 8 + hi) * g.block_size + off0 + lo) * X;
-      E *v_cache = vc_base + (int64_t)((cg * 8 + hi) * X + lo) * g.block_size + off0;
-      const int nc = FULL_GROUPS ? 8 : min(8, chunks_per_head - 8 * cg);  // chunks in this group
-      if (SCATTER) {
-        if (lo < nc) {
-          *reinterpret_cast<uint4 *>(ks + hi * KP + lo * X) = *reinterpret_cast<const uint4 *>(k_tok);
-          *reinterpret_cast<uint4 *>(vs + hi * VP + lo * X) = *reinterpret_cast<const uint4 *>(v_tok);
-        }
-        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the slab is private to this wavefront
-        if (hi < nc) {
-          *reinterpret_cast<uint4 *>(k_cache) = *reinterpret_cast<const uint4 *>(ks + lo * KP + hi * X);
-          uint4 o;
-          E *oe = reinterpret_cast<E *>(&o);
-#pragma unroll
-          for (int t = 0; t < 8; t++) oe[t] = vs[t * VP + lane];  // element (hi, lo) of token t
-          *reinterpret_cast<uint4 *>(v_cache) = o;
-        }
-      } else {
-        if (hi < nc) {
-          *reinterpret_cast<uint4 *>(ks + lo * KP + hi * X) = load16_once(k_cache);
-          const uint4 vin = load16_once(v_cache);
-          const E *ve = reinterpret_cast<const E *>(&vin);
-#pragma unroll
-          for (int t = 0; t < 8; t++) vs[t * VP + lane] = ve[t];
-        }
-        __builtin_amdgcn_s_waitcnt(0xc07f);
-        if (lo < nc) {
-          *reinterpret_cast<uint4 *>(k_tok) = *reinterpret_cast<const uint4 *>(ks + hi * KP + lo * X);
-          *reinterpret_cast<uint4 *>(v_tok) = *reinterpret_cast<const uint4 *>(vs + hi * VP + lo * X);
-        }
+    // the others, eight tokens at a time: lane (token hi of the eight, chunk lo)
+    for (unsigned left = rest; left != 0;) {
+      unsigned mine = left;
+      for (int k = 0; k < hi; k++) mine &= mine - 1;
+      const int at = mine != 0 ? __builtin_ctz(mine) : 0;
+      const int64_t one = ((int64_t)__shfl((int)(slot >> 32), at, 64) << 32) | (unsigned)__shfl((int)slot, at, 64);
+      if (mine != 0 && lo < nc) {
+        const int64_t blk = one / g.block_size;
+        const int off = (int)(one % g.block_size), c = cg * 8 + lo;
+        move_token_chunk<E, SCATTER>(key + (t0 + at) * key_tok_stride + h * key_head_stride + c * X,
+                                     value + (t0 + at) * val_tok_stride + h * val_head_stride + c * X,
+                                     key_cache + blk * g.k_block_stride + h * g.k_head_stride + ((int64_t)c * g.block_size + off) * X,
+                                     value_cache + blk * g.v_block_stride + h * g.v_head_stride + (int64_t)c * X * g.block_size + off,
+                                     g.block_size);
       }
-      __builtin_amdgcn_s_waitcnt(0xc07f);  // slab reads done before the next item overwrites it
-      continue;
-    }
-    // per-token path for this group of 8: lane = chunk of the 64-element group, tokens in turn
-    for (int t = 0; t < 8; t++) {
-      const int64_t token = t0 + t;
-      if (token >= num_tokens) break;
-      const int64_t slot = (int64_t)slot_mapping[token];
-      if (slot < 0) continue;
-      const int64_t blk = slot / g.block_size;
-      if (blk >= g.num_blocks) continue;
-      const int off = (int)(slot % g.block_size);
-      if (lane < (FULL_GROUPS ? 8 : min(8, chunks_per_head - 8 * cg))) {
-        const int c = cg * 8 + lane;
-        E *kp = key + token * key_tok_stride + h * key_head_stride + c * X;
-        E *vp = value + token * val_tok_stride + h * val_head_stride + c * X;
-        E *kc = key_cache + blk * g.k_block_stride + h * g.k_head_stride + ((int64_t)c * g.block_size + off) * X;
-        E *vc = value_cache + blk * g.v_block_stride + h * g.v_head_stride + (int64_t)c * X * g.block_size + off;
-        move_token_chunk<E, SCATTER>(kp, vp, kc, vc, g.block_size);
-      }
+      for (int k = 0; k < 8; k++) left &= left - 1;
     }
   }
 }
@@ -560,22 +528,37 @@ void launch_move(const hipattn_tensor *key, const hipattn_tensor *value,
                    g.k_head_stride % X == 0 && g.head_size % X == 0;
   dim3 grid((unsigned)T);
   if constexpr (sizeof(E) == 2) {
-    // long inputs (prompts): 8-token workgroups with the transposing fast path
-    if (vec && T >= 1024 && g.block_size % 8 == 0 && aligned16(vc) && g.v_block_stride % 8 == 0 &&
-        g.v_head_stride % 8 == 0) {
-      // The LDS-transposing kernel pays off (whole rows on both sides) once there are enough 16-token
-      // workgroups to hide its load -> LDS -> store chains.
-      if (T >= 16384 && tuning().cache_move_lds != 0) {
-        // head sizes that are multiples of 64 have no partial chunk group: their instance carries no guards
-        if (g.head_size % 64 == 0)
-          cache_move_tile_kernel<Slot, SCATTER, true><<<dim3((unsigned)((T + 15) / 16)), 256, 0, stream>>>(
-              kp, vp, kc, vc, sp, T, key->strides[0], key->strides[1], value->strides[0], value->strides[1], g);
-        else
-          cache_move_tile_kernel<Slot, SCATTER, false><<<dim3((unsigned)((T + 15) / 16)), 256, 0, stream>>>(
-              kp, vp, kc, vc, sp, T, key->strides[0], key->strides[1], value->strides[0], value->strides[1], g);
-        check_launch(SCATTER ? "reshape_and_cache" : "gather_cached_kv");
-        return;
+    // prompts (and whatever comes with them): the transposing kernels
+    const bool vec_v = vec && g.block_size % 8 == 0 && aligned16(vc) && g.v_block_stride % 8 == 0 && g.v_head_stride % 8 == 0;
+    if (vec_v && T >= 128 && g.block_size % 16 == 0 && tuning().cache_move_lds != 0) {
+      // One item (a head's 64 elements of 16 tokens) per wavefront while that is no more than 32 wavefronts per compute unit, up
+      // to eight beyond (the slots are looked at once per wavefront).
+      const int64_t groups = (T + 15) / 16;
+      CacheGeom gt = g;
+      if (key->strides[1] == g.head_size && value->strides[1] == g.head_size && g.k_head_stride == (int64_t)g.head_size * g.block_size &&
+          g.v_head_stride == g.k_head_stride && (int64_t)g.num_heads * g.head_size <= (1 << 20)) {
+        // heads that lie end to end in the rows and in the cache are one wide head: chunk groups run across them (head size
+        // 80: five full groups per four heads instead of eight, half of them with two chunks)
+        gt.head_size *= gt.num_heads;
+        gt.num_heads = 1;
       }
+      const int items = gt.num_heads * ((gt.head_size / X + 7) / 8);
+      const int per_wave = (int)std::min<int64_t>(8, std::max<int64_t>(1, groups * items / 8192));
+      const int waves_per_group = (items + per_wave - 1) / per_wave;
+      const dim3 tiles((unsigned)((groups * waves_per_group + 3) / 4));
+      // head sizes that are multiples of 64 have no partial chunk group: their instance carries no guards
+      if (gt.head_size % 64 == 0)
+        cache_move_tile_kernel<Slot, SCATTER, true><<<tiles, 256, 0, stream>>>(
+            kp, vp, kc, vc, sp, T, key->strides[0], key->strides[1], value->strides[0], value->strides[1], gt, per_wave,
+            waves_per_group);
+      else
+        cache_move_tile_kernel<Slot, SCATTER, false><<<tiles, 256, 0, stream>>>(
+            kp, vp, kc, vc, sp, T, key->strides[0], key->strides[1], value->strides[0], value->strides[1], gt, per_wave,
+            waves_per_group);
+      check_launch(SCATTER ? "reshape_and_cache" : "gather_cached_kv");
+      return;
+    }
+    if (vec_v && T >= 1024) {
       // about two thousand workgroups, if the heads allow: a few hundred of them leave most of the memory
       // system idle (2168 tokens of 32 heads x 80: 60 us with one workgroup per 16 tokens)
       const int64_t groups = (T + 15) / 16;

@@ -114,6 +114,38 @@ def test_long_inputs_runs_of_tokens_mixed_with_everything_else(device, dtype, st
     assert torch.equal(bits(ko), bits(want_k)) and torch.equal(bits(vo), bits(want_v))
 
 
+@pytest.mark.parametrize("bs,d,H", [(16, 128, 3), (16, 80, 2), (32, 64, 1), (48, 8, 5), (16, 64, 2)])
+@pytest.mark.parametrize("T", [127, 128, 129, 160, 300, 1023])
+def test_tiles_start_at_any_token(device, bs, d, H, T):
+    """Batches of short sequences laid end to end: their full rows of 16 slots start at every token index modulo 16, next to
+    single tokens, beginnings in the middle of a block, ends, padding slots and slots past the cache."""
+    g = torch.Generator().manual_seed(1000 * bs + T)
+    nb = 2 * T // bs + 60
+    order = torch.randperm(nb, generator=g).tolist()
+    slots = []
+    while len(slots) < T:
+        n = int(torch.randint(1, 60, (1,), generator=g)) if len(slots) % 3 else 1
+        first = int(torch.randint(0, bs, (1,), generator=g)) if n % 4 == 0 else 0
+        blocks = [order.pop() for _ in range((first + n + bs - 1) // bs)] if len(order) > 6 else []
+        slots += [blocks[(first + i) // bs] * bs + (first + i) % bs for i in range(n)] if blocks else [-1]
+    slots = torch.tensor(slots[:T], dtype=torch.int64)
+    slots[T // 3], slots[T // 2] = -1, nb * bs + 7
+    key, value = (torch.randn((T, H, d), generator=g).to(torch.bfloat16) for _ in range(2))
+    kc, vc = make_cache(nb, H, d, bs, torch.bfloat16, fill=-3.0)
+    kc_ref, vc_ref = kc.clone(), vc.clone()
+    ok = (slots >= 0) & (slots < nb * bs)
+    ref.reshape_and_cache(key[ok], value[ok], kc_ref, vc_ref, slots[ok])
+    kd, vd = kc.to(device), vc.to(device)
+    K.reshape_and_cache(key.to(device), value.to(device), kd, vd, slots.to(device))
+    assert torch.equal(bits(kd), bits(kc_ref)) and torch.equal(bits(vd), bits(vc_ref))
+    ko = torch.full((T, H, d), 9.0, dtype=torch.bfloat16, device=device)
+    vo = torch.full_like(ko, 9.0)
+    K.gather_cached_kv(ko, vo, kd, vd, slots.to(torch.int32).to(device))
+    want_k, want_v = key.clone(), value.clone()
+    want_k[~ok], want_v[~ok] = 9.0, 9.0
+    assert torch.equal(bits(ko), bits(want_k)) and torch.equal(bits(vo), bits(want_v))
+
+
 def test_config1_scatter_bit_exact(device):
     p, extra = W.config1()
     nb = extra["pool_blocks"]
