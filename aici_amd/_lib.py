@@ -87,6 +87,8 @@ _ERR_FUNCS = {
     "hipattn_reshape_and_cache": [TP, TP, TP, TP, TP, c_void_p],
     "hipattn_gather_cached_kv": [TP, TP, TP, TP, TP, c_void_p],
     "hipattn_copy_blocks_2": [TP, TP, TP, TP, c_void_p],
+    "hipattn_copy_blocks_host": [POINTER(c_void_p), POINTER(c_void_p), c_int64, POINTER(c_int64), c_int64, c_int64,
+                                 c_void_p],
     "hipattn_swap_blocks": [TP, c_int, TP, c_int, POINTER(c_int64), c_int64, c_void_p],
     "hipattn_rotary_embedding": [TP, TP, TP, c_int, TP, c_bool, c_void_p],
     "hipattn_rotary_embedding_and_cache": [TP, TP, TP, TP, c_int, TP, c_bool, TP, TP, TP, c_void_p],

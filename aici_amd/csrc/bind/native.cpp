@@ -18,6 +18,7 @@
 #include <string>
 #include <tuple>
 #include <utility>
+#include <vector>
 
 #include "../../../include/hipattn.h"
 
@@ -243,6 +244,81 @@ PyMethodDef method(const char *fn, const char *names) {
   Binding<Fn>::names = names;
   return {fn, (PyCFunction)(void (*)(void))Binding<Fn>::call, METH_FASTCALL, names};
 }
+
+// copy_blocks(key_caches, value_caches, pairs): lists of every layer's caches and of src, dst, src, dst, ...  True if done;
+// False where the caches are not what hipattn_copy_blocks_host takes (the caller then has its own checks).
+PyObject *copy_blocks(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  if (n != 3) {
+    PyErr_Format(PyExc_TypeError, "copy_blocks takes 3 arguments (key_caches,value_caches,pairs), got %zd", n);
+    return nullptr;
+  }
+  Call c{"copy_blocks", "key_caches,value_caches,pairs"};
+  std::vector<void *> ptrs[2];
+  hipattn_tensor first{};
+  int64_t bytes = 1;
+  PyObject *held[3] = {nullptr, nullptr, nullptr};
+  struct Release {
+    PyObject **held;
+    ~Release() {
+      for (int i = 0; i < 3; i++) Py_XDECREF(held[i]);
+    }
+  } release{held};
+  for (int i = 0; i < 3; i++)
+    if ((held[i] = PySequence_Fast(args[i], "copy_blocks: expected sequences")) == nullptr) return nullptr;
+  for (int side = 0; side < 2; side++) {
+    const Py_ssize_t layers = PySequence_Fast_GET_SIZE(held[side]);
+    for (Py_ssize_t l = 0; l < layers; l++) {
+      PyObject *o = PySequence_Fast_GET_ITEM(held[side], l);
+      hipattn_tensor d{};
+      DLTensor t;
+      if (!PyObject_TypeCheck(o, g_tensor_type) || g_exchange->dltensor_from_py_object_no_sync(o, &t) != 0) {
+        PyErr_Clear();
+        Py_RETURN_FALSE;
+      }
+      if ((t.device.device_type != kDLROCM && t.device.device_type != kDLCUDA) || t.ndim < 1 || t.ndim > HIPATTN_MAX_DIMS ||
+          !dtype_of(t.dtype, &d.dtype) || (d.dtype != HIPATTN_F16 && d.dtype != HIPATTN_BF16) || !describe(o, side, c, &d)) {
+        PyErr_Clear();
+        Py_RETURN_FALSE;
+      }
+      int64_t dense = 1, all = 1;
+      bool contiguous = true;
+      for (int i = d.ndim - 1; i >= 0; i--) {
+        contiguous = contiguous && (d.sizes[i] == 1 || d.strides[i] == dense);
+        dense *= d.sizes[i];
+        if (i > 0) all *= d.sizes[i];
+      }
+      if (side == 0 && l == 0) {
+        first = d;
+        bytes = all * 2;
+      }
+      int64_t first_numel = 1;
+      for (int i = 0; i < first.ndim; i++) first_numel *= first.sizes[i];
+      if (!contiguous || dense != first_numel || t.device.device_id != c.device ||
+          (reinterpret_cast<uintptr_t>(d.data) & 15) != 0) Py_RETURN_FALSE;
+      ptrs[side].push_back(d.data);
+    }
+  }
+  if (bytes <= 0 || bytes % 16 != 0 || ptrs[0].size() != ptrs[1].size() || ptrs[0].empty()) Py_RETURN_FALSE;
+  const Py_ssize_t count = PySequence_Fast_GET_SIZE(held[2]);
+  std::vector<int64_t> pairs((size_t)count);
+  for (Py_ssize_t i = 0; i < count; i++)
+    if (!to_i64(PySequence_Fast_GET_ITEM(held[2], i), &pairs[(size_t)i])) return nullptr;
+  void *stream = nullptr;
+  if (g_exchange->current_work_stream((DLDeviceType)c.device_type, c.device, &stream) != 0) {
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "no current stream");
+    return nullptr;
+  }
+  char *err;
+  Py_BEGIN_ALLOW_THREADS
+  err = hipattn_copy_blocks_host(ptrs[0].data(), ptrs[1].data(), (int64_t)ptrs[0].size(), pairs.data(), count / 2, bytes, stream);
+  Py_END_ALLOW_THREADS
+  if (err != nullptr) {
+    PyErr_Format(g_error, "hipattn_copy_blocks_host: %s", err);
+    hipattn_free_error(err);
+    return nullptr;
+  }
+  Py_RETURN_TRUE;
+}
 #define BIND(name, names) method<hipattn_##name>(#name, names)
 
 PyMethodDef g_methods[] = {
@@ -258,6 +334,7 @@ PyMethodDef g_methods[] = {
                              "block_tables,context_lens,block_size,max_context_len,alibi"),
     BIND(reshape_and_cache, "key,value,key_cache,value_cache,slot_mapping"),
     BIND(gather_cached_kv, "key,value,key_cache,value_cache,slot_mapping"),
+    {"copy_blocks", (PyCFunction)(void (*)(void))copy_blocks, METH_FASTCALL, "key_caches,value_caches,pairs"},
     BIND(rotary_embedding, "positions,query,key,head_size,cos_sin_cache,is_neox"),
     BIND(rotary_embedding_and_cache, "positions,query,key,value,head_size,cos_sin_cache,is_neox,key_cache,value_cache,"
                                      "slot_mapping"),

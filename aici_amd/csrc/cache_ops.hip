@@ -725,6 +725,36 @@ __global__ __launch_bounds__(256) void copy_blocks_kernel(const int64_t *__restr
   }
 }
 
+// The same with the addresses and the pairs in the kernel's arguments: nothing goes to the device in front of the launch.
+// grid (layers, pairs).  Whole rows of 16 bytes (the entry point checks), four of K and four of V on their way per thread.
+constexpr int kCopyLayers = 64, kCopyPairs = 128;  // per launch: 3 KB of arguments
+struct CopyArgs {
+  char *key[kCopyLayers], *value[kCopyLayers];
+  int64_t pairs[kCopyPairs][2];
+};
+__global__ __launch_bounds__(256) void copy_blocks_args_kernel(const CopyArgs a, int64_t bytes_per_block) {
+  const int64_t src = a.pairs[blockIdx.y][0] * bytes_per_block, dst = a.pairs[blockIdx.y][1] * bytes_per_block;
+  char *kc = a.key[blockIdx.x], *vc = a.value[blockIdx.x];
+  const uint4 *ks = reinterpret_cast<const uint4 *>(kc + src), *vs = reinterpret_cast<const uint4 *>(vc + src);
+  uint4 *kd = reinterpret_cast<uint4 *>(kc + dst), *vd = reinterpret_cast<uint4 *>(vc + dst);
+  const int64_t n = bytes_per_block / 16;
+  for (int64_t i = threadIdx.x; i < n; i += 1024) {
+    uint4 k[4], v[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (i + j * 256 < n) {
+        k[j] = ks[i + j * 256];
+        v[j] = vs[i + j * 256];
+      }
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (i + j * 256 < n) {
+        kd[i + j * 256] = k[j];
+        vd[i + j * 256] = v[j];
+      }
+  }
+}
+
 }  // namespace
 
 }  // namespace hipattn
@@ -788,6 +818,35 @@ extern "C" char *hipattn_copy_blocks_2(const hipattn_tensor *key_cache_ptrs,
         static_cast<const int64_t *>(value_cache_ptrs->data),
         static_cast<const int64_t *>(block_mapping->data), bytes);
     check_launch("copy_blocks");
+  });
+}
+
+extern "C" char *hipattn_copy_blocks_host(void *const *key_caches, void *const *value_caches, int64_t layers,
+                                          const int64_t *block_mapping, int64_t n_pairs, int64_t bytes_per_block,
+                                          void *stream_arg) {
+  HA_PROTECT({
+    HA_CHECK(layers >= 0 && n_pairs >= 0 && bytes_per_block >= 0, "copy_blocks: negative sizes");
+    if (layers == 0 || n_pairs == 0 || bytes_per_block == 0) return nullptr;
+    HA_CHECK(key_caches != nullptr && value_caches != nullptr && block_mapping != nullptr, "copy_blocks: NULL array");
+    HA_CHECK(bytes_per_block % 16 == 0, "copy_blocks: a block of %lld bytes is not a multiple of 16", (long long)bytes_per_block);
+    for (int64_t i = 0; i < layers; i++)
+      HA_CHECK(key_caches[i] != nullptr && value_caches[i] != nullptr && aligned16(key_caches[i]) && aligned16(value_caches[i]),
+               "copy_blocks: the caches of layer %lld must start on a 16-byte boundary", (long long)i);
+    hipStream_t stream = resolve_stream(stream_arg);
+    CopyArgs a;
+    for (int64_t l0 = 0; l0 < layers; l0 += kCopyLayers) {
+      const int64_t nl = std::min<int64_t>(kCopyLayers, layers - l0);
+      for (int64_t i = 0; i < nl; i++) {
+        a.key[i] = static_cast<char *>(key_caches[l0 + i]);
+        a.value[i] = static_cast<char *>(value_caches[l0 + i]);
+      }
+      for (int64_t p0 = 0; p0 < n_pairs; p0 += kCopyPairs) {
+        const int64_t np = std::min<int64_t>(kCopyPairs, n_pairs - p0);
+        memcpy(a.pairs, block_mapping + 2 * p0, (size_t)np * sizeof a.pairs[0]);
+        copy_blocks_args_kernel<<<dim3((unsigned)nl, (unsigned)np), 256, 0, stream>>>(a, bytes_per_block);
+        check_launch("copy_blocks");
+      }
+    }
   });
 }
 

@@ -182,13 +182,16 @@ def copy_blocks(key_caches: List[torch.Tensor], value_caches: List[torch.Tensor]
         return
     device = key_caches[0].device
     tsize = key_caches[0].numel()
-    for e in list(key_caches) + list(value_caches):
-        assert e.device == device and e.numel() == tsize and e.is_contiguous()
-        assert e.dtype in (torch.float16, torch.bfloat16)
     pairs: List[int] = []
     for src, dsts in block_mapping.items():
         for dst in dsts:
             pairs += [int(src), int(dst)]
+    # addresses and pairs as arguments of the launch; False for blocks that are not whole 16-byte rows
+    if _native.copy_blocks(key_caches, value_caches, pairs):
+        return
+    for e in list(key_caches) + list(value_caches):
+        assert e.device == device and e.numel() == tsize and e.is_contiguous()
+        assert e.dtype in (torch.float16, torch.bfloat16)
     kp = torch.tensor([t.data_ptr() for t in key_caches], dtype=torch.int64).to(device)
     vp = torch.tensor([t.data_ptr() for t in value_caches], dtype=torch.int64).to(device)
     bm = torch.tensor(pairs, dtype=torch.int64).to(device)

@@ -239,6 +239,16 @@ char *hipattn_copy_blocks_2(const hipattn_tensor *key_cache_ptrs,
                             const hipattn_tensor *block_mapping,
                             const hipattn_tensor *key0, void *stream);
 
+/* The same from host arrays: the caches' base addresses of every layer and the
+ * (src,dst) pairs are read before the call returns and travel as arguments of
+ * the launches (64 layers x 128 pairs each), so that no upload goes in front
+ * of the copy and the call may be captured.  Caches must start on 16-byte
+ * boundaries and bytes_per_block be a multiple of 16. */
+char *hipattn_copy_blocks_host(void *const *key_caches, void *const *value_caches,
+                               int64_t layers, const int64_t *block_mapping,
+                               int64_t n_pairs, int64_t bytes_per_block,
+                               void *stream);
+
 /* Replaces swap_blocks (cache_kernels.cu:12-50; the Rust wrapper is a stub,
  * lib.rs:236-243).  src/dst are whole caches of equal block shape; direction
  * is given by where each lives (0 = host, 1 = device); block_mapping is a host

@@ -146,6 +146,23 @@ def test_tiles_start_at_any_token(device, bs, d, H, T):
     assert torch.equal(bits(ko), bits(want_k)) and torch.equal(bits(vo), bits(want_v))
 
 
+@pytest.mark.parametrize("layers,pairs,d", [(1, 1, 8), (3, 129, 64), (65, 2, 80), (2, 0, 64)])
+def test_copy_blocks_with_more_than_one_launch_holds(device, layers, pairs, d):
+    """Layers and pairs beyond what one launch's arguments hold; and the former entry point, from device arrays."""
+    g = torch.Generator().manual_seed(layers + pairs)
+    nb = 2 * pairs + 3
+    caches = [make_cache(nb, 2, d, 16, torch.float16, fill=0.0) for _ in range(layers)]
+    caches = [(torch.randn(k.shape, generator=g).half(), torch.randn(v.shape, generator=g).half()) for k, v in caches]
+    order = torch.randperm(nb, generator=g).tolist()
+    mapping = {order[i]: [order[pairs + i]] for i in range(pairs)}
+    dev = [(k.to(device), v.to(device)) for k, v in caches]
+    K.copy_blocks([k for k, _ in dev], [v for _, v in dev], mapping)
+    for (k, v), (kd, vd) in zip(caches, dev):
+        for src, (dst,) in mapping.items():
+            k[dst], v[dst] = k[src], v[src]
+        assert torch.equal(bits(kd), bits(k)) and torch.equal(bits(vd), bits(v))
+
+
 def test_config1_scatter_bit_exact(device):
     p, extra = W.config1()
     nb = extra["pool_blocks"]
