@@ -84,6 +84,34 @@ def test_context_edge_lengths_and_stale_cache_contents(device, dtype):
     assert (got.float() - want).abs().max().item() <= TOL[dtype]
 
 
+@pytest.mark.parametrize("S,heads,longest,part_blocks", [
+    (1, (32, 8, 128), 129, 0), (2, (8, 8, 64), 256, 0), (16, (32, 8, 128), 257, 0), (16, (8, 8, 96), 512, 0),   # a context per
+    (18, (32, 8, 128), 1024, 0), (65, (16, 2, 64), 1009, 0),                                                     # workgroup
+    (3, (32, 8, 128), 8 * 32, 2), (3, (8, 8, 80), 9 * 32, 2), (3, (16, 1, 64), 16 * 32, 2), (2, (8, 2, 256), 17 * 32, 2)])
+def test_whole_contexts_per_workgroup_and_merges_of_few_partitions(device, tuning, S, heads, longest, part_blocks):
+    """Contexts of 0, 1, one pair per wavefront and one more, and the longest, where eight wavefronts share a context; and 8, 9, 16 and
+    17 partitions, on both sides of what the small merge kernels take.  Uncovered cache slots hold NaN."""
+    Hq, Hkv, d = heads
+    tuning("decode_part_blocks", part_blocks)
+    c = W.decode_inputs(50 + S, S, longest, longest, Hq, Hkv, d, torch.bfloat16, S * ((longest + 15) // 16) + 3)
+    lens = np.random.default_rng(S).integers(0, longest + 1, size=S).astype(np.int32)
+    edges = [longest, 0, 1, min(256, longest), min(257, longest), 31][:S]
+    lens[:len(edges)] = edges
+    c.context_lens = torch.from_numpy(lens)
+    for s, n in enumerate(lens.tolist()):
+        for b in range(n // 16, c.block_tables.size(1)):
+            first = n % 16 if b == n // 16 else 0
+            c.value_cache[int(c.block_tables[s, b]), :, :, first:] = float("nan")
+            c.key_cache[int(c.block_tables[s, b]), :, :, first:] = float("nan")
+    got = run_v1(c, device)
+    clean = W.DecodeInputs(**{**c.__dict__, "key_cache": c.key_cache.nan_to_num(0.0), "value_cache": c.value_cache.nan_to_num(0.0)})
+    want = oracle(clean)
+    assert not torch.isnan(got).any()
+    live = c.context_lens > 0
+    assert (got[live].float() - want[live]).abs().max().item() <= TOL[torch.bfloat16]
+    assert torch.all(got[~live] == 0)
+
+
 def test_single_partition_path_and_many_partitions_agree_with_oracle(device):
     # S large -> one partition per sequence; S = 1 -> the context is split many ways.
     big = W.decode_inputs(13, 300, 100, 400, 8, 2, 128, torch.float16, 8000)
