@@ -28,8 +28,8 @@
 //   11 + 11 + 10 bits, each summing the mass per bucket of the tokens that match the bits fixed so far, until the image
 //   of the last kept value -- and with it the mass above and the number of equal values kept -- is known.
 //
-// 128 rows of 128256 bf16 logits, 5 % allowed, top-p 0.9: any row 198 us, counting 48 us (the logits themselves
-// take 5 us to read once).
+// 128 rows of 128256 bf16 logits, 5 % allowed, top-p 0.9: any row 199 us, counting 43 us; all allowed 221 / 55, one row
+// 177 / 40; fp16 203 / 60 (the logits take 5 us to read once; a pass over one row on one compute unit takes 6 to 12).
 #include "common.h"
 #include "device_types.h"
 
@@ -76,6 +76,8 @@ struct Scratch {
   int wave_int[kWaves];
   float wave_f[kWaves];
   int pick, last;
+  int n_others;
+  uint16_t others[kThreads];
 };
 
 __device__ __forceinline__ float block_max(float v, Scratch &s) {
@@ -129,21 +131,22 @@ __device__ __forceinline__ u64 block_exclusive(u64 v, Scratch &s) {
 }
 
 // The counted values of a 16-bit float type: magnitudes above kLo (2^-16 / 2^-8) of either sign, numbered by their bits;
-// smaller ones share number 0.  kBins values from the row's largest down have a counter.
+// smaller ones share number 0.  kBins values have a counter: of bf16 all from 2^16 (number kTop) down to -2^16, so that the
+// largest is found among the counters; fp16 has more, and the counters go from the row's largest down, found in a pass before.
 template <typename T>
 struct Counted {
   static constexpr bool possible = false;
-  static constexpr int kBins = 1, kLo = 0, kInf = 0;
+  static constexpr int kBins = 1, kLo = 0, kInf = 0, kTop = 0;
 };
 template <>
 struct Counted<bf16_t> {
   static constexpr bool possible = true;
-  static constexpr int kBins = 8192, kLo = 0x3780, kInf = 0x7f80;
+  static constexpr int kBins = 8192, kLo = 0x3780, kTop = 4096;
 };
 template <>
 struct Counted<half_t> {
   static constexpr bool possible = true;
-  static constexpr int kBins = 28672, kLo = 0x1c00, kInf = 0x7c00;
+  static constexpr int kBins = 28672, kLo = 0x1c00, kInf = 0x7c00, kTop = 0;
 };
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
@@ -196,100 +199,151 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
     return to_float(bit_cast<T>(b));
   };
 
-  // The largest image.
-  u16x2 top = {0, 0};
-  for (int base = g0; base < g1; base += 64 * U) {
-    uint4 raw[U];
-    unsigned bits[U];
+  // numbers of two values: their bits above kLo, with the sign
+  auto numbers = [](unsigned w, u16x2 &mag) {
+    typedef short i16x2 __attribute__((ext_vector_type(2)));
+    const u16x2 sign = bit_cast<u16x2>(bit_cast<i16x2>(w) >> (short)15);
+    mag = __builtin_elementwise_sub_sat(bit_cast<u16x2>(w & 0x7fff7fffu), (u16x2)(unsigned short)C::kLo);
+    return (mag ^ sign) - sign;
+  };
+  // every group of eight of this wavefront: f(raw, allow-bits)
+  auto for_groups = [&](auto &&f) {
+    for (int base = g0; base < g1; base += 64 * U) {
+      uint4 raw[U];
+      unsigned bits[U];
 #pragma unroll
-    for (int u = 0; u < U; u++) load(base + u * 64 + lane, g1, raw[u], bits[u]);
+      for (int u = 0; u < U; u++) load(base + u * 64 + lane, g1, raw[u], bits[u]);
 #pragma unroll
-    for (int u = 0; u < U; u++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const unsigned lo = __builtin_amdgcn_sbfe((int)bits[u], 2 * i, 1), hi = __builtin_amdgcn_sbfe((int)bits[u], 2 * i + 1, 1);
-        const unsigned allowed = (lo & 0xffffu) | (hi & 0xffff0000u);
-        top = __builtin_elementwise_max(top, bit_cast<u16x2>(images(pair(raw[u], i)) & allowed));
-      }
-  }
-#pragma unroll
-  for (int i = 0; i < kOwn; i++) bins[tid + i * kThreads] = 0;
-  const int image_max = (int)block_max((float)max(top[0], top[1]), s);
-  if (image_max <= (int)(0x7fffu - C::kInf)) {  // nothing allowed (or -inf alone): no distribution to draw from
-    if (tid == 0) *out = 0;
-    return true;
-  }
-  const bool positive = (image_max & 0x8000) != 0;
-  const int top_mag = (positive ? image_max & 0x7fff : 0x7fff - image_max) - C::kLo;
-  if (image_max >= (0x8000 | C::kInf) || top_mag <= 0 || !(temp < 1e15f)) return false;
-  const int top_number = positive ? top_mag : -top_mag;
-  const float m = value((unsigned)image_max) / temp;
-  if (!(fabsf(m) < INFINITY)) return false;
-  auto mass = [&](float v) -> u64 {
-    const float x = v / temp;
-    return x > -INFINITY ? (u64)(__builtin_amdgcn_exp2f((x - m) * kLog2e) * kMassUnit) : 0ull;
+      for (int u = 0; u < U; u++) f(raw[u], bits[u]);
+    }
   };
 
-  // Tokens per value.  Those of a small magnitude, or too far below the largest to have a counter, are few: their mass
-  // is summed one by one.
-  u64 small = 0, low = 0;
-  for (int base = g0; base < g1; base += 64 * U) {
-    uint4 raw[U];
-    unsigned bits[U];
 #pragma unroll
-    for (int u = 0; u < U; u++) load(base + u * 64 + lane, g1, raw[u], bits[u]);
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      if (!__any((int)bits[u])) continue;
-      typedef short i16x2 __attribute__((ext_vector_type(2)));
-      u16x2 off[4], least = {0xffff, 0xffff}, most = {0, 0};
+  for (int i = 0; i < kOwn; i++) bins[tid + i * kThreads] = 0;
+  if (tid == 0) s.n_others = 0;
+  int top_number = C::kTop;  // of counter 0
+  if constexpr (C::kTop == 0) {
+    u16x2 top = {0, 0};
+    for_groups([&](const uint4 &raw, unsigned bits) {
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const unsigned w = pair(raw[u], i);
-        const u16x2 sign = bit_cast<u16x2>(bit_cast<i16x2>(w) >> (short)15);
-        const u16x2 mag = __builtin_elementwise_sub_sat(bit_cast<u16x2>(w & 0x7fff7fffu), (u16x2)(unsigned short)C::kLo);
-        off[i] = (u16x2)(unsigned short)top_number - ((mag ^ sign) - sign);
-        least = __builtin_elementwise_min(least, mag);
-        most = __builtin_elementwise_max(most, off[i]);
+        const unsigned lo = __builtin_amdgcn_sbfe((int)bits, 2 * i, 1), hi = __builtin_amdgcn_sbfe((int)bits, 2 * i + 1, 1);
+        const unsigned allowed = (lo & 0xffffu) | (hi & 0xffff0000u);
+        top = __builtin_elementwise_max(top, bit_cast<u16x2>(images(pair(raw, i)) & allowed));
       }
-      const bool all_counted = min(least[0], least[1]) > 0 && max(most[0], most[1]) < C::kBins;
-      if (all_counted) {
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-          if ((bits[u] >> j) & 1) atomicAdd(&bins[off[j / 2][j & 1]], 1u);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-          if ((bits[u] >> j) & 1) {
-            const int o = off[j / 2][j & 1];
-            if (o != top_number && o < C::kBins) {
-              atomicAdd(&bins[o], 1u);
-            } else {
-              const u64 w = mass(to_float(bit_cast<T>((unsigned short)(pair(raw[u], j / 2) >> (16 * (j & 1))))));
-              if (o == top_number) small += w;
-              else low += w;
-            }
-          }
-      }
+    });
+    const int image_max = (int)block_max((float)max(top[0], top[1]), s);
+    if (image_max <= (int)(0x7fffu - C::kInf)) {  // nothing allowed (or -inf alone): no distribution to draw from
+      if (tid == 0) *out = 0;
+      return true;
     }
+    const bool positive = (image_max & 0x8000) != 0;
+    const int top_mag = (positive ? image_max & 0x7fff : 0x7fff - image_max) - C::kLo;
+    if (image_max >= (0x8000 | C::kInf) || top_mag <= 0) return false;
+    top_number = positive ? top_mag : -top_mag;
+  } else {
+    __syncthreads();
   }
-  if (__syncthreads_or((small | low) != 0)) {  // (behind the barrier the counts are complete)
-    small = block_sum(small, s);
-    low = block_sum(low, s);
-  }
-  // Thread t owns counters [kOwn t, kOwn (t + 1)): thread order is descending order of the values.
+
+  // Tokens per value.
+  // Allowed ones of a small magnitude, or without a counter, are few, but every large batch has rows with some: listed.
+  for_groups([&](const uint4 &raw, unsigned bits) {
+    if (!__any((int)bits)) return;
+    u16x2 off[4], least = {0xffff, 0xffff}, most = {0, 0};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      u16x2 mag;
+      off[i] = (u16x2)(unsigned short)top_number - numbers(pair(raw, i), mag);
+      least = __builtin_elementwise_min(least, mag);
+      most = __builtin_elementwise_max(most, off[i]);
+    }
+    if (min(least[0], least[1]) > 0 && max(most[0], most[1]) < C::kBins) {
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        if ((bits >> j) & 1) atomicAdd(&bins[off[j / 2][j & 1]], 1u);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        if ((bits >> j) & 1) {
+          const int o = off[j / 2][j & 1];
+          if (o != top_number && o < C::kBins) atomicAdd(&bins[o], 1u);
+          else {
+            const int at = atomicAdd(&s.n_others, 1);
+            if (at < kThreads) s.others[at] = (uint16_t)(pair(raw, j / 2) >> (16 * (j & 1)));
+          }
+        }
+    }
+  });
+  __syncthreads();
+  const int others = s.n_others;
+
   auto bin_image = [&](int o) {
     const int number = top_number - o;  // 0: the small ones
     return (unsigned)(number >= 0 ? 0x8000 + number + C::kLo : 0x7fff + number - C::kLo);
   };
-  auto bin_mass = [&](int o) -> u64 {
-    if (o == top_number) return small;
-    const unsigned n = bins[o];
-    return n ? n * mass(value(bin_image(o))) : 0ull;
+  int largest = 0;  // counter of the row's largest value
+  if constexpr (C::kTop != 0) {
+    int found = C::kBins;
+#pragma unroll
+    for (int i = kOwn - 1; i >= 0; i--)
+      if (bins[kOwn * tid + i] != 0) found = kOwn * tid + i;
+    largest = C::kBins - (int)block_max((float)(C::kBins - found), s);
+    if (largest == C::kBins) {
+      if (others > 0) return false;
+      if (tid == 0) *out = 0;  // nothing allowed: no distribution to draw from
+      return true;
+    }
+    if (others > 0 && largest > top_number) return false;  // a small one may be the largest
+  }
+  if (!(temp < 1e15f)) return false;
+  const float m = value(bin_image(largest)) / temp;
+  if (!(fabsf(m) < INFINITY)) return false;
+  auto mass_f = [&](float v) {  // before it is cut to an integer
+    const float x = v / temp;
+    return x > -INFINITY ? __builtin_amdgcn_exp2f((x - m) * kLog2e) * kMassUnit : 0.f;
   };
+  auto mass = [&](float v) -> u64 { return (u64)mass_f(v); };
+  u64 small = 0, low = 0;  // mass of the small ones and of those below the counters
+  if (others > 0) {
+    bool above = false;
+    auto add = [&](unsigned b) {
+      const u64 w = mass(to_float(bit_cast<T>((unsigned short)b)));
+      if ((int)(b & 0x7fffu) <= C::kLo) small += w;
+      else if (b & 0x8000u) low += w;
+      else above = true;  // fixed counters only: beyond 2^16, infinite, or not a number
+    };
+    if (others <= kThreads) {
+      if (tid < others) add(s.others[tid]);
+    } else {
+      for_groups([&](const uint4 &raw, unsigned bits) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          u16x2 mag;
+          const u16x2 off = (u16x2)(unsigned short)top_number - numbers(pair(raw, i), mag);
+#pragma unroll
+          for (int k = 0; k < 2; k++)
+            if (((bits >> (2 * i + k)) & 1) && (mag[k] == 0 || off[k] >= C::kBins)) add((pair(raw, i) >> (16 * k)) & 0xffffu);
+        }
+      });
+    }
+    if (__syncthreads_or(above)) return false;
+    small = block_sum(small, s);
+    low = block_sum(low, s);
+  }
+  // Thread t owns counters [kOwn t, kOwn (t + 1)): thread order is descending order of the values.  From here on a counter holds
+  // the mass of one token of its value (a float), for the draw to look up.
+  unsigned count[kOwn];
   u64 own = 0;
-#pragma unroll 4
-  for (int i = 0; i < kOwn; i++) own += bin_mass(kOwn * tid + i);
+#pragma unroll
+  for (int i = 0; i < kOwn; i++) {
+    const int o = kOwn * tid + i;
+    count[i] = bins[o];
+    float f = 0.f;
+    if (count[i] != 0) f = mass_f(value(bin_image(o)));
+    bins[o] = __float_as_uint(f);
+    own += count[i] * (u64)f;
+    if (o == top_number) own += small;
+  }
   const u64 z = block_sum(own, s) + low + (top_number >= C::kBins ? small : 0ull);
   unsigned kstar = 0;  // image of the last kept value; below every image that is counted: everything is kept
   int n_keep = 0;
@@ -302,12 +356,16 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
     // exactly one thread's values cross the target (from below it to it or beyond), or none
     if (own && (before < target || (target == 0 && before == 0)) && before + own >= target) {
       u64 above = before;
+      bool found = false;
+#pragma unroll
       for (int i = 0; i < kOwn; i++) {
-        const u64 h = bin_mass(kOwn * tid + i);
-        if (h && above + h >= target) {
-          s.pick = kOwn * tid + i;
+        const int o = kOwn * tid + i;
+        const u64 h = o == top_number ? small : count[i] * (u64)__uint_as_float(bins[o]);
+        if (!found && h && above + h >= target) {
+          found = true;
+          s.pick = o;
           s.hist[0] = above;
-          break;
+          s.cnt[0] = count[i];
         }
         above += h;
       }
@@ -316,9 +374,9 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
     const int chosen = s.pick;
     if (chosen < 0 || chosen == top_number) return false;  // among the small or the low ones
     const u64 mass_gt = s.hist[0];
-    const unsigned ties = bins[chosen];
+    const unsigned ties = s.cnt[0];
     kstar = bin_image(chosen);
-    m_star = mass(value(kstar));
+    m_star = (u64)__uint_as_float(bins[chosen]);
     u64 need = (m_star && target > mass_gt) ? (target - mass_gt + m_star - 1) / m_star : 1;
     if (need < 1) need = 1;
     if (need > ties) need = ties;
@@ -326,27 +384,30 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
     total = mass_gt + (u64)n_keep * m_star;
   }
 
+  __syncthreads();  // every counter holds its mass
   // The draw, in id order: mass and ties per wavefront, then all share the tokens of the one that holds the winner.
   const float u01 = fminf(fmaxf(uniform, 0.f), 1.f);  // outside [0, 1): the first or the last kept token
   u64 c = (u64)((double)u01 * (double)total);
   if (c >= total) c = total - 1;  // u * total rounded up to the total itself: the last token with a weight
   // bit j: token j of the group is above kstar / equal to it
   auto kept = [&](const uint4 &raw, unsigned bits, unsigned &ties) {
-    unsigned gt = 0;
-    ties = 0;
+    unsigned gt = 0, other = 0;  // first bits 2i (even tokens) and 16 + 2i (odd ones)
+    const u16x2 limit = (u16x2)(unsigned short)kstar, one = {1, 1};
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const unsigned w = images(pair(raw, i));
-      const unsigned lo = w & 0xffffu, hi = w >> 16;
-      gt |= (lo > kstar ? 1u << (2 * i) : 0u) | (hi > kstar ? 2u << (2 * i) : 0u);
-      ties |= (lo == kstar ? 1u << (2 * i) : 0u) | (hi == kstar ? 2u << (2 * i) : 0u);
+      const u16x2 w = bit_cast<u16x2>(images(pair(raw, i)));
+      gt |= bit_cast<unsigned>(__builtin_elementwise_min(__builtin_elementwise_sub_sat(w, limit), one)) << (2 * i);
+      other |= bit_cast<unsigned>(__builtin_elementwise_min((u16x2)(w ^ limit), one)) << (2 * i);
     }
-    ties = n_keep > 0 ? ties & bits : 0u;
-    return gt & bits;
+    ties = n_keep > 0 ? ~(other | other >> 15) & 0xffu & bits : 0u;
+    return (gt | gt >> 15) & 0xffu & bits;
   };
   auto token_mass = [&](const uint4 &raw, int j) {
-    const unsigned w = pair(raw, j >> 1);
-    return mass(to_float(bit_cast<T>((unsigned short)(w >> (16 * (j & 1))))));
+    const unsigned b = (pair(raw, j >> 1) >> (16 * (j & 1))) & 0xffffu;
+    const int mag = (int)(b & 0x7fffu) - C::kLo;
+    const int o = top_number - ((b & 0x8000u) ? -mag : mag);
+    if (mag > 0 && (unsigned)o < (unsigned)C::kBins) return (u64)__uint_as_float(bins[o]);
+    return mass(to_float(bit_cast<T>((unsigned short)b)));
   };
   auto mass_of = [&](const uint4 &raw, unsigned gt) {
     u64 sum = 0;
@@ -359,19 +420,12 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
   };
   u64 my_gt = 0;
   int my_ties = 0;
-  for (int base = g0; base < g1; base += 64 * U) {
-    uint4 raw[U];
-    unsigned bits[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) load(base + u * 64 + lane, g1, raw[u], bits[u]);
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      unsigned ties;
-      const unsigned gt = kept(raw[u], bits[u], ties);
-      my_gt += mass_of(raw[u], gt);
-      my_ties += __builtin_popcount(ties);
-    }
-  }
+  for_groups([&](const uint4 &raw, unsigned bits) {
+    unsigned ties;
+    const unsigned gt = kept(raw, bits, ties);
+    my_gt += mass_of(raw, gt);
+    my_ties += __builtin_popcount(ties);
+  });
   my_gt = wave_sum(my_gt);
   my_ties = (int)wave_sum((u64)my_ties);
   __syncthreads();
