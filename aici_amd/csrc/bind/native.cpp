@@ -298,11 +298,13 @@ PyObject *copy_blocks(PyObject *, PyObject *const *args, Py_ssize_t n) {
       ptrs[side].push_back(d.data);
     }
   }
-  if (bytes <= 0 || bytes % 16 != 0 || ptrs[0].size() != ptrs[1].size() || ptrs[0].empty()) Py_RETURN_FALSE;
+  if (bytes <= 0 || bytes % 16 != 0 || bytes > (1 << 26) || ptrs[0].size() != ptrs[1].size() || ptrs[0].empty()) Py_RETURN_FALSE;
   const Py_ssize_t count = PySequence_Fast_GET_SIZE(held[2]);
   std::vector<int64_t> pairs((size_t)count);
   for (Py_ssize_t i = 0; i < count; i++)
     if (!to_i64(PySequence_Fast_GET_ITEM(held[2], i), &pairs[(size_t)i])) return nullptr;
+  for (int64_t b : pairs)
+    if (b < INT32_MIN || b > INT32_MAX) Py_RETURN_FALSE;
   void *stream = nullptr;
   if (g_exchange->current_work_stream((DLDeviceType)c.device_type, c.device, &stream) != 0) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "no current stream");

@@ -241,9 +241,10 @@ char *hipattn_copy_blocks_2(const hipattn_tensor *key_cache_ptrs,
 
 /* The same from host arrays: the caches' base addresses of every layer and the
  * (src,dst) pairs are read before the call returns and travel as arguments of
- * the launches (64 layers x 128 pairs each), so that no upload goes in front
+ * the launches (64 layers x 256 pairs each), so that no upload goes in front
  * of the copy and the call may be captured.  Caches must start on 16-byte
- * boundaries and bytes_per_block be a multiple of 16. */
+ * boundaries, bytes_per_block be a multiple of 16 (at most 64 MiB) and block
+ * numbers fit 32 bits. */
 char *hipattn_copy_blocks_host(void *const *key_caches, void *const *value_caches,
                                int64_t layers, const int64_t *block_mapping,
                                int64_t n_pairs, int64_t bytes_per_block,

@@ -146,7 +146,7 @@ def test_tiles_start_at_any_token(device, bs, d, H, T):
     assert torch.equal(bits(ko), bits(want_k)) and torch.equal(bits(vo), bits(want_v))
 
 
-@pytest.mark.parametrize("layers,pairs,d", [(1, 1, 8), (3, 129, 64), (65, 2, 80), (2, 0, 64)])
+@pytest.mark.parametrize("layers,pairs,d", [(1, 1, 8), (3, 257, 64), (65, 2, 80), (130, 3, 8), (2, 0, 64)])
 def test_copy_blocks_with_more_than_one_launch_holds(device, layers, pairs, d):
     """Layers and pairs beyond what one launch's arguments hold; and the former entry point, from device arrays."""
     g = torch.Generator().manual_seed(layers + pairs)
