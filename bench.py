@@ -511,9 +511,8 @@ def llama_step_leg(dev, stream, steps: int, layers: int, share_cache: bool) -> d
     """One full engine step of a Llama-3-8B-shaped model (random weights): 128 sequences decoding
     one token each over contexts U[1024,16384] (seed 5), every layer with its own paged KV cache,
     then the AICI step (5 % of the vocabulary allowed per sequence, packed bit masks) and greedy
-    arg-max.  q/k/v, gate/up and lm_head are library GEMMs; o_proj and down_proj (few rows of the weight: a
-    library GEMM leaves most of the device idle) and everything else run through the C ABI.
-    `ms_per_step_library_gemms_only` is the same step with those two projections as library GEMMs as well."""
+    arg-max.  lm_head is a library GEMM at this many sequences; every other projection and everything else run
+    through the C ABI.  `ms_per_step_library_gemms_only` is the same step with every projection a library GEMM."""
     import numpy as np
     import torch
 
