@@ -225,7 +225,9 @@ __global__ __launch_bounds__(256) void cache_move_run8_kernel(
 //
 // A tile is 16 consecutive tokens that fill 16 consecutive slots from a multiple of 16 on.  The sequences of a batch lie
 // end to end, so tiles start at any token: a wavefront takes the tile that starts among its 16 tokens, wherever it ends, and the
-// tokens of its own that belong to no tile (ends of sequences, decode rows) one by one, eight at a time.  Tiles cut at
+// tokens of its own that belong to no tile (ends of sequences, decode rows) one by one, eight at a time -- or, below 1024
+// tokens, leaves them to workgroups of their own behind the tiles', one per token (128 decode rows x 8 heads x 128: 3.7 us a
+// token per workgroup alone, 6.4 eight at a time, 3.8 so; from 1024 tokens on eight at a time is as fast).  Tiles cut at
 // multiples of 16 of the token index (as before) fit the first sequence of a ragged batch only.
 //
 // us, before -> now (fp16): 1375 tokens of 4 sequences x 32 heads x 128 27 -> 9.3, 40012 tokens of 32 sequences x 2 heads x 64 34.7 -> 11.0,
@@ -235,9 +237,29 @@ __global__ __launch_bounds__(256) void cache_move_tile_kernel(
     uint16_t *__restrict__ key, uint16_t *__restrict__ value, uint16_t *__restrict__ key_cache,
     uint16_t *__restrict__ value_cache, const Slot *__restrict__ slot_mapping, int64_t num_tokens,
     int64_t key_tok_stride, int64_t key_head_stride, int64_t val_tok_stride,
-    int64_t val_head_stride, CacheGeom g, int items_per_wave, int waves_per_group) {
+    int64_t val_head_stride, CacheGeom g, int items_per_wave, int waves_per_group, int tile_wgs) {
   typedef uint16_t E;
   constexpr int X = 8;
+  if ((int)blockIdx.x >= tile_wgs) {  // a token that is in no tile
+    const int64_t token = blockIdx.x - tile_wgs;
+    const int64_t slot = (int64_t)slot_mapping[token];
+    if (slot < 0 || slot / g.block_size >= g.num_blocks) return;
+    const int64_t first = token - slot % 16;  // where its tile would start
+    const int l = threadIdx.x & 15;
+    const bool there = first >= 0 && first + 15 < num_tokens && (int64_t)slot_mapping[first + l] == slot - slot % 16 + l;
+    if (__all(there)) return;
+    const int64_t blk = slot / g.block_size;
+    const int off = (int)(slot % g.block_size), chunks = g.head_size / X;
+    for (int i = threadIdx.x; i < g.num_heads * chunks; i += 256) {
+      const int h = i / chunks, c = i % chunks;
+      move_token_chunk<E, SCATTER>(key + token * key_tok_stride + h * key_head_stride + c * X,
+                                   value + token * val_tok_stride + h * val_head_stride + c * X,
+                                   key_cache + blk * g.k_block_stride + h * g.k_head_stride + ((int64_t)c * g.block_size + off) * X,
+                                   value_cache + blk * g.v_block_stride + h * g.v_head_stride + (int64_t)c * X * g.block_size + off,
+                                   g.block_size);
+    }
+    return;
+  }
   constexpr int KP = 72;  // K slab row pitch in elements: 8 chunks + 16 bytes, keeps the transposed 16-byte reads apart
   constexpr int VP = 64;  // V slab row pitch: the 2-byte column accesses of a wavefront fall in one row
   __shared__ __attribute__((aligned(16))) E slab[4][16 * KP + 16 * VP];
@@ -265,7 +287,7 @@ __global__ __launch_bounds__(256) void cache_move_tile_kernel(
   const unsigned later = starts & 0xffff0000u;
   unsigned owned = ~0u << __builtin_ctz(own_starts);
   if (later != 0) owned &= (1u << __builtin_ctz(later)) - 1u;
-  unsigned rest = owned & valid;
+  unsigned rest = (int)gridDim.x > tile_wgs ? 0u : owned & valid;
   const int tile_at = tile != 0 ? __builtin_ctz(tile) : 0;
   if (tile != 0) rest &= ~(0xffffu << tile_at);
   const int64_t tile_slot = ((int64_t)__builtin_amdgcn_readlane((int)(slot >> 32), tile_at) << 32) |
@@ -530,7 +552,10 @@ void launch_move(const hipattn_tensor *key, const hipattn_tensor *value,
   if constexpr (sizeof(E) == 2) {
     // prompts (and whatever comes with them): the transposing kernels
     const bool vec_v = vec && g.block_size % 8 == 0 && aligned16(vc) && g.v_block_stride % 8 == 0 && g.v_head_stride % 8 == 0;
-    if (vec_v && T >= 128 && g.block_size % 16 == 0 && tuning().cache_move_lds != 0) {
+    // (few tokens of narrow rows are launch-bound either way: 128 .. 1000 prompt tokens x 2 heads x 64 2.5 .. 3.5 us a token per
+    // workgroup, 2.9 .. 3.2 by tiles)
+    if (vec_v && T >= 128 && (T >= 1024 || g.num_heads * g.head_size > 256) && g.block_size % 16 == 0 &&
+        tuning().cache_move_lds != 0) {
       // One item (a head's 64 elements of 16 tokens) per wavefront while that is no more than 32 wavefronts per compute unit, up
       // to eight beyond (the slots are looked at once per wavefront).
       const int64_t groups = (T + 15) / 16;
@@ -545,16 +570,17 @@ void launch_move(const hipattn_tensor *key, const hipattn_tensor *value,
       const int items = gt.num_heads * ((gt.head_size / X + 7) / 8);
       const int per_wave = (int)std::min<int64_t>(8, std::max<int64_t>(1, groups * items / 8192));
       const int waves_per_group = (items + per_wave - 1) / per_wave;
-      const dim3 tiles((unsigned)((groups * waves_per_group + 3) / 4));
+      const int tile_wgs = (int)((groups * waves_per_group + 3) / 4);
+      const dim3 tiles((unsigned)(tile_wgs + (T < 1024 ? T : 0)));
       // head sizes that are multiples of 64 have no partial chunk group: their instance carries no guards
       if (gt.head_size % 64 == 0)
         cache_move_tile_kernel<Slot, SCATTER, true><<<tiles, 256, 0, stream>>>(
             kp, vp, kc, vc, sp, T, key->strides[0], key->strides[1], value->strides[0], value->strides[1], gt, per_wave,
-            waves_per_group);
+            waves_per_group, tile_wgs);
       else
         cache_move_tile_kernel<Slot, SCATTER, false><<<tiles, 256, 0, stream>>>(
             kp, vp, kc, vc, sp, T, key->strides[0], key->strides[1], value->strides[0], value->strides[1], gt, per_wave,
-            waves_per_group);
+            waves_per_group, tile_wgs);
       check_launch(SCATTER ? "reshape_and_cache" : "gather_cached_kv");
       return;
     }

@@ -114,8 +114,8 @@ def test_long_inputs_runs_of_tokens_mixed_with_everything_else(device, dtype, st
     assert torch.equal(bits(ko), bits(want_k)) and torch.equal(bits(vo), bits(want_v))
 
 
-@pytest.mark.parametrize("bs,d,H", [(16, 128, 3), (16, 80, 2), (32, 64, 1), (48, 8, 5), (16, 64, 2)])
-@pytest.mark.parametrize("T", [127, 128, 129, 160, 300, 1023])
+@pytest.mark.parametrize("bs,d,H", [(16, 128, 3), (16, 80, 4), (32, 64, 5), (48, 8, 40), (16, 64, 2)])
+@pytest.mark.parametrize("T", [127, 128, 129, 160, 300, 1023, 1024])
 def test_tiles_start_at_any_token(device, bs, d, H, T):
     """Batches of short sequences laid end to end: their full rows of 16 slots start at every token index modulo 16, next to
     single tokens, beginnings in the middle of a block, ends, padding slots and slots past the cache."""
