@@ -255,9 +255,9 @@ class BatchInfo:
     multi_context_lens: Optional[torch.Tensor] = None
 
     def to(self, device) -> "BatchInfo":
-        """The batch with its arrays on `device`.  On the way from the host to a GPU all of them travel as one copy:
-        a pageable copy per array costs some 12 us and waits for the stream each time, and a step has ten of them.
-        The staging buffer is torch's pinned memory, which goes back to its pool once the copy has run."""
+        """The batch with its arrays on `device`, there when the call returns: they may be used on any stream.  On the way
+        from the host to a GPU all of them travel as one copy, waited for once: a pageable copy per array costs some
+        12 us, the wait included, and a step has ten of them."""
         device = torch.device(device)
         tensors = {k: v for k, v in self.__dict__.items() if isinstance(v, torch.Tensor)}
         kw = dict(self.__dict__)
@@ -274,7 +274,7 @@ class BatchInfo:
             if w:
                 host[at:at + w] = v.numpy().reshape(-1).view(np.int32)
             at += p
-        parts = staged.to(device, non_blocking=True).split(padded)
+        parts = staged.to(device).split(padded)  # waits for the copy
         for (k, v), w, part in zip(tensors.items(), words, parts):
             if w != part.numel():
                 part = part[:w]

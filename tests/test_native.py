@@ -28,6 +28,34 @@ def _batch(lens):
     return b.finish()
 
 
+def test_batch_upload_waits_for_its_copy(monkeypatch):
+    """No array may still be on its way when `to` returns: a caller uploads on one stream and runs the model on another."""
+    asked = []
+    empty = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, pin_memory=False, **kw: empty(*a, **kw))  # no pinned memory without a GPU
+    monkeypatch.setattr(torch.Tensor, "to", lambda t, *a, **kw: asked.append((a, kw)) or t.clone())
+    got = _batch([(37, 0), (5, 4)]).to("cuda")
+    assert len(asked) == 1 and got.slot_mapping.numel() == 38
+    (args, kw), = asked
+    assert not kw.get("non_blocking", False) and not any(a is True for a in args)
+
+
+@pytest.mark.gpu
+def test_batch_uploaded_behind_queued_work_is_there_for_other_streams(device):
+    host = _batch([(37, 0), (5, 4), (300, 299)])
+    a = torch.randn((4096, 4096), device=device)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(20):  # some milliseconds in front of the upload
+            a @ a
+        dev = host.to(device)
+    for name, want in host.__dict__.items():  # read on the default stream, which waits for nothing
+        if isinstance(want, torch.Tensor):
+            assert torch.equal(getattr(dev, name).clone().cpu(), want), name
+    side.synchronize()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("lens", [[(1, 0)], [(37, 0), (5, 4), (100, 99)], [(64, 17)], [(3, 2), (300, 299)]])
 def test_batch_upload_keeps_every_array(device, lens):
