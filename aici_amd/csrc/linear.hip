@@ -490,7 +490,7 @@ struct LinearPlan {
   int waves;    // tile kernel: wavefronts per workgroup
   int splits;   // ranges of k
   int stages_per_split;
-  size_t partial_bytes;
+  size_t partial_bytes;  // fp32 sums of every range, [range][128 rows][N]; not used by the few-rows kernel
 };
 
 // The ranges of k depend on the weight alone (see above).  At least 1024 wavefronts' worth of (16 rows, range) pairs, four per
@@ -514,7 +514,7 @@ LinearPlan plan_linear(int M, int N, int K) {
   pl.waves = ((int64_t)((N + 63) / 64) * splits <= 256 || (splits == 1 && M <= 32)) ? 4 : 8;
   if (tn.linear_tiles > 0) pl.waves = 4 * tn.linear_tiles;
   if (tn.linear_waves > 0) pl.waves = tn.linear_waves;
-  pl.partial_bytes = pl.splits > 1 && !pl.stream ? (size_t)pl.splits * (N / 16) * kLinMT * 64 * sizeof(f32x4_t) : 0;
+  pl.partial_bytes = (size_t)pl.splits * kLinMaxRows * N * sizeof(float);
   return pl;
 }
 
@@ -599,10 +599,9 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
   LinearPlan pl = plan_linear((int)M, (int)N, (int)K);
   const int64_t outputs = gated ? N / 2 : N;
   const bool with_norm = norm_out != nullptr || ws_query_with_norm;
-  // rows of sums for the norm: [range][128 rows][N] fp32 -- the size the tiles of sums take as well.  (The few-rows kernel leaves
-  // finished rows: a launch of rms_norm normalises them.)
-  if (with_norm && !pl.stream) pl.partial_bytes = (size_t)pl.splits * kLinMaxRows * (size_t)N * sizeof(float);
-  if (ws_query != nullptr) {
+  // the norm's launch takes rows of sums, however few the ranges
+  if (pl.splits == 1 && !with_norm) pl.partial_bytes = 0;
+  if (ws_query != nullptr) {  // whatever the rows of x: a buffer sized with one serves a step of 128
     *ws_query = (int64_t)pl.partial_bytes;
     return;
   }
@@ -682,7 +681,7 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
   p.total_stages = (int)(K / kLinStageK);
   p.half = gated ? (int)(N / 2) : 0;
   hipStream_t stream = resolve_stream(stream_arg);
-  if (pl.partial_bytes > 0) {
+  if (pl.partial_bytes > 0 && !pl.stream) {  // (the few-rows kernel leaves finished rows: a launch of rms_norm normalises them)
     if (workspace != nullptr) {
       check_tensor(workspace, "workspace", 1);
       HA_CHECK(workspace->dtype == HIPATTN_U8 && workspace->strides[0] == 1, "linear: workspace must be contiguous u8");

@@ -316,12 +316,13 @@ char *hipattn_fused_add_rms_norm(hipattn_tensor *input,
  * prompt).  Rounding: fp32 sums over K, + bias in fp32, rounded to the data
  * type; with a residual, that value + residual rounded again (the separate
  * addition of llama.rs:166, 173).  The same bits on every run.  When weight has
- * too few rows to occupy the device the inner dimension is split between
- * workgroups and a second launch adds the parts, in fp32, from `workspace`
- * (u8, hipattn_linear_workspace_size bytes; 0 when no split is needed) or,
- * when that is NULL, from a scratch buffer that the library keeps per stream
- * (with what hipattn_paged_attention_v1 says about captures and overlapping
- * calls). */
+ * too few rows to occupy the device the inner dimension is split, and from 17
+ * rows of x on a second launch adds the parts, in fp32, from `workspace` (u8,
+ * hipattn_linear_workspace_size bytes: a function of weight alone, 0 when no
+ * split is needed, so that a buffer sized with any number of rows serves every
+ * other) or, when that is NULL, from a scratch buffer that the library keeps
+ * per stream (with what hipattn_paged_attention_v1 says about captures and
+ * overlapping calls).  Up to 16 rows take one launch and no workspace. */
 char *hipattn_linear(hipattn_tensor *out, const hipattn_tensor *x,
                      const hipattn_tensor *weight, const hipattn_tensor *bias,
                      const hipattn_tensor *residual,
@@ -337,17 +338,18 @@ char *hipattn_linear_silu_and_mul(hipattn_tensor *out, const hipattn_tensor *x,
                                   const hipattn_tensor *weight,
                                   const hipattn_tensor *workspace, void *stream);
 
-/* hipattn_linear followed by the RMS norm of the finished rows, in the launch
- * that adds up the ranges of the inner dimension: out = x . weight^T (+ bias)
- * (+ residual) as above, norm_out = rms_norm(out, norm_weight, epsilon) with the
+/* hipattn_linear followed by the RMS norm of the finished rows, from 17 rows of
+ * x on in the launch that adds up the ranges of the inner dimension, below in
+ * a launch of its own: out = x . weight^T (+ bias) (+ residual) as above, norm_out = rms_norm(out, norm_weight, epsilon) with the
  * arithmetic of hipattn_rms_norm -- the same bits as the two calls one after
  * the other.  It is the pair that closes every residual branch of the decoder
  * (llama.rs:166 + 169, 173 + 165 of the next block, 173 + 207), with no
  * counterpart of its own in the reference's extern "C" block.  Operands as
  * for hipattn_linear, and: N a multiple of 8, at most 8192; norm_weight [N],
  * norm_out [M, N]; rows of out, norm_out and residual on 16-byte boundaries.
- * The workspace (hipattn_linear_rms_norm_workspace_size bytes, or the
- * library's per-stream scratch when NULL) is used whatever the shape. */
+ * The workspace (hipattn_linear_rms_norm_workspace_size bytes, a function of
+ * weight alone, or the library's per-stream scratch when NULL) is used
+ * whatever the weight, from 17 rows of x on. */
 char *hipattn_linear_rms_norm(hipattn_tensor *out, hipattn_tensor *norm_out,
                               const hipattn_tensor *x,
                               const hipattn_tensor *weight,

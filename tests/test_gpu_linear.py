@@ -145,6 +145,19 @@ def test_workspace_from_the_caller(device):
     assert K.linear_workspace_size(xd, wd) == 0
 
 
+def test_workspace_sized_with_one_row_serves_every_batch(device):
+    x, w, _ = operands(128, 4096, 4096, torch.bfloat16, seed=43)
+    xd, wd = x.to(device), w.to(device)
+    nw = torch.ones((4096,), dtype=torch.bfloat16, device=device)
+    ws = torch.empty((K.linear_workspace_size(xd[:1], wd),), dtype=torch.uint8, device=device)
+    ws_norm = torch.empty((K.linear_rms_norm_workspace_size(xd[:1], wd),), dtype=torch.uint8, device=device)
+    for m in (1, 16, 17, 128):
+        want, want_n = K.linear_rms_norm(xd[:m], wd, nw, 1e-5)
+        assert torch.equal(K.linear(xd[:m], wd, workspace=ws), want)
+        out, normed = K.linear_rms_norm(xd[:m], wd, nw, 1e-5, workspace=ws_norm)
+        assert torch.equal(out, want) and torch.equal(normed, want_n)
+
+
 @pytest.mark.parametrize("splits", [0, 1, 3, 8])
 def test_linear_rms_norm_gives_the_bits_of_the_two_calls(device, splits):
     K.tuning_set("linear_splits", splits)

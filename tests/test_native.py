@@ -1,8 +1,10 @@
 """The CPython binding of the hot entry points (csrc/bind/native.cpp) and the one-copy upload of a batch."""
+import ctypes
+
 import pytest
 import torch
 
-from aici_amd import _lib, _native, paged
+from aici_amd import _lib, _native, kernels, paged
 
 
 def test_arguments_are_checked_before_the_call():
@@ -17,6 +19,20 @@ def test_arguments_are_checked_before_the_call():
         _native.rms_norm(x)
     with pytest.raises(_lib.HipAttnError, match="hipattn_reshape_and_cache: .*NULL"):
         _native.reshape_and_cache(None, None, None, None, None)
+
+
+@pytest.mark.parametrize("fn", ["hipattn_linear_workspace_size", "hipattn_linear_rms_norm_workspace_size"])
+@pytest.mark.parametrize("shape", [(4096, 14336), (6144, 4096), (16, 256), (512, 512)])
+def test_linear_workspace_depends_on_the_weight_alone(fn, shape):
+    """An engine asks once, with whatever batch it has then.  (Descriptors of host tensors do: nothing is read.)"""
+    desc = lambda t: kernels._desc(t, device=False)
+    sizes = set()
+    for m in (1, 16, 17, 128):
+        n = ctypes.c_int64(-1)
+        _lib.call(fn, desc(torch.empty((m, shape[1]), dtype=torch.bfloat16)), desc(torch.empty(shape, dtype=torch.bfloat16)),
+                  ctypes.byref(n))
+        sizes.add(n.value)
+    assert len(sizes) == 1 and sizes.pop() > 0
 
 
 def _batch(lens):
