@@ -62,6 +62,7 @@ struct LinearParams {
   // with an RMS norm behind the layer: the sums go to the workspace as rows ([range][128 rows][N] fp32), and the
   // launch that adds them up also normalises the finished row
   int row_sums;
+  int tile_sums;  // the sums go to the workspace as tiles, and a second launch finishes them
   const void *norm_w;
   void *norm_out;
   int64_t ldn;
@@ -366,7 +367,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_tile_kernel(const LinearPar
         if (mt < p.mtiles)
           *reinterpret_cast<f32x4_t *>(p.partial + ((int64_t)split * kLinMaxRows + mt * 16 + col) * p.N + n) = acc[mt];
     }
-  } else if (p.splits > 1) {
+  } else if (p.tile_sums) {
     if (n_tile < n_end) {
       const int nt = (part * p.half + n_tile) / 16;
       f32x4_t *dst = reinterpret_cast<f32x4_t *>(p.partial) + ((int64_t)(split * (p.N / 16) + nt) * kLinMT) * 64 + lane;
@@ -568,7 +569,7 @@ void launch_linear(const LinearParams &p, const LinearPlan &pl, hipStream_t stre
     if (threads > 1024) threads = 1024;  // (the entry point bounds N)
     hipLaunchKernelGGL((linear_reduce_norm_kernel<T>), dim3((unsigned)p.M), dim3((unsigned)threads), 0, stream, p);
     check_launch("linear (sum of the ranges + rms_norm)");
-  } else if (pl.splits > 1) {
+  } else if (p.tile_sums) {
     const int64_t threads = (int64_t)((GATED ? p.half : p.N) / 16) * p.mtiles * 64;
     hipLaunchKernelGGL((linear_reduce_kernel<T, GATED>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, p);
     check_launch("linear (sum of the ranges)");
@@ -576,6 +577,23 @@ void launch_linear(const LinearParams &p, const LinearPlan &pl, hipStream_t stre
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+// Whether rows of two 2-byte matrices may share memory.  Column ranges of one wider matrix lie between each other without.
+bool rows_overlap(const hipattn_tensor *a, const hipattn_tensor *b) {
+  struct Span {
+    int64_t lo, hi;  // bytes, hi past the end
+  };
+  auto span = [](const hipattn_tensor *t) {
+    const int64_t at = (int64_t)reinterpret_cast<uintptr_t>(t->data), reach = (t->sizes[0] - 1) * t->strides[0] * 2;
+    return Span{at + (reach < 0 ? reach : 0), at + (reach > 0 ? reach : 0) + t->sizes[1] * 2};
+  };
+  const Span sa = span(a), sb = span(b);
+  if (sa.hi <= sb.lo || sb.hi <= sa.lo) return false;
+  const int64_t ld = a->strides[0] * 2, off = (int64_t)reinterpret_cast<uintptr_t>(b->data) - (int64_t)reinterpret_cast<uintptr_t>(a->data);
+  if (ld <= 0 || a->strides[0] != b->strides[0]) return true;
+  const int64_t within = ((off % ld) + ld) % ld;  // where b's columns start in a's rows
+  return within < a->sizes[1] * 2 || within + b->sizes[1] * 2 > ld;
+}
 
 // With `norm_out` the RMS norm of the finished rows (weight `norm_weight`, `eps`) is written there by the launch
 // that adds up the ranges' sums; the workspace is then needed whatever the number of ranges.
@@ -619,6 +637,14 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
            "linear: rows of x and weight must start on 16-byte boundaries");
   HA_CHECK(out->strides[0] % 4 == 0 && (reinterpret_cast<uintptr_t>(out->data) & 7) == 0,
            "linear: rows of out must start on 8-byte boundaries");
+
+  // Output rows over rows of x: both kernels write while other workgroups still read x, so every row of sums goes to the workspace
+  // and a second launch finishes it.
+  const bool overlap = rows_overlap(x, out);
+  if (overlap) {
+    pl.stream = false;
+    pl.partial_bytes = (size_t)pl.splits * kLinMaxRows * N * sizeof(float);
+  }
 
   // offsets between eight rows are 32 bits
   HA_CHECK(weight->strides[0] >= 0 && weight->strides[0] < (1 << 28) && x->strides[0] >= 0 && x->strides[0] < (1 << 28),
@@ -676,6 +702,7 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
     p.ldn = norm_out->strides[0];
     p.eps = eps;
   }
+  p.tile_sums = !pl.stream && !p.row_sums && (pl.splits > 1 || overlap);
   p.splits = pl.splits;
   p.stages_per_split = pl.stages_per_split;
   p.total_stages = (int)(K / kLinStageK);

@@ -322,7 +322,10 @@ char *hipattn_fused_add_rms_norm(hipattn_tensor *input,
  * split is needed, so that a buffer sized with any number of rows serves every
  * other) or, when that is NULL, from a scratch buffer that the library keeps
  * per stream (with what hipattn_paged_attention_v1 says about captures and
- * overlapping calls).  Up to 16 rows take one launch and no workspace. */
+ * overlapping calls).  Up to 16 rows take one launch and no workspace.  out
+ * may lie over x, in this call and in the two below: the sums then go through
+ * the workspace whatever the shape (splits x 128 x N x 4 bytes; a caller's own
+ * that is smaller is refused). */
 char *hipattn_linear(hipattn_tensor *out, const hipattn_tensor *x,
                      const hipattn_tensor *weight, const hipattn_tensor *bias,
                      const hipattn_tensor *residual,

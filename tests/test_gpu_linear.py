@@ -3,6 +3,7 @@ the oracle's fp64 product, on the projection shapes of the configured models and
 import pytest
 import torch
 
+from aici_amd import _native
 from aici_amd import kernels as K
 from aici_amd._lib import HipAttnError
 from oracle import refkernels as ref
@@ -143,6 +144,40 @@ def test_workspace_from_the_caller(device):
         K.linear(xd, wd, workspace=ws[: need - 256])
     K.tuning_set("linear_splits", 1)
     assert K.linear_workspace_size(xd, wd) == 0
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 128])
+@pytest.mark.parametrize("N", [512, 4096, 16384])  # the last: k is not cut
+def test_output_over_the_input(device, M, N):
+    """out = x's own memory, shifted against it, and between its rows."""
+    Kd = 512
+    x, w, g = operands(M, N, Kd, torch.bfloat16, seed=M + N)
+    wd = w.to(device)
+    want = K.linear(x.to(device), wd)
+    nw = torch.ones((N,), dtype=torch.bfloat16, device=device)
+    want_n = torch.empty_like(want)
+    if N <= 8192:
+        K.rms_norm(want_n, want, nw, 1e-5)
+    for at, ld in [(0, N), (64, N + 64), (Kd, N + Kd)]:  # the last: out's columns behind x's, in the same rows
+        def buffer():
+            buf = torch.zeros((M * ld + 64 + N,), dtype=torch.bfloat16, device=device)
+            xv = buf.as_strided((M, Kd), (ld, 1))
+            xv.copy_(x)
+            return xv, buf.as_strided((M, N), (ld, 1), at)
+        xv, out = buffer()
+        assert torch.equal(K.linear(xv, wd, out=out), want)
+        if at == Kd:
+            assert torch.equal(xv.cpu(), x)
+        if N <= 8192 and at != Kd:
+            xv, out = buffer()
+            normed = torch.empty_like(want)
+            _native.linear_rms_norm(out, normed, xv, wd, None, None, nw, 1e-5, None)
+            assert torch.equal(normed, want_n)
+            assert torch.equal(out, want)
+        xv, out = buffer()
+        half = out[:, : N // 2]
+        _native.linear_silu_and_mul(half, xv, wd, None)
+        assert torch.equal(half, K.linear_silu_and_mul(x.to(device), wd))
 
 
 def test_workspace_sized_with_one_row_serves_every_batch(device):
