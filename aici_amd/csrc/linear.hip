@@ -696,6 +696,9 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
                  aligned16(norm_weight->data) && (bias == nullptr || aligned16(bias->data)) &&
                  (residual == nullptr || (residual->strides[0] % 8 == 0 && aligned16(residual->data))),
              "linear_rms_norm: rows of out, norm_out and residual, and bias and norm_weight, must start on 16-byte boundaries");
+    // The launch of rms_norm behind the few-rows kernel takes rows that lie end to end; other rows (a slice of a wider matrix) go the
+    // way of larger batches, with the same bits.
+    if (!is_contiguous(out) || !is_contiguous(norm_out)) pl.stream = false;
     p.row_sums = pl.stream ? 0 : 1;
     p.norm_w = norm_weight->data;
     p.norm_out = norm_out->data;

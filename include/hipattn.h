@@ -342,8 +342,8 @@ char *hipattn_linear_silu_and_mul(hipattn_tensor *out, const hipattn_tensor *x,
                                   const hipattn_tensor *workspace, void *stream);
 
 /* hipattn_linear followed by the RMS norm of the finished rows, from 17 rows of
- * x on in the launch that adds up the ranges of the inner dimension, below in
- * a launch of its own: out = x . weight^T (+ bias) (+ residual) as above, norm_out = rms_norm(out, norm_weight, epsilon) with the
+ * x on (and for rows of out or norm_out that lie apart) in the launch that adds
+ * up the ranges of the inner dimension, below in a launch of its own: out = x . weight^T (+ bias) (+ residual) as above, norm_out = rms_norm(out, norm_weight, epsilon) with the
  * arithmetic of hipattn_rms_norm -- the same bits as the two calls one after
  * the other.  It is the pair that closes every residual branch of the decoder
  * (llama.rs:166 + 169, 173 + 165 of the next block, 173 + 207), with no
@@ -352,7 +352,7 @@ char *hipattn_linear_silu_and_mul(hipattn_tensor *out, const hipattn_tensor *x,
  * norm_out [M, N]; rows of out, norm_out and residual on 16-byte boundaries.
  * The workspace (hipattn_linear_rms_norm_workspace_size bytes, a function of
  * weight alone, or the library's per-stream scratch when NULL) is used
- * whatever the weight, from 17 rows of x on. */
+ * whatever the weight, from 17 rows of x on and for rows that lie apart. */
 char *hipattn_linear_rms_norm(hipattn_tensor *out, hipattn_tensor *norm_out,
                               const hipattn_tensor *x,
                               const hipattn_tensor *weight,

@@ -168,7 +168,7 @@ def test_output_over_the_input(device, M, N):
         assert torch.equal(K.linear(xv, wd, out=out), want)
         if at == Kd:
             assert torch.equal(xv.cpu(), x)
-        if N <= 8192 and at != Kd:
+        if N <= 8192:
             xv, out = buffer()
             normed = torch.empty_like(want)
             _native.linear_rms_norm(out, normed, xv, wd, None, None, nw, 1e-5, None)
@@ -191,6 +191,23 @@ def test_workspace_sized_with_one_row_serves_every_batch(device):
         assert torch.equal(K.linear(xd[:m], wd, workspace=ws), want)
         out, normed = K.linear_rms_norm(xd[:m], wd, nw, 1e-5, workspace=ws_norm)
         assert torch.equal(out, want) and torch.equal(normed, want_n)
+
+
+@pytest.mark.parametrize("M", [1, 2, 16, 17])
+@pytest.mark.parametrize("wide", ["out", "norm_out", "both"])
+def test_linear_rms_norm_into_rows_that_lie_apart(device, M, wide):
+    N, Kd = 1024, 4096
+    x, w, g = operands(M, N, Kd, torch.float16, seed=M)
+    xd, wd = x.to(device), w.to(device)
+    nw = (1.0 + 0.1 * torch.randn((N,), generator=g)).half().to(device)
+    res = torch.randn((M, 2 * N), generator=g).half().to(device)[:, N:]
+    want, want_n = K.linear_rms_norm(xd, wd, nw, 1e-5, residual=res)
+    bufs = [torch.full((M, N + 8 * (wide in (name, "both"))), 7.0, dtype=torch.float16, device=device) for name in ("out", "norm_out")]
+    ws = torch.empty((K.linear_rms_norm_workspace_size(xd, wd),), dtype=torch.uint8, device=device)
+    for workspace in (None, ws):
+        _native.linear_rms_norm(bufs[0][:, :N], bufs[1][:, :N], xd, wd, None, res, nw, 1e-5, workspace)
+        assert torch.equal(bufs[0][:, :N], want) and torch.equal(bufs[1][:, :N], want_n)
+        assert torch.all(bufs[0][:, N:] == 7.0) and torch.all(bufs[1][:, N:] == 7.0)
 
 
 @pytest.mark.parametrize("splits", [0, 1, 3, 8])
