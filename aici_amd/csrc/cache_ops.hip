@@ -856,9 +856,10 @@ extern "C" char *hipattn_copy_blocks_host(void *const *key_caches, void *const *
     for (int64_t i = 0; i < layers; i++)
       HA_CHECK(key_caches[i] != nullptr && value_caches[i] != nullptr && aligned16(key_caches[i]) && aligned16(value_caches[i]),
                "copy_blocks: the caches of layer %lld must start on a 16-byte boundary", (long long)i);
-    for (int64_t i = 0; i < 2 * n_pairs; i++)
-      HA_CHECK(block_mapping[i] >= INT32_MIN && block_mapping[i] <= INT32_MAX, "copy_blocks: block %lld does not fit 32 bits",
-               (long long)block_mapping[i]);
+    for (int64_t i = 0; i < 2 * n_pairs; i++) {
+      HA_CHECK(block_mapping[i] >= 0, "copy_blocks: pair %lld has block %lld", (long long)(i / 2), (long long)block_mapping[i]);
+      HA_CHECK(block_mapping[i] <= INT32_MAX, "copy_blocks: block %lld does not fit 32 bits", (long long)block_mapping[i]);
+    }
     hipStream_t stream = resolve_stream(stream_arg);
     const int64_t rows = bytes_per_block / 16;
     HA_CHECK(rows <= (1 << 22), "copy_blocks: a block of %lld bytes is too large", (long long)bytes_per_block);

@@ -183,9 +183,12 @@ def copy_blocks(key_caches: List[torch.Tensor], value_caches: List[torch.Tensor]
     device = key_caches[0].device
     tsize = key_caches[0].numel()
     pairs: List[int] = []
+    blocks = key_caches[0].size(0)
     for src, dsts in block_mapping.items():
         for dst in dsts:
             pairs += [int(src), int(dst)]
+            if not (0 <= pairs[-2] < blocks and 0 <= pairs[-1] < blocks):
+                raise HipAttnError(f"copy_blocks: pair {src} -> {dst} out of range, the caches have {blocks} blocks")
     # addresses and pairs as arguments of the launch; False for blocks that are not whole 16-byte rows
     if _native.copy_blocks(key_caches, value_caches, pairs):
         return

@@ -244,7 +244,9 @@ char *hipattn_copy_blocks_2(const hipattn_tensor *key_cache_ptrs,
  * the launches (64 layers x 256 pairs each), so that no upload goes in front
  * of the copy and the call may be captured.  Caches must start on 16-byte
  * boundaries, bytes_per_block be a multiple of 16 (at most 64 MiB) and block
- * numbers fit 32 bits. */
+ * numbers lie between 0 and what 32 bits hold; a negative one is refused before
+ * any launch.  That they lie within the caches is the caller's to see to: the
+ * call does not know how many blocks there are. */
 char *hipattn_copy_blocks_host(void *const *key_caches, void *const *value_caches,
                                int64_t layers, const int64_t *block_mapping,
                                int64_t n_pairs, int64_t bytes_per_block,

@@ -35,6 +35,22 @@ def test_linear_workspace_depends_on_the_weight_alone(fn, shape):
     assert len(sizes) == 1 and sizes.pop() > 0
 
 
+@pytest.mark.parametrize("mapping", [{-1: [0]}, {0: [-1]}, {4: [0]}, {0: [1, 4]}, {0: [2 ** 31]}, {-(2 ** 40): [1]}])
+def test_copy_blocks_refuses_blocks_outside_the_caches(mapping):
+    """Before anything is launched (and before the caches are looked at: they need not be on a GPU here)."""
+    kc, vc = torch.zeros((4, 2, 1, 16, 8), dtype=torch.float16), torch.zeros((4, 2, 8, 16), dtype=torch.float16)
+    with pytest.raises(_lib.HipAttnError, match="out of range"):
+        kernels.copy_blocks([kc], [vc], mapping)
+
+
+@pytest.mark.parametrize("pair,message", [((-1, 0), "pair 1 has block -1"), ((0, -5), "pair 1 has block -5"),
+                                          ((0, 2 ** 31), "does not fit 32 bits")])
+def test_copy_blocks_host_refuses_bad_numbers_before_any_launch(pair, message):
+    ptr = (ctypes.c_void_p * 1)(4096)  # never read: the numbers are looked at first
+    with pytest.raises(_lib.HipAttnError, match=message):
+        _lib.call("hipattn_copy_blocks_host", ptr, ptr, 1, (ctypes.c_int64 * 4)(0, 1, *pair), 2, 4096, None)
+
+
 def _batch(lens):
     alloc = paged.BlockAllocator(16, 256)
     b = paged.BatchInfoBuilder(16, 4096, 1)
