@@ -163,7 +163,10 @@ def paged_attention_v2(out: torch.Tensor, exp_sums: torch.Tensor, max_logits: to
 
 def reshape_and_cache(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor,
                       slot_mapping: torch.Tensor) -> None:
-    """lib.rs:192-213.  The reference's wrapper widens the slots to int64; the kernels read either width."""
+    """lib.rs:192-213.  The reference's wrapper widens the slots to int64; the kernels read either width, so int32 slots that
+    lie end to end are taken as they are."""
+    if slot_mapping.dtype != torch.int32 or not slot_mapping.is_contiguous():
+        slot_mapping = slot_mapping.to(torch.int64)
     _native.reshape_and_cache(key, value, key_cache, value_cache, slot_mapping)
 
 

@@ -114,6 +114,20 @@ def test_long_inputs_runs_of_tokens_mixed_with_everything_else(device, dtype, st
     assert torch.equal(bits(ko), bits(want_k)) and torch.equal(bits(vo), bits(want_v))
 
 
+@pytest.mark.parametrize("slots", [torch.tensor([35, 2, -1, 60], dtype=torch.int16), torch.tensor([35, 2, 7, 60], dtype=torch.uint8),
+                                   torch.tensor([35, 0, 2, 0, -1, 0, 60, 0], dtype=torch.int32)[::2]])
+def test_slots_of_other_types_and_strided_ones(device, slots):
+    g = torch.Generator().manual_seed(3)
+    key, value = (torch.randn((4, 2, 64), generator=g).half() for _ in range(2))
+    kc, vc = make_cache(4, 2, 64, 16, torch.float16, fill=-3.0)
+    kd, vd = kc.to(device), vc.to(device)
+    ref.reshape_and_cache(key, value, kc, vc, slots.to(torch.int64))
+    on_device = slots.to(device) if slots.is_contiguous() else torch.stack([slots, slots], 1).to(device)[:, 0]
+    assert on_device.is_contiguous() == slots.is_contiguous()
+    K.reshape_and_cache(key.to(device), value.to(device), kd, vd, on_device)
+    assert torch.equal(bits(kd), bits(kc)) and torch.equal(bits(vd), bits(vc))
+
+
 @pytest.mark.parametrize("bs,d,H", [(16, 128, 3), (16, 80, 4), (32, 64, 5), (48, 8, 40), (16, 64, 2)])
 @pytest.mark.parametrize("T", [127, 128, 129, 160, 300, 1023, 1024])
 def test_tiles_start_at_any_token(device, bs, d, H, T):

@@ -1,5 +1,6 @@
 """The CPython binding of the hot entry points (csrc/bind/native.cpp) and the one-copy upload of a batch."""
 import ctypes
+import types
 
 import pytest
 import torch
@@ -49,6 +50,17 @@ def test_copy_blocks_host_refuses_bad_numbers_before_any_launch(pair, message):
     ptr = (ctypes.c_void_p * 1)(4096)  # never read: the numbers are looked at first
     with pytest.raises(_lib.HipAttnError, match=message):
         _lib.call("hipattn_copy_blocks_host", ptr, ptr, 1, (ctypes.c_int64 * 4)(0, 1, *pair), 2, 4096, None)
+
+
+@pytest.mark.parametrize("slots", [torch.tensor([3, 1], dtype=d) for d in (torch.int8, torch.int16, torch.uint8, torch.int64)]
+                         + [torch.tensor([3, 0, 1], dtype=torch.int32)[::2], torch.tensor([3, 1], dtype=torch.int32)])
+def test_slots_of_every_integer_type_reach_the_kernel(slots, monkeypatch):
+    seen = []
+    monkeypatch.setattr(kernels, "_native", types.SimpleNamespace(reshape_and_cache=lambda *a: seen.append(a[4])))
+    kernels.reshape_and_cache(None, None, None, None, slots)
+    (got,) = seen
+    assert got.dtype in (torch.int32, torch.int64) and got.is_contiguous() and got.tolist() == [3, 1]
+    assert got is slots or slots.dtype not in (torch.int32, torch.int64) or not slots.is_contiguous()
 
 
 def _batch(lens):
