@@ -37,6 +37,8 @@
 #include "device_types.h"
 #include "workspace.h"
 
+#include <type_traits>
+
 // The copies set M0, and say so; the compiler reports that it is a reserved register.
 #pragma clang diagnostic ignored "-Winline-asm"
 
@@ -62,6 +64,7 @@ struct LinearParams {
   // with an RMS norm behind the layer: the sums go to the workspace as rows ([range][128 rows][N] fp32), and the
   // launch that adds them up also normalises the finished row
   int row_sums;
+  int wide;       // rows of x or W more than 2^28 elements apart
   int tile_sums;  // the sums go to the workspace as tiles, and a second launch finishes them
   const void *norm_w;
   void *norm_out;
@@ -129,27 +132,34 @@ __device__ __forceinline__ const P *uniform_base(const P *ptr) {
 }
 
 // What a copy instruction brings of a stage: 128 bytes of each of eight rows (first .. first + 7; rows past `last` repeat
-// it, and what is made of them is never stored).  One scalar base for the eight rows, a 32-bit offset per lane.
+// it, and what is made of them is never stored).  One scalar base for the eight rows, a 32-bit offset per lane (WIDE, for rows further
+// apart than that reaches: 64-bit, and the address in vector registers).
+template <bool WIDE>
 struct CopySource {
   const char *base;
-  uint32_t off;
+  typename std::conditional<WIDE, int64_t, uint32_t>::type off;
 };
-template <typename T>
-__device__ __forceinline__ CopySource copy_source(const void *rows, int64_t ld, int first, int last, int stage0) {
+template <typename T, bool WIDE>
+__device__ __forceinline__ CopySource<WIDE> copy_source(const void *rows, int64_t ld, int first, int last, int stage0) {
   const int lane = threadIdx.x & 63, r = lane >> 3, q = (lane & 7) ^ r;  // run q of row r goes to this lane's place
   const int b = min(first, last);
-  CopySource s;
+  CopySource<WIDE> s;
   s.base = uniform_base(reinterpret_cast<const char *>(static_cast<const T *>(rows) + b * ld + (int64_t)stage0 * kLinStageK));
-  s.off = (uint32_t)min(first + r, last) - (uint32_t)b;
-  s.off = s.off * (uint32_t)(ld * 2) + q * 16;
+  const int rows_on = min(first + r, last) - b;
+  if constexpr (WIDE)
+    s.off = (int64_t)rows_on * ld * 2 + q * 16;
+  else
+    s.off = (uint32_t)rows_on * (uint32_t)(ld * 2) + q * 16;
   return s;
 }
 
 // 64 lanes x 16 bytes of stage st, global -> LDS: lane l's bytes go to lds + 16 l.  ONCE: with the read-once hint.
-template <bool ONCE>
-__device__ __forceinline__ void copy_1k(uint32_t lds, const CopySource &s, int st) {
+template <bool ONCE, bool WIDE>
+__device__ __forceinline__ void copy_1k(uint32_t lds, const CopySource<WIDE> &s, int st) {
   const char *base = s.base + (int64_t)st * (kLinStageK * 2);
-  if (ONCE)
+  if constexpr (WIDE)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(base + s.off) : "memory", "m0");
+  else if constexpr (ONCE)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(s.off), "s"(base) : "memory", "m0");
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(s.off), "s"(base) : "memory", "m0");
@@ -190,20 +200,20 @@ __global__ __launch_bounds__(WAVES * 64) void linear_stream_kernel(const LinearP
   const int stage0 = first_range * p.stages_per_split;
   const int nst = max(0, min(ranges * p.stages_per_split, p.total_stages - stage0));
 
-  CopySource wsrc[kCopiesW], xsrc[kCopiesX];
+  CopySource<false> wsrc[kCopiesW], xsrc[kCopiesX];
 #pragma unroll
   for (int i = 0; i < kCopiesW; i++)
-    wsrc[i] = copy_source<T>(p.w, p.ldw, part * p.half + n_tile + i * 8, part * p.half + n_end - 1, stage0);
+    wsrc[i] = copy_source<T, false>(p.w, p.ldw, part * p.half + n_tile + i * 8, part * p.half + n_end - 1, stage0);
 #pragma unroll
-  for (int i = 0; i < kCopiesX; i++) xsrc[i] = copy_source<T>(p.x, p.ldx, i * 8, p.M - 1, stage0);
+  for (int i = 0; i < kCopiesX; i++) xsrc[i] = copy_source<T, false>(p.x, p.ldx, i * 8, p.M - 1, stage0);
   const char *mine = ring + wave * S * kStageBytes;
   const uint32_t mine_lds = lds_address(ring) + wave * S * kStageBytes;
   auto ask = [&](int slot, int st) {
     const uint32_t at = mine_lds + slot * kStageBytes;
 #pragma unroll
-    for (int i = 0; i < kCopiesX; i++) copy_1k<false>(at + (kCopiesW + i) * 1024, xsrc[i], st);
+    for (int i = 0; i < kCopiesX; i++) copy_1k<false, false>(at + (kCopiesW + i) * 1024, xsrc[i], st);
 #pragma unroll
-    for (int i = 0; i < kCopiesW; i++) copy_1k<true>(at + i * 1024, wsrc[i], st);
+    for (int i = 0; i < kCopiesW; i++) copy_1k<true, false>(at + i * 1024, wsrc[i], st);
   };
   f32x4_t acc[NT];
 #pragma unroll
@@ -282,7 +292,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_stream_kernel(const LinearP
 
 // Up to 16 MT rows of x: a workgroup owns 16 WAVES rows of W over one range of k.  GATED: the second half of the
 // wavefronts takes the up rows that belong to the gate rows of the first.
-template <typename T, int MT, int S, int WAVES, bool GATED>
+template <typename T, int MT, int S, int WAVES, bool GATED, bool WIDE>
 __global__ __launch_bounds__(WAVES * 64) void linear_tile_kernel(const LinearParams p) {
   using vec8 = typename Vec8<T>::type;
   // The read-once hint on W (stream kernel: always) measured 3 to 8 % faster here as well, except on the short ranges that the
@@ -307,22 +317,22 @@ __global__ __launch_bounds__(WAVES * 64) void linear_tile_kernel(const LinearPar
   const int stage0 = split * p.stages_per_split;
   const int nst = max(0, min(p.stages_per_split, p.total_stages - stage0));
 
-  CopySource wsrc[kCopiesW], xsrc[kCopiesX];
+  CopySource<WIDE> wsrc[kCopiesW], xsrc[kCopiesX];
 #pragma unroll
   for (int i = 0; i < kCopiesW; i++)
-    wsrc[i] = copy_source<T>(p.w, p.ldw, part * p.half + n_tile + i * 8, part * p.half + n_end - 1, stage0);
+    wsrc[i] = copy_source<T, WIDE>(p.w, p.ldw, part * p.half + n_tile + i * 8, part * p.half + n_end - 1, stage0);
   // Where the copies of x do not divide evenly some are made twice (the same bytes to the same place): every wavefront
   // counts the same number of copies per stage.
 #pragma unroll
-  for (int i = 0; i < kCopiesX; i++) xsrc[i] = copy_source<T>(p.x, p.ldx, ((wave + i * WAVES) % kAllX) * 8, p.M - 1, stage0);
+  for (int i = 0; i < kCopiesX; i++) xsrc[i] = copy_source<T, WIDE>(p.x, p.ldx, ((wave + i * WAVES) % kAllX) * 8, p.M - 1, stage0);
   const uint32_t ring_lds = lds_address(ring);
   auto ask = [&](int slot, int st) {
     const uint32_t at = ring_lds + slot * kStageBytes;
 #pragma unroll
     for (int i = 0; i < kCopiesX; i++)
-      copy_1k<false>(at + (kCopiesW * WAVES + (wave + i * WAVES) % kAllX) * 1024, xsrc[i], st);
+      copy_1k<false, WIDE>(at + (kCopiesW * WAVES + (wave + i * WAVES) % kAllX) * 1024, xsrc[i], st);
 #pragma unroll
-    for (int i = 0; i < kCopiesW; i++) copy_1k<kOnce>(at + (wave * kCopiesW + i) * 1024, wsrc[i], st);
+    for (int i = 0; i < kCopiesW; i++) copy_1k<kOnce, WIDE>(at + (wave * kCopiesW + i) * 1024, wsrc[i], st);
   };
   f32x4_t acc[MT];
 #pragma unroll
@@ -528,14 +538,19 @@ constexpr int ring_stages() {
   return s > 6 ? 6 : s;
 }
 
-template <typename T, int MT, bool GATED>
+// WIDE: MT and the workgroup are those of the largest call, which every smaller one fits.
+template <typename T, int MT, bool GATED, bool WIDE = false>
 void launch_tile(const LinearParams &p, const LinearPlan &pl, hipStream_t stream) {
-  const int n = GATED ? p.half : p.N, per_wg = pl.waves * 16 / (GATED ? 2 : 1);
-  const dim3 grid((n + per_wg - 1) / per_wg, pl.splits), block(pl.waves * 64);
-  if (pl.waves == 8)
-    hipLaunchKernelGGL((linear_tile_kernel<T, MT, ring_stages<MT, 8>(), 8, GATED>), grid, block, 0, stream, p);
-  else
-    hipLaunchKernelGGL((linear_tile_kernel<T, MT, ring_stages<MT, 4>(), 4, GATED>), grid, block, 0, stream, p);
+  const int waves = WIDE ? 8 : pl.waves;
+  const int n = GATED ? p.half : p.N, per_wg = waves * 16 / (GATED ? 2 : 1);
+  const dim3 grid((n + per_wg - 1) / per_wg, pl.splits), block(waves * 64);
+  if constexpr (!WIDE) {
+    if (waves == 4) {
+      hipLaunchKernelGGL((linear_tile_kernel<T, MT, ring_stages<MT, 4>(), 4, GATED, false>), grid, block, 0, stream, p);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((linear_tile_kernel<T, MT, ring_stages<MT, 8>(), 8, GATED, WIDE>), grid, block, 0, stream, p);
 }
 
 template <typename T, bool GATED>
@@ -555,7 +570,9 @@ void launch_linear(const LinearParams &p, const LinearPlan &pl, hipStream_t stre
     check_launch("linear (few rows)");
     return;
   }
-  if (p.M <= 32)
+  if (p.wide)
+    launch_tile<T, 8, GATED, true>(p, pl, stream);
+  else if (p.M <= 32)
     launch_tile<T, 2, GATED>(p, pl, stream);
   else if (p.M <= 64)
     launch_tile<T, 4, GATED>(p, pl, stream);
@@ -646,10 +663,6 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
     pl.partial_bytes = (size_t)pl.splits * kLinMaxRows * N * sizeof(float);
   }
 
-  // offsets between eight rows are 32 bits
-  HA_CHECK(weight->strides[0] >= 0 && weight->strides[0] < (1 << 28) && x->strides[0] >= 0 && x->strides[0] < (1 << 28),
-           "linear: row strides %lld / %lld of x / weight out of range", (long long)x->strides[0], (long long)weight->strides[0]);
-
   LinearParams p{};
   p.x = x->data;
   p.w = weight->data;
@@ -658,8 +671,13 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
   p.N = (int)N;
   p.K = (int)K;
   p.mtiles = (int)((M + 15) / 16);
-  p.ldx = x->strides[0];
+  p.ldx = M == 1 ? 0 : x->strides[0];
   p.ldw = weight->strides[0];
+  // seven rows on must be within 32 bits of bytes, else one instance of the tile kernel serves all sizes (the last position of every
+  // sequence of a [sequences, 65536, 4096] activation lies 2^28 elements apart)
+  auto far = [](int64_t ld) { return ld < 0 || ld >= (1 << 28); };
+  p.wide = far(p.ldx) || far(p.ldw);
+  if (p.wide) pl.stream = false;
   p.ldo = out->strides[0];
   if (bias != nullptr) {
     check_tensor(bias, "bias", 1);

@@ -122,6 +122,29 @@ def test_row_strides_of_every_operand(device):
     assert torch.all(out_wide[:, N:] == 7.0)  # nothing written past a row's end
 
 
+@pytest.mark.parametrize("M,N,ldx,ldw", [(1, 64, 1 << 30, None), (2, 1024, 1 << 28, None), (17, 16384, (1 << 28) + 64, None),
+                                         (5, 16, None, 1 << 28), (128, 48, 640, (1 << 28) + 8)])
+def test_rows_further_apart_than_32_bits_of_bytes(device, M, N, ldx, ldw):
+    """One position per sequence of a long activation; a slice of an enormous weight."""
+    Kd = 512
+    x, w, g = operands(M, N, Kd, torch.bfloat16, seed=M)
+
+    def spread(t, ld):
+        if ld is None:
+            return t.to(device)
+        far = torch.empty(((t.size(0) - 1) * ld + t.size(1),), dtype=t.dtype, device=device).as_strided(t.shape, (ld, 1))
+        return far.copy_(t)
+    xd, wd = x.to(device), w.to(device)
+    xf, wf = spread(x, ldx), spread(w, ldw)
+    assert torch.equal(K.linear(xf, wf), K.linear(xd, wd))
+    if N % 32 == 0:
+        assert torch.equal(K.linear_silu_and_mul(xf, wf), K.linear_silu_and_mul(xd, wd))
+    if N <= 8192:
+        nw = torch.ones((N,), dtype=torch.bfloat16, device=device)
+        for got, want in zip(K.linear_rms_norm(xf, wf, nw, 1e-5), K.linear_rms_norm(xd, wd, nw, 1e-5)):
+            assert torch.equal(got, want)
+
+
 def test_same_bits_on_every_run_and_rows_do_not_mix(device):
     x, w, _ = operands(128, 4096, 14336, torch.bfloat16, seed=33)
     xd, wd = x.to(device), w.to(device)
