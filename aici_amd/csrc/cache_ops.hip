@@ -8,6 +8,8 @@
 #include "device_types.h"
 #include "workspace.h"
 
+#include <type_traits>
+
 namespace hipattn {
 
 namespace {
@@ -215,16 +217,17 @@ __global__ __launch_bounds__(256) void cache_move_run8_kernel(
   }
 }
 
-// Coalesced on both sides (2-byte elements, head size a multiple of 8, blocks of a multiple of 16 tokens; the last group of a head
+// Coalesced on both sides (2-byte elements, head size a multiple of 8, blocks of a multiple of 8 tokens; the last group of a head
 // has fewer than 8 chunks when it is not a multiple of 64, and the lanes beyond them sit out).  The input is
 // token-major, the cache chunk-major, so some side of a direct copy always touches 16-byte pieces 256 bytes apart.
-// Here a wavefront moves a tile of 16 tokens x 8 chunks (64 head elements) of one head through a private LDS
+// Here a wavefront moves a tile of TT tokens x 8 chunks (64 head elements) of one head through a private LDS
 // slab: it reads the source in the source's order, transposes in LDS, and writes the destination in the
 // destination's order -- whole rows of the cache ([chunk][16 tokens] = 256 bytes of K, [16 tokens] = 32 bytes of
-// each V element, 1 KiB contiguous per instruction), whole 128-byte runs of a token.
+// each V element, 1 KiB contiguous per instruction), whole 128-byte runs of a token.  TT = 16 where blocks are multiples of
+// 16 tokens, else 8.
 //
-// A tile is 16 consecutive tokens that fill 16 consecutive slots from a multiple of 16 on.  The sequences of a batch lie
-// end to end, so tiles start at any token: a wavefront takes the tile that starts among its 16 tokens, wherever it ends, and the
+// A tile is TT consecutive tokens that fill TT consecutive slots from a multiple of TT on.  The sequences of a batch lie
+// end to end, so tiles start at any token: a wavefront takes the tile that starts among its TT tokens, wherever it ends, and the
 // tokens of its own that belong to no tile (ends of sequences, decode rows) one by one, eight at a time -- or, below 1024
 // tokens, leaves them to workgroups of their own behind the tiles', one per token (128 decode rows x 8 heads x 128: 3.7 us a
 // token per workgroup alone, 6.4 eight at a time, 3.8 so; from 1024 tokens on eight at a time is as fast).  Tiles cut at
@@ -232,7 +235,7 @@ __global__ __launch_bounds__(256) void cache_move_run8_kernel(
 //
 // us, before -> now (fp16): 1375 tokens of 4 sequences x 32 heads x 128 27 -> 9.3, 40012 tokens of 32 sequences x 2 heads x 64 34.7 -> 11.0,
 // 32768 tokens of 8 sequences x 8 heads x 128 44 -> 43.5.
-template <typename Slot, bool SCATTER, bool FULL_GROUPS>
+template <typename Slot, bool SCATTER, bool FULL_GROUPS, int TT>
 __global__ __launch_bounds__(256) void cache_move_tile_kernel(
     uint16_t *__restrict__ key, uint16_t *__restrict__ value, uint16_t *__restrict__ key_cache,
     uint16_t *__restrict__ value_cache, const Slot *__restrict__ slot_mapping, int64_t num_tokens,
@@ -240,13 +243,15 @@ __global__ __launch_bounds__(256) void cache_move_tile_kernel(
     int64_t val_head_stride, CacheGeom g, int items_per_wave, int waves_per_group, int tile_wgs) {
   typedef uint16_t E;
   constexpr int X = 8;
+  constexpr int RUNS = TT / 8;  // 16-byte pieces of a V row in the tile
+  constexpr unsigned kOwn = (1u << TT) - 1, kSeen = (unsigned)((1ull << (2 * TT)) - 1);
   if ((int)blockIdx.x >= tile_wgs) {  // a token that is in no tile
     const int64_t token = blockIdx.x - tile_wgs;
     const int64_t slot = (int64_t)slot_mapping[token];
     if (slot < 0 || slot / g.block_size >= g.num_blocks) return;
-    const int64_t first = token - slot % 16;  // where its tile would start
-    const int l = threadIdx.x & 15;
-    const bool there = first >= 0 && first + 15 < num_tokens && (int64_t)slot_mapping[first + l] == slot - slot % 16 + l;
+    const int64_t first = token - slot % TT;  // where its tile would start
+    const int l = threadIdx.x & (TT - 1);
+    const bool there = first >= 0 && first + TT <= num_tokens && (int64_t)slot_mapping[first + l] == slot - slot % TT + l;
     if (__all(there)) return;
     const int64_t blk = slot / g.block_size;
     const int off = (int)(slot % g.block_size), chunks = g.head_size / X;
@@ -262,43 +267,43 @@ __global__ __launch_bounds__(256) void cache_move_tile_kernel(
   }
   constexpr int KP = 72;  // K slab row pitch in elements: 8 chunks + 16 bytes, keeps the transposed 16-byte reads apart
   constexpr int VP = 64;  // V slab row pitch: the 2-byte column accesses of a wavefront fall in one row
-  __shared__ __attribute__((aligned(16))) E slab[4][16 * KP + 16 * VP];
+  __shared__ __attribute__((aligned(16))) E slab[4][TT * KP + TT * VP];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  E *ks = slab[wave], *vs = slab[wave] + 16 * KP;
+  E *ks = slab[wave], *vs = slab[wave] + TT * KP;
   const int64_t w = (int64_t)blockIdx.x * 4 + wave;
-  const int64_t t0 = w / waves_per_group * 16;
+  const int64_t t0 = w / waves_per_group * TT;
   if (t0 >= num_tokens) return;
   const int chunks_per_head = g.head_size / X;
   const int groups_per_head = (chunks_per_head + 7) / 8;  // the last group of a head may hold fewer than 8 chunks
   const int item0 = (int)(w % waves_per_group) * items_per_wave;
   const int item1 = min(item0 + items_per_wave, g.num_heads * groups_per_head);
 
-  // Lanes 0 .. 31 look at tokens t0 .. t0 + 31: a tile that starts among the first 16 ends among them.
-  const int64_t t = t0 + (lane & 31);
+  // Lanes 0 .. 2 TT - 1 look at tokens t0 .. t0 + 2 TT - 1: a tile that starts among the first TT ends among them.
+  const int64_t t = t0 + (lane & (2 * TT - 1));
   int64_t slot = t < num_tokens ? (int64_t)slot_mapping[t] : -1;
   if (slot >= 0 && slot / g.block_size >= g.num_blocks) slot = -1;  // never outside the cache
-  const bool follows = t > 0 && t < num_tokens && slot > 0 && slot % 16 != 0 && (int64_t)slot_mapping[t - 1] == slot - 1;
-  const unsigned starts = (unsigned)__ballot(!follows), valid = (unsigned)__ballot(slot >= 0);
-  const unsigned own_starts = starts & 0xffffu;
-  if (own_starts == 0) return;  // all 16 belong to the tile of the wavefront before
-  // no other start among the 15 tokens behind it: all of them follow one another within the row of 16 slots
-  const bool is_tile = lane < 16 && !follows && slot >= 0 && slot % 16 == 0 && ((starts >> (lane + 1)) & 0x7fffu) == 0;
+  const bool follows = t > 0 && t < num_tokens && slot > 0 && slot % TT != 0 && (int64_t)slot_mapping[t - 1] == slot - 1;
+  const unsigned starts = (unsigned)__ballot(!follows) & kSeen, valid = (unsigned)__ballot(slot >= 0);
+  const unsigned own_starts = starts & kOwn;
+  if (own_starts == 0) return;  // all TT belong to the tile of the wavefront before
+  // no other start among the TT - 1 tokens behind it: all of them follow one another within the row of TT slots
+  const bool is_tile = lane < TT && !follows && slot >= 0 && slot % TT == 0 && ((starts >> (lane + 1)) & (kOwn >> 1)) == 0;
   const unsigned tile = (unsigned)__ballot(is_tile);  // at most one
-  const unsigned later = starts & 0xffff0000u;
+  const unsigned later = starts & ~kOwn;
   unsigned owned = ~0u << __builtin_ctz(own_starts);
   if (later != 0) owned &= (1u << __builtin_ctz(later)) - 1u;
   unsigned rest = (int)gridDim.x > tile_wgs ? 0u : owned & valid;
   const int tile_at = tile != 0 ? __builtin_ctz(tile) : 0;
-  if (tile != 0) rest &= ~(0xffffu << tile_at);
+  if (tile != 0) rest &= ~(kOwn << tile_at);
   const int64_t tile_slot = ((int64_t)__builtin_amdgcn_readlane((int)(slot >> 32), tile_at) << 32) |
                             (unsigned)__builtin_amdgcn_readlane((int)slot, tile_at);
   const int hi = lane >> 3, lo = lane & 7;
-  const int tok = lane & 15, c4 = lane >> 4;
-  const int th = lane & 1;  // which 8 tokens of a V row
+  const int tok = lane & (TT - 1), c4 = lane / TT;
+  const int th = lane & (RUNS - 1);  // which 8 tokens of a V row
   // In wider blocks a tile's pieces of V are parts of cache lines: with the hint a line goes to memory once per part, and comes
   // back once per part (us, hint / plain, on caches that are in no cache, 16000 tokens x 8 heads x 128: scatter 47.8 / 38.7 and gather
   // 34.2 / 31.4 in 32-token blocks, 63.7 / 40.6 and 39.3 / 32.8 in 64-token ones).
-  const bool whole_rows = g.block_size == 16;
+  const bool whole_rows = g.block_size == TT;
 
   for (int item = item0; item < item1; item++) {
     const int h = item / groups_per_head, cg = item % groups_per_head;
@@ -310,31 +315,31 @@ __global__ __launch_bounds__(256) void cache_move_tile_kernel(
       E *k_tok = key + (t0 + tile_at + hi) * key_tok_stride + h * key_head_stride + (cg * 8 + lo) * X;
       E *v_tok = value + (t0 + tile_at + hi) * val_tok_stride + h * val_head_stride + (cg * 8 + lo) * X;
       if (SCATTER) {
-        uint4 kk[2], vv[2];
+        uint4 kk[RUNS], vv[RUNS];
 #pragma unroll
-        for (int half = 0; half < 2; half++)  // tokens hi and hi + 8, chunk lo
+        for (int half = 0; half < RUNS; half++)  // tokens hi and hi + 8, chunk lo
           if (lo < nc) {
             kk[half] = *reinterpret_cast<const uint4 *>(k_tok + 8 * half * key_tok_stride);
             vv[half] = *reinterpret_cast<const uint4 *>(v_tok + 8 * half * val_tok_stride);
           }
 #pragma unroll
-        for (int half = 0; half < 2; half++)
+        for (int half = 0; half < RUNS; half++)
           if (lo < nc) {
             *reinterpret_cast<uint4 *>(ks + (8 * half + hi) * KP + lo * X) = kk[half];
             *reinterpret_cast<uint4 *>(vs + (8 * half + hi) * VP + lo * X) = vv[half];
           }
         __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the slab is private to this wavefront
 #pragma unroll
-        for (int i = 0; i < 2; i++) {  // chunk rows 4i + c4: 4 rows x 256 bytes per instruction
-          const int c = 4 * i + c4;
+        for (int i = 0; i < RUNS; i++) {  // TT = 16: chunk rows 4i + c4, 4 rows x 256 bytes per instruction
+          const int c = 64 / TT * i + c4;
           if (c < nc)
             // (the cache is not read again before a later step: stored with the written-once hint, 47.8 -> 44.1 us
             // for 32768 tokens x 8 kv heads x 128)
             store16_once(kc_base + ((int64_t)c * g.block_size + tok) * X, *reinterpret_cast<const uint4 *>(ks + tok * KP + c * X));
         }
 #pragma unroll
-        for (int i = 0; i < 2; i++) {  // head elements 32i + lane / 2: 32 rows x 32 bytes per instruction
-          const int e = 32 * i + (lane >> 1);
+        for (int i = 0; i < RUNS; i++) {  // TT = 16: head elements 32i + lane / 2, 32 rows x 32 bytes per instruction
+          const int e = 64 / RUNS * i + lane / RUNS;
           uint4 o;
           E *oe = reinterpret_cast<E *>(&o);
 #pragma unroll
@@ -346,10 +351,10 @@ __global__ __launch_bounds__(256) void cache_move_tile_kernel(
           }
         }
       } else {
-        uint4 kk[2], vv[2];
+        uint4 kk[RUNS], vv[RUNS];
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-          const int c = 4 * i + c4, e = 32 * i + (lane >> 1);
+        for (int i = 0; i < RUNS; i++) {
+          const int c = 64 / TT * i + c4, e = 64 / RUNS * i + lane / RUNS;
           if (c < nc) kk[i] = load16_once(kc_base + ((int64_t)c * g.block_size + tok) * X);
           if (e < nc * X) {
             const E *at = vc_base + (int64_t)e * g.block_size + 8 * th;
@@ -357,8 +362,8 @@ __global__ __launch_bounds__(256) void cache_move_tile_kernel(
           }
         }
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-          const int c = 4 * i + c4, e = 32 * i + (lane >> 1);
+        for (int i = 0; i < RUNS; i++) {
+          const int c = 64 / TT * i + c4, e = 64 / RUNS * i + lane / RUNS;
           if (c < nc) *reinterpret_cast<uint4 *>(ks + tok * KP + c * X) = kk[i];
           if (e < nc * X) {
             const E *ve = reinterpret_cast<const E *>(&vv[i]);
@@ -368,7 +373,7 @@ __global__ __launch_bounds__(256) void cache_move_tile_kernel(
         }
         __builtin_amdgcn_s_waitcnt(0xc07f);
 #pragma unroll
-        for (int half = 0; half < 2; half++)
+        for (int half = 0; half < RUNS; half++)
           if (lo < nc) {
             *reinterpret_cast<uint4 *>(k_tok + 8 * half * key_tok_stride) =
                 *reinterpret_cast<const uint4 *>(ks + (8 * half + hi) * KP + lo * X);
@@ -565,11 +570,14 @@ void launch_move(const hipattn_tensor *key, const hipattn_tensor *value,
     const bool vec_v = vec && g.block_size % 8 == 0 && aligned16(vc) && g.v_block_stride % 8 == 0 && g.v_head_stride % 8 == 0;
     // (few tokens of narrow rows are launch-bound either way: 128 .. 1000 prompt tokens x 2 heads x 64 2.5 .. 3.5 us a token per
     // workgroup, 2.9 .. 3.2 by tiles)
-    if (vec_v && T >= 128 && (T >= 1024 || g.num_heads * g.head_size > 256) && g.block_size % 16 == 0 &&
-        tuning().cache_move_lds != 0) {
+    // Tiles of 8 tokens, for blocks that are no multiple of 16, from 16384 tokens on (us, the kernel of runs of 8 / tiles, caches that are
+    // in no cache, 8-token blocks: 32768 x 8 x 128 scatter 74.1 / 62.5, gather 62.5 / 61.6; 16384 x 8 x 128 46.3 / 32.9 and 34.8 /
+    // 31.6; 16384 unrelated slots, which no prompt has, 181 / 181 and 96 / 112).
+    const int tt = g.block_size % 16 == 0 ? 16 : 8;
+    if (vec_v && T >= (tt == 16 ? 128 : 16384) && (T >= 1024 || g.num_heads * g.head_size > 256) && tuning().cache_move_lds != 0) {
       // One item (a head's 64 elements of 16 tokens) per wavefront while that is no more than 32 wavefronts per compute unit, up
       // to eight beyond (the slots are looked at once per wavefront).
-      const int64_t groups = (T + 15) / 16;
+      const int64_t groups = (T + tt - 1) / tt;
       CacheGeom gt = g;
       if (key->strides[1] == g.head_size && value->strides[1] == g.head_size && g.k_head_stride == (int64_t)g.head_size * g.block_size &&
           g.v_head_stride == g.k_head_stride && (int64_t)g.num_heads * g.head_size <= (1 << 20)) {
@@ -584,14 +592,17 @@ void launch_move(const hipattn_tensor *key, const hipattn_tensor *value,
       const int tile_wgs = (int)((groups * waves_per_group + 3) / 4);
       const dim3 tiles((unsigned)(tile_wgs + (T < 1024 ? T : 0)));
       // head sizes that are multiples of 64 have no partial chunk group: their instance carries no guards
-      if (gt.head_size % 64 == 0)
-        cache_move_tile_kernel<Slot, SCATTER, true><<<tiles, 256, 0, stream>>>(
+      auto launch = [&](auto full, auto tokens) {
+        cache_move_tile_kernel<Slot, SCATTER, decltype(full)::value, decltype(tokens)::value><<<tiles, 256, 0, stream>>>(
             kp, vp, kc, vc, sp, T, key->strides[0], key->strides[1], value->strides[0], value->strides[1], gt, per_wave,
             waves_per_group, tile_wgs);
-      else
-        cache_move_tile_kernel<Slot, SCATTER, false><<<tiles, 256, 0, stream>>>(
-            kp, vp, kc, vc, sp, T, key->strides[0], key->strides[1], value->strides[0], value->strides[1], gt, per_wave,
-            waves_per_group, tile_wgs);
+      };
+      auto launch_tokens = [&](auto full) {
+        if (tt == 16) launch(full, std::integral_constant<int, 16>{});
+        else launch(full, std::integral_constant<int, 8>{});
+      };
+      if (gt.head_size % 64 == 0) launch_tokens(std::true_type{});
+      else launch_tokens(std::false_type{});
       check_launch(SCATTER ? "reshape_and_cache" : "gather_cached_kv");
       return;
     }

@@ -128,11 +128,12 @@ def test_slots_of_other_types_and_strided_ones(device, slots):
     assert torch.equal(bits(kd), bits(kc)) and torch.equal(bits(vd), bits(vc))
 
 
-@pytest.mark.parametrize("bs,d,H", [(16, 128, 3), (16, 80, 4), (32, 64, 5), (48, 8, 40), (16, 64, 2)])
+@pytest.mark.parametrize("bs,d,H", [(16, 128, 3), (16, 80, 4), (32, 64, 5), (48, 8, 40), (16, 64, 2), (8, 128, 3), (24, 80, 5), (40, 64, 6)])
 @pytest.mark.parametrize("T", [127, 128, 129, 160, 300, 1023, 1024])
 def test_tiles_start_at_any_token(device, bs, d, H, T):
     """Batches of short sequences laid end to end: their full rows of 16 slots start at every token index modulo 16, next to
-    single tokens, beginnings in the middle of a block, ends, padding slots and slots past the cache."""
+    single tokens, beginnings in the middle of a block, ends, padding slots and slots past the cache.  (Blocks of 8, 24 and 40 tokens:
+    a token per workgroup, and from 1024 tokens on runs of 8.)"""
     g = torch.Generator().manual_seed(1000 * bs + T)
     nb = 2 * T // bs + 60
     order = torch.randperm(nb, generator=g).tolist()
@@ -158,6 +159,32 @@ def test_tiles_start_at_any_token(device, bs, d, H, T):
     want_k, want_v = key.clone(), value.clone()
     want_k[~ok], want_v[~ok] = 9.0, 9.0
     assert torch.equal(bits(ko), bits(want_k)) and torch.equal(bits(vo), bits(want_v))
+
+
+@pytest.mark.parametrize("bs,d,H,T", [(16, 128, 8, 16500), (8, 128, 8, 16387), (16, 72, 17, 16500), (24, 72, 17, 16384)])
+def test_tiles_of_several_items_per_wavefront(device, bs, d, H, T):
+    """More (tile, 64 elements) pairs than twice the device's wavefronts: a wavefront takes two and more, and its LDS slab is
+    used again; whole chunk groups, and a last one of fewer chunks (17 x 72 = 19 groups and an eighth)."""
+    assert (T + (16 if bs % 16 == 0 else 8) - 1) // (16 if bs % 16 == 0 else 8) * ((H * d + 63) // 64) >= 16384
+    g = torch.Generator().manual_seed(bs + d)
+    nb = T // bs + 40
+    slots = (torch.randperm(nb, generator=g)[:, None] * bs + torch.arange(bs)).reshape(-1)[3:T + 3].clone()
+    slots[100:200] = slots[100:200][torch.randperm(100, generator=g)]  # decode-like: unrelated slots
+    slots[T // 3], slots[T // 2], slots[T - 2] = -1, nb * bs + 7, -1
+    key, value = (torch.randint(-2 ** 15, 2 ** 15, (T, H, d), generator=g, dtype=torch.int16).view(torch.float16) for _ in range(2))
+    ok = (slots >= 0) & (slots < nb * bs)
+    kd, vd = (torch.zeros(s, dtype=torch.float16, device=device) for s in ((nb, H, d // 8, bs, 8), (nb, H, d, bs)))
+    kr, vr = kd.clone().view(torch.int16), vd.clone().view(torch.int16)
+    key_d, value_d = key.to(device), value.to(device)
+    at = slots[ok].to(device)
+    kr[at // bs, :, :, at % bs] = key_d[ok.to(device)].view(torch.int16).view(-1, H, d // 8, 8)
+    vr[at // bs, :, :, at % bs] = value_d[ok.to(device)].view(torch.int16)
+    K.reshape_and_cache(key_d, value_d, kd, vd, slots.to(device))
+    assert torch.equal(kd.view(torch.int16), kr) and torch.equal(vd.view(torch.int16), vr)
+    ko, vo = torch.full_like(key_d, 9.0), torch.full_like(value_d, 9.0)
+    K.gather_cached_kv(ko, vo, kd, vd, slots.to(torch.int32).to(device))
+    key_d[~ok.to(device)], value_d[~ok.to(device)] = 9.0, 9.0
+    assert torch.equal(ko.view(torch.int16), key_d.view(torch.int16)) and torch.equal(vo.view(torch.int16), value_d.view(torch.int16))
 
 
 @pytest.mark.parametrize("layers,pairs,d", [(1, 1, 8), (3, 257, 64), (65, 2, 80), (130, 3, 8), (2, 0, 64)])
