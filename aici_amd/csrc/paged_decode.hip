@@ -1102,14 +1102,19 @@ DecodePlan plan_decode(int64_t S, int Hq, int Hkv, int head_size, int block_size
       // A whole context per workgroup of eight wavefronts instead of partitions and their merge.  The merge costs about 3 us;
       // each block pair a wavefront takes after its first costs 2.4 us where only a few compute units run (head size 128; 1.5
       // at 64), and nothing where the launch is bound by memory.  So: contexts of one pair per wavefront, two pairs of small
-      // heads, and whatever fits one lane-held slice of the table once 128 workgroups share the memory; from 1024
-      // workgroups on the partitions win (one workgroup of eight per compute unit).  us, partitions / one workgroup:
-      //   32 q / 8 kv x 128: 1 x 256 8.5 / 6.8, 1 x 512 8.3 / 9.7, 1 x 700 9.2 / 11.7, 16 x 512 12.5 / 11.2, 64 x 512 30.2 / 27.6,
-      //   128 x 512 50.0 / 52.1; 32 / 32 x 80: 1 x 512 8.1 / 7.7, 4 x 512 9.9 / 8.4, 1 x 1023 8.7 / 11.2; 16 / 2 x 64: 1 x 512 7.2 / 6.4,
-      //   16 x 1023 8.5 / 9.6, 128 x 1023 20.3 / 14.7.
+      // heads, and whatever fits one lane-held slice of the table once the workgroups share the memory (128 of them; 192 for
+      // the longest contexts of larger heads, which otherwise end last and alone).  Beyond two such workgroups per compute unit
+      // they gain nothing, and their last round loses, but at small heads, which keep winning up to 1024.  us, partitions / one
+      // workgroup, all contexts of that length (lengths uniform up to it):
+      //   32 q / 8 kv x 128: 1 x 256 8.5 / 6.8, 1 x 512 8.3 / 9.7, 1 x 700 9.2 / 11.7, 16 x 512 13.6 / 12.5 (11.6 / 10.9), 16 x 1024 20.3 /
+      //   20.1 (15.1 / 17.1), 24 x 1024 26.2 / 22.5 (20.2 / 18.5), 40 x 512 23.0 / 24.7 (18.4 / 15.8), 40 x 1024 36.7 / 40.9 (26.2 / 23.6),
+      //   64 x 512 30.2 / 27.6, 72 x 512 35.6 / 38.6 (25.8 / 24.7), 104 x 512 47.4 / 51.5 (32.6 / 34.3); 32 / 32 x 80: 1 x 512 8.1 / 7.7,
+      //   4 x 512 9.9 / 8.4, 1 x 1023 8.7 / 11.2, 26 x 200 19.2 / 21.1 (15.0 / 16.9); 16 / 2 x 64: 1 x 512 7.2 / 6.4, 16 x 1023 8.5 / 9.6,
+      //   64 x 1024 14.0 / 12.0 (12.8 / 10.7), 508 x 512 33.6 / 31.2 (24.5 / 22.1).
       const int64_t wgs = S * Hkv * col_groups;
-      const bool one_wg = max_blocks <= 16 || (max_blocks <= 32 && (head_size <= 64 || wgs >= 128)) || (max_blocks <= 64 && wgs >= 128);
-      if (tuning().decode_part_blocks <= 0 && head_size <= 128 && max_blocks > pl.part_blocks && wgs < 1024 && one_wg) {
+      const bool small = head_size <= 64;
+      const bool one_wg = max_blocks <= 16 || (max_blocks <= 32 && small) || (max_blocks <= 64 && wgs >= (small || max_blocks <= 48 ? 128 : 192));
+      if (tuning().decode_part_blocks <= 0 && head_size <= 128 && max_blocks > pl.part_blocks && wgs <= (small ? 1023 : 512) && one_wg) {
         pl.part_blocks = 64;
         pl.waves = 8;
       }
