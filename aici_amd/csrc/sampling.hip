@@ -133,20 +133,24 @@ __device__ __forceinline__ u64 block_exclusive(u64 v, Scratch &s) {
 // The counted values of a 16-bit float type: magnitudes above kLo (2^-16 / 2^-8) of either sign, numbered by their bits;
 // smaller ones share number 0.  kBins values have a counter: of bf16 all from 2^16 (number kTop) down to -2^16, so that the
 // largest is found among the counters; fp16 has more, and the counters go from the row's largest down, found in a pass before.
+// The counters cost the same whatever the vocabulary, the other way's passes (three more with a nucleus to cut) grow with it: rows
+// are counted from kLeastCut tokens on, or kLeastAll without a cut.  us, any row / counting, 128 rows, 5 % allowed, bf16: with a cut 2000
+// tokens 22.1 / 21.8, 4096 23.3 / 22.2; without 8192 15.5 / 18.2, 12000 19.6 / 19.7, 16384 23.0 / 19.6; fp16: 8192 27.7 / 32.6, 12000
+// 33.0 / 33.7, 16384 39.0 / 34.4; without 24000 31.2 / 31.2, all allowed 32000 39.5 / 41.7, 40000 46.2 / 45.3.
 template <typename T>
 struct Counted {
   static constexpr bool possible = false;
-  static constexpr int kBins = 1, kLo = 0, kInf = 0, kTop = 0;
+  static constexpr int kBins = 1, kLo = 0, kInf = 0, kTop = 0, kLeastCut = 0, kLeastAll = 0;
 };
 template <>
 struct Counted<bf16_t> {
   static constexpr bool possible = true;
-  static constexpr int kBins = 8192, kLo = 0x3780, kTop = 4096;
+  static constexpr int kBins = 8192, kLo = 0x3780, kTop = 4096, kLeastCut = 2048, kLeastAll = 16384;
 };
 template <>
 struct Counted<half_t> {
   static constexpr bool possible = true;
-  static constexpr int kBins = 28672, kLo = 0x1c00, kInf = 0x7c00, kTop = 0;
+  static constexpr int kBins = 28672, kLo = 0x1c00, kInf = 0x7c00, kTop = 0, kLeastCut = 16384, kLeastAll = 40000;
 };
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
@@ -475,7 +479,8 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
   return true;
 }
 
-template <typename T, int MODE /*0 = f32 bias rows, 1 = packed allow-bits*/>
+// COUNT: with the counting way and the LDS that it takes.
+template <typename T, int MODE /*0 = f32 bias rows, 1 = packed allow-bits*/, bool COUNT>
 __global__ __launch_bounds__(kThreads) void bias_sample_kernel(SampleParams p) {
   __shared__ Scratch s;
   const int tid = threadIdx.x;
@@ -560,12 +565,14 @@ __global__ __launch_bounds__(kThreads) void bias_sample_kernel(SampleParams p) {
     return;
   }
 
-  if constexpr (MODE == 1 && Counted<T>::possible) {
+  const float top_p = p.top_p ? p.top_p[seq] : 1.0f;
+  const bool cut = top_p > 0.f && top_p < 1.0f;
+  if constexpr (COUNT) {
     __shared__ unsigned bins[Counted<T>::kBins];
-    if (sample_counted<T>(p, s, bins, lg, p.mask + row * p.mask_stride, temp, p.top_p ? p.top_p[seq] : 1.0f, p.uniforms[seq],
-                          p.out_tokens + seq))
-      return;
-    __syncthreads();
+    if (V >= (cut ? Counted<T>::kLeastCut : Counted<T>::kLeastAll)) {
+      if (sample_counted<T>(p, s, bins, lg, p.mask + row * p.mask_stride, temp, top_p, p.uniforms[seq], p.out_tokens + seq)) return;
+      __syncthreads();
+    }
   }
 
   // logits / temperature as the reference forms it: a true division
@@ -609,11 +616,10 @@ __global__ __launch_bounds__(kThreads) void bias_sample_kernel(SampleParams p) {
 
   // The nucleus: the image `kstar` of the smallest kept value, the mass above it, and how many of the
   // tokens equal to it are kept (the first n_keep in id order).
-  const float top_p = p.top_p ? p.top_p[seq] : 1.0f;
   unsigned kstar = 0;  // below every image: everything is kept
   int n_keep = 0;
   u64 mass_gt = 0, m_star = 0, total = z;
-  if (top_p > 0.f && top_p < 1.0f) {
+  if (cut) {
     const u64 target = (u64)((double)top_p * (double)z);
     unsigned prefix = 0;  // the bits of kstar fixed so far, in place
     int fixed_bits = 0;
@@ -810,9 +816,11 @@ void bias_sample_impl(const hipattn_tensor *logits, const hipattn_tensor *bias, 
   p.uniforms = static_cast<const float *>(uniforms->data);
   p.out_tokens = static_cast<int32_t *>(out_tokens->data);
   HA_CHECK(S <= 0x7fffffff, "%s: too many sequences", op);
-#define HA_BS(TT)                                                                   \
-  if (bias) bias_sample_kernel<TT, 0><<<dim3((unsigned)S), kThreads, 0, stream>>>(p); \
-  else bias_sample_kernel<TT, 1><<<dim3((unsigned)S), kThreads, 0, stream>>>(p)
+#define HA_BS(TT)                                                                                                   \
+  if (bias) bias_sample_kernel<TT, 0, false><<<dim3((unsigned)S), kThreads, 0, stream>>>(p);                         \
+  else if (!Counted<TT>::possible || p.vocab < Counted<TT>::kLeastCut)                                               \
+    bias_sample_kernel<TT, 1, false><<<dim3((unsigned)S), kThreads, 0, stream>>>(p);                                 \
+  else bias_sample_kernel<TT, 1, Counted<TT>::possible><<<dim3((unsigned)S), kThreads, 0, stream>>>(p)
   switch (logits->dtype) {
     case HIPATTN_F32: HA_BS(float); break;
     case HIPATTN_F16: HA_BS(half_t); break;

@@ -288,7 +288,9 @@ def test_bias_sample_equal_values_and_distribution(device):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("V,share", [(128256, 0.05), (128256, 1.0), (50003, 0.0005), (1001, 0.5), (7, 1.0)])
+@pytest.mark.parametrize("V,share", [(128256, 0.05), (128256, 1.0), (50003, 0.0005), (1001, 0.5), (7, 1.0),
+                                     (2047, 0.5), (2048, 0.5), (16383, 0.1), (16384, 0.1), (40000, 1.0),  # where counting begins
+                                     (262149, 0.3)])  # a wavefront's tokens are searched in three rounds
 def test_bias_sample_counts_equal_logits_to_the_same_tokens(device, dtype, V, share):
     """16-bit logits under allow-bits are sampled by counting equal values, float32 ones are not: the same values give
     the same token either way, whatever their range -- ordinary logits, all below zero, equal ones, ones too small or too
