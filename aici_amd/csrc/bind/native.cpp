@@ -303,8 +303,15 @@ PyObject *copy_blocks(PyObject *, PyObject *const *args, Py_ssize_t n) {
   std::vector<int64_t> pairs((size_t)count);
   for (Py_ssize_t i = 0; i < count; i++)
     if (!to_i64(PySequence_Fast_GET_ITEM(held[2], i), &pairs[(size_t)i])) return nullptr;
-  for (int64_t b : pairs)
-    if (b < INT32_MIN || b > INT32_MAX) Py_RETURN_FALSE;
+  for (Py_ssize_t i = 0; i + 1 < count; i += 2) {
+    const int64_t src = pairs[(size_t)i], dst = pairs[(size_t)i + 1], blocks = first.sizes[0];
+    if (src < 0 || src >= blocks || dst < 0 || dst >= blocks) {
+      PyErr_Format(g_error, "copy_blocks: pair %lld -> %lld out of range, the caches have %lld blocks", (long long)src, (long long)dst,
+                   (long long)blocks);
+      return nullptr;
+    }
+  }
+  if (first.sizes[0] > INT32_MAX) Py_RETURN_FALSE;
   void *stream = nullptr;
   if (g_exchange->current_work_stream((DLDeviceType)c.device_type, c.device, &stream) != 0) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "no current stream");

@@ -186,15 +186,16 @@ def copy_blocks(key_caches: List[torch.Tensor], value_caches: List[torch.Tensor]
     device = key_caches[0].device
     tsize = key_caches[0].numel()
     pairs: List[int] = []
-    blocks = key_caches[0].size(0)
     for src, dsts in block_mapping.items():
         for dst in dsts:
             pairs += [int(src), int(dst)]
-            if not (0 <= pairs[-2] < blocks and 0 <= pairs[-1] < blocks):
-                raise HipAttnError(f"copy_blocks: pair {src} -> {dst} out of range, the caches have {blocks} blocks")
     # addresses and pairs as arguments of the launch; False for blocks that are not whole 16-byte rows
     if _native.copy_blocks(key_caches, value_caches, pairs):
         return
+    blocks = key_caches[0].size(0)
+    for src, dst in zip(pairs[::2], pairs[1::2]):
+        if not (0 <= src < blocks and 0 <= dst < blocks):
+            raise HipAttnError(f"copy_blocks: pair {src} -> {dst} out of range, the caches have {blocks} blocks")
     for e in list(key_caches) + list(value_caches):
         assert e.device == device and e.numel() == tsize and e.is_contiguous()
         assert e.dtype in (torch.float16, torch.bfloat16)

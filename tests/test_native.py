@@ -44,6 +44,16 @@ def test_copy_blocks_refuses_blocks_outside_the_caches(mapping):
         kernels.copy_blocks([kc], [vc], mapping)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("mapping", [{-1: [0]}, {0: [-1]}, {4: [0]}, {0: [1, 4]}, {0: [2 ** 31]}, {-(2 ** 40): [1]}])
+def test_copy_blocks_refuses_blocks_outside_caches_on_the_device(device, mapping):
+    """The binding's own look at the pairs, before any launch."""
+    kc = torch.zeros((4, 2, 1, 16, 8), dtype=torch.float16, device=device)
+    vc = torch.zeros((4, 2, 8, 16), dtype=torch.float16, device=device)
+    with pytest.raises(_lib.HipAttnError, match="out of range, the caches have 4 blocks"):
+        kernels.copy_blocks([kc], [vc], mapping)
+
+
 @pytest.mark.parametrize("pair,message", [((-1, 0), "pair 1 has block -1"), ((0, -5), "pair 1 has block -5"),
                                           ((0, 2 ** 31), "does not fit 32 bits")])
 def test_copy_blocks_host_refuses_bad_numbers_before_any_launch(pair, message):
