@@ -1,5 +1,6 @@
 """reshape_and_cache / gather_cached_kv / copy_blocks / swap_blocks through the C ABI against
 the oracle: bit-exact."""
+import numpy as np
 import pytest
 import torch
 
@@ -58,12 +59,10 @@ def test_reshape_and_cache_and_gather_bit_exact(device, dtype, slot_dtype, strid
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("strided", [False, True])
-@pytest.mark.parametrize("d,first", [(96, 512), (128, 512),      # the register-tile kernel (under 16384 tokens)
-                                     (128, 16000), (64, 16000),   # the LDS-tile kernel
-                                     (96, 16000), (80, 16000)])   # ... with a partial last chunk group per head
+@pytest.mark.parametrize("d,first", [(96, 512), (128, 512), (128, 16000), (64, 16000),
+                                     (96, 16000), (80, 16000)])   # (head sizes with a partial last chunk group where heads lie apart)
 def test_long_inputs_runs_of_tokens_mixed_with_everything_else(device, dtype, strided, d, first):
-    """More than 1024 tokens: the kernels move aligned runs of 8 tokens as tiles and fall back per
-    token elsewhere.  The slot list mixes prompts that fill permuted blocks in order (lengths not
+    """More than 1024 tokens: rows of 16 slots are moved as tiles, the other tokens one by one.  The slot list mixes prompts that fill permuted blocks in order (lengths not
     multiples of 8, so runs straddle sequences), a prompt that starts in the middle of a block,
     padding slots inside a run, decode-like random slots, a slot past the cache and a ragged tail."""
     g = torch.Generator().manual_seed(7)
@@ -129,7 +128,7 @@ def test_slots_of_other_types_and_strided_ones(device, slots):
 
 
 @pytest.mark.parametrize("bs,d,H", [(16, 128, 3), (16, 80, 4), (32, 64, 5), (48, 8, 40), (16, 64, 2), (8, 128, 3), (24, 80, 5), (40, 64, 6)])
-@pytest.mark.parametrize("T", [127, 128, 129, 160, 300, 1023, 1024])
+@pytest.mark.parametrize("T", [127, 128, 129, 160, 300, 1023, 1024, 1501])
 def test_tiles_start_at_any_token(device, bs, d, H, T):
     """Batches of short sequences laid end to end: their full rows of 16 slots start at every token index modulo 16, next to
     single tokens, beginnings in the middle of a block, ends, padding slots and slots past the cache.  (Blocks of 8, 24 and 40 tokens:
@@ -189,7 +188,7 @@ def test_tiles_of_several_items_per_wavefront(device, bs, d, H, T):
 
 @pytest.mark.parametrize("layers,pairs,d", [(1, 1, 8), (3, 257, 64), (65, 2, 80), (130, 3, 8), (2, 0, 64)])
 def test_copy_blocks_with_more_than_one_launch_holds(device, layers, pairs, d):
-    """Layers and pairs beyond what one launch's arguments hold; and the former entry point, from device arrays."""
+    """Layers and pairs beyond what one launch's arguments hold."""
     g = torch.Generator().manual_seed(layers + pairs)
     nb = 2 * pairs + 3
     caches = [make_cache(nb, 2, d, 16, torch.float16, fill=0.0) for _ in range(layers)]
@@ -202,6 +201,37 @@ def test_copy_blocks_with_more_than_one_launch_holds(device, layers, pairs, d):
         for src, (dst,) in mapping.items():
             k[dst], v[dst] = k[src], v[src]
         assert torch.equal(bits(kd), bits(k)) and torch.equal(bits(vd), bits(v))
+
+
+@pytest.mark.parametrize("route", ["device arrays", "python"])
+@pytest.mark.parametrize("shape,dtype", [((2, 8, 16, 8), torch.float16),   # whole 16-byte rows
+                                         ((2, 3, 5), torch.bfloat16),      # 60 bytes: copied byte by byte
+                                         ((4, 8), torch.float16)])         # ... and caches that start on no 16-byte boundary
+@pytest.mark.parametrize("layers,pairs", [(1, 1), (3, 40)])
+def test_copy_blocks_from_device_arrays(device, route, shape, dtype, layers, pairs):
+    """hipattn_copy_blocks_2 itself, and copy_blocks of caches that the launch by arguments does not take."""
+    from aici_amd.kernels import _desc, _stream, call
+    g = torch.Generator().manual_seed(layers + pairs)
+    nb = 2 * pairs + 3
+    n = nb * int(np.prod(shape))
+    shift = 4 if shape == (4, 8) else 0  # elements: 8 bytes
+    bufs = [[torch.randn((n + shift,), generator=g).to(dtype) for _ in range(layers)] for _ in range(2)]
+    want = [[b[shift:].clone().view(nb, *shape) for b in side] for side in bufs]
+    dev = [[b.to(device)[shift:].view(nb, *shape) for b in side] for side in bufs]
+    assert all(t.data_ptr() % 16 == 2 * shift for side in dev for t in side)
+    order = torch.randperm(nb, generator=g).tolist()
+    mapping = {order[i]: [order[pairs + i]] for i in range(pairs)}
+    if route == "python":
+        K.copy_blocks(*dev, mapping)
+    else:
+        kp, vp = (torch.tensor([t.data_ptr() for t in side], dtype=torch.int64, device=device) for side in dev)
+        flat = torch.tensor([b for s, (d,) in mapping.items() for b in (s, d)], dtype=torch.int64, device=device)
+        call("hipattn_copy_blocks_2", _desc(kp), _desc(vp), _desc(flat), _desc(dev[0][0]), _stream(kp))
+    for side, refs in zip(dev, want):
+        for got, ref_t in zip(side, refs):
+            for s, (d,) in mapping.items():
+                ref_t[d] = ref_t[s]
+            assert torch.equal(bits(got), bits(ref_t))
 
 
 def test_config1_scatter_bit_exact(device):
