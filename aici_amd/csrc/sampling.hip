@@ -145,7 +145,7 @@ struct Counted {
 template <>
 struct Counted<bf16_t> {
   static constexpr bool possible = true;
-  static constexpr int kBins = 8192, kLo = 0x3780, kTop = 4096, kLeastCut = 2048, kLeastAll = 16384;
+  static constexpr int kBins = 8192, kLo = 0x3780, kInf = 0x7f80, kTop = 4096, kLeastCut = 2048, kLeastAll = 16384;
 };
 template <>
 struct Counted<half_t> {
@@ -348,7 +348,8 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
     own += count[i] * (u64)f;
     if (o == top_number) own += small;
   }
-  const u64 z = block_sum(own, s) + low + (top_number >= C::kBins ? small : 0ull);
+  static_assert((C::kTop != 0 ? C::kTop : C::kInf - C::kLo) < C::kBins, "number 0, the small ones, is among the counters' numbers or above");
+  const u64 z = block_sum(own, s) + low;
   unsigned kstar = 0;  // image of the last kept value; below every image that is counted: everything is kept
   int n_keep = 0;
   u64 m_star = 0, total = z;
