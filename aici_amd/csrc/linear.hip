@@ -8,7 +8,7 @@
 // operands of v_mfma_f32_16x16x32 are read from LDS without bank conflicts.  What bounds them is how many whole
 // cache lines are on their way: the same loop with W loaded straight into the operands (16 rows x 64 bytes per instruction, so
 // every line asked for twice, and both copies of it held in the 32 KB L1) reached 5.1 TB/s on a 28672 x 4096 weight and one row of x,
-// 4.0 with sixteen; this form 6.0 and 5.5 (library GEMM: 3.9 / 3.9).
+// 4.0 with sixteen; this form 5.9 and 5.4 (library GEMM: 4.0 / 3.9).
 //
 //   linear_stream_kernel, up to 16 rows of x: a wavefront owns 16 (or 64) rows of W and keeps a private ring, its own copy of
 //   the rows of x in it, so nothing waits for anything but the wavefront's own copies; wavefronts that share rows of W
@@ -28,8 +28,11 @@
 //   28672 x 4096        58.8 -> 40.1   59.8 -> 43.7   51.2 -> 43.0   51.4 -> 47.2   53.9 -> 53.1
 //     + silu_and_mul    62.9 -> 41.7   64.2 -> 44.0   56.8 -> 43.1   57.9 -> 49.7   61.0 -> 54.8
 //   128256 x 4096       183 -> 166     186 -> 166     196 -> 186     208 -> 211     232 -> 248
-// (one row of 28672 x 4096 is 5.9 TB/s; what bounds the many-row end is the LDS: 128 rows of x are read from it by every
-// wavefront, eight times the bytes of W, and a workgroup has the compute unit to itself, its start and end open.)
+// (one row of 28672 x 4096 is 5.9 TB/s, 128 rows are 4.4.  At that end every workgroup copies as many bytes of x into LDS as of W and
+// has the compute unit to itself, its start and end open; the reads of x from LDS, eight times the bytes of W, are not what bounds it:
+// a third fewer of them changed nothing.)
+// Narrower weights keep these kernels' lead: 1024 x 4096 13.6 -> 6.4 with one row and 18.3 -> 12.7 with 128 against a kernel that cut them
+// into up to 32 ranges and always added the ranges up in a second launch, 1024 x 14336 with 16 rows 22.0 -> 19.4.
 //
 // Rounding points: fp32 accumulation over k, + bias in fp32, rounded to T -- what a library GEMM with a bias epilogue
 // does; then, if a residual is given, T(y + residual): the separate addition of llama.rs:166, 173, rounded again.
@@ -504,9 +507,9 @@ struct LinearPlan {
   size_t partial_bytes;  // fp32 sums of every range, [range][128 rows][N]; not used by the few-rows kernel
 };
 
-// The ranges of k depend on the weight alone (see above).  At least 1024 wavefronts' worth of (16 rows, range) pairs, four per
-// compute unit, and no range longer than 2048 once k is cut at all: 4096 x 4096 and 6144 x 4096 four, 4096 x 14336
-// eight, weights of 16384 rows and more none.
+// The ranges of k depend on the weight alone (see above).  As far as eight ranges allow: 1024 wavefronts' worth of (16 rows, range)
+// pairs, four per compute unit, and no range longer than 2048 once k is cut at all -- 4096 x 4096 and 6144 x 4096 four, 4096 x
+// 14336 eight, weights of 16384 rows and more none.
 LinearPlan plan_linear(int M, int N, int K) {
   const Tuning &tn = tuning();
   LinearPlan pl;
