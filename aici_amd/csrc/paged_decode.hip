@@ -1072,6 +1072,8 @@ int choose_part_blocks(int64_t S, int Hkv, int col_groups, int max_ctx) {
   return (int)pb;
 }
 
+constexpr size_t kStaticScratchBytes = (size_t)16 << 20;  // of hipattn_paged_attention_v1_static
+
 DecodePlan plan_decode(int64_t S, int Hq, int Hkv, int head_size, int block_size, int dtype, int max_context_len) {
   DecodePlan pl;
   pl.generic = takes_generic_kernel(dtype, block_size, head_size);
@@ -1104,8 +1106,9 @@ DecodePlan plan_decode(int64_t S, int Hq, int Hkv, int head_size, int block_size
       // at 64), and nothing where the launch is bound by memory.  So: contexts of one pair per wavefront, two pairs of small
       // heads, and whatever fits one lane-held slice of the table once the workgroups share the memory (128 of them; 192 for
       // the longest contexts of larger heads, which otherwise end last and alone).  Beyond two such workgroups per compute unit
-      // they gain nothing, and their last round loses, but at small heads, which keep winning up to 1024.  us, partitions / one
-      // workgroup, all contexts of that length (lengths uniform up to it):
+      // they gain nothing, and their last round loses, but at small heads, which keep winning up to 1024, and but where the partitions'
+      // results would not fit the built-in array (sixteen query heads per kv head, a thousand contexts), so that the entry point
+      // that uses it can serve them.  us, partitions / one workgroup, all contexts of that length (lengths uniform up to it):
       //   32 q / 8 kv x 128: 1 x 256 8.5 / 6.8, 1 x 512 8.3 / 9.7, 1 x 700 9.2 / 11.7, 16 x 512 13.6 / 12.5 (11.6 / 10.9), 16 x 1024 20.3 /
       //   20.1 (15.1 / 17.1), 24 x 1024 26.2 / 22.5 (20.2 / 18.5), 40 x 512 23.0 / 24.7 (18.4 / 15.8), 40 x 1024 36.7 / 40.9 (26.2 / 23.6),
       //   64 x 512 30.2 / 27.6, 72 x 512 35.6 / 38.6 (25.8 / 24.7), 104 x 512 47.4 / 51.5 (32.6 / 34.3); 32 / 32 x 80: 1 x 512 8.1 / 7.7,
@@ -1114,7 +1117,9 @@ DecodePlan plan_decode(int64_t S, int Hq, int Hkv, int head_size, int block_size
       const int64_t wgs = S * Hkv * col_groups;
       const bool small = head_size <= 64;
       const bool one_wg = max_blocks <= 16 || (max_blocks <= 32 && small) || (max_blocks <= 64 && wgs >= (small || max_blocks <= 48 ? 128 : 192));
-      if (tuning().decode_part_blocks <= 0 && head_size <= 128 && max_blocks > pl.part_blocks && wgs <= (small ? 1023 : 512) && one_wg) {
+      const size_t partials = (size_t)S * Hq * ((max_blocks + pl.part_blocks - 1) / pl.part_blocks) * (head_size + 2) * sizeof(float);
+      const int64_t most_wgs = small || partials > kStaticScratchBytes ? 1023 : 512;
+      if (tuning().decode_part_blocks <= 0 && head_size <= 128 && max_blocks > pl.part_blocks && wgs <= most_wgs && one_wg) {
         pl.part_blocks = 64;
         pl.waves = 8;
       }
@@ -1138,7 +1143,6 @@ struct Scratch {
 // The scratch array of hipattn_paged_attention_v1_static, the entry point that allocates nothing: device
 // memory that exists from the moment the code object is loaded, one copy per device.  In host code the
 // array's name is only a handle for hipGetSymbolAddress; kernels get the address that call returns.
-constexpr size_t kStaticScratchBytes = (size_t)16 << 20;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
 // The address of `scratch` on the current device, asked of the runtime once per device.

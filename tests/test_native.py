@@ -22,6 +22,12 @@ def test_arguments_are_checked_before_the_call():
         _native.reshape_and_cache(None, None, None, None, None)
 
 
+@pytest.mark.parametrize("S,Hkv,longest,d", [(1000, 1, 1024, 128), (1000, 1, 1024, 80), (1023, 1, 513, 128), (500, 2, 1024, 112), (250, 4, 1024, 96)])
+def test_static_scratch_holds_what_contexts_of_1024_tokens_need(S, Hkv, longest, d):
+    """Sixteen query heads per kv head: the partitions of that many contexts would not fit the built-in array."""
+    assert kernels.paged_attention_workspace_size(S, 16 * Hkv, Hkv, d, 16, longest, torch.bfloat16) <= 16 << 20
+
+
 @pytest.mark.parametrize("fn", ["hipattn_linear_workspace_size", "hipattn_linear_rms_norm_workspace_size"])
 @pytest.mark.parametrize("shape", [(4096, 14336), (6144, 4096), (16, 256), (512, 512)])
 def test_linear_workspace_depends_on_the_weight_alone(fn, shape):
