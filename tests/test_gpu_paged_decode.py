@@ -86,8 +86,8 @@ def test_context_edge_lengths_and_stale_cache_contents(device, dtype):
 
 @pytest.mark.parametrize("S,heads,longest,part_blocks", [
     (1, (32, 8, 128), 129, 0), (2, (8, 8, 64), 256, 0), (16, (32, 8, 128), 257, 0), (16, (8, 8, 96), 512, 0),   # a context per
-    (18, (32, 8, 128), 1024, 0), (65, (16, 2, 64), 1009, 0),                                                     # workgroup
-    (25, (32, 8, 128), 1024, 0), (64, (32, 8, 128), 300, 0), (65, (32, 8, 128), 300, 0), (511, (16, 2, 64), 40, 0),  # (or beyond)
+    (25, (32, 8, 128), 1024, 0), (65, (16, 2, 64), 1009, 0), (64, (32, 8, 128), 300, 0),                         # workgroup
+    (18, (32, 8, 128), 1024, 0), (65, (32, 8, 128), 300, 0), (512, (16, 2, 64), 200, 0),                         # no longer so
     (3, (32, 8, 128), 8 * 32, 2), (3, (8, 8, 80), 9 * 32, 2), (3, (16, 1, 64), 16 * 32, 2), (2, (8, 2, 256), 17 * 32, 2)])
 def test_whole_contexts_per_workgroup_and_merges_of_few_partitions(device, tuning, S, heads, longest, part_blocks):
     """Contexts of 0, 1, one pair per wavefront and one more, and the longest, where eight wavefronts share a context; and 8, 9, 16 and
