@@ -274,12 +274,14 @@ class BatchInfo:
             if w:
                 host[at:at + w] = v.numpy().reshape(-1).view(np.int32)
             at += p
-        parts = staged.to(device).split(padded)  # waits for the copy
-        for (k, v), w, part in zip(tensors.items(), words, parts):
+        there = torch.empty((sum(padded),), dtype=torch.int32, device=device)
+        for (k, v), w, part in zip(tensors.items(), words, there.split(padded)):
             if w != part.numel():
                 part = part[:w]
             kw[k] = (part if v.dtype == torch.int32 else part.view(v.dtype)).view(v.shape)
-        return BatchInfo(**kw)
+        batch = BatchInfo(**kw)
+        there.copy_(staged)  # waits for the copy, and so for the work queued before it: nothing is left to do behind it
+        return batch
 
 
 def _np(ptr, n: int, dtype) -> np.ndarray:

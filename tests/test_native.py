@@ -91,13 +91,17 @@ def _batch(lens):
 def test_batch_upload_waits_for_its_copy(monkeypatch):
     """No array may still be on its way when `to` returns: a caller uploads on one stream and runs the model on another."""
     asked = []
-    empty = torch.empty
-    monkeypatch.setattr(torch, "empty", lambda *a, pin_memory=False, **kw: empty(*a, **kw))  # no pinned memory without a GPU
+    empty, copy_ = torch.empty, torch.Tensor.copy_
+    monkeypatch.setattr(torch, "empty", lambda *a, pin_memory=False, device=None, **kw: empty(*a, **kw))  # there is no GPU here
     monkeypatch.setattr(torch.Tensor, "to", lambda t, *a, **kw: asked.append((a, kw)) or t.clone())
-    got = _batch([(37, 0), (5, 4)]).to("cuda")
-    assert len(asked) == 1 and got.slot_mapping.numel() == 38
+    monkeypatch.setattr(torch.Tensor, "copy_", lambda t, src, *a, **kw: asked.append((a, kw)) or copy_(t, src))
+    host = _batch([(37, 0), (5, 4)])
+    got = host.to("cuda")
     (args, kw), = asked
     assert not kw.get("non_blocking", False) and not any(a is True for a in args)
+    for name, want in host.__dict__.items():
+        if isinstance(want, torch.Tensor):
+            assert torch.equal(getattr(got, name), want), name
 
 
 @pytest.mark.gpu
