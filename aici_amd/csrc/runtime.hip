@@ -137,6 +137,21 @@ void *library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream) {
   return ws.ptr;
 }
 
+void *try_library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream) {
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (capturing != hipStreamCaptureStatusNone) return nullptr;
+  try {
+    return library_workspace(user, bytes, stream);
+  } catch (const Error &) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+}
+
 }  // namespace hipattn
 
 using namespace hipattn;

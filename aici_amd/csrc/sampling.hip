@@ -16,7 +16,8 @@
 //   Without a top-p cut the reference asks torch for `multinomial`, which draws from the same distribution
 //   by other means; here the same inverse-CDF rule is used for both.
 //
-// One workgroup of 1024 threads per row; the row is re-read from L2 in every pass.  Probability mass is
+// One workgroup of 1024 threads per row (bf16 rows of many tokens: one that finishes what several have counted, see
+// PieceCounts); the row is re-read from L2 in every pass.  Probability mass is
 // carried as an integer -- exp(x - max) in units of 2^-40 -- so sums do not depend on the order in which they
 // are formed: a launch gives the same token every time, whatever the scheduling, and whichever of the two ways below
 // is taken.  What bounds both is the vector unit (125 tokens per thread and pass at 128256 tokens), not memory.
@@ -29,9 +30,11 @@
 //   of the last kept value -- and with it the mass above and the number of equal values kept -- is known.
 //
 // 128 rows of 128256 bf16 logits, 5 % allowed, top-p 0.9: any row 199 us, counting 43 us; all allowed 221 / 55, one row
-// 177 / 40; fp16 203 / 60 (the logits take 5 us to read once; a pass over one row on one compute unit takes 6 to 12).
+// 177 / 40; fp16 203 / 60 (the logits take 5 us to read once; a pass over one row on one compute unit takes 6 to 12).  Counted in
+// pieces, bf16: 26 and, all allowed, 29 us; one row 15.
 #include "common.h"
 #include "device_types.h"
+#include "workspace.h"
 
 namespace hipattn {
 
@@ -92,42 +95,52 @@ __device__ __forceinline__ float block_max(float v, Scratch &s) {
   return r;
 }
 
-__device__ __forceinline__ u64 shfl_xor_u64(u64 v, int o) {
-  const unsigned lo = __shfl_xor((unsigned)v, o, 64), hi = __shfl_xor((unsigned)(v >> 32), o, 64);
+// v of the lane that DPP control CTRL names, zero where there is none.
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ u64 dpp_u64(u64 v) {
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)v, CTRL, ROWS, 0xf, false);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(v >> 32), CTRL, ROWS, 0xf, false);
   return ((u64)hi << 32) | lo;
 }
-__device__ __forceinline__ u64 shfl_up_u64(u64 v, int o) {
-  const unsigned lo = __shfl_up((unsigned)v, o, 64), hi = __shfl_up((unsigned)(v >> 32), o, 64);
+__device__ __forceinline__ u64 lane_u64(u64 v, int lane) {
+  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)v, lane), hi = __builtin_amdgcn_readlane((int)(unsigned)(v >> 32), lane);
   return ((u64)hi << 32) | lo;
 }
+// Inclusive prefix over the 16 lanes of a row, and over the wavefront.
+__device__ __forceinline__ u64 row_inclusive(u64 v) {
+  v += dpp_u64<0x111>(v);  // row_shr:1, 2, 4, 8
+  v += dpp_u64<0x112>(v);
+  v += dpp_u64<0x114>(v);
+  v += dpp_u64<0x118>(v);
+  return v;
+}
+__device__ __forceinline__ u64 wave_inclusive(u64 v) {
+  v = row_inclusive(v);
+  v += dpp_u64<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3, row_bcast:31 into rows 2 and 3
+  v += dpp_u64<0x143, 0xc>(v);
+  return v;
+}
+__device__ __forceinline__ u64 wave_sum(u64 v) { return lane_u64(wave_inclusive(v), 63); }
 
 __device__ __forceinline__ u64 block_sum(u64 v, Scratch &s) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += shfl_xor_u64(v, o);
+  static_assert(kWaves == 16, "a wavefront's sum per lane of a row");
+  v = wave_sum(v);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) s.wave_u64[threadIdx.x >> 6] = v;
   __syncthreads();
-  u64 r = 0;
-#pragma unroll
-  for (int w = 0; w < kWaves; w++) r += s.wave_u64[w];
-  return r;
+  return lane_u64(row_inclusive(s.wave_u64[threadIdx.x & 15]), 15);
 }
 
-// Exclusive prefix over the threads of the workgroup, in thread order.
-__device__ __forceinline__ u64 block_exclusive(u64 v, Scratch &s) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  u64 inc = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const u64 t = shfl_up_u64(inc, o);
-    if (lane >= o) inc += t;
-  }
+// Exclusive prefix over the threads of the workgroup, in thread order; `all`: the sum of them all.
+__device__ __forceinline__ u64 block_exclusive(u64 v, Scratch &s, u64 *all = nullptr) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const u64 inc = wave_inclusive(v);
   __syncthreads();
   if (lane == 63) s.wave_u64[wave] = inc;
   __syncthreads();
-  u64 before = 0;
-  for (int w = 0; w < wave; w++) before += s.wave_u64[w];
-  return before + inc - v;
+  const u64 waves = row_inclusive(s.wave_u64[lane & 15]);
+  if (all != nullptr) *all = lane_u64(waves, 15);
+  return (wave > 0 ? lane_u64(waves, wave - 1) : 0) + inc - v;
 }
 
 // The counted values of a 16-bit float type: magnitudes above kLo (2^-16 / 2^-8) of either sign, numbered by their bits;
@@ -154,10 +167,157 @@ struct Counted<half_t> {
 };
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ u64 wave_sum(u64 v) {
+// Tokens 8g .. 8g + 7 of a row of 16-bit logits and their allow-bits; nothing from group `end` on.
+template <typename T>
+__device__ __forceinline__ void load_tokens(const SampleParams &p, const T *lg, const uint8_t *mask, int g, int end, uint4 &raw,
+                                            unsigned &bits) {
+  const int V = p.vocab;
+  raw = make_uint4(0, 0, 0, 0);
+  bits = 0;
+  if (g >= end) return;
+  bits = g < p.mask_bytes ? mask[g] : 0u;
+  if (V - g * 8 >= 8) {
+    __builtin_memcpy(&raw, lg + g * 8, 16);
+  } else {
+    const unsigned short *e = reinterpret_cast<const unsigned short *>(lg) + g * 8;
+    unsigned w[4] = {0, 0, 0, 0};
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += shfl_xor_u64(v, o);
-  return v;
+    for (int j = 0; j < 8; j++)
+      if (j < V - g * 8) w[j / 2] |= (unsigned)e[j] << (16 * (j & 1));
+    raw = make_uint4(w[0], w[1], w[2], w[3]);
+    bits &= (1u << (V - g * 8)) - 1u;
+  }
+}
+__device__ __forceinline__ unsigned token_pair(const uint4 &raw, int i) {
+  return i == 0 ? raw.x : i == 1 ? raw.y : i == 2 ? raw.z : raw.w;
+}
+// order-preserving images of two values
+__device__ __forceinline__ unsigned value_images(unsigned w) {
+  typedef short i16x2 __attribute__((ext_vector_type(2)));
+  const unsigned sign = bit_cast<unsigned>(bit_cast<i16x2>(w) >> (short)15);
+  return w ^ (sign | 0x80008000u);
+}
+template <typename T>
+__device__ __forceinline__ float image_value(unsigned image) {  // of a 16-bit image
+  const unsigned short b = (unsigned short)((image & 0x8000u) ? (image & 0x7fffu) : ~image);
+  return to_float(bit_cast<T>(b));
+}
+// numbers of two values: their bits above kLo, with the sign
+template <typename T>
+__device__ __forceinline__ u16x2 value_numbers(unsigned w, u16x2 &mag) {
+  typedef short i16x2 __attribute__((ext_vector_type(2)));
+  const u16x2 sign = bit_cast<u16x2>(bit_cast<i16x2>(w) >> (short)15);
+  mag = __builtin_elementwise_sub_sat(bit_cast<u16x2>(w & 0x7fff7fffu), (u16x2)(unsigned short)Counted<T>::kLo);
+  return (mag ^ sign) - sign;
+}
+
+// Probability mass of a row's tokens: exp(x / temp - m) in units of 2^-40.  bins[o] holds, once filled, the mass of a token of
+// counter o's value as a float.
+template <typename T>
+struct Masses {
+  const unsigned *bins;
+  int top_number;  // of counter 0
+  float temp, m;
+
+  __device__ __forceinline__ unsigned image(int o) const {  // of counter o's value
+    const int number = top_number - o;                      // 0: the small ones
+    return (unsigned)(number >= 0 ? 0x8000 + number + Counted<T>::kLo : 0x7fff + number - Counted<T>::kLo);
+  }
+  __device__ __forceinline__ float value_mass_f(float v) const {  // before it is cut to an integer
+    const float x = v / temp;
+    return x > -INFINITY ? __builtin_amdgcn_exp2f((x - m) * kLog2e) * kMassUnit : 0.f;
+  }
+  __device__ __forceinline__ u64 value_mass(float v) const { return (u64)value_mass_f(v); }
+  __device__ __forceinline__ u64 token(const uint4 &raw, int j) const {
+    const unsigned b = (token_pair(raw, j >> 1) >> (16 * (j & 1))) & 0xffffu;
+    const int mag = (int)(b & 0x7fffu) - Counted<T>::kLo;
+    const int o = top_number - ((b & 0x8000u) ? -mag : mag);
+    if (mag > 0 && (unsigned)o < (unsigned)Counted<T>::kBins) return (u64)__uint_as_float(bins[o]);
+    return value_mass(to_float(bit_cast<T>((unsigned short)b)));
+  }
+  __device__ __forceinline__ u64 tokens(const uint4 &raw, unsigned which) const {
+    u64 sum = 0;
+    // many per thread: all looked up at once
+    if (__any(__builtin_popcount(which) > 2)) {
+      unsigned counted = 0;
+      float w[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const unsigned b = (token_pair(raw, j >> 1) >> (16 * (j & 1))) & 0xffffu;
+        const int mag = (int)(b & 0x7fffu) - Counted<T>::kLo;
+        const int o = top_number - ((b & 0x8000u) ? -mag : mag);
+        const bool has = mag > 0 && (unsigned)o < (unsigned)Counted<T>::kBins && ((which >> j) & 1);
+        counted |= has ? 1u << j : 0u;
+        w[j] = __uint_as_float(bins[has ? o : 0]);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; j++) sum += (counted >> j) & 1 ? (u64)w[j] : 0;
+      which &= ~counted;
+    }
+    while (which) {
+      const int j = __builtin_ctz(which);
+      which &= which - 1;
+      sum += token(raw, j);
+    }
+    return sum;
+  }
+};
+
+// The allowed tokens of a group above the value of image kstar, and (want_ties) those equal to it: bit j for token j.
+__device__ __forceinline__ unsigned kept_tokens(const uint4 &raw, unsigned bits, unsigned kstar, bool want_ties, unsigned &ties) {
+  unsigned gt = 0, other = 0;  // first bits 2i (even tokens) and 16 + 2i (odd ones)
+  const u16x2 limit = (u16x2)(unsigned short)kstar, one = {1, 1};
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const u16x2 w = bit_cast<u16x2>(value_images(token_pair(raw, i)));
+    gt |= bit_cast<unsigned>(__builtin_elementwise_min(__builtin_elementwise_sub_sat(w, limit), one)) << (2 * i);
+    other |= bit_cast<unsigned>(__builtin_elementwise_min((u16x2)(w ^ limit), one)) << (2 * i);
+  }
+  ties = want_ties ? ~(other | other >> 15) & 0xffu & bits : 0u;
+  return (gt | gt >> 15) & 0xffu & bits;
+}
+
+// Adds a group's allowed tokens to the counters of their values.  Those of a small magnitude, or without a counter, go to
+// listed(16 bits).
+template <typename T, typename F>
+__device__ __forceinline__ void count_tokens(unsigned *bins, int top_number, const uint4 &raw, unsigned bits, F &&listed) {
+  using C = Counted<T>;
+  if (!__any((int)bits)) return;
+  u16x2 off[4], least = {0xffff, 0xffff}, most = {0, 0};
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    u16x2 mag;
+    off[i] = (u16x2)(unsigned short)top_number - value_numbers<T>(token_pair(raw, i), mag);
+    least = __builtin_elementwise_min(least, mag);
+    most = __builtin_elementwise_max(most, off[i]);
+  }
+  if (min(least[0], least[1]) > 0 && max(most[0], most[1]) < C::kBins) {
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      if ((bits >> j) & 1) atomicAdd(&bins[off[j / 2][j & 1]], 1u);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      if ((bits >> j) & 1) {
+        const int o = off[j / 2][j & 1];
+        if (o != top_number && o < C::kBins) atomicAdd(&bins[o], 1u);
+        else listed((uint16_t)(token_pair(raw, j / 2) >> (16 * (j & 1))));
+      }
+  }
+}
+
+// ... and what such tokens weigh: f(16 bits) for each of the group's.
+template <typename T, typename F>
+__device__ __forceinline__ void for_listed(int top_number, const uint4 &raw, unsigned bits, F &&f) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    u16x2 mag;
+    const u16x2 off = (u16x2)(unsigned short)top_number - value_numbers<T>(token_pair(raw, i), mag);
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+      if (((bits >> (2 * i + k)) & 1) && (mag[k] == 0 || off[k] >= Counted<T>::kBins))
+        f((token_pair(raw, i) >> (16 * k)) & 0xffffu);
+  }
 }
 
 // The counting way.  False (for the whole workgroup): the row is not one it can decide, nothing was written -- a NaN or an
@@ -174,42 +334,7 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
   // a wavefront owns consecutive tokens (the draw goes in id order), its lanes take neighbouring groups
   const int per_wave = (groups + kWaves - 1) / kWaves;
   const int g0 = wave * per_wave, g1 = min(g0 + per_wave, groups);
-  auto load = [&](int g, int end, uint4 &raw, unsigned &bits) {
-    raw = make_uint4(0, 0, 0, 0);
-    bits = 0;
-    if (g >= end) return;
-    bits = g < p.mask_bytes ? mask[g] : 0u;
-    if (V - g * 8 >= 8) {
-      __builtin_memcpy(&raw, lg + g * 8, 16);
-    } else {
-      const unsigned short *e = reinterpret_cast<const unsigned short *>(lg) + g * 8;
-      unsigned w[4] = {0, 0, 0, 0};
-#pragma unroll
-      for (int j = 0; j < 8; j++)
-        if (j < V - g * 8) w[j / 2] |= (unsigned)e[j] << (16 * (j & 1));
-      raw = make_uint4(w[0], w[1], w[2], w[3]);
-      bits &= (1u << (V - g * 8)) - 1u;
-    }
-  };
-  auto pair = [](const uint4 &raw, int i) { return i == 0 ? raw.x : i == 1 ? raw.y : i == 2 ? raw.z : raw.w; };
-  // order-preserving images of two values
-  auto images = [](unsigned w) {
-    typedef short i16x2 __attribute__((ext_vector_type(2)));
-    const unsigned sign = bit_cast<unsigned>(bit_cast<i16x2>(w) >> (short)15);
-    return w ^ (sign | 0x80008000u);
-  };
-  auto value = [](unsigned image) {  // of a 16-bit image
-    const unsigned short b = (unsigned short)((image & 0x8000u) ? (image & 0x7fffu) : ~image);
-    return to_float(bit_cast<T>(b));
-  };
-
-  // numbers of two values: their bits above kLo, with the sign
-  auto numbers = [](unsigned w, u16x2 &mag) {
-    typedef short i16x2 __attribute__((ext_vector_type(2)));
-    const u16x2 sign = bit_cast<u16x2>(bit_cast<i16x2>(w) >> (short)15);
-    mag = __builtin_elementwise_sub_sat(bit_cast<u16x2>(w & 0x7fff7fffu), (u16x2)(unsigned short)C::kLo);
-    return (mag ^ sign) - sign;
-  };
+  auto load = [&](int g, int end, uint4 &raw, unsigned &bits) { load_tokens(p, lg, mask, g, end, raw, bits); };
   // every group of eight of this wavefront: f(raw, allow-bits)
   auto for_groups = [&](auto &&f) {
     for (int base = g0; base < g1; base += 64 * U) {
@@ -233,7 +358,7 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
       for (int i = 0; i < 4; i++) {
         const unsigned lo = __builtin_amdgcn_sbfe((int)bits, 2 * i, 1), hi = __builtin_amdgcn_sbfe((int)bits, 2 * i + 1, 1);
         const unsigned allowed = (lo & 0xffffu) | (hi & 0xffff0000u);
-        top = __builtin_elementwise_max(top, bit_cast<u16x2>(images(pair(raw, i)) & allowed));
+        top = __builtin_elementwise_max(top, bit_cast<u16x2>(value_images(token_pair(raw, i)) & allowed));
       }
     });
     const int image_max = (int)block_max((float)max(top[0], top[1]), s);
@@ -252,39 +377,15 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
   // Tokens per value.
   // Allowed ones of a small magnitude, or without a counter, are few, but every large batch has rows with some: listed.
   for_groups([&](const uint4 &raw, unsigned bits) {
-    if (!__any((int)bits)) return;
-    u16x2 off[4], least = {0xffff, 0xffff}, most = {0, 0};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      u16x2 mag;
-      off[i] = (u16x2)(unsigned short)top_number - numbers(pair(raw, i), mag);
-      least = __builtin_elementwise_min(least, mag);
-      most = __builtin_elementwise_max(most, off[i]);
-    }
-    if (min(least[0], least[1]) > 0 && max(most[0], most[1]) < C::kBins) {
-#pragma unroll
-      for (int j = 0; j < 8; j++)
-        if ((bits >> j) & 1) atomicAdd(&bins[off[j / 2][j & 1]], 1u);
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; j++)
-        if ((bits >> j) & 1) {
-          const int o = off[j / 2][j & 1];
-          if (o != top_number && o < C::kBins) atomicAdd(&bins[o], 1u);
-          else {
-            const int at = atomicAdd(&s.n_others, 1);
-            if (at < kThreads) s.others[at] = (uint16_t)(pair(raw, j / 2) >> (16 * (j & 1)));
-          }
-        }
-    }
+    count_tokens<T>(bins, top_number, raw, bits, [&](uint16_t b) {
+      const int at = atomicAdd(&s.n_others, 1);
+      if (at < kThreads) s.others[at] = b;
+    });
   });
   __syncthreads();
   const int others = s.n_others;
 
-  auto bin_image = [&](int o) {
-    const int number = top_number - o;  // 0: the small ones
-    return (unsigned)(number >= 0 ? 0x8000 + number + C::kLo : 0x7fff + number - C::kLo);
-  };
+  Masses<T> masses{bins, top_number, temp, 0.f};
   int largest = 0;  // counter of the row's largest value
   if constexpr (C::kTop != 0) {
     int found = C::kBins;
@@ -300,18 +401,13 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
     if (others > 0 && largest > top_number) return false;  // a small one may be the largest
   }
   if (!(temp < 1e15f)) return false;
-  const float m = value(bin_image(largest)) / temp;
-  if (!(fabsf(m) < INFINITY)) return false;
-  auto mass_f = [&](float v) {  // before it is cut to an integer
-    const float x = v / temp;
-    return x > -INFINITY ? __builtin_amdgcn_exp2f((x - m) * kLog2e) * kMassUnit : 0.f;
-  };
-  auto mass = [&](float v) -> u64 { return (u64)mass_f(v); };
+  masses.m = image_value<T>(masses.image(largest)) / temp;
+  if (!(fabsf(masses.m) < INFINITY)) return false;
   u64 small = 0, low = 0;  // mass of the small ones and of those below the counters
   if (others > 0) {
     bool above = false;
     auto add = [&](unsigned b) {
-      const u64 w = mass(to_float(bit_cast<T>((unsigned short)b)));
+      const u64 w = masses.value_mass(to_float(bit_cast<T>((unsigned short)b)));
       if ((int)(b & 0x7fffu) <= C::kLo) small += w;
       else if (b & 0x8000u) low += w;
       else above = true;  // fixed counters only: beyond 2^16, infinite, or not a number
@@ -319,16 +415,7 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
     if (others <= kThreads) {
       if (tid < others) add(s.others[tid]);
     } else {
-      for_groups([&](const uint4 &raw, unsigned bits) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          u16x2 mag;
-          const u16x2 off = (u16x2)(unsigned short)top_number - numbers(pair(raw, i), mag);
-#pragma unroll
-          for (int k = 0; k < 2; k++)
-            if (((bits >> (2 * i + k)) & 1) && (mag[k] == 0 || off[k] >= C::kBins)) add((pair(raw, i) >> (16 * k)) & 0xffffu);
-        }
-      });
+      for_groups([&](const uint4 &raw, unsigned bits) { for_listed<T>(top_number, raw, bits, add); });
     }
     if (__syncthreads_or(above)) return false;
     small = block_sum(small, s);
@@ -343,7 +430,7 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
     const int o = kOwn * tid + i;
     count[i] = bins[o];
     float f = 0.f;
-    if (count[i] != 0) f = mass_f(value(bin_image(o)));
+    if (count[i] != 0) f = masses.value_mass_f(image_value<T>(masses.image(o)));
     bins[o] = __float_as_uint(f);
     own += count[i] * (u64)f;
     if (o == top_number) own += small;
@@ -380,7 +467,7 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
     if (chosen < 0 || chosen == top_number) return false;  // among the small or the low ones
     const u64 mass_gt = s.hist[0];
     const unsigned ties = s.cnt[0];
-    kstar = bin_image(chosen);
+    kstar = masses.image(chosen);
     m_star = (u64)__uint_as_float(bins[chosen]);
     u64 need = (m_star && target > mass_gt) ? (target - mass_gt + m_star - 1) / m_star : 1;
     if (need < 1) need = 1;
@@ -394,41 +481,12 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
   const float u01 = fminf(fmaxf(uniform, 0.f), 1.f);  // outside [0, 1): the first or the last kept token
   u64 c = (u64)((double)u01 * (double)total);
   if (c >= total) c = total - 1;  // u * total rounded up to the total itself: the last token with a weight
-  // bit j: token j of the group is above kstar / equal to it
-  auto kept = [&](const uint4 &raw, unsigned bits, unsigned &ties) {
-    unsigned gt = 0, other = 0;  // first bits 2i (even tokens) and 16 + 2i (odd ones)
-    const u16x2 limit = (u16x2)(unsigned short)kstar, one = {1, 1};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const u16x2 w = bit_cast<u16x2>(images(pair(raw, i)));
-      gt |= bit_cast<unsigned>(__builtin_elementwise_min(__builtin_elementwise_sub_sat(w, limit), one)) << (2 * i);
-      other |= bit_cast<unsigned>(__builtin_elementwise_min((u16x2)(w ^ limit), one)) << (2 * i);
-    }
-    ties = n_keep > 0 ? ~(other | other >> 15) & 0xffu & bits : 0u;
-    return (gt | gt >> 15) & 0xffu & bits;
-  };
-  auto token_mass = [&](const uint4 &raw, int j) {
-    const unsigned b = (pair(raw, j >> 1) >> (16 * (j & 1))) & 0xffffu;
-    const int mag = (int)(b & 0x7fffu) - C::kLo;
-    const int o = top_number - ((b & 0x8000u) ? -mag : mag);
-    if (mag > 0 && (unsigned)o < (unsigned)C::kBins) return (u64)__uint_as_float(bins[o]);
-    return mass(to_float(bit_cast<T>((unsigned short)b)));
-  };
-  auto mass_of = [&](const uint4 &raw, unsigned gt) {
-    u64 sum = 0;
-    while (gt) {
-      const int j = __builtin_ctz(gt);
-      gt &= gt - 1;
-      sum += token_mass(raw, j);
-    }
-    return sum;
-  };
   u64 my_gt = 0;
   int my_ties = 0;
   for_groups([&](const uint4 &raw, unsigned bits) {
     unsigned ties;
-    const unsigned gt = kept(raw, bits, ties);
-    my_gt += mass_of(raw, gt);
+    const unsigned gt = kept_tokens(raw, bits, kstar, n_keep > 0, ties);
+    my_gt += masses.tokens(raw, gt);
     my_ties += __builtin_popcount(ties);
   });
   my_gt = wave_sum(my_gt);
@@ -453,16 +511,16 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
     uint4 raw;
     unsigned bits, ties;
     load(base + tid, end, raw, bits);
-    const unsigned gt = kept(raw, bits, ties);
+    const unsigned gt = kept_tokens(raw, bits, kstar, n_keep > 0, ties);
     const int n_ties = __builtin_popcount(ties);
     const int first_rank = n_keep > 0 ? rank + (int)block_exclusive((u64)n_ties, s) : 0;
-    const u64 sum = mass_of(raw, gt) + (u64)max(0, min(n_ties, n_keep - first_rank)) * m_star;
+    const u64 sum = masses.tokens(raw, gt) + (u64)max(0, min(n_ties, n_keep - first_rank)) * m_star;
     u64 at = run + block_exclusive(sum, s);
     if (sum > 0 && at <= c && at + sum > c) {
       int r = first_rank, token = 0;
       for (int j = 0; j < 8; j++) {
         u64 w = 0;
-        if ((gt >> j) & 1) w = token_mass(raw, j);
+        if ((gt >> j) & 1) w = masses.token(raw, j);
         else if ((ties >> j) & 1) w = r++ < n_keep ? m_star : 0;
         at += w;
         if (w && at > c) {
@@ -480,9 +538,334 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
   return true;
 }
 
-// COUNT: with the counting way and the LDS that it takes.
-template <typename T, int MODE /*0 = f32 bias rows, 1 = packed allow-bits*/, bool COUNT>
-__global__ __launch_bounds__(kThreads) void bias_sample_kernel(SampleParams p) {
+// The counting way with a row's tokens dealt out to several workgroups: pieces of kPieceTokens consecutive tokens are counted by
+// a workgroup each (sample_count_kernel), which leaves the counters in memory; the row's workgroup (sample_pieces) adds them up, finds
+// the nucleus from them, knows from a piece's own counters what the piece weighs, and looks at the tokens of one piece only.
+// us, 128256 tokens, 5 % allowed, top-p 0.9, one workgroup / pieces: 1 row 38.3 / 15.4, 32 rows 42.7 / 19.8, 128 rows 44.6 / 25.9 (12 of
+// them the count, which moves 52 MB with its counters, 13 the row's part: a chain of barriers and instructions on one compute
+// unit), 256 rows 48.1 / 36.9; all allowed without a cut, 128 rows, 70.6 / 35.6.  Pieces from 24576 tokens on: 20000 tokens, 256 rows, no
+// cut 28.5 / 29.6 (with a cut 25.0 / 19.9), 32000 tokens 32.0 / 30.9 (26.4 / 21.2).  Only what is not all zero written and read of the
+// counters: 0.7 us less in the count, 0.7 more in the row's part.
+constexpr int kPieceTokens = 16384;  // no counter above 16 bits
+constexpr int kCountThreads = 512;   // four workgroups per compute unit, by LDS and by wavefronts
+constexpr int kLeastPieces = 24576;  // tokens
+constexpr int kMaxPieces = kWaves;   // a wavefront of the row's workgroup for each
+constexpr int kPieceListed = 1016;
+struct PieceCounts {
+  uint16_t counts[Counted<bf16_t>::kBins];
+  int n_others, pad[3];
+  uint16_t others[kPieceListed];
+};
+
+template <typename T>
+__global__ __launch_bounds__(kCountThreads) void sample_count_kernel(SampleParams p, PieceCounts *scratch) {
+  using C = Counted<T>;
+  static_assert(C::kTop != 0, "counters that do not depend on the row's largest value");
+  constexpr int kOwn = 8;                                   // counters per 16-byte store
+  constexpr int U = kPieceTokens / 8 / kCountThreads;       // groups of 8 tokens per thread, all in flight
+  __shared__ __align__(16) unsigned bins[C::kBins];
+  __shared__ uint16_t listed[kPieceListed];
+  __shared__ int n_others;
+  const int tid = threadIdx.x, piece = blockIdx.x;
+  const int64_t seq = blockIdx.y;
+  if (!((p.temperature ? p.temperature[seq] : 0.f) >= kSamplingEps)) return;  // greedy: nothing is drawn
+  int64_t row = p.rows ? (int64_t)p.rows[seq] : seq;
+  row = row < 0 ? 0 : (row >= p.nrows ? p.nrows - 1 : row);
+  const T *lg = static_cast<const T *>(p.logits) + seq * p.logit_stride;
+  const uint8_t *mask = p.mask + row * p.mask_stride;
+  const int groups = (p.vocab + 7) / 8, g0 = piece * (kPieceTokens / 8), end = min(g0 + kPieceTokens / 8, groups);
+  uint4 raw[U];
+  unsigned bits[U];
+#pragma unroll
+  for (int u = 0; u < U; u++) load_tokens(p, lg, mask, g0 + u * kCountThreads + tid, end, raw[u], bits[u]);
+#pragma unroll
+  for (int i = 0; i < C::kBins / 4 / kCountThreads; i++) *reinterpret_cast<uint4 *>(bins + 4 * (tid + i * kCountThreads)) = make_uint4(0, 0, 0, 0);
+  if (tid == 0) n_others = 0;
+  auto list = [&](unsigned b, int n) {
+    for (int at = atomicAdd(&n_others, n), to = min(at + n, kPieceListed); at < to; at++) listed[at] = (uint16_t)b;
+  };
+  __syncthreads();
+  // Places here: 4096 magnitudes above kLo in ascending order, positive, then negative.  A value's place takes no comparison of
+  // signs, and the order that the row's workgroup wants is made when the counters leave.
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    if (!__any((int)bits[u])) continue;
+    unsigned mag[4], at[4], far = 0;  // at: byte offsets of the places
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      mag[i] = bit_cast<unsigned>((u16x2)(bit_cast<u16x2>(token_pair(raw[u], i)) - (u16x2)(unsigned short)(C::kLo + 1)));
+      at[i] = ((mag[i] << 2) & 0x3ffc3ffcu) | ((mag[i] >> 1) & 0x40004000u);
+      far |= mag[i];
+    }
+    if ((far & 0x70007000u) == 0) {
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        if ((bits[u] >> j) & 1) atomicAdd(&bins[((at[j / 2] >> (16 * (j & 1))) & 0xffffu) / 4], 1u);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        if ((bits[u] >> j) & 1) {
+          if (((mag[j / 2] >> (16 * (j & 1))) & 0x7000u) == 0) atomicAdd(&bins[((at[j / 2] >> (16 * (j & 1))) & 0xffffu) / 4], 1u);
+          else list((token_pair(raw[u], j / 2) >> (16 * (j & 1))) & 0xffffu, 1);
+        }
+    }
+  }
+  __syncthreads();
+  static_assert(C::kTop == 4096 && C::kBins == 2 * C::kTop, "the places above");
+  if (const unsigned n = bins[C::kBins - 1]) {  // -2^16: the row's counters end just above it
+    if (tid == 0) list(0x8000u | (C::kLo + C::kTop), (int)n);
+    __syncthreads();
+  }
+  PieceCounts &out = scratch[seq * gridDim.x + piece];
+  // counters 0 .. 4095 are the positive values from the largest down, 4096 the listed ones', then the negative ones
+#pragma unroll
+  for (int i = 0; i < C::kBins / kOwn / kCountThreads; i++) {
+    const int o = kOwn * (tid + i * kCountThreads);
+    const bool positive = o < C::kTop;
+    const unsigned *src = bins + (positive ? C::kTop - kOwn - o : o);
+    const uint4 a = *reinterpret_cast<const uint4 *>(src), b = *reinterpret_cast<const uint4 *>(src + 4);
+    const unsigned before = o <= C::kTop ? 0u : bins[o - 1];
+    *reinterpret_cast<uint4 *>(out.counts + o) =
+        positive ? make_uint4(b.w | b.z << 16, b.y | b.x << 16, a.w | a.z << 16, a.y | a.x << 16)
+                 : make_uint4(before | a.x << 16, a.y | a.z << 16, a.w | b.x << 16, b.y | b.z << 16);
+  }
+  const int others = n_others;
+  if (tid == 0) out.n_others = others;
+  for (int i = tid; i < min(others, kPieceListed); i += kCountThreads) out.others[i] = listed[i];
+}
+
+// The row's part of it.  False (for the whole workgroup) under the same conditions as sample_counted, and the same token otherwise.
+template <typename T>
+__device__ __forceinline__ bool sample_pieces(const SampleParams &p, Scratch &s, unsigned *bins, const PieceCounts *pieces, int n_pieces,
+                                              const T *lg, const uint8_t *mask, float temp, float top_p, float uniform, int32_t *out) {
+  using C = Counted<T>;
+  constexpr int kOwn = C::kBins / kThreads;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int groups = (p.vocab + 7) / 8;
+  const PieceCounts &mine = pieces[min(wave, n_pieces - 1)];  // a wavefront for each piece
+  const int my_others = wave < n_pieces ? mine.n_others : 0;
+  // (What this costs is instructions: sixteen wavefronts share four SIMDs.  So: wavefronts whose counters are all zero -- half of
+  // them -- skip what they can, three pieces' counters are added two at a time before they are taken apart (3 x 16384 fits), and
+  // what is the same for all is worked out by one wavefront where it is long.)
+  unsigned count[kOwn] = {};
+  for (int q0 = 0; q0 < n_pieces; q0 += 8) {
+    uint4 c[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      c[i] = make_uint4(0, 0, 0, 0);
+      if (q0 + i < n_pieces) c[i] = *reinterpret_cast<const uint4 *>(pieces[q0 + i].counts + kOwn * tid);
+    }
+    unsigned any = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) any |= c[i].x | c[i].y | c[i].z | c[i].w;
+    if (__any((int)any)) {
+#pragma unroll
+      for (int i = 0; i < 8; i += 3)
+#pragma unroll
+        for (int k = 0; k < kOwn / 2; k++) {
+          u16x2 n = bit_cast<u16x2>(token_pair(c[i], k)) + bit_cast<u16x2>(token_pair(c[i + 1], k));
+          if (i + 2 < 8) n += bit_cast<u16x2>(token_pair(c[i + 2 < 8 ? i + 2 : 0], k));
+          count[2 * k] += n[0];
+          count[2 * k + 1] += n[1];
+        }
+    }
+  }
+  unsigned present = 0;  // bit i: counter i of this thread is not zero
+#pragma unroll
+  for (int i = 0; i < kOwn; i++) present |= count[i] != 0 ? 1u << i : 0u;
+  const u64 lanes = __ballot(present != 0);
+  const bool wave_empty = lanes == 0;
+  if (lane == 0) s.wave_int[wave] = my_others > 0;
+  if (lanes != 0 && lane == __builtin_ctzll(lanes)) s.cnt[wave] = kOwn * tid + __builtin_ctz(present);
+  if (lanes == 0 && lane == 0) s.cnt[wave] = C::kBins;
+  __syncthreads();
+  const unsigned wave_first = s.cnt[lane & 15];  // a wavefront's first counter that is not zero: its largest value
+  const u64 not_empty = __ballot(wave_first != C::kBins);
+  const bool any_others = __any(s.wave_int[lane & 15]);
+  const int largest = not_empty == 0 ? C::kBins : __builtin_amdgcn_readlane((int)wave_first, __builtin_ctzll(not_empty));
+  if (not_empty == 0) {
+    if (any_others) return false;
+    if (tid == 0) *out = 0;  // nothing allowed: no distribution to draw from
+    return true;
+  }
+  if (any_others && largest > C::kTop) return false;  // a small one may be the largest
+  if (!(temp < 1e15f)) return false;
+  Masses<T> masses{bins, C::kTop, temp, 0.f};
+  masses.m = image_value<T>(masses.image(largest)) / temp;
+  if (!(fabsf(masses.m) < INFINITY)) return false;
+  u64 my_small = 0, my_low = 0, small = 0, low = 0;  // mass of this wavefront's, of all pieces' small tokens and of those below the counters
+  if (any_others) {
+    bool above = false;
+    auto add = [&](unsigned b) {
+      const u64 w = masses.value_mass(to_float(bit_cast<T>((unsigned short)b)));
+      if ((int)(b & 0x7fffu) <= C::kLo) my_small += w;
+      else if (b & 0x8000u) my_low += w;
+      else above = true;  // beyond 2^16, infinite, or not a number
+    };
+    if (my_others <= kPieceListed) {
+      for (int i = lane; i < my_others; i += 64) add(mine.others[i]);
+    } else {
+      const int g0 = wave * (kPieceTokens / 8), end = min(g0 + kPieceTokens / 8, groups);
+      for (int g = g0 + lane; g < end; g += 64) {
+        uint4 raw;
+        unsigned bits;
+        load_tokens(p, lg, mask, g, end, raw, bits);
+        for_listed<T>(C::kTop, raw, bits, add);
+      }
+    }
+    if (__syncthreads_or(above)) return false;
+    my_small = wave_sum(my_small);
+    my_low = wave_sum(my_low);
+    small = block_sum(lane == 0 ? my_small : 0, s);
+    low = block_sum(lane == 0 ? my_low : 0, s);
+  }
+  // Thread t owns counters [kOwn t, kOwn (t + 1)): thread order is descending order of the values.
+  u64 own = 0;
+  float weight[kOwn] = {};  // of one token of the counter's value
+  if (!wave_empty) {
+#pragma unroll
+    for (int i = 0; i < kOwn; i++)
+      if (count[i] != 0) {
+        weight[i] = masses.value_mass_f(image_value<T>(masses.image(kOwn * tid + i)));
+        own += count[i] * (u64)weight[i];
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < kOwn; i += 4)
+    *reinterpret_cast<f32x4_t *>(bins + kOwn * tid + i) = f32x4_t{weight[i], weight[i + 1], weight[i + 2], weight[i + 3]};
+  static_assert(C::kTop % kOwn == 0, "the small ones stand first among their thread's counters, and have no counts");
+  if (tid == C::kTop / kOwn) own += small;
+  if (tid == 0) s.pick = -1;
+  u64 z;
+  const u64 before = block_exclusive(own, s, &z);
+  z += low;
+  const bool cut = top_p > 0.f && top_p < 1.0f;
+  unsigned kstar = 0;  // image of the last kept value; below every image that is counted: everything is kept
+  int n_keep = 0, chosen = C::kBins;
+  u64 m_star = 0, total = z;
+  if (cut) {
+    // exactly one thread's values cross the target (from below it to it or beyond), or none; it works out what follows
+    const u64 target = (u64)((double)top_p * (double)z);
+    if (own && (before < target || (target == 0 && before == 0)) && before + own >= target) {
+      u64 above = before, gt = 0, one = 0;
+      int o = -1;
+      unsigned ties = 0;
+#pragma unroll
+      for (int i = 0; i < kOwn; i++) {
+        const u64 w = (u64)weight[i], h = (i == 0 && tid == C::kTop / kOwn) ? small : count[i] * w;
+        if (o < 0 && h && above + h >= target) {
+          o = kOwn * tid + i;
+          gt = above;
+          one = w;
+          ties = count[i];
+        }
+        above += h;
+      }
+      u64 need = (one && target > gt) ? (target - gt + one - 1) / one : 1;
+      if (need < 1) need = 1;
+      if (need > ties) need = ties;
+      s.pick = o;
+      s.n_others = (int)need;
+      s.hist[0] = one;
+      s.hist[1] = gt + need * one;
+    }
+    __syncthreads();
+    chosen = s.pick;
+    if (chosen < 0 || chosen == C::kTop) return false;  // among the small or the low ones
+    kstar = masses.image(chosen);
+    n_keep = s.n_others;
+    m_star = s.hist[0];
+    total = s.hist[1];
+  }
+  // What each piece weighs: its wavefront adds its counters from the row's largest value down to the last kept one.  (The barriers
+  // above, in block_exclusive or behind it, say that every counter's weight is in its place.)
+  {
+    u64 sum = 0;
+    int ties = 0;
+    if (wave < n_pieces) {
+      for (int base = largest & ~511; base < chosen; base += 2048) {
+        uint4 c[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) c[i] = *reinterpret_cast<const uint4 *>(mine.counts + min(base + 512 * i, C::kBins - 512) + kOwn * lane);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int o = base + 512 * i + kOwn * lane;
+          if (o >= chosen || (c[i].x | c[i].y | c[i].z | c[i].w) == 0) continue;
+          const f32x4_t w0 = *reinterpret_cast<const f32x4_t *>(bins + o), w1 = *reinterpret_cast<const f32x4_t *>(bins + o + 4);
+#pragma unroll
+          for (int k = 0; k < kOwn; k++) {
+            const unsigned n = (token_pair(c[i], k / 2) >> (16 * (k & 1))) & 0xffffu;
+            if (n != 0 && o + k < chosen) sum += n * (u64)(k < 4 ? w0[k & 3] : w1[k & 3]);
+          }
+        }
+      }
+      sum = wave_sum(sum);
+      if (chosen > C::kTop) sum += my_small;
+      if (!cut) sum += my_low;
+      if (n_keep > 0) ties = mine.counts[chosen];
+    }
+    if (lane == 0) {
+      s.hist[16 + wave] = sum;  // (wave_u64 may still be read by a wavefront that is in block_exclusive)
+      s.wave_int[wave] = ties;
+    }
+  }
+  __syncthreads();
+  // The draw, in id order: the piece that holds the winner, and its tokens, sixteen per thread.
+  const float u01 = fminf(fmaxf(uniform, 0.f), 1.f);  // outside [0, 1): the first or the last kept token
+  u64 c = (u64)((double)u01 * (double)total);
+  if (c >= total) c = total - 1;  // u * total rounded up to the total itself: the last token with a weight
+  // lane i: piece i
+  const int p_ties = (lane & 15) < n_pieces ? s.wave_int[lane & 15] : 0;
+  const u64 p_gt = (lane & 15) < n_pieces ? s.hist[16 + (lane & 15)] : 0;
+  const u64 ties_to = row_inclusive((u64)p_ties), gt_to = row_inclusive(p_gt);
+  const u64 weight_to = gt_to + min(ties_to, (u64)n_keep) * m_star;
+  const u64 reaches = __ballot(weight_to > c) & ((1u << n_pieces) - 1u);
+  const int winner = reaches != 0 ? __builtin_ctzll(reaches) : n_pieces - 1;
+  const u64 rank0 = winner > 0 ? lane_u64(ties_to, winner - 1) : 0, gt0 = winner > 0 ? lane_u64(gt_to, winner - 1) : 0;
+  const int first = winner * (kPieceTokens / 8), end = min(first + kPieceTokens / 8, groups);
+  uint4 raw[2];
+  unsigned bits[2], gt[2], ties[2];
+#pragma unroll
+  for (int u = 0; u < 2; u++) load_tokens(p, lg, mask, first + 2 * tid + u, end, raw[u], bits[u]);
+#pragma unroll
+  for (int u = 0; u < 2; u++) gt[u] = kept_tokens(raw[u], bits[u], kstar, n_keep > 0, ties[u]);
+  const u64 my_ties = __builtin_popcount(ties[0] | ties[1] << 8);
+  const u64 my_gt = masses.tokens(raw[0], gt[0]) + masses.tokens(raw[1], gt[1]);
+  // weight of everything in front of this thread's tokens: the values above the last kept one, and as many of those as are kept
+  u64 rank = rank0, ahead = gt0;
+  {
+    const u64 ties_in = n_keep > 0 ? wave_inclusive(my_ties) : 0, gt_in = wave_inclusive(my_gt);
+    if (lane == 63) {
+      s.wave_u64[wave] = gt_in;
+      s.hist[wave] = ties_in;
+    }
+    __syncthreads();
+    const u64 waves_gt = row_inclusive(s.wave_u64[lane & 15]), waves_ties = row_inclusive(s.hist[lane & 15]);
+    rank += (wave > 0 ? lane_u64(waves_ties, wave - 1) : 0) + ties_in - my_ties;
+    ahead += (wave > 0 ? lane_u64(waves_gt, wave - 1) : 0) + gt_in - my_gt;
+  }
+  u64 at = ahead + min(rank, (u64)n_keep) * m_star;
+  const u64 to = ahead + my_gt + min(rank + my_ties, (u64)n_keep) * m_star;
+  if (at <= c && to > c) {
+    int token = 0;
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+      for (unsigned left = gt[u] | ties[u]; left != 0; left &= left - 1) {
+        const int j = __builtin_ctz(left);
+        const u64 w = (gt[u] >> j) & 1 ? masses.token(raw[u], j) : rank++ < (u64)n_keep ? m_star : 0;
+        if (w && at <= c && at + w > c) token = (first + 2 * tid + u) * 8 + j;
+        at += w;
+      }
+    *out = token;
+  }
+  return true;
+}
+
+enum { SAMPLE_ANY = 0, SAMPLE_COUNTED = 1, SAMPLE_PIECES = 2 };
+
+// HOW: with the counting way and the LDS that it takes, or with the row's part of it behind sample_count_kernel.
+template <typename T, int MODE /*0 = f32 bias rows, 1 = packed allow-bits*/, int HOW>
+__global__ __launch_bounds__(kThreads) void bias_sample_kernel(SampleParams p, const PieceCounts *pieces, int n_pieces) {
   __shared__ Scratch s;
   const int tid = threadIdx.x;
   const int64_t seq = blockIdx.x;
@@ -490,7 +873,9 @@ __global__ __launch_bounds__(kThreads) void bias_sample_kernel(SampleParams p) {
   row = row < 0 ? 0 : (row >= p.nrows ? p.nrows - 1 : row);  // a bad row index reads a wrong row, never outside
   const T *lg = static_cast<const T *>(p.logits) + seq * p.logit_stride;
   const int V = p.vocab;
+  // (asked for together: one after the other they are three waits)
   const float temp = p.temperature ? p.temperature[seq] : 0.f;
+  const float top_p = p.top_p ? p.top_p[seq] : 1.0f, uniform = p.uniforms[seq];
   const bool greedy = !(temp >= kSamplingEps);
   const int groups = (V + 7) / 8;  // tokens are handled eight at a time: one mask byte, 16 bytes of 2-byte logits
 
@@ -566,12 +951,17 @@ __global__ __launch_bounds__(kThreads) void bias_sample_kernel(SampleParams p) {
     return;
   }
 
-  const float top_p = p.top_p ? p.top_p[seq] : 1.0f;
   const bool cut = top_p > 0.f && top_p < 1.0f;
-  if constexpr (COUNT) {
+  if constexpr (HOW == SAMPLE_PIECES) {
+    __shared__ __align__(16) unsigned bins[Counted<T>::kBins];
+    if (sample_pieces<T>(p, s, bins, pieces + seq * n_pieces, n_pieces, lg, p.mask + row * p.mask_stride, temp, top_p, uniform, p.out_tokens + seq))
+      return;
+    __syncthreads();
+  }
+  if constexpr (HOW == SAMPLE_COUNTED) {
     __shared__ unsigned bins[Counted<T>::kBins];
     if (V >= (cut ? Counted<T>::kLeastCut : Counted<T>::kLeastAll)) {
-      if (sample_counted<T>(p, s, bins, lg, p.mask + row * p.mask_stride, temp, top_p, p.uniforms[seq], p.out_tokens + seq)) return;
+      if (sample_counted<T>(p, s, bins, lg, p.mask + row * p.mask_stride, temp, top_p, uniform, p.out_tokens + seq)) return;
       __syncthreads();
     }
   }
@@ -690,7 +1080,7 @@ __global__ __launch_bounds__(kThreads) void bias_sample_kernel(SampleParams p) {
   }
 
   // The draw, in id order: thread t owns the contiguous token groups [t C, (t + 1) C).
-  const float u = fminf(fmaxf(p.uniforms[seq], 0.f), 1.f);  // outside [0, 1): the first or the last kept token
+  const float u = fminf(fmaxf(uniform, 0.f), 1.f);  // outside [0, 1): the first or the last kept token
   const u64 c = (u64)((double)u * (double)total);
   const int C = (groups + kThreads - 1) / kThreads;
   const int g_begin = min(tid * C, groups), g_end = min(g_begin + C, groups);
@@ -817,11 +1207,24 @@ void bias_sample_impl(const hipattn_tensor *logits, const hipattn_tensor *bias, 
   p.uniforms = static_cast<const float *>(uniforms->data);
   p.out_tokens = static_cast<int32_t *>(out_tokens->data);
   HA_CHECK(S <= 0x7fffffff, "%s: too many sequences", op);
+  // Pieces, where there are several and workgroups for them: the scratch memory then stays below 40 MB.  Under capture the row's
+  // workgroup does it alone: the graph may be replayed beside other calls on this stream's scratch memory.
+  const int64_t n_pieces = (V + kPieceTokens - 1) / kPieceTokens;
+  PieceCounts *pieces = nullptr;
+  if (mask && logits->dtype == HIPATTN_BF16 && V >= kLeastPieces && n_pieces <= kMaxPieces && S * n_pieces <= 2048)
+    pieces = static_cast<PieceCounts *>(try_library_workspace(WS_SAMPLE, (size_t)(S * n_pieces) * sizeof(PieceCounts), stream));
+  if (pieces != nullptr) {
+    sample_count_kernel<bf16_t><<<dim3((unsigned)n_pieces, (unsigned)S), kCountThreads, 0, stream>>>(p, pieces);
+    check_launch(op);
+    bias_sample_kernel<bf16_t, 1, SAMPLE_PIECES><<<dim3((unsigned)S), kThreads, 0, stream>>>(p, pieces, (int)n_pieces);
+    check_launch(op);
+    return;
+  }
 #define HA_BS(TT)                                                                                                   \
-  if (bias) bias_sample_kernel<TT, 0, false><<<dim3((unsigned)S), kThreads, 0, stream>>>(p);                         \
+  if (bias) bias_sample_kernel<TT, 0, SAMPLE_ANY><<<dim3((unsigned)S), kThreads, 0, stream>>>(p, nullptr, 0);        \
   else if (!Counted<TT>::possible || p.vocab < Counted<TT>::kLeastCut)                                               \
-    bias_sample_kernel<TT, 1, false><<<dim3((unsigned)S), kThreads, 0, stream>>>(p);                                 \
-  else bias_sample_kernel<TT, 1, Counted<TT>::possible><<<dim3((unsigned)S), kThreads, 0, stream>>>(p)
+    bias_sample_kernel<TT, 1, SAMPLE_ANY><<<dim3((unsigned)S), kThreads, 0, stream>>>(p, nullptr, 0);                \
+  else bias_sample_kernel<TT, 1, Counted<TT>::possible ? SAMPLE_COUNTED : SAMPLE_ANY><<<dim3((unsigned)S), kThreads, 0, stream>>>(p, nullptr, 0)
   switch (logits->dtype) {
     case HIPATTN_F32: HA_BS(float); break;
     case HIPATTN_F16: HA_BS(half_t); break;

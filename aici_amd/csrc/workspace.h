@@ -8,7 +8,7 @@
 namespace hipattn {
 
 // Which op a library-owned scratch buffer belongs to: ops never share one.
-enum WorkspaceUser { WS_PAGED_ATTENTION = 0, WS_BIAS_ARGMAX = 1, WS_LINEAR = 2 };
+enum WorkspaceUser { WS_PAGED_ATTENTION = 0, WS_BIAS_ARGMAX = 1, WS_LINEAR = 2, WS_SAMPLE = 3 };
 
 // Returns at least `bytes` of device memory on the current device for `user`,
 // private to `stream`: calls on different streams never share a buffer, so
@@ -18,6 +18,10 @@ enum WorkspaceUser { WS_PAGED_ATTENTION = 0, WS_BIAS_ARGMAX = 1, WS_LINEAR = 2 }
 // that is being captured cannot grow its buffer: the call fails with a
 // message that says so.
 void *library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream);
+
+// The same for an op that has another way without scratch memory: null while the stream is being captured (also where the buffer is
+// there: a graph may be replayed on any stream, beside calls that use it) and where there is no memory to be had.
+void *try_library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream);
 
 // Switches for tuning and for tests that want one particular kernel; read
 // from the environment (HIPATTN_<NAME in capitals>) once, when the library is

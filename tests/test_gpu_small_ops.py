@@ -316,6 +316,45 @@ def test_bias_sample_counts_equal_logits_to_the_same_tokens(device, dtype, V, sh
     assert torch.equal(got, want), torch.nonzero(got != want).flatten().tolist()
 
 
+@pytest.mark.parametrize("V", [24575, 24576, 32768, 32776, 128256, 262144, 262152])
+def test_bias_sample_in_pieces_gives_the_same_tokens(device, V):
+    """bf16 rows of 24576 to 262144 tokens are counted by a workgroup per 16384 of them.  The same values in float32 take the
+    other way: the same tokens, whatever the values -- at and beyond both ends of the counters (2^-16, 2^16), small ones too
+    many to be listed, whole rows of one value, pieces without an allowed token -- and however many pieces; and a captured call,
+    which keeps to one workgroup per row, replays them."""
+    g = torch.Generator().manual_seed(V)
+    n = torch.randn((9, V), generator=g)
+    edge = torch.tensor([-65536.0, 65536.0, 2.0 ** -16, -2.0 ** -16, 65280.0, 0.0, -0.0, 1.0])
+    edge = edge[torch.randint(0, 8, (2, V), generator=g)]
+    kinds = torch.stack([n[0] * 2.5, n[1] * 0.5 - 30, n[2] * 0, n[3].round(), torch.where(n[4] > 0.5, n[4] * 0, n[4]), n[5] * 1e-6,
+                         n[6] * 40, n[7] * 0 + 1.5, edge[0], torch.where(edge[1] > 2, edge[1] * 0 + 3, edge[1])])
+    rows = kinds.repeat_interleave(6, 0).to(torch.bfloat16)
+    S = rows.size(0)
+    allowed = torch.rand((S, V), generator=g) < torch.tensor([0.05, 1.0, 0.001]).repeat(S // 3)[:, None]
+    allowed[1::4, :16384] = False
+    allowed[:, V - 1] = True
+    allowed[5] = False
+    mask = torch.from_numpy(np.stack([aici.pack_allowed(a) for a in allowed.numpy()])).to(device)
+    temperature = torch.tensor([0.8, 0.3, 1.5, 20.0, 0.0]).repeat(S // 5).to(device)
+    top_p = torch.tensor([0.9, 1.0, 0.5, 0.9999]).repeat(S // 4 + 1)[:S].to(device)
+    u = torch.rand((S,), generator=g)
+    u[::7], u[3::11] = 0.0, 0.99999994
+    u, rows = u.to(device), rows.to(device)
+    want = K.bias_sample(rows.float(), temperature, top_p, u, mask=mask)
+    got = K.bias_sample(rows, temperature, top_p, u, mask=mask)
+    assert torch.equal(got, want), torch.nonzero(got != want).flatten().tolist()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        replayed = K.bias_sample(rows, temperature, top_p, u, mask=mask)
+    for _ in range(2):
+        replayed.zero_()
+        graph.replay()
+        assert torch.equal(replayed, want)
+        assert torch.equal(K.bias_sample(rows, temperature, top_p, u, mask=mask), want)
+
+
 def test_bias_sample_corner_rows(device):
     """Rows outside what the reference defines still give a defined, allowed token: an infinite logit (its first
     holder), uniform numbers outside [0, 1) (the first / the last token with weight), an infinite temperature
