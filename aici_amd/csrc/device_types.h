@@ -106,9 +106,17 @@ __device__ __forceinline__ V bit_cast(const U &u) {
 // Sums over a wavefront and over the workgroup (every thread receives the result); the order of the additions
 // is fixed by the thread numbers alone, so two kernels that hand these the same per-thread values get the same
 // bits.
+// The wavefront's: pairs 32, 16, 8, 4, 2 and 1 lanes apart, in registers (through LDS permutes each step is a wait of its own: a
+// row's norm at 4096 elements holds two such sums, and every wavefront of a linear layer that normalises its rows two per row).
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  const auto halves = __builtin_amdgcn_permlane32_swap(bit_cast<unsigned>(v), bit_cast<unsigned>(v), false, false);
+  v = bit_cast<float>((unsigned)halves[0]) + bit_cast<float>((unsigned)halves[1]);
+  const auto rows = __builtin_amdgcn_permlane16_swap(bit_cast<unsigned>(v), bit_cast<unsigned>(v), false, false);
+  v = bit_cast<float>((unsigned)rows[0]) + bit_cast<float>((unsigned)rows[1]);
+  v += bit_cast<float>(__builtin_amdgcn_update_dpp(0, bit_cast<int>(v), 0x128, 0xf, 0xf, true));  // row_ror:8
+  v += bit_cast<float>(__builtin_amdgcn_update_dpp(0, bit_cast<int>(v), 0x124, 0xf, 0xf, true));  // row_ror:4 (lanes 8 apart are equal now)
+  v += bit_cast<float>(__builtin_amdgcn_update_dpp(0, bit_cast<int>(v), 0x4e, 0xf, 0xf, true));   // quad_perm 2, 3, 0, 1
+  v += bit_cast<float>(__builtin_amdgcn_update_dpp(0, bit_cast<int>(v), 0xb1, 0xf, 0xf, true));   // quad_perm 1, 0, 3, 2
   return v;
 }
 __device__ __forceinline__ float block_sum(float v, float *smem /* >= 17 floats */) {

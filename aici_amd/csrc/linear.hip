@@ -52,6 +52,9 @@ constexpr int kLinMaxRows = 128;  // rows of x
 constexpr int kLinMT = 8;         // 16-row tiles of x
 constexpr int kLinStageK = 64;    // values of k per stage: 128 bytes of a row
 constexpr int kLinStreamRows = 16;
+constexpr int kLinHeldRows = 4;
+constexpr int kLinHeldBytes = 40 * 1024;  // of x and the norm's weight: two workgroups per compute unit
+constexpr int kHeldStages = 4;
 constexpr int kLinMaxRanges = 8;  // ranges of k that the library itself chooses
 
 struct LinearParams {
@@ -73,6 +76,7 @@ struct LinearParams {
   void *norm_out;
   int64_t ldn;
   float eps;
+  int norm_in;  // the norm is that of the rows of x, in front of the layer
 };
 
 template <typename T>
@@ -177,6 +181,17 @@ __device__ __forceinline__ const uint4 *staged_run(const char *rows, int r, int 
   return reinterpret_cast<const uint4 *>(rows + r * (kLinStageK * 2) + ((q ^ (r & 7)) * 16));
 }
 
+// The sums of a tile's ranges, first to last.
+__device__ __forceinline__ f32x4_t add_ranges(const f32x4_t *src, int splits) {
+  f32x4_t total = src[0];
+  for (int i = 1; i < splits; i++) {
+    const f32x4_t v = src[i * 64];
+#pragma unroll
+    for (int r = 0; r < 4; r++) total[r] += v[r];
+  }
+  return total;
+}
+
 // Up to 16 rows of x.  WAVES wavefronts; each owns 16 NT rows of W.  GATED: odd wavefronts take the up rows that
 // belong to the gate rows of the wavefront before them.
 template <typename T, int NT, int S, int WAVES, bool GATED>
@@ -276,20 +291,169 @@ __global__ __launch_bounds__(WAVES * 64) void linear_stream_kernel(const LinearP
       const int n = (blockIdx.x * tiles + wave) * 16 + 4 * kg;
       f32x4_t total[kParts];
 #pragma unroll
-      for (int q = 0; q < kParts; q++) {
-        const f32x4_t *src = sums + (wave * kParts + q) * p.splits * 64 + lane;
-        total[q] = src[0];
-        for (int i = 1; i < p.splits; i++) {
-          const f32x4_t v = src[i * 64];
-#pragma unroll
-          for (int r = 0; r < 4; r++) total[q][r] += v[r];
-        }
-      }
+      for (int q = 0; q < kParts; q++) total[q] = add_ranges(sums + (wave * kParts + q) * p.splits * 64 + lane, p.splits);
       if constexpr (GATED)
         linear_finish_gated<T>(p, total[0], total[1], col, n);
       else
         linear_finish<T>(p, total[0], col, n);
     }
+  }
+}
+
+// RMS norm of up to ROWS rows of x and the layer behind it.  The rows are held in LDS whole and normalised there, with the arithmetic
+// and the order of additions of rms_norm_vec8_kernel, so with its bits, while the first stages of W are on their way: a launch of
+// rms_norm less, whose time is all latency.  The rows' part repeats in every workgroup and costs about 1 us per row, so it ends at few
+// rows.  LDS: ring | sums of ranges | rows of x | the norm's weight.
+__host__ __device__ constexpr int held_pitch(int K) { return (K * 2 + 1023) / 1024 * 1024; }
+template <typename T, int S, int ROWS, bool GATED>
+__global__ __launch_bounds__(256) void norm_linear_kernel(const LinearParams p) {
+  using vec8 = typename Vec8<T>::type;
+  constexpr int WAVES = 4, kParts = GATED ? 2 : 1;
+  constexpr int kStageBytes = 2048;
+  extern __shared__ __align__(1024) char lds[];
+  __shared__ float part_sums[ROWS * 16];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, kg = lane >> 4;
+  const int per_tile = min(p.splits, WAVES / kParts), ranges = p.splits / per_tile;
+  const int part = GATED ? wave & 1 : 0;
+  const int tile = (wave / kParts) / per_tile, first_range = ((wave / kParts) % per_tile) * ranges;
+  const int tiles = WAVES / kParts / per_tile;
+  const int n_tile = (blockIdx.x * tiles + tile) * 16;
+  const int n_end = GATED ? p.half : p.N;
+  const int stage0 = first_range * p.stages_per_split;
+  const int nst = max(0, min(ranges * p.stages_per_split, p.total_stages - stage0));
+  f32x4_t *sums = reinterpret_cast<f32x4_t *>(lds + WAVES * S * kStageBytes);
+  const int pitch = held_pitch(p.K);
+  char *xrows = lds + WAVES * S * kStageBytes + tiles * kParts * p.splits * 1024;
+  char *normw = xrows + p.M * pitch;
+
+  // rows of x (and the norm's weight behind them), 1 KB a piece: run q of row r goes to place q ^ (r & 7) of its row
+  {
+    const int per_row = pitch / 1024, pieces = (p.M + 1) * per_row, last = p.K / 8 - 1;
+    const uint32_t at = lds_address(xrows);
+    for (int i = wave; i < pieces; i += WAVES) {
+      const int r = i / per_row, q0 = (i % per_row) * 64;
+      CopySource<false> src;
+      src.base = uniform_base(static_cast<const char *>(r == p.M ? p.norm_w : static_cast<const T *>(p.x) + r * p.ldx));
+      src.off = (uint32_t)min(q0 + (lane ^ (r == p.M ? 0 : r & 7)), last) * 16;
+      copy_1k<false, false>(at + i * 1024, src, 0);
+    }
+  }
+  CopySource<false> wsrc[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+    wsrc[i] = copy_source<T, false>(p.w, p.ldw, part * p.half + n_tile + i * 8, part * p.half + n_end - 1, stage0);
+  const char *mine = lds + wave * S * kStageBytes;
+  const uint32_t mine_lds = lds_address(lds) + wave * S * kStageBytes;
+  auto ask = [&](int slot, int st) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) copy_1k<true, false>(mine_lds + slot * kStageBytes + i * 1024, wsrc[i], st);
+  };
+#pragma unroll
+  for (int j = 0; j < S; j++)
+    if (j < nst) ask(j, j);
+  if (nst >= S)
+    wait_copies<2 * S>();
+  else
+    wait_copies<0>();
+  asm volatile("s_barrier" ::: "memory");
+  {
+    // rms_norm_vec8_kernel's thread t owns run t of a row: a wavefront here takes the place of one of its wavefronts at a time
+    const int runs = p.K / 8, waves = (runs + 63) / 64;
+    auto at = [&](int r, int q) { return reinterpret_cast<uint4 *>(xrows + r * pitch + (q ^ (r & 7)) * 16); };
+    for (int w = wave; w < waves; w += WAVES) {
+      const int q = w * 64 + lane;
+      uint4 raw[ROWS];
+      float ss[ROWS] = {};
+#pragma unroll
+      for (int r = 0; r < ROWS; r++) raw[r] = *at(min(r, p.M - 1), min(q, runs - 1));
+#pragma unroll
+      for (int r = 0; r < ROWS; r++) {
+        const T *e = reinterpret_cast<const T *>(&raw[r]);
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = to_float(e[j]);
+#pragma unroll
+        for (int j = 0; j < 8; j++) ss[r] += v[j] * v[j];
+        ss[r] = wave_sum(q < runs ? ss[r] : 0.f);
+        if (lane == 0) part_sums[r * 16 + w] = ss[r];
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    float inv[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) inv[r] = rsqrtf(wave_sum(lane < waves ? part_sums[r * 16 + (lane & 15)] : 0.f) / (float)p.K + p.eps);
+    for (int w = wave; w < waves; w += WAVES) {
+      const int q = min(w * 64 + lane, runs - 1);
+      uint4 raw[ROWS];
+      const uint4 wr = *reinterpret_cast<const uint4 *>(normw + q * 16);
+      const T *we = reinterpret_cast<const T *>(&wr);
+#pragma unroll
+      for (int r = 0; r < ROWS; r++) raw[r] = *at(min(r, p.M - 1), q);
+#pragma unroll
+      for (int r = 0; r < ROWS; r++) {
+        const T *e = reinterpret_cast<const T *>(&raw[r]);
+        uint4 o;
+        T *oe = reinterpret_cast<T *>(&o);
+#pragma unroll
+        for (int j = 0; j < 8; j++) oe[j] = from_float<T>(to_float(from_float<T>(to_float(e[j]) * inv[r])) * to_float(we[j]));
+        if (r < p.M && w * 64 + lane < runs) *at(r, q) = o;
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+  const int xr = min(col, p.M - 1);
+  const char *xrow = xrows + xr * pitch + stage0 * (kLinStageK * 2);
+  f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  f32x4_t *range_sums = sums + ((tile * kParts + part) * p.splits + first_range) * 64 + lane;
+  int left = p.stages_per_split, range = 0;  // of the range in hand
+  for (int base = 0; base < nst; base += S) {
+#pragma unroll
+    for (int j = 0; j < S; j++) {
+      const int st = base + j;
+      if (st < nst) {
+        if (st + S - 1 < nst)
+          wait_copies<(S - 1) * 2>();
+        else
+          wait_copies<0>();
+        const char *stage = mine + j * kStageBytes;
+        uint4 wf[2], xf[2];
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          wf[s] = *staged_run(stage, col, 4 * s + kg);
+          xf[s] = *reinterpret_cast<const uint4 *>(xrow + st * (kLinStageK * 2) + ((4 * s + kg) ^ (xr & 7)) * 16);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage is in registers: its place can be filled again
+        if (st + S < nst) ask(j, st + S);
+#pragma unroll
+        for (int s = 0; s < 2; s++) acc = LinMfma<T>::run(bit_cast<vec8>(wf[s]), bit_cast<vec8>(xf[s]), acc);
+        if (ranges > 1 && --left == 0) {
+          range_sums[range++ * 64] = acc;
+          acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          left = p.stages_per_split;
+        }
+      }
+    }
+  }
+  if (!GATED && p.splits == 1) {
+    linear_finish<T>(p, acc, col, n_tile + 4 * kg);
+    return;
+  }
+  for (; range < ranges; range++) {  // what is left of the last range; ranges past the end of k are zero
+    range_sums[range * 64] = acc;
+    acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  __syncthreads();
+  if (wave < tiles) {
+    const int n = (blockIdx.x * tiles + wave) * 16 + 4 * kg;
+    f32x4_t total[kParts];
+#pragma unroll
+    for (int q = 0; q < kParts; q++) total[q] = add_ranges(sums + (wave * kParts + q) * p.splits * 64 + lane, p.splits);
+    if constexpr (GATED)
+      linear_finish_gated<T>(p, total[0], total[1], col, n);
+    else
+      linear_finish<T>(p, total[0], col, n);
   }
 }
 
@@ -510,7 +674,7 @@ struct LinearPlan {
 // The ranges of k depend on the weight alone (see above).  As far as eight ranges allow: 1024 wavefronts' worth of (16 rows, range)
 // pairs, four per compute unit, and no range longer than 2048 once k is cut at all -- 4096 x 4096 and 6144 x 4096 four, 4096 x
 // 14336 eight, weights of 16384 rows and more none.
-LinearPlan plan_linear(int M, int N, int K) {
+LinearPlan plan_linear(int M, int N, int K, bool norm_in) {
   const Tuning &tn = tuning();
   LinearPlan pl;
   const int stages = K / kLinStageK;
@@ -519,8 +683,8 @@ LinearPlan plan_linear(int M, int N, int K) {
   while (splits > 1 && splits < kLinMaxRanges && K / splits > 2048) splits *= 2;
   while (splits > stages) splits /= 2;
   pl.stream = M <= kLinStreamRows;
-  if (tn.linear_splits > 0) splits = tn.linear_splits < stages ? tn.linear_splits : stages;
-  if (tn.linear_splits > 0 || tn.linear_waves > 0 || tn.linear_tiles > 0) pl.stream = false;
+  if (tn.linear_splits > 0 && !norm_in) splits = tn.linear_splits < stages ? tn.linear_splits : stages;
+  if ((tn.linear_splits > 0 || tn.linear_waves > 0 || tn.linear_tiles > 0) && !norm_in) pl.stream = false;
   pl.splits = splits;
   pl.stages_per_split = (stages + splits - 1) / splits;
   // Workgroups of 64 rows while the device holds all of them at once, one per compute unit, or where 32 rows of x leave the copies of x
@@ -556,8 +720,35 @@ void launch_tile(const LinearParams &p, const LinearPlan &pl, hipStream_t stream
   hipLaunchKernelGGL((linear_tile_kernel<T, MT, ring_stages<MT, 8>(), 8, GATED, WIDE>), grid, block, 0, stream, p);
 }
 
+template <typename T, int ROWS, bool GATED>
+void launch_norm_linear(const LinearParams &p, hipStream_t stream) {
+  constexpr int S = kHeldStages;
+  static bool attr_set = false;  // benign race: setting twice is harmless
+  auto kernel = norm_linear_kernel<T, S, ROWS, GATED>;
+  if (!attr_set) {
+    HA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               4 * S * 2048 + 16 * 1024 + kLinHeldBytes));
+    attr_set = true;
+  }
+  const int parts = GATED ? 2 : 1, n = GATED ? p.half : p.N;
+  const int per_tile = p.splits < 4 / parts ? p.splits : 4 / parts, tiles = 4 / parts / per_tile;
+  const int rows = 16 * tiles;
+  const size_t bytes = 4 * S * 2048 + tiles * parts * p.splits * 1024 + (size_t)(p.M + 1) * held_pitch(p.K);
+  hipLaunchKernelGGL(kernel, dim3((n + rows - 1) / rows), dim3(256), bytes, stream, p);
+  check_launch("rms_norm_linear");
+}
+
 template <typename T, bool GATED>
 void launch_linear(const LinearParams &p, const LinearPlan &pl, hipStream_t stream) {
+  if (p.norm_in) {
+    if (p.M == 1)
+      launch_norm_linear<T, 1, GATED>(p, stream);
+    else if (p.M == 2)
+      launch_norm_linear<T, 2, GATED>(p, stream);
+    else
+      launch_norm_linear<T, kLinHeldRows, GATED>(p, stream);
+    return;
+  }
   if (pl.stream) {
     if (!GATED && p.splits == 1 && p.N >= 65536) {
       // A vocabulary's rows: 512 per workgroup, so that one round of workgroups covers the device (128256 x 4096, 16 rows: 161
@@ -620,7 +811,7 @@ bool rows_overlap(const hipattn_tensor *a, const hipattn_tensor *b) {
 void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_tensor *weight, const hipattn_tensor *bias,
                  const hipattn_tensor *residual, const hipattn_tensor *workspace, void *stream_arg, int64_t *ws_query,
                  hipattn_tensor *norm_out = nullptr, const hipattn_tensor *norm_weight = nullptr, float eps = 0.f,
-                 bool ws_query_with_norm = false, bool gated = false) {
+                 bool ws_query_with_norm = false, bool gated = false, bool norm_in = false) {
   check_tensor(x, "x", 2);
   check_tensor(weight, "weight", 2);
   const int dt = x->dtype;
@@ -634,7 +825,7 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
   HA_CHECK(N % 16 == 0, "linear: the number of rows of weight (%lld) must be a multiple of 16", (long long)N);
   HA_CHECK(N < (1 << 24) && K < (1 << 24), "linear: sizes out of range");
   HA_CHECK(!gated || N % 32 == 0, "linear_silu_and_mul: gate and up rows (%lld together) must be multiples of 16 each", (long long)N);
-  LinearPlan pl = plan_linear((int)M, (int)N, (int)K);
+  LinearPlan pl = plan_linear((int)M, (int)N, (int)K, norm_in);
   const int64_t outputs = gated ? N / 2 : N;
   const bool with_norm = norm_out != nullptr || ws_query_with_norm;
   // the norm's launch takes rows of sums, however few the ranges
@@ -661,6 +852,17 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
   // Output rows over rows of x: both kernels write while other workgroups still read x, so every row of sums goes to the workspace
   // and a second launch finishes it.
   const bool overlap = rows_overlap(x, out);
+  if (norm_in) {
+    HA_CHECK(M <= kLinHeldRows && K <= 8192 && N < 65536 && (M + 1) * held_pitch((int)K) <= kLinHeldBytes,
+             "rms_norm_linear: %lld rows of %lld and a weight of %lld rows; it takes at most %d rows of up to 8192, %d bytes with the norm's weight, and fewer than 65536 rows of weight",
+             (long long)M, (long long)K, (long long)N, kLinHeldRows, kLinHeldBytes);
+    HA_CHECK(!overlap, "rms_norm_linear: out lies over x");
+    check_tensor(norm_weight, "norm_weight", 1);
+    HA_CHECK(norm_weight->dtype == dt && norm_weight->sizes[0] == K && norm_weight->strides[0] == 1,
+             "rms_norm_linear: norm_weight must be %lld contiguous %s", (long long)K, dtype_name(dt));
+    check_data(norm_weight, "norm_weight");
+    HA_CHECK(aligned16(norm_weight->data), "rms_norm_linear: norm_weight must start on a 16-byte boundary");
+  }
   if (overlap) {
     pl.stream = false;
     pl.partial_bytes = (size_t)pl.splits * kLinMaxRows * N * sizeof(float);
@@ -681,6 +883,12 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
   auto far = [](int64_t ld) { return ld < 0 || ld >= (1 << 28); };
   p.wide = far(p.ldx) || far(p.ldw);
   if (p.wide) pl.stream = false;
+  if (norm_in) {
+    HA_CHECK(pl.stream, "rms_norm_linear: rows of x or weight lie too far apart");
+    p.norm_in = 1;
+    p.norm_w = norm_weight->data;
+    p.eps = eps;
+  }
   p.ldo = out->strides[0];
   if (bias != nullptr) {
     check_tensor(bias, "bias", 1);
@@ -773,6 +981,12 @@ extern "C" char *hipattn_linear(hipattn_tensor *out, const hipattn_tensor *x, co
 extern "C" char *hipattn_linear_silu_and_mul(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_tensor *weight,
                                              const hipattn_tensor *workspace, void *stream) {
   HA_PROTECT(linear_impl(out, x, weight, nullptr, nullptr, workspace, stream, nullptr, nullptr, nullptr, 0.f, false, true));
+}
+
+extern "C" char *hipattn_rms_norm_linear(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_tensor *norm_weight,
+                                         float epsilon, const hipattn_tensor *weight, bool silu_and_mul, void *stream) {
+  HA_PROTECT(linear_impl(out, x, weight, nullptr, nullptr, nullptr, stream, nullptr, nullptr, norm_weight, epsilon, false, silu_and_mul,
+                         true));
 }
 
 extern "C" char *hipattn_linear_workspace_size(const hipattn_tensor *x, const hipattn_tensor *weight, int64_t *bytes) {

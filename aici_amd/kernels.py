@@ -282,6 +282,25 @@ def linear_rms_norm(x: torch.Tensor, weight: torch.Tensor, norm_weight: torch.Te
     return out, normed
 
 
+RMS_NORM_LINEAR_MAX_ROWS = 4
+
+
+def rms_norm_linear_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether `rms_norm_linear` accepts these operands (else a caller makes the two calls)."""
+    return (linear_takes(x, weight) and x.size(0) <= RMS_NORM_LINEAR_MAX_ROWS and x.size(1) <= 8192
+            and (x.size(0) + 1) * ((x.size(1) * 2 + 1023) // 1024) <= 40 and weight.size(0) < 65536 and weight.size(0) % 32 == 0
+            and 0 < weight.stride(0) < 1 << 28 and (x.size(0) == 1 or 0 <= x.stride(0) < 1 << 28))
+
+
+def rms_norm_linear(x: torch.Tensor, norm_weight: torch.Tensor, epsilon: float, weight: torch.Tensor,
+                    silu_and_mul: bool = False) -> torch.Tensor:
+    """rms_norm(x) @ weight.T, or with silu_and_mul behind it (weight [2 n, K], the gate rows first), in one launch for the few
+    rows of a small step (llama.rs:165 + 81-83, 169 + 135-142): the bits of the two calls."""
+    out = torch.empty((x.size(0), weight.size(0) // 2 if silu_and_mul else weight.size(0)), dtype=x.dtype, device=x.device)
+    _native.rms_norm_linear(out, x, norm_weight, epsilon, weight, silu_and_mul)
+    return out
+
+
 def linear_rms_norm_workspace_size(x: torch.Tensor, weight: torch.Tensor) -> int:
     n = ctypes.c_int64(0)
     call("hipattn_linear_rms_norm_workspace_size", _desc(x, "x"), _desc(weight, "weight"), ctypes.byref(n))

@@ -7,7 +7,8 @@ The embedding is a library gather.  The projections of a step of at most 128 row
 the head of any step with at most that many sequences, go through the C ABI's linear
 kernels: the weight is read once at the rate of the memory, silu_and_mul happens where the
 gate and up products are finished, and so do the residual addition and, from 17 rows on, the
-RMS norm that follow o_proj and down_proj.  Projections of more rows are library GEMMs
+RMS norm that follow o_proj and down_proj; up to 4 rows are normalised by the projections
+behind the norm.  Projections of more rows are library GEMMs
 (torch on ROCm).
 Everything else -- rms_norm, rotary, the paged-KV attention composition,
 silu_and_mul, bias + argmax -- goes through the C ABI as well.  Weights are random
@@ -116,6 +117,12 @@ class Llama:
         kernels.rms_norm(out, x, weight, self.cfg.rms_norm_eps)
         return out
 
+    def _norm_in_proj(self, x: torch.Tensor, weight: torch.Tensor) -> bool:
+        """Whether the projection normalises its rows itself, the same bits (us, 4096 columns, norm and projection / one launch: 6144
+        rows 13.1 / 11.2 with one row of x, 13.3 / 13.1 with four; 28672 rows 45.9 / 43.1 and 45.9 / 43.8)."""
+        return (x.size(0) <= kernels.RMS_NORM_LINEAR_MAX_ROWS and self.skinny_linear and self.fused_norm
+                and kernels.rms_norm_linear_takes(x, weight))
+
     def _proj(self, x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         """x @ weight.T (llama.rs:81-83, 210).  A vocabulary's rows with more than 48 sequences stay with the library
         (128256 x 4096, us, library / C ABI: 48 rows 206 / 203, 64 rows 208 / 211, 128 rows 232 / 248)."""
@@ -132,12 +139,14 @@ class Llama:
         kernels.silu_and_mul(act, gu)
         return act
 
-    def _proj_add_norm(self, y: torch.Tensor, weight: torch.Tensor, x: torch.Tensor, norm_weight: torch.Tensor):
+    def _proj_add_norm(self, y: torch.Tensor, weight: torch.Tensor, x: torch.Tensor, norm_weight: torch.Tensor, behind=None):
         """x' = y @ weight.T + x (llama.rs:96 + 166, 143 + 173) and the RMS norm of x' that follows it (:169, :165 of the
-        next block, :207).  Few rows: the C ABI's kernel, which splits the inner dimension over the device and finishes the
+        next block, :207), or None where the projection `behind` normalises its rows itself.  Few rows: the C ABI's kernel, which splits the inner dimension over the device and finishes the
         rows -- residual and norm -- in the launch that adds the parts up; else a library GEMM, an addition and
         rms_norm.  The same bits either way as far as the norm goes."""
         if self.skinny_linear and weight.size(0) <= 8192 and kernels.linear_takes(y, weight):
+            if behind is not None and self._norm_in_proj(x, behind):
+                return kernels.linear(y, weight, residual=x), None
             if self.fused_norm:
                 return kernels.linear_rms_norm(y, weight, norm_weight, self.cfg.rms_norm_eps, residual=x)
             x = kernels.linear(y, weight, residual=x)
@@ -155,9 +164,13 @@ class Llama:
         Hq, Hkv, d = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
         x = self.wte.index_select(0, batch_info.tokens.long())                   # llama.rs:203
         T = x.size(0)
-        h = self._rms(x, self.layers[0]["rms_1"])                               # :165
+        # h: the normalised rows, None where the projection that takes them does it
+        h = None if self._norm_in_proj(x, self.layers[0]["qkv"]) else self._rms(x, self.layers[0]["rms_1"])  # :165
         for li, (layer, (kc, vc)) in enumerate(zip(self.layers, caches)):
-            qkv = self._proj(h, layer["qkv"])                                   # :81-83
+            if h is None:
+                qkv = kernels.rms_norm_linear(x, layer["rms_1"], cfg.rms_norm_eps, layer["qkv"])
+            else:
+                qkv = self._proj(h, layer["qkv"])                               # :81-83
             if fused:
                 q, k, v = qkv.split([Hq * d, Hkv * d, Hkv * d], dim=1)
                 v = v.view(T, Hkv, d)
@@ -168,11 +181,14 @@ class Llama:
                 q, k, v = (t.contiguous() for t in qkv.split([Hq * d, Hkv * d, Hkv * d], dim=1))
                 q, k = self.rotary.forward(batch_info.positions, q, k)          # :85 (in place on the copies)
                 y = varlen_attn(q, k, v.reshape(T, Hkv, d), batch_info, kc, vc, paged_prefill=paged_prefill)  # :93
-            x, h = self._proj_add_norm(y, layer["o"], x, layer["rms_2"])         # :96, :166, :169
-            act = self._gate_up_silu(h, layer["gate_up"])                       # :135-142
+            x, h = self._proj_add_norm(y, layer["o"], x, layer["rms_2"], layer["gate_up"])  # :96, :166, :169
+            if h is None:
+                act = kernels.rms_norm_linear(x, layer["rms_2"], cfg.rms_norm_eps, layer["gate_up"], silu_and_mul=True)
+            else:
+                act = self._gate_up_silu(h, layer["gate_up"])                   # :135-142
             # the norm behind the block is the next block's first one, or the model's last (:165, :207)
-            after = self.layers[li + 1]["rms_1"] if li + 1 < len(self.layers) else self.ln_f
-            x, h = self._proj_add_norm(act, layer["down"], x, after)            # :143, :173
+            behind = self.layers[li + 1] if li + 1 < len(self.layers) else {"rms_1": self.ln_f, "qkv": None}
+            x, h = self._proj_add_norm(act, layer["down"], x, behind["rms_1"], behind["qkv"])  # :143, :173
         x0 = h
         sel = x0.index_select(0, batch_info.logit_idxs.long())                  # :209 extract_positions
         return self._proj(sel, self.lm_head)                                    # :210

@@ -366,6 +366,17 @@ char *hipattn_linear_rms_norm_workspace_size(const hipattn_tensor *x,
                                              const hipattn_tensor *weight,
                                              int64_t *bytes);
 
+/* hipattn_rms_norm of the rows of x and the linear layer behind it (llama.rs:165 + 81-83, 169 + 135-142) in one launch, for the few
+ * rows that a workgroup can hold: out = rms_norm(x, norm_weight, epsilon) . weight^T, or with silu_and_mul as in
+ * hipattn_linear_silu_and_mul; the bits of the two calls; the normalised rows are not written to memory.  Operands as for
+ * hipattn_linear, and: x at most HIPATTN_RMS_NORM_LINEAR_ROWS rows of at most 8192 (rows and norm_weight together at most 40 KB),
+ * fewer than 65536 rows of weight, norm_weight [K] on a 16-byte boundary, out not over x.  No workspace. */
+#define HIPATTN_RMS_NORM_LINEAR_ROWS 4
+char *hipattn_rms_norm_linear(hipattn_tensor *out, const hipattn_tensor *x,
+                              const hipattn_tensor *norm_weight, float epsilon,
+                              const hipattn_tensor *weight, bool silu_and_mul,
+                              void *stream);
+
 /* Replace silu_and_mul_C / gelu_new_C / gelu_fast_C (lib.rs:162-166;
  * activation_kernels.cu:15-115). */
 char *hipattn_silu_and_mul(hipattn_tensor *out, const hipattn_tensor *input,

@@ -327,3 +327,41 @@ def test_vocabulary_rows(device, m):
     x, w, _ = operands(m, 65536 + 80, 256, torch.bfloat16, seed=m)
     y = K.linear(x.to(device), w.to(device))
     check(y, x, w)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Kd,N,M", [(256, 32, 1), (768, 1056, 4), (4096, 6144, 1), (4096, 4096, 2), (4096, 28672, 3), (2560, 2560, 4),
+                                   (8192, 96, 1), (5120, 480, 3), (14336 // 2, 64, 1)])
+def test_rms_norm_linear_gives_the_bits_of_the_two_calls(device, dtype, Kd, N, M):
+    """The norm inside the projection: the bits of rms_norm and linear (or linear_silu_and_mul) one after the other, from rows
+    that lie apart as well, for one range of k and several, rows and weights that end inside a 1 KB piece."""
+    g = torch.Generator().manual_seed(Kd + N + M)
+    wide = (torch.randn((M, Kd + 24), generator=g) * torch.linspace(0.01, 30, M)[:, None]).to(dtype).to(device)
+    x = wide[:, 8:Kd + 8]
+    weight = (torch.randn((N, Kd), generator=g) / Kd ** 0.5).to(dtype).to(device)
+    norm = (1 + 0.2 * torch.randn((Kd,), generator=g)).to(dtype).to(device)
+    h = torch.empty((M, Kd), dtype=dtype, device=device)
+    K.rms_norm(h, x.contiguous(), norm, 1e-5)
+    assert K.rms_norm_linear_takes(x, weight)
+    before = wide.clone()
+    for _ in range(2):
+        assert torch.equal(K.rms_norm_linear(x, norm, 1e-5, weight), K.linear(h, weight))
+        assert torch.equal(K.rms_norm_linear(x, norm, 1e-5, weight, silu_and_mul=True), K.linear_silu_and_mul(h, weight))
+    assert torch.equal(wide, before)
+
+
+def test_rms_norm_linear_refusals(device):
+    x = torch.zeros((5, 4096), dtype=torch.bfloat16, device=device)
+    w = torch.zeros((64, 4096), dtype=torch.bfloat16, device=device)
+    norm = torch.ones((4096,), dtype=torch.bfloat16, device=device)
+    assert not K.rms_norm_linear_takes(x, w)
+    with pytest.raises(HipAttnError, match="at most 4 rows"):
+        K.rms_norm_linear(x, norm, 1e-5, w)
+    with pytest.raises(HipAttnError, match="at most 4 rows"):  # 3 rows of 8192: more than 40 KB with the norm's weight
+        K.rms_norm_linear(torch.zeros((3, 8192), dtype=torch.bfloat16, device=device), torch.ones(8192, dtype=torch.bfloat16,
+                                device=device), 1e-5, torch.zeros((64, 8192), dtype=torch.bfloat16, device=device))
+    with pytest.raises(HipAttnError, match="norm_weight must be 4096"):
+        K.rms_norm_linear(x[:2], norm[:2048], 1e-5, w)
+    square = torch.zeros((4096, 4096), dtype=torch.bfloat16, device=device)
+    with pytest.raises(HipAttnError, match="over x"):
+        _native.rms_norm_linear(x[:2], x[:2], norm, 1e-5, square, False)
