@@ -22,6 +22,8 @@ struct PrefillParams {
   const int32_t *cu_q, *cu_k, *seqused_k;
   int batch, Hq, Hkv, G, d;
   int max_q;      // caller's bound on Lq; sizes the grid
+  int max_k;      // ... and on Lk
+  int64_t total_q;  // query rows of all sequences
   int lse_pitch;  // elements between (batch, head) rows of lse
   int n_qblocks;
   float scale_log2;

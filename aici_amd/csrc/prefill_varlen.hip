@@ -441,7 +441,7 @@ __global__ __launch_bounds__(256) void prefill_varlen_kernel(PrefillParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Eight-wavefront kernel for head sizes up to 128.  512 threads own 256 query rows (32 per wavefront) and run
+// Kernel of eight wavefronts for head sizes up to 128 (its form with four: NW below).  512 threads own 256 query rows (32 per wavefront) and run
 // two wavefronts per SIMD within 256 registers each: every accumulator lives in a vector register the vector
 // ALU can touch directly.  Three forms (MODE below) differ in how the 64-key tiles reach LDS and in the loop:
 //   rows of k / v and block images of the paged cache: global -> LDS copies (no staging registers) into five
@@ -450,9 +450,17 @@ __global__ __launch_bounds__(256) void prefill_varlen_kernel(PrefillParams p) {
 //     (read with ds_read_b64_tr_b16) or, from the cache, as the [d][16 tokens] images that ds_read_b128 takes;
 //   staged (paged cache, head sizes below 32 or on request): tiles through registers into three padded stages
 //     (TileW8 below: K rows and V^T rows), one software-pipelined loop per wavefront.
+// NW = 4: workgroups of four wavefronts and three stages, three to a compute unit, so that every SIMD has a wavefront of each.
+// The alternation of the two pipes is left to chance; what it gains is that a workgroup's set-up and wind-down (block ids, Q, the
+// first tile; the output) pass while the other two work.  Head sizes up to 64 always, larger ones, with tiles of 32 keys to fit the
+// registers and the LDS of a third of a compute unit, where contexts are short (four_wavefronts_pay).
 // ---------------------------------------------------------------------------
 // Where the eight-wavefront kernel takes its K/V tiles from.
 enum { W8_ROWS = 0, W8_PAGED = 1, W8_PAGED_DMA = 2, W8_PAGED_DMA_PART = 3 };
+
+// Keys per tile and wavefronts per SIMD of the forms with eight and four wavefronts.
+constexpr int w8_tile_keys(int hdp, int nw) { return nw == 4 && hdp > 64 ? 32 : 64; }
+constexpr int w8_wavefronts(int hdp, int nw) { return nw == 4 ? 3 : 2; }
 
 // LDS geometry of the staged form.
 template <int HDP>
@@ -465,10 +473,11 @@ struct TileW8 {
   static constexpr size_t LDS_BYTES = 3 * (size_t)STAGE_ELEMS * 2;
 };
 
-template <typename T, int HDP, int MODE>
-__global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams p) {
+template <typename T, int HDP, int MODE, int NW = 8>
+__global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varlen_w8_kernel(PrefillParams p) {
   typedef typename Vec8<T>::type vec8;
   typedef TileW8<HDP> TL;
+  constexpr int BN = w8_tile_keys(HDP, NW), NKT = BN / 32;  // keys per tile, halves of 32
   constexpr bool PAGED = MODE != W8_ROWS;
   constexpr bool ROWS = MODE == W8_ROWS;
   constexpr bool DMA = MODE == W8_PAGED_DMA || MODE == W8_PAGED_DMA_PART;
@@ -478,6 +487,7 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
   // forms run the alternating MFMA / softmax blocks.
   constexpr bool KIMG = DMA || ROWS;      // K tiles lie in LDS as block images
   constexpr bool PINGPONG = DMA || ROWS;
+  static_assert(NW == 8 || (NW == 4 && PINGPONG), "eight wavefronts, or four without staged tiles");
   // W8_PAGED_DMA_PART: head sizes below HDP (Phi-2's 80 in the 96-wide instance).  An image then fills only the
   // first d / HDP of its place in LDS; the rest is cleared once, so the contraction steps and output rows past d
   // work on zeros.
@@ -485,7 +495,7 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
   // W8_PAGED_DMA keeps a tile as the four block images of the cache, unpadded, in four stages.
   // Block images and rows: five stages (all of the 160 KB at head size 128) and one barrier per tile; staged:
   // three.  No tile is padded; where reads would collide, runs change places within their row (see v_rows_dma).
-  constexpr int NST = PINGPONG ? 5 : 3;
+  constexpr int NST = NW == 4 ? 3 : PINGPONG ? 5 : 3;
   constexpr int K_ELEMS = KIMG ? BN * HDP : TL::K_ELEMS;
   constexpr int STAGE_ELEMS = PINGPONG ? 2 * BN * HDP : K_ELEMS + TL::V_ELEMS;
   constexpr int KSTEPS = HDP / 16;
@@ -506,7 +516,7 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
   // LDS) times 8 >> hl groups of 32 query rows.  With several heads per workgroup all wavefronts sit at
   // about the same rows, reach the diagonal of the causal mask together and skip the same tiles.
   const int hl = p.wg_heads_log2;
-  const int BM = 256 >> hl;
+  const int BM = (NW * 32) >> hl;
 
   // Workgroups in launch order: query head fastest (the heads of a kv group land on one XCD and share its
   // L2), then the row blocks of a sequence, last rows -- the longest stretch of keys under the causal mask --
@@ -537,7 +547,7 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
   // Wavefronts w and w + 4 share a SIMD.  Under the causal mask a wavefront's work grows with its rows'
   // position in the block, so with one head per workgroup the two of a SIMD take row groups (w, 7 - w):
   // every SIMD gets the same sum.
-  const int row_group = hl == 0 ? (wave < 4 ? wave : 11 - wave) : wave >> hl;
+  const int row_group = hl == 0 ? (wave < 4 ? wave : 11 - wave) : wave >> hl;  // (four wavefronts: one per SIMD)
   const int wave_row0 = wg_row0 + row_group * 32;
   const int wave_last_row = wave_row0 + 31;
 
@@ -553,7 +563,7 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
   constexpr int QSTR = HDP + 8;  // row pitch of the turned Q tile, elements
   // The alternating-block forms turn Q through stages 2.., so that tiles 0 and 1 can be on their way meanwhile.
   constexpr int Q_STAGE0 = PINGPONG ? 2 : 1;
-  constexpr bool Q_VIA_LDS = (size_t)8 * 32 * QSTR <= (size_t)(NST - Q_STAGE0) * STAGE_ELEMS;
+  constexpr bool Q_VIA_LDS = (size_t)NW * 32 * QSTR <= (size_t)(NST - Q_STAGE0) * STAGE_ELEMS;
   constexpr int CPRQ = HDP / 8;
   constexpr int NQL = (32 * CPRQ + 63) / 64;
   vec8 qreg[KSTEPS];
@@ -597,6 +607,10 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
 #pragma unroll
       for (int ks = 0; ks < KSTEPS; ks++)
         qreg[ks] = *reinterpret_cast<const vec8 *>(qst + c * QSTR + (2 * ks + g) * 8);
+    } else {
+      // (a use the compiler sees: its wait for these loads belongs here, not in front of every tile's first product)
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ks++) asm volatile("" : "+v"(qreg[ks]));
     }
   };
   auto load_q = [&]() {
@@ -679,37 +693,49 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
   constexpr int BLK_ELEMS = HDP * 16;
   constexpr int NDMA = HDP / 32;  // instructions per wavefront and tile
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)smem_raw;
-  const int dma_v = wave_u & 1, dma_r = wave_u >> 1;
-  const unsigned dma_lane = dma_v ? c * 32 + g * 16 : lane * 16;
-  const char *dma_base = reinterpret_cast<const char *>(dma_v ? vp : kp);
-  const int64_t dma_blk_bytes = (dma_v ? p.vc_block : p.kc_block) * (int64_t)sizeof(T);
+  constexpr int BPT = BN / 16, TPG = 64 / BPT;  // blocks per tile, tiles per 64 table columns
+  constexpr int IMG = 2 * BPT / NW;  // images per wavefront: one, or K and V of block w
+  auto dma_v = [&](int im) { return IMG == 1 ? wave_u & 1 : im; };
+  const int dma_r = IMG == 1 ? wave_u >> 1 : wave_u;
+  unsigned dma_lane[IMG];
+  const char *dma_base[IMG];
+  int64_t dma_blk_bytes[IMG];
   // The last piece of an image that is shorter than HDP: K lanes past the image's last 16-byte run and V
   // lanes whose row lies past d fetch nothing (what lies there belongs to the next head or block).
   const int dma_tail = p.d - 32 * (NDMA - 1);  // head elements in the last piece, 32 when d == HDP
-  const bool dma_last_ok = !DMA_PART || (dma_v ? c < dma_tail : lane < 2 * dma_tail);
-  int64_t tbl_off = 0;
-  auto ids_to_offsets = [&](int blk) -> int64_t {
+  bool dma_last_ok[IMG];
+  int64_t tbl_off[IMG];
+#pragma unroll
+  for (int im = 0; im < IMG; im++) {
+    dma_lane[im] = dma_v(im) ? c * 32 + g * 16 : lane * 16;
+    dma_base[im] = reinterpret_cast<const char *>(dma_v(im) ? vp : kp);
+    dma_blk_bytes[im] = (dma_v(im) ? p.vc_block : p.kc_block) * (int64_t)sizeof(T);
+    dma_last_ok[im] = !DMA_PART || (dma_v(im) ? c < dma_tail : lane < 2 * dma_tail);
+    tbl_off[im] = 0;
+  }
+  auto ids_to_offsets = [&](int blk) {
     const int64_t bid = blk < 0 ? 0 : (blk >= p.num_blocks ? p.num_blocks - 1 : (int64_t)blk);
-    return bid * dma_blk_bytes;
+#pragma unroll
+    for (int im = 0; im < IMG; im++) tbl_off[im] = bid * dma_blk_bytes[im];
   };
-  auto dma_piece = [&](int tile, int i) {
-    const int idx = (tile & 15) * 4 + dma_r;
-    const unsigned lo = __builtin_amdgcn_readlane((int)(uint32_t)tbl_off, idx);
-    const unsigned hi = __builtin_amdgcn_readlane((int)(uint32_t)(tbl_off >> 32), idx);
+  auto dma_piece = [&](int tile, int i, int im) {
+    const int idx = (tile % TPG) * BPT + dma_r;
+    const unsigned lo = __builtin_amdgcn_readlane((int)(uint32_t)tbl_off[im], idx);
+    const unsigned hi = __builtin_amdgcn_readlane((int)(uint32_t)(tbl_off[im] >> 32), idx);
     // (an "s" operand is not made a scalar for the asm when the compiler holds the value in vector registers)
-    const uint64_t src_v = reinterpret_cast<uint64_t>(dma_base) + (((uint64_t)hi << 32) | lo);
+    const uint64_t src_v = reinterpret_cast<uint64_t>(dma_base[im]) + (((uint64_t)hi << 32) | lo);
     const char *src = reinterpret_cast<const char *>(
         ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(src_v >> 32)) << 32) |
         (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)src_v));
     // the instruction's offset field moves both ends of the copy: the address in memory and the one in LDS
     const unsigned dst = (unsigned)__builtin_amdgcn_readfirstlane(
-        (int)(lds0 + (unsigned)(((tile % NST) * STAGE_ELEMS + dma_v * K_ELEMS + dma_r * BLK_ELEMS) * (int)sizeof(T))));
+        (int)(lds0 + (unsigned)(((tile % NST) * STAGE_ELEMS + dma_v(im) * K_ELEMS + dma_r * BLK_ELEMS) * (int)sizeof(T))));
 #define HA_DMA_PIECE(OFF)                                                                          \
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:" #OFF \
                :                                                                                   \
-               : "s"(dst), "v"(dma_lane), "s"(src)                                                 \
+               : "s"(dst), "v"(dma_lane[im]), "s"(src)                                                 \
                : "memory", "m0")
-    if (!DMA_PART || i < NDMA - 1 || dma_last_ok) {
+    if (!DMA_PART || i < NDMA - 1 || dma_last_ok[im]) {
       switch (i) {
         case 0: HA_DMA_PIECE(0); break;
         case 1: HA_DMA_PIECE(1024); break;
@@ -718,23 +744,25 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
       }
     }
 #undef HA_DMA_PIECE
-    if (i == NDMA - 1) {
-      if ((tile & 15) == 14) tbl_nxt = load_ids((tile >> 4) + 1);
-      if ((tile & 15) == 15) tbl_off = ids_to_offsets(tbl_nxt);
+    if (i == NDMA - 1 && im == IMG - 1) {
+      if (tile % TPG == TPG - 2) tbl_nxt = load_ids(tile / TPG + 1);
+      if (tile % TPG == TPG - 1) ids_to_offsets(tbl_nxt);
     }
   };
   auto dma_tile = [&](int tile) {
 #pragma unroll
-    for (int i = 0; i < NDMA; i++) dma_piece(tile, i);
+    for (int im = 0; im < IMG; im++)
+#pragma unroll
+      for (int i = 0; i < NDMA; i++) dma_piece(tile, i, im);
   };
   // W8_PAGED_DMA_PART: clears what the images leave untouched in stages first..last: per block the K runs of
   // head elements d..HDP and, in the last V piece, the rows d..HDP of both 8-token halves.
   auto clear_image_tails = [&](int first, int last) {
     if constexpr (DMA_PART) {
       const int R = HDP - p.d;       // a multiple of 8 below 32
-      const int per_stage = 16 * R;  // 16-byte runs: 4 blocks x (2 R of K + 2 R of V)
+      const int per_stage = 4 * BPT * R;  // 16-byte runs: per block 2 R of K + 2 R of V
       for (int st = first; st <= last; st++)
-        for (int idx = tid; idx < per_stage; idx += 512) {
+        for (int idx = tid; idx < per_stage; idx += NW * 64) {
           const int r = idx / (4 * R), rem = idx % (4 * R);
           int e;
           if (rem < 2 * R) {
@@ -752,10 +780,10 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
   // cache contents may be NaN, which a zero probability would not neutralise.
   auto dma_wait = [&](int tile, bool newer) {
     if (newer)
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NDMA * IMG) : "memory");
     else
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (dma_v && tile * BN + BN > Lk) {
+    if (dma_v(IMG - 1) && tile * BN + BN > Lk) {
       T *vs = smem + (tile % NST) * STAGE_ELEMS + K_ELEMS + dma_r * BLK_ELEMS;
       const int alive = Lk - (tile * BN + dma_r * 16 + g * 8);  // tokens of this lane's runs inside the context
       if (alive < 8) {
@@ -779,7 +807,7 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
   // l % 16.  On a full tile the lane's offset is the same for every piece (the piece's own part is added to
   // the scalar base); only the last piece of a block clamps runs past d, and the last tile keys past Lk.
   constexpr int KPB = HDP / 32;   // pieces per block
-  constexpr int KNP = 4 * KPB;    // pieces per tile
+  constexpr int KNP = BPT * KPB;  // pieces per tile
   const int kd_tok = lane & 15, kd_run = lane >> 4;
   const uint32_t kd_off = (uint32_t)(((int64_t)kd_tok * p.k_row + kd_run * 8) * (int64_t)sizeof(T));
   const uint32_t kd_off_last =
@@ -789,12 +817,12 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
   // of the sequence's keys (one scalar pointer for the whole loop), a tile's and a piece's place go into the
   // lane's 32-bit byte offset (the host sends launches whose keys span more than that to the other kernel), and a
   // piece's place in LDS is its number times 1 KiB.
-  constexpr int KW = (KNP + 7) / 8;  // pieces per wavefront
+  constexpr int KW = (KNP + NW - 1) / NW;  // pieces per wavefront
   uint32_t k_off0[KW];
   if constexpr (ROWS) {
 #pragma unroll
     for (int i = 0; i < KW; i++) {
-      const int q = wave_u + 8 * i, r = q / KPB, pi = q % KPB;
+      const int q = wave_u + NW * i, r = q / KPB, pi = q % KPB;
       k_off0[i] = (pi == KPB - 1 ? kd_off_last : kd_off) + (uint32_t)(((int64_t)16 * r * p.k_row + 32 * pi) * (int64_t)sizeof(T));
     }
   }
@@ -810,15 +838,15 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
     const uint32_t tile_off = (uint32_t)tile * k_tile_bytes;
 #pragma unroll
     for (int i = 0; i < KW; i++) {
-      const int q = wave_u + 8 * i;
-      if (KNP % 8 == 0 || q < KNP) {
+      const int q = wave_u + NW * i;
+      if (KNP % NW == 0 || q < KNP) {
         uint32_t off = k_off0[i] + tile_off;
         if (k0 + BN > Lk) {
           const int r = q / KPB, pi = q % KPB;
           const int key = min(k0 + 16 * r + kd_tok, Lk - 1);
           off = (uint32_t)(((int64_t)key * p.k_row + min(4 * pi + kd_run, d_chunks - 1) * 8) * (int64_t)sizeof(T));
         }
-        const unsigned dst = dst0 + (unsigned)i * 8192u;
+        const unsigned dst = dst0 + (unsigned)i * (NW * 1024u);
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                      :
                      : "s"(dst), "v"(off), "s"(kp_u)
@@ -835,13 +863,13 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
   // output nobody stores), keys past Lk the last real key (their probabilities are zero).
   constexpr int CPRV = HDP / 8;          // runs per row
   constexpr int VNP = BN * CPRV / 64;    // pieces per tile
-  constexpr int VNPW = (VNP + 7) / 8;    // ... per wavefront
+  constexpr int VNPW = (VNP + NW - 1) / NW;  // ... per wavefront
   auto vswz = [](int r) -> int { return HDP == 128 ? (r & 3) << 2 : (HDP == 64 ? ((r >> 1) & 1) << 2 : 0); };
   uint32_t vd_off[VNPW];
   if constexpr (ROWS) {
 #pragma unroll
     for (int i = 0; i < VNPW; i++) {
-      const int u = (wave + 8 * i) * 64 + lane;  // the lane's run of the tile, in LDS order
+      const int u = (wave + NW * i) * 64 + lane;  // the lane's run of the tile, in LDS order
       const int r = u / CPRV, pc = u % CPRV;
       vd_off[i] = (uint32_t)(((int64_t)r * p.v_row + min(pc ^ vswz(r), d_chunks - 1) * 8) * (int64_t)sizeof(T));
     }
@@ -852,8 +880,8 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
     const uint32_t tile_off = (uint32_t)tile * v_tile_bytes;
 #pragma unroll
     for (int i = 0; i < VNPW; i++) {
-      const int q = wave_u + 8 * i;
-      if (VNP % 8 == 0 || q < VNP) {
+      const int q = wave_u + NW * i;
+      if (VNP % NW == 0 || q < VNP) {
         uint32_t off = vd_off[i] + tile_off;
         if (k0 + BN > Lk) {
           // (the lane number through an opaque copy: hoisted out of the loop, what is derived from it here
@@ -864,7 +892,7 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
           const int r = u / CPRV, pc = u % CPRV;
           off = (uint32_t)(((int64_t)min(k0 + r, Lk - 1) * p.v_row + min(pc ^ vswz(r), d_chunks - 1) * 8) * (int64_t)sizeof(T));
         }
-        const unsigned dst = dst0 + (unsigned)i * 8192u;
+        const unsigned dst = dst0 + (unsigned)i * (NW * 1024u);
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                      :
                      : "s"(dst), "v"(off), "s"(vp_u)
@@ -917,14 +945,14 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
   if constexpr (PINGPONG) q_issue();
   if (PAGED && n_tiles > 0) tbl_cur = load_ids(0);
   if constexpr (DMA) {
-    tbl_off = ids_to_offsets(tbl_cur);
+    ids_to_offsets(tbl_cur);
     if (n_tiles > 0) dma_tile(0);
     if (n_tiles > 1) dma_tile(1);
     clear_image_tails(0, 1);
     q_finish();
     if (n_tiles > 0) dma_wait(0, n_tiles > 1);
     __syncthreads();
-    if (n_tiles > 2) dma_tile(2);
+    if (NST > 3 && n_tiles > 2) dma_tile(2);
     clear_image_tails(2, NST - 1);  // seen by all after the barrier in front of the loop
   } else if constexpr (ROWS) {
     if (n_tiles > 0) {
@@ -938,7 +966,7 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
     q_finish();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (n_tiles > 2) {
+    if (NST > 3 && n_tiles > 2) {
       k_rows_dma(2);
       v_rows_dma(2);
     }
@@ -977,27 +1005,27 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
 
   // S^T = K . Q^T of one tile on its own (used for tile 0): both 32-key halves,
   // LDS reads two contraction steps ahead of the MFMAs that consume them.
-  auto phase_qk = [&](int buf, f32x16_t(&s)[2]) {
+  auto phase_qk = [&](int buf, f32x16_t(&s)[NKT]) {
     const T *ks_base = smem + buf * STAGE_ELEMS;
     auto rd = [&](int kt, int ks) -> vec8 {
       return *reinterpret_cast<const vec8 *>(ks_base + k_lane_off + kt * K_HALF + ks * K_STEP);
     };
-    vec8 ka[3][2];
-    ka[0][0] = rd(0, 0);
-    ka[0][1] = rd(1, 0);
+    vec8 ka[3][NKT];
+#pragma unroll
+    for (int kt = 0; kt < NKT; kt++) ka[0][kt] = rd(kt, 0);
     if (KSTEPS > 1) {
-      ka[1][0] = rd(0, 1);
-      ka[1][1] = rd(1, 1);
+#pragma unroll
+      for (int kt = 0; kt < NKT; kt++) ka[1][kt] = rd(kt, 1);
     }
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ks++) {
       if (ks + 2 < KSTEPS) {
-        ka[(ks + 2) % 3][0] = rd(0, ks + 2);
-        ka[(ks + 2) % 3][1] = rd(1, ks + 2);
+#pragma unroll
+        for (int kt = 0; kt < NKT; kt++) ka[(ks + 2) % 3][kt] = rd(kt, ks + 2);
       }
       __builtin_amdgcn_sched_barrier(0);
-      s[0] = Mfma32<T>::run(ka[ks % 3][0], qreg[ks], ks == 0 ? zero : s[0]);
-      s[1] = Mfma32<T>::run(ka[ks % 3][1], qreg[ks], ks == 0 ? zero : s[1]);
+#pragma unroll
+      for (int kt = 0; kt < NKT; kt++) s[kt] = Mfma32<T>::run(ka[ks % 3][kt], qreg[ks], ks == 0 ? zero : s[kt]);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -1011,14 +1039,15 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
   // runs with the staging of tile j+2 (registers -> LDS) and the loads of tile
   // j+3 in its shadow.  Three LDS buffers: iteration j reads K of (j+1)%3 and V
   // of j%3 and writes (j+2)%3; one barrier per iteration.
-  constexpr int NQ = 2 * KSTEPS;   // MFMAs of one S tile: step n = (contraction step n/2, key half n%2)
+  constexpr int NQ = 2 * KSTEPS;   // MFMAs of one S tile of 64 keys: step n = (contraction step n/2, key half n%2)
   constexpr int MAXS = NQ / 4;     // of which the first MAXS shadow the row maximum,
   constexpr int EXPS = NQ - MAXS;  // the rest the exponentials
   constexpr int QK_DEPTH = 3;      // K operands read ahead of their MFMA
 
   // DO_QK: S(j+1) is wanted (written to sn); the softmax of S(j) (in s) always runs.
-  auto qk_softmax = [&](auto do_qk, int j, f32x16_t(&s)[2], f32x16_t(&sn)[2], vec8(&pk)[2][2]) {
+  auto qk_softmax = [&](auto do_qk, int j, f32x16_t(&s)[NKT], f32x16_t(&sn)[NKT], vec8(&pk)[NKT][2]) {
     constexpr bool DO_QK = decltype(do_qk)::value;
+    static_assert(!DO_QK || NKT == 2, "tiles of 64 keys");
     const int k0 = j * BN;
     const T *ks_base = smem + ((j + 1) % NST) * STAGE_ELEMS;
     auto rd = [&](int n) -> vec8 {
@@ -1030,7 +1059,7 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
       for (int n = 0; n < QK_DEPTH && n < NQ; n++) ka[n] = rd(n);
     }
     auto qk_step = [&](int n) {
-      if (DO_QK) {
+      if constexpr (DO_QK) {
         if (n + QK_DEPTH < NQ) ka[(n + QK_DEPTH) % (QK_DEPTH + 1)] = rd(n + QK_DEPTH);
         __builtin_amdgcn_sched_barrier(0);
         sn[n & 1] = Mfma32<T>::run(ka[n % (QK_DEPTH + 1)], qreg[n >> 1], (n >> 1) == 0 ? zero : sn[n & 1]);
@@ -1044,7 +1073,7 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
       int limit = p.causal ? row + off : Lk - 1;
       limit = min(limit, Lk - 1);
 #pragma unroll
-      for (int kt = 0; kt < 2; kt++)
+      for (int kt = 0; kt < NKT; kt++)
 #pragma unroll
         for (int i = 0; i < 16; i++) {
           const int key = KIMG ? k0 + kt * 32 + ((i >> 3) & 1) * 16 + g * 8 + ((i >> 2) & 1) * 4 + (i & 3)
@@ -1053,16 +1082,18 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
         }
     }
     // row maximum in the shadow of the first MAXS MFMAs
-    float mx = fmaxf(s[0][0], s[1][0]);
+    float mx = fmaxf(s[0][0], s[NKT - 1][NKT == 2 ? 0 : 1]);
 #pragma unroll
     for (int n = 0; n < MAXS; n++) {
       qk_step(n);
 #pragma unroll
       for (int i = 16 * n / MAXS; i < 16 * (n + 1) / MAXS; i++)
-        if (i > 0) mx = max3(mx, s[0][i], s[1][i]);
+        if (NKT == 2 ? i > 0 : (i > 0 && i % 2 == 0)) mx = max3(mx, s[0][i], s[NKT - 1][NKT == 2 ? i : i + 1]);
     }
     mx = max_across_halves(mx) * p.scale_log2;
-    const bool grow = mx > m_run + p.rescale_thr;
+    // (tiles of 32 keys: behind the second one the reference is the largest of 64 keys, as with tiles of 64 behind the first, so that this
+    // one's probability is exactly 1 in either; without, the output is 2 to 5 % further from float64)
+    const bool grow = mx > m_run + (NKT == 1 && j == 1 ? 0.f : p.rescale_thr);
     if (__builtin_expect(__any(grow), 0)) {
       const float m_new = grow ? mx : m_run;
       const float alpha = grow ? fast_exp2(m_run - m_new) : 1.0f;
@@ -1079,7 +1110,7 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
     for (int n = 0; n < EXPS; n++) {
       qk_step(MAXS + n);
 #pragma unroll
-      for (int v = 32 * n / EXPS; v < 32 * (n + 1) / EXPS; v++) {
+      for (int v = 16 * NKT * n / EXPS; v < 16 * NKT * (n + 1) / EXPS; v++) {
         const float e = fast_exp2(s[v / 16][v % 16] * p.scale_log2 - msub);
         psum += e;
         pk[v / 16][(v % 16) / 8][v % 8] = from_float<T>(e);
@@ -1088,8 +1119,8 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
     l_run += psum;
   };
 
-  constexpr int PV_STEPS = NDT * 4;
-  f32x16_t s_a[2], s_b[2];
+  constexpr int PV_STEPS = NDT * 2 * NKT;
+  f32x16_t s_a[NKT], s_b[NKT];
   if constexpr (PINGPONG) {
     // ---- block images and rows: the two wavefronts of a SIMD alternate between the matrix pipe and the vector ALU ----
     // A wavefront that issues MFMAs and vector instructions in turn has its vector instructions held up
@@ -1106,7 +1137,7 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
     // M(t), and swap in the middle.
     // Measured on 8 x 4096 tokens from the paged cache: 1.118 -> 1.058 ms with four stages and a barrier per
     // half period, 1.091 -> 1.075 ms from there to five stages and one barrier.
-    vec8 pk[2][2];
+    vec8 pk[NKT][2];
     auto pv_images = [&](int j) {
       const T *vs_base = smem + (j % NST) * STAGE_ELEMS + K_ELEMS;
       // Step n = (contraction step n / NDT, output tile n % NDT): consecutive MFMAs go to different
@@ -1159,6 +1190,14 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
         }
       }
     };
+    auto send_tile = [&](int t) {
+      if constexpr (DMA) {
+        dma_tile(t);
+      } else {
+        k_rows_dma(t);
+        v_rows_dma(t);
+      }
+    };
     auto m_block = [&](int t) {
       if (t >= 1 && !skip_tile(t - 1)) pv_images(t - 1);
       if (t < n_tiles && !skip_tile(t)) phase_qk(t % NST, s_a);
@@ -1178,8 +1217,25 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
         }
       }
     };
+    if constexpr (NW == 4) {
+      // Four wavefronts, one per SIMD, with two more workgroups on the compute unit to fill the pipes: three stages.  A period sends tile
+      // t + 2 into the place of tile t - 1 first of all and ends when it is there.
+      m_block(0);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (DMA && n_tiles > 1) dma_wait(1, false);
+      lds_barrier();
+      asm volatile(".p2align 6");
+      for (int j = 0; j < n_tiles; j++) {
+        if (j + 2 < n_tiles) send_tile(j + 2);
+        if (!skip_tile(j)) qk_softmax(std::false_type{}, j, s_a, s_b, pk);
+        m_block(j + 1);
+        if (DMA && j + 2 < n_tiles) dma_wait(j + 2, false);
+        if (ROWS) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        lds_barrier();
+      }
+    } else {
     // The prologue has sent tiles 0, 1 and 2; tiles 0 and 1 have to be complete before the first period.
-    const bool second_group = wave_u >= 4;
+    const bool second_group = wave_u >= 4;  // (none with four wavefronts: its SIMD mates are another workgroup's)
     if constexpr (DMA) {
       if (!second_group) m_block(0);
       if (n_tiles > 1) dma_wait(1, n_tiles > 2);
@@ -1208,6 +1264,7 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
       }
       m_block(n_tiles);
       lds_barrier();
+    }
     }
   } else {
     // ---- staged tiles: one software-pipelined loop per wavefront ----
@@ -1336,18 +1393,46 @@ __global__ __launch_bounds__(512, 2) void prefill_varlen_w8_kernel(PrefillParams
   }
 }
 
-template <typename T, int HDP, int MODE = W8_ROWS>
-void launch_prefill_w8(PrefillParams p, hipStream_t stream) {
+// hl: log2 of the query heads per workgroup.
+template <typename T, int HDP, int MODE, int NW>
+void launch_prefill_nw(PrefillParams p, int hl, hipStream_t stream) {
   static bool attr_set = false;  // benign race: setting twice is harmless
-  auto kernel = prefill_varlen_w8_kernel<T, HDP, MODE>;
-  constexpr size_t lds_bytes = MODE >= W8_PAGED_DMA ? (size_t)5 * 2 * BN * HDP * 2
-                               : MODE == W8_ROWS   ? (size_t)5 * 2 * BN * HDP * 2
-                                                   : TileW8<HDP>::LDS_BYTES;
+  auto kernel = prefill_varlen_w8_kernel<T, HDP, MODE, NW>;
+  constexpr size_t lds_bytes = MODE == W8_PAGED ? TileW8<HDP>::LDS_BYTES : (size_t)(NW == 4 ? 3 : 5) * 2 * w8_tile_keys(HDP, NW) * HDP * 2;
   if (!attr_set) {
     HA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)lds_bytes));
     attr_set = true;
   }
+  p.wg_heads_log2 = hl;
+  const int bm = (NW * 32) >> hl;
+  p.n_qblocks = (p.max_q + bm - 1) / bm;
+  const int64_t n_wg = (int64_t)p.n_qblocks * p.batch * (p.Hq >> hl);
+  HA_CHECK(n_wg <= 0x7fffffff, "mha_varlen_fwd: too many workgroups");
+  kernel<<<dim3((unsigned)n_wg), NW * 64, lds_bytes, stream>>>(p);
+  check_launch("mha_varlen_fwd");
+}
+
+// Whether a launch of head sizes above 64 takes workgroups of four wavefronts.  They hide a workgroup's set-up and wind-down behind the
+// two others on the compute unit (about 8 us per workgroup of eight, which has the compute unit to itself), but their tiles of 32
+// keys cost more per key.  So: more workgroups of eight than compute units, and contexts short enough that those 8 us count.  us,
+// eight / four wavefronts (32 q / 8 kv x 128; 32 / 32 x 80; 32 / 32 x 128), by sequences and lengths:
+//   64 x 30..300     70 / 52      94 / 57      93 / 67       16 x 20..256     22 / 19      27 / 19      29 / 21
+//   32 x 512        130 / 114    125 / 106    140 / 142      16 x 100..1000   98 / 88     100 / 86     110 / 97
+//   32 x 1024       346 / 353    335 / 319    393 / 387      16 x 2048       591 / 624    537 / 570    628 / 662
+//   8 x 512          39 / 40      38 / 37      40 / 41       8 x 384             -         29 / 23      30 / 25
+//   4 x 512          20 / 22      22 / 25      24 / 27       1 x 1024         29 / 32      28 / 32      30 / 33
+// (8 x 512 is two full rounds of 256 workgroups of eight, and one and a third of 768 of four: between one round and two the
+// contexts have to be shorter.)  With keys cached in front of the queries only the longest context is known here.
+bool four_wavefronts_pay(const PrefillParams &p, int heads) {
+  const int bm = 256 / heads;
+  const int64_t wgs = (p.total_q / bm + p.batch / 2) * (p.Hq / heads);
+  const int64_t keys = p.block_tables == nullptr ? p.total_k / p.batch : p.max_k > p.max_q ? p.max_k : p.total_q / p.batch;
+  return wgs > 300 && keys <= (wgs < 600 ? 400 : 640);
+}
+
+template <typename T, int HDP, int MODE = W8_ROWS>
+void launch_prefill_w8(const PrefillParams &p, hipStream_t stream) {
   // Heads per workgroup: the largest power of two up to four (or up to the tuning switch prefill_wg_heads, when
   // that is set) that divides the GQA ratio: a workgroup then covers 64 rows of each of four heads that share
   // their K / V tiles instead of 256 rows of one, and a sequence's last, partly filled row block idles fewer
@@ -1358,13 +1443,20 @@ void launch_prefill_w8(PrefillParams p, hipStream_t stream) {
   int hl = 0;
   const int limit = tuning().prefill_wg_heads > 0 ? tuning().prefill_wg_heads : 4;
   while (hl < 3 && p.G % (2 << hl) == 0 && (2 << hl) <= limit) hl++;
-  p.wg_heads_log2 = hl;
-  const int bm = 256 >> hl;
-  p.n_qblocks = (p.max_q + bm - 1) / bm;
-  const int64_t n_wg = (int64_t)p.n_qblocks * p.batch * (p.Hq >> hl);
-  HA_CHECK(n_wg <= 0x7fffffff, "mha_varlen_fwd: too many workgroups");
-  kernel<<<dim3((unsigned)n_wg), 512, lds_bytes, stream>>>(p);
-  check_launch("mha_varlen_fwd");
+  if constexpr (MODE == W8_PAGED) {
+    launch_prefill_nw<T, HDP, MODE, 8>(p, hl, stream);
+  } else if constexpr (HDP <= 64) {
+    // One wavefront's chain of a tile (scores, softmax, products) is as long as the work of two on a SIMD: a third one is free.  us,
+    // eight wavefronts per workgroup / four, 16 q / 2 kv heads x 64: 32 x 1..2048 213 / 190, 64 x 30..300 28 / 21, 64 x 2048 855 / 731,
+    // 8 x 8000 1264 / 1190, 1 x 300 10.0 / 9.1, 1 x 8000 160 / 163.
+    launch_prefill_nw<T, HDP, MODE, 4>(p, hl < 2 ? hl : 2, stream);
+  } else {
+    const int force = tuning().prefill_kernel;
+    if (force == 5 || (force != 1 && four_wavefronts_pay(p, 1 << (hl < 2 ? hl : 2))))
+      launch_prefill_nw<T, HDP, MODE, 4>(p, hl < 2 ? hl : 2, stream);
+    else
+      launch_prefill_nw<T, HDP, MODE, 8>(p, hl, stream);
+  }
 }
 
 template <typename T, int HDP, int QT, bool PAGED = false>
@@ -1399,7 +1491,7 @@ void pick_qt(const PrefillParams &p, int64_t total_q, hipStream_t stream) {
                       (p.total_k + 64) * p.v_row * (int64_t)sizeof(T) < span;
     // it knows the causal mask and no mask; other windows go to the four-wavefront kernel
     const bool plain = p.win_left < 0 && p.win_right <= 0;
-    if (plain && fits && (force == 0 || force == 1)) {
+    if (plain && fits && (force == 0 || force == 1 || force == 5)) {
       launch_prefill_w8<T, HDP>(p, stream);
       return;
     }
@@ -1539,6 +1631,8 @@ void mha_varlen_fwd_impl(const hipattn_tensor *q, const hipattn_tensor *k, const
   p.G = Hq / Hkv;
   p.d = d;
   p.max_q = max_q;
+  p.max_k = max_k;
+  p.total_q = total_q;
   p.lse_pitch = lse ? (int)lse->sizes[2] : 0;
   p.scale_log2 = scale * kLog2e;
   p.causal = causal ? 1 : 0;
@@ -1681,6 +1775,8 @@ void mha_varlen_fwd_paged_impl(const hipattn_tensor *q, const hipattn_tensor *ke
   p.G = Hq / Hkv;
   p.d = d;
   p.max_q = max_q;
+  p.max_k = max_k;
+  p.total_q = total_q;
   p.lse_pitch = lse ? (int)lse->sizes[2] : 0;
   p.scale_log2 = scale * kLog2e;
   p.causal = causal ? 1 : 0;

@@ -345,3 +345,46 @@ def test_several_heads_of_a_kv_group_per_workgroup(device, tuning, limit):
         for b, lq in enumerate(p.lens_q):   # rows past a sequence's length are not written
             assert torch.equal(got_lse[b, :, :lq], want_lse[b, :, :lq])
         assert (got.cpu().double() - fp64(p)).abs().max().item() <= TOL[dtype]
+
+
+@pytest.mark.parametrize("heads", [(8, 2, 128), (4, 4, 80), (6, 2, 96), (8, 1, 120), (4, 1, 64), (2, 2, 48), (2, 1, 32)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_workgroups_of_four_wavefronts(device, tuning, kernel_choice, dtype, heads):
+    """Head sizes up to 64 always, larger ones on short contexts (here: on request) run in workgroups of four wavefronts with three
+    stages, above 64 with tiles of 32 keys: lengths around the edges of tiles, row blocks and stages, alone and behind cached keys,
+    from rows and from the paged cache, masked and not, against float64."""
+    if kernel_choice != "auto":
+        pytest.skip("forces its own kernel")
+    Hq, Hkv, d = heads
+    lens_q = [1, 31, 32, 33, 64, 65, 96, 97, 127, 129, 160, 0, 300, 17]
+    lens_k = [1, 31, 40, 33, 64, 129, 96, 97, 191, 129, 161, 32, 300, 2000]
+    p = general_inputs(71, lens_q, lens_k, Hq, Hkv, d, dtype)
+    tuning("prefill_kernel", 5)
+    want = fp64(p)
+    got, lse = run(p, device, return_lse=True)
+    assert (got.cpu().double() - want).abs().max().item() <= TOL[dtype]
+    unmasked = run(p, device, causal=False)
+    assert (unmasked.cpu().double() - fp64(p, causal=False)).abs().max().item() <= TOL[dtype]
+    # the cache that holds the same keys and values, its blocks in a random order
+    blocks = [(n + 15) // 16 for n in lens_k]
+    order = torch.randperm(sum(blocks) + 3, generator=torch.Generator().manual_seed(7)).tolist()
+    tables = torch.zeros((len(lens_k), max(blocks)), dtype=torch.int32)
+    slots = []
+    for i, (n, nb) in enumerate(zip(lens_k, blocks)):
+        mine, order = order[:nb], order[nb:]
+        tables[i, :nb] = torch.tensor(mine, dtype=torch.int32)
+        slots += [mine[t // 16] * 16 + t % 16 for t in range(n)]
+    pool = sum(blocks) + 3
+    kc = torch.full((pool, Hkv, d // 8, 16, 8), float("nan"), dtype=dtype, device=device)
+    vc = torch.full((pool, Hkv, d, 16), float("nan"), dtype=dtype, device=device)
+    K.reshape_and_cache(p.k.to(device), p.v.to(device), kc, vc, torch.tensor(slots, dtype=torch.int64, device=device))
+    ctx = torch.tensor(lens_k, dtype=torch.int32, device=device)
+    paged, paged_lse = K.flash_attn_varlen_paged(p.q.to(device), kc, vc, tables.to(device), p.cu_q.to(device), ctx, p.max_q, p.max_k,
+                                                 p.scale, True, return_lse=True)
+    assert torch.equal(paged, got)
+    for i, n in enumerate(lens_q):
+        assert torch.equal(paged_lse[i, :, :n], lse[i, :, :n])
+    if d > 64:
+        tuning("prefill_kernel", 1)
+        eight = run(p, device)
+        assert (eight.float() - got.float()).abs().max().item() <= TOL[dtype]
