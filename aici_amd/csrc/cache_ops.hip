@@ -436,6 +436,44 @@ __global__ __launch_bounds__(256) void cache_move_scalar_kernel(
   }
 }
 
+// Block and offset of a slot; block -1: not cached (negative, or past the cache).
+__device__ __forceinline__ int64_t slot_block(int64_t slot, const CacheGeom &g, int &off) {
+  int64_t blk = -1;
+  off = 0;
+  if (slot >= 0 && slot <= 0x7fffffff) {  // (a 64-bit division is some hundred instructions in front of every store)
+    const unsigned b = (unsigned)slot / (unsigned)g.block_size;
+    off = (int)((unsigned)slot - b * (unsigned)g.block_size);
+    blk = b;
+  } else if (slot >= 0) {
+    blk = slot / g.block_size;
+    off = (int)(slot % g.block_size);
+  }
+  return blk < g.num_blocks ? blk : -1;
+}
+
+// One pair of 8-element runs of a head, r elements into either half: rotated in place (NeoX) where `rotate`, and handed back.
+template <typename T>
+__device__ __forceinline__ void rotate_pair(T *arr, const T *cos_ptr, int embed, int r, bool rotate, uint4 &xo, uint4 &yo) {
+  const uint4 xr = *reinterpret_cast<const uint4 *>(arr + r);
+  const uint4 yr = *reinterpret_cast<const uint4 *>(arr + embed + r);
+  xo = xr;
+  yo = yr;
+  if (rotate) {
+    const uint4 cr = *reinterpret_cast<const uint4 *>(cos_ptr + r);
+    const uint4 sr = *reinterpret_cast<const uint4 *>(cos_ptr + embed + r);
+    const T *x = reinterpret_cast<const T *>(&xr), *y = reinterpret_cast<const T *>(&yr);
+    const T *c = reinterpret_cast<const T *>(&cr), *sn = reinterpret_cast<const T *>(&sr);
+    T *xe = reinterpret_cast<T *>(&xo), *ye = reinterpret_cast<T *>(&yo);
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      xe[j] = sub_t(mul_t(x[j], c[j]), mul_t(y[j], sn[j]));
+      ye[j] = add_t(mul_t(y[j], c[j]), mul_t(x[j], sn[j]));
+    }
+    *reinterpret_cast<uint4 *>(arr + r) = xo;
+    *reinterpret_cast<uint4 *>(arr + embed + r) = yo;
+  }
+}
+
 // rotary_embedding followed by reshape_and_cache for the new tokens of a step, in one launch (a decode step
 // is bound by its launches, not by these few kilobytes): a workgroup per token rotates the query heads in
 // place, rotates the key heads in place and writes them to the cache from the same registers, and
@@ -443,7 +481,7 @@ __global__ __launch_bounds__(256) void cache_move_scalar_kernel(
 // rotary_neox_vec8_kernel, so the results equal the two calls bit for bit.  A position outside the table
 // leaves its row unrotated (it is still cached); a negative slot or one past the cache is not cached.
 template <typename T, typename Pos, typename Slot>
-__global__ __launch_bounds__(256) void rotary_cache_kernel(const Pos *__restrict__ positions, T *__restrict__ query,
+__global__ __launch_bounds__(512) void rotary_cache_kernel(const Pos *__restrict__ positions, T *__restrict__ query,
                                                            T *__restrict__ key, const T *__restrict__ value,
                                                            const T *__restrict__ cos_sin, int rot_dim, int64_t max_pos,
                                                            int64_t q_stride, int64_t k_stride, int64_t v_tok_stride,
@@ -453,34 +491,13 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(const Pos *__restrict
   const int64_t token = blockIdx.x;
   const int64_t pos = (int64_t)positions[token];
   const bool rotate = pos >= 0 && pos < max_pos;
-  const int64_t slot = (int64_t)slot_mapping[token];
-  const int64_t blk = slot >= 0 ? slot / g.block_size : -1;
-  const bool cache = blk >= 0 && blk < g.num_blocks;
-  const int off = cache ? (int)(slot % g.block_size) : 0;
+  int off;
+  const int64_t blk = slot_block((int64_t)slot_mapping[token], g, off);
+  const bool cache = blk >= 0;
   const int hd = g.head_size;
   const int embed = rot_dim / 2;
   const int per_head = embed / 8;
   const T *cos_ptr = cos_sin + (rotate ? pos : 0) * rot_dim;
-  auto rotate8 = [&](T *arr, int r, uint4 &xo, uint4 &yo) {
-    const uint4 xr = *reinterpret_cast<const uint4 *>(arr + r);
-    const uint4 yr = *reinterpret_cast<const uint4 *>(arr + embed + r);
-    xo = xr;
-    yo = yr;
-    if (rotate) {
-      const uint4 cr = *reinterpret_cast<const uint4 *>(cos_ptr + r);
-      const uint4 sr = *reinterpret_cast<const uint4 *>(cos_ptr + embed + r);
-      const T *x = reinterpret_cast<const T *>(&xr), *y = reinterpret_cast<const T *>(&yr);
-      const T *c = reinterpret_cast<const T *>(&cr), *sn = reinterpret_cast<const T *>(&sr);
-      T *xe = reinterpret_cast<T *>(&xo), *ye = reinterpret_cast<T *>(&yo);
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        xe[j] = sub_t(mul_t(x[j], c[j]), mul_t(y[j], sn[j]));
-        ye[j] = add_t(mul_t(y[j], c[j]), mul_t(x[j], sn[j]));
-      }
-      *reinterpret_cast<uint4 *>(arr + r) = xo;
-      *reinterpret_cast<uint4 *>(arr + embed + r) = yo;
-    }
-  };
   T *kc_tok = key_cache + (cache ? blk : 0) * g.k_block_stride + (int64_t)off * 8;
   T *vc_tok = value_cache + (cache ? blk : 0) * g.v_block_stride + off;
   const int pass_per_head = (hd - rot_dim) / 8;
@@ -491,10 +508,10 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(const Pos *__restrict
   for (int i = threadIdx.x; i < n_q + n_k + n_pass + n_v; i += blockDim.x) {
     uint4 xo, yo;
     if (i < n_q) {
-      if (rotate) rotate8(query + token * q_stride + (int64_t)(i / per_head) * hd, (i % per_head) * 8, xo, yo);
+      if (rotate) rotate_pair<T>(query + token * q_stride + (int64_t)(i / per_head) * hd, cos_ptr, embed, (i % per_head) * 8, true, xo, yo);
     } else if (i < n_q + n_k) {
       const int j = i - n_q, h = j / per_head, r = (j % per_head) * 8;
-      rotate8(key + token * k_stride + (int64_t)h * hd, r, xo, yo);
+      rotate_pair<T>(key + token * k_stride + (int64_t)h * hd, cos_ptr, embed, r, rotate, xo, yo);
       if (cache) {
         T *kc = kc_tok + h * g.k_head_stride;
         *reinterpret_cast<uint4 *>(kc + (int64_t)(r / 8) * g.block_size * 8) = xo;
@@ -514,6 +531,75 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(const Pos *__restrict
       for (int e = 0; e < 8; e++) vc[(int64_t)e * g.block_size] = ve[e];
     }
   }
+}
+
+// The same for many tokens: a workgroup takes 16 consecutive tokens and either two query heads or one kv head.  Values are turned through
+// LDS, so that a store instruction writes four whole rows of 16 tokens of a block ([head element][16 tokens]) where the tokens' slots
+// follow one another -- the token's own workgroup writes 2 bytes at a time, and a cache line is finished by sixteen of them.
+constexpr int kGroupTokens = 16, kGroupHead = 256;  // largest head size
+// From here on.  us, a workgroup per token / per group (32 q / 8 kv x 128; 32 / 32 x 80): prompts of 722 tokens together 10.1 / 7.0 and 16.6 /
+// 10.1, 2054 20.2 / 12.0 and 39 / 19, 4098 38 / 21 and 130 / 51; one token of each of 64 sequences 6.1 / 6.0 and 5.8 / 4.8, 128 5.1 / 4.8 and
+// 7.3 / 6.3; fewer are the same either way (the launch).
+constexpr int kGroupLeast = 64;
+template <typename T, typename Pos, typename Slot>
+__global__ __launch_bounds__(256) void rotary_cache_group_kernel(const Pos *__restrict__ positions, T *__restrict__ query,
+                                                                 T *__restrict__ key, const T *__restrict__ value,
+                                                                 const T *__restrict__ cos_sin, int rot_dim, int64_t max_pos,
+                                                                 int64_t q_stride, int64_t k_stride, int64_t v_tok_stride,
+                                                                 int64_t v_head_stride, int num_q_heads,
+                                                                 T *__restrict__ key_cache, T *__restrict__ value_cache,
+                                                                 const Slot *__restrict__ slot_mapping, CacheGeom g,
+                                                                 int64_t tokens) {
+  __shared__ uint16_t rows[kGroupTokens * (kGroupHead + 2)];
+  const int tid = threadIdx.x;
+  const int64_t t0 = (int64_t)blockIdx.x * kGroupTokens;
+  const int n = (int)min((int64_t)kGroupTokens, tokens - t0);
+  const int hd = g.head_size, embed = rot_dim / 2, per_head = embed / 8;
+  const int q_jobs = (num_q_heads + 1) / 2;
+  uint4 xo, yo;
+  if ((int)blockIdx.y < q_jobs) {
+    const int h0 = blockIdx.y * 2, heads = min(2, num_q_heads - h0);
+    for (int i = tid; i < n * heads * per_head; i += 256) {
+      const int tok = i / (heads * per_head), rem = i % (heads * per_head);
+      const int64_t t = t0 + tok, pos = (int64_t)positions[t];
+      if (pos >= 0 && pos < max_pos)
+        rotate_pair<T>(query + t * q_stride + (int64_t)(h0 + rem / per_head) * hd, cos_sin + pos * rot_dim, embed, (rem % per_head) * 8,
+                       true, xo, yo);
+    }
+    return;
+  }
+  const int h = blockIdx.y - q_jobs, pitch = hd + 2;
+  for (int i = tid; i < n * (hd / 8); i += 256) {
+    const int tok = i / (hd / 8), ch = i % (hd / 8);
+    const uint4 v = *reinterpret_cast<const uint4 *>(value + (t0 + tok) * v_tok_stride + h * v_head_stride + ch * 8);
+    unsigned *dst = reinterpret_cast<unsigned *>(rows + tok * pitch + ch * 8);
+    dst[0] = v.x, dst[1] = v.y, dst[2] = v.z, dst[3] = v.w;
+  }
+  // a thread keeps to one token (the fastest index, so that a store covers neighbouring places of a block)
+  const int tok = tid % kGroupTokens;
+  const int64_t t = t0 + min(tok, n - 1), pos = (int64_t)positions[t];
+  const bool rotate = pos >= 0 && pos < max_pos;
+  int off;
+  const int64_t blk = slot_block((int64_t)slot_mapping[t], g, off);
+  T *kc = key_cache + (blk < 0 ? 0 : blk) * g.k_block_stride + h * g.k_head_stride + (int64_t)off * 8;
+  T *vc = value_cache + (blk < 0 ? 0 : blk) * g.v_block_stride + h * g.v_head_stride + off;
+  T *row = key + t * k_stride + (int64_t)h * hd;
+  if (tok < n) {
+    for (int i = tid / kGroupTokens; i < per_head; i += 256 / kGroupTokens) {
+      rotate_pair<T>(row, cos_sin + (rotate ? pos : 0) * rot_dim, embed, i * 8, rotate, xo, yo);
+      if (blk >= 0) {
+        *reinterpret_cast<uint4 *>(kc + (int64_t)i * g.block_size * 8) = xo;
+        *reinterpret_cast<uint4 *>(kc + (int64_t)(per_head + i) * g.block_size * 8) = yo;
+      }
+    }
+    if (blk >= 0)
+      for (int ch = 2 * per_head + tid / kGroupTokens; ch < hd / 8; ch += 256 / kGroupTokens)
+        *reinterpret_cast<uint4 *>(kc + (int64_t)ch * g.block_size * 8) = *reinterpret_cast<const uint4 *>(row + ch * 8);
+  }
+  __syncthreads();
+  if (tok < n && blk >= 0)
+    for (int e = tid / kGroupTokens; e < hd; e += 256 / kGroupTokens)
+      vc[(int64_t)e * g.block_size] = bit_cast<T>(rows[tok * pitch + e]);
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -728,15 +814,26 @@ void rotary_and_cache(const hipattn_tensor *positions, hipattn_tensor *query, hi
   check_data(value, "value");
   check_data(cos_sin, "cos_sin_cache");
   const int Hq = (int)(query->sizes[1] / head_size);
+  const bool group = T >= kGroupLeast && head_size <= kGroupHead && (Hq + 1) / 2 + g.num_heads <= 65535;
+  const dim3 groups((unsigned)((T + kGroupTokens - 1) / kGroupTokens), (unsigned)((Hq + 1) / 2 + g.num_heads));
+  const int64_t items = ((int64_t)Hq + g.num_heads) * (rot_dim / 16) + g.num_heads * ((head_size - rot_dim) / 8 + head_size / 8);
 #define HA_RC(TT, PP, SS)                                                                                            \
-  rotary_cache_kernel<TT, PP, SS><<<dim3((unsigned)T), 256, 0, stream>>>(                                             \
+  if (group)                                                                                                         \
+    rotary_cache_group_kernel<TT, PP, SS><<<groups, 256, 0, stream>>>(                                                \
+        static_cast<const PP *>(positions->data), static_cast<TT *>(query->data), static_cast<TT *>(key->data),       \
+        static_cast<const TT *>(value->data), static_cast<const TT *>(cos_sin->data), rot_dim, cos_sin->sizes[0],     \
+        query->strides[0], key->strides[0], value->strides[0], value->strides[1], Hq,                                 \
+        static_cast<TT *>(key_cache->data), static_cast<TT *>(value_cache->data),                                     \
+        static_cast<const SS *>(slot_mapping->data), g, T);                                                           \
+  else                                                                                                               \
+  rotary_cache_kernel<TT, PP, SS><<<dim3((unsigned)T), items > 256 ? 512 : 256, 0, stream>>>(                         \
       static_cast<const PP *>(positions->data), static_cast<TT *>(query->data), static_cast<TT *>(key->data),         \
       static_cast<const TT *>(value->data), static_cast<const TT *>(cos_sin->data), rot_dim, cos_sin->sizes[0],       \
       query->strides[0], key->strides[0], value->strides[0], value->strides[1], Hq, static_cast<TT *>(key_cache->data), \
       static_cast<TT *>(value_cache->data), static_cast<const SS *>(slot_mapping->data), g)
 #define HA_RC_S(TT, PP)                                     \
-  if (slot_mapping->dtype == HIPATTN_I64) HA_RC(TT, PP, int64_t); \
-  else HA_RC(TT, PP, int32_t)
+  if (slot_mapping->dtype == HIPATTN_I64) { HA_RC(TT, PP, int64_t); } \
+  else { HA_RC(TT, PP, int32_t); }
 #define HA_RC_P(TT)                                      \
   if (positions->dtype == HIPATTN_I64) { HA_RC_S(TT, int64_t); } \
   else { HA_RC_S(TT, int32_t); }

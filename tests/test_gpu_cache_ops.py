@@ -435,3 +435,39 @@ def test_rotary_and_cache_equals_the_two_calls(device, case):
     assert torch.equal(bits(qd), bits(q_ref)) and torch.equal(bits(kd), bits(k_ref))
     assert torch.equal(bits(kcd), bits(kc_ref)) and torch.equal(bits(vcd), bits(vc_ref))
     assert torch.equal(bits(vd), bits(v))
+
+
+@pytest.mark.parametrize("heads,rot", [((32, 8, 128), 128), ((3, 1, 80), 32), ((5, 5, 256), 240), ((2, 1, 264), 256), ((4, 2, 8 * 9), 64)])
+@pytest.mark.parametrize("T", [1, 5, 63, 64, 65, 79, 230])
+def test_rotary_and_cache_by_token_and_by_groups_of_tokens(device, heads, rot, T):
+    """From 64 tokens on workgroups take 16 tokens each: both against rotary_embedding and reshape_and_cache, bit for bit, for tokens whose
+    slots follow one another from anywhere in a block, jump, or are not cached, blocks of 8, 16 and 32 tokens, numbers of query heads
+    that do not pair up, heads wider than a group takes, and slots beyond 32 bits."""
+    Hq, Hkv, d = heads
+    g = torch.Generator().manual_seed(T + d)
+    for bs in (8, 16, 32):
+        nb = (2 * T + 100) // bs + 4
+        qkv = torch.randn((T, (Hq + 2 * Hkv) * d), generator=g).to(torch.bfloat16).to(device)
+        pos = torch.randint(0, 300, (T,), generator=g)
+        pos[T // 2] = 400
+        slots = torch.arange(T, dtype=torch.int64) + 5
+        slots[T // 3:] += bs + 3
+        slots[T // 2:] += torch.randperm(T - T // 2, generator=g) - torch.arange(T - T // 2)
+        slots[0] = -1
+        if T > 4:
+            slots[3], slots[4] = (1 << 33) + 7, nb * bs
+        slots, pos = slots.to(device), pos.to(device)
+        table = ref.rotary_table(rot, 10000.0, 300, torch.bfloat16).to(device)
+        caches = [t.to(device) for t in make_cache(nb, Hkv, d, bs, torch.bfloat16, fill=-2.0)]
+        both = []
+        for fused in (True, False):
+            x, kc, vc = qkv.clone(), caches[0].clone(), caches[1].clone()
+            q, k, v = x[:, :Hq * d], x[:, Hq * d:(Hq + Hkv) * d], x[:, (Hq + Hkv) * d:].view(T, Hkv, d)
+            if fused:
+                K.rotary_embedding_and_cache(pos, q, k, v, d, table, True, kc, vc, slots)
+            else:
+                K.rotary_embedding(pos, q, k, d, table, True)
+                K.reshape_and_cache(k.view(T, Hkv, d), v, kc, vc, slots)
+            both.append((x, kc, vc))
+        for a, b in zip(*both):
+            assert torch.equal(bits(a), bits(b))
