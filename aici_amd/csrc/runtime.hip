@@ -144,12 +144,20 @@ void *try_library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream
     return nullptr;
   }
   if (capturing != hipStreamCaptureStatusNone) return nullptr;
-  try {
-    return library_workspace(user, bytes, stream);
-  } catch (const Error &) {
+  // A capture on some other stream forbids allocations, in every thread unless the thread says otherwise.
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
+  void *ws = nullptr;
+  try {
+    ws = library_workspace(user, bytes, stream);
+  } catch (const Error &) {
+    (void)hipGetLastError();
+  }
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  return ws;
 }
 
 }  // namespace hipattn

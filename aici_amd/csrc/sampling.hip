@@ -32,6 +32,8 @@
 // 128 rows of 128256 bf16 logits, 5 % allowed, top-p 0.9: any row 199 us, counting 43 us; all allowed 221 / 55, one row
 // 177 / 40; fp16 203 / 60 (the logits take 5 us to read once; a pass over one row on one compute unit takes 6 to 12).  Counted in
 // pieces, bf16: 26 and, all allowed, 29 us; one row 15.
+#include <mutex>
+
 #include "common.h"
 #include "device_types.h"
 #include "workspace.h"
@@ -1209,10 +1211,17 @@ void bias_sample_impl(const hipattn_tensor *logits, const hipattn_tensor *bias, 
   HA_CHECK(S <= 0x7fffffff, "%s: too many sequences", op);
   // Pieces, where there are several and workgroups for them: the scratch memory then stays below 40 MB.  Under capture the row's
   // workgroup does it alone: the graph may be replayed beside other calls on this stream's scratch memory.
+  // Two launches that share it stay next to one another where several threads use one stream; hipStreamPerThread names a stream of each
+  // thread's own by one handle, so it has no scratch memory.
+  static std::mutex pair_mutex;
+  std::unique_lock<std::mutex> pair(pair_mutex, std::defer_lock);
   const int64_t n_pieces = (V + kPieceTokens - 1) / kPieceTokens;
   PieceCounts *pieces = nullptr;
-  if (mask && logits->dtype == HIPATTN_BF16 && V >= kLeastPieces && n_pieces <= kMaxPieces && S * n_pieces <= 2048)
+  if (mask && logits->dtype == HIPATTN_BF16 && V >= kLeastPieces && n_pieces <= kMaxPieces && S * n_pieces <= 2048 &&
+      stream != hipStreamPerThread) {
+    pair.lock();
     pieces = static_cast<PieceCounts *>(try_library_workspace(WS_SAMPLE, (size_t)(S * n_pieces) * sizeof(PieceCounts), stream));
+  }
   if (pieces != nullptr) {
     sample_count_kernel<bf16_t><<<dim3((unsigned)n_pieces, (unsigned)S), kCountThreads, 0, stream>>>(p, pieces);
     check_launch(op);

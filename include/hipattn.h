@@ -432,7 +432,12 @@ char *hipattn_bias_argmax(const hipattn_tensor *logits,
  * clamped.  A token with bias -inf is never drawn, whatever the temperature.
  * A row that holds +inf (where the reference's softmax has no answer) yields
  * the first such token, a row with nothing allowed token 0.
- * out_tokens int32 [S]. */
+ * out_tokens int32 [S].
+ * bf16 rows of 24576 to 262144 tokens under a mask are read by several
+ * workgroups each, which leave their counts in a buffer of the library's that
+ * belongs to the stream (up to 58 MB, kept until hipattn_shutdown).  While the stream
+ * is being captured, or without memory for the buffer, one workgroup reads the
+ * row, as for other rows: the same tokens. */
 char *hipattn_bias_sample(const hipattn_tensor *logits,
                           const hipattn_tensor *bias,
                           const hipattn_tensor *mask,

@@ -1,10 +1,12 @@
 """rotary_embedding, rms_norm, activations, bias_argmax and the runtime plumbing through the
 C ABI against the oracle."""
+import threading
+
 import numpy as np
 import pytest
 import torch
 
-from aici_amd import attn, kernels as K
+from aici_amd import _native, attn, kernels as K
 from aici_amd import workloads as W
 from aici_amd._lib import HipAttnError
 from oracle import aici
@@ -353,6 +355,52 @@ def test_bias_sample_in_pieces_gives_the_same_tokens(device, V):
         graph.replay()
         assert torch.equal(replayed, want)
         assert torch.equal(K.bias_sample(rows, temperature, top_p, u, mask=mask), want)
+
+
+def test_bias_sample_in_pieces_from_several_threads(device):
+    """Two threads on one stream share its scratch memory: each still gets its own tokens.  A first call on a stream while another
+    one is being captured neither fails nor spoils the capture."""
+    V, S = 32768, 5
+    g = torch.Generator().manual_seed(3)
+    rows = [(torch.randn((S, V), generator=g) * (1 + i)).to(torch.bfloat16).to(device) for i in range(2)]
+    mask = torch.full((S, V // 8), 255, dtype=torch.uint8, device=device)
+    ones = torch.ones((S,), device=device)
+    u = [torch.rand((S,), generator=g).to(device) for _ in range(2)]
+    want = [K.bias_sample(rows[i].float(), ones, 0.9 * ones, u[i], mask=mask) for i in range(2)]
+    got = [[], []]
+
+    def calls(i):
+        for _ in range(200):
+            got[i].append(K.bias_sample(rows[i], ones, 0.9 * ones, u[i], mask=mask))
+
+    threads = [threading.Thread(target=calls, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert all(len(got[i]) == 200 and all(torch.equal(t, want[i]) for t in got[i]) for i in range(2))
+
+    top_p = 0.9 * ones
+    first, out = torch.cuda.Stream(), torch.zeros((S,), dtype=torch.int32, device=device)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+
+    def on_first():
+        with torch.cuda.stream(first):
+            _native.bias_sample(rows[1], None, mask, None, ones, top_p, u[1], out)
+
+    with torch.cuda.graph(graph):
+        captured = rows[0] * 2
+        t = threading.Thread(target=on_first)
+        t.start()
+        t.join()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want[1])
+    for _ in range(2):
+        captured.zero_()
+        graph.replay()
+        assert torch.equal(captured, rows[0] * 2)
 
 
 def test_bias_sample_corner_rows(device):
