@@ -285,9 +285,9 @@ def linear_rms_norm(x: torch.Tensor, weight: torch.Tensor, norm_weight: torch.Te
 RMS_NORM_LINEAR_MAX_ROWS = 4
 
 
-def rms_norm_linear_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
+def rms_norm_linear_takes(x: torch.Tensor, norm_weight: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether `rms_norm_linear` accepts these operands (else a caller makes the two calls)."""
-    return (linear_takes(x, weight) and x.size(0) <= RMS_NORM_LINEAR_MAX_ROWS and x.size(1) <= 8192
+    return (linear_takes(x, weight) and norm_weight.data_ptr() % 16 == 0 and norm_weight.is_contiguous() and x.size(0) <= RMS_NORM_LINEAR_MAX_ROWS and x.size(1) <= 8192
             and (x.size(0) + 1) * ((x.size(1) * 2 + 1023) // 1024) <= 40 and weight.size(0) < 65536 and weight.size(0) % 32 == 0
             and 0 < weight.stride(0) < 1 << 28 and (x.size(0) == 1 or 0 <= x.stride(0) < 1 << 28))
 

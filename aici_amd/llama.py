@@ -117,11 +117,11 @@ class Llama:
         kernels.rms_norm(out, x, weight, self.cfg.rms_norm_eps)
         return out
 
-    def _norm_in_proj(self, x: torch.Tensor, weight: torch.Tensor) -> bool:
+    def _norm_in_proj(self, x: torch.Tensor, norm_weight: torch.Tensor, weight: torch.Tensor) -> bool:
         """Whether the projection normalises its rows itself, the same bits (us, 4096 columns, norm and projection / one launch: 6144
         rows 13.1 / 11.2 with one row of x, 13.3 / 13.1 with four; 28672 rows 45.9 / 43.1 and 45.9 / 43.8)."""
         return (x.size(0) <= kernels.RMS_NORM_LINEAR_MAX_ROWS and self.skinny_linear and self.fused_norm
-                and kernels.rms_norm_linear_takes(x, weight))
+                and kernels.rms_norm_linear_takes(x, norm_weight, weight))
 
     def _proj(self, x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         """x @ weight.T (llama.rs:81-83, 210).  A vocabulary's rows with more than 48 sequences stay with the library
@@ -145,7 +145,7 @@ class Llama:
         rows -- residual and norm -- in the launch that adds the parts up; else a library GEMM, an addition and
         rms_norm.  The same bits either way as far as the norm goes."""
         if self.skinny_linear and weight.size(0) <= 8192 and kernels.linear_takes(y, weight):
-            if behind is not None and self._norm_in_proj(x, behind):
+            if behind is not None and self._norm_in_proj(x, norm_weight, behind):
                 return kernels.linear(y, weight, residual=x), None
             if self.fused_norm:
                 return kernels.linear_rms_norm(y, weight, norm_weight, self.cfg.rms_norm_eps, residual=x)
@@ -165,7 +165,8 @@ class Llama:
         x = self.wte.index_select(0, batch_info.tokens.long())                   # llama.rs:203
         T = x.size(0)
         # h: the normalised rows, None where the projection that takes them does it
-        h = None if self._norm_in_proj(x, self.layers[0]["qkv"]) else self._rms(x, self.layers[0]["rms_1"])  # :165
+        first = self.layers[0]
+        h = None if self._norm_in_proj(x, first["rms_1"], first["qkv"]) else self._rms(x, first["rms_1"])  # :165
         for li, (layer, (kc, vc)) in enumerate(zip(self.layers, caches)):
             if h is None:
                 qkv = kernels.rms_norm_linear(x, layer["rms_1"], cfg.rms_norm_eps, layer["qkv"])

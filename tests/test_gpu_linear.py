@@ -342,7 +342,7 @@ def test_rms_norm_linear_gives_the_bits_of_the_two_calls(device, dtype, Kd, N, M
     norm = (1 + 0.2 * torch.randn((Kd,), generator=g)).to(dtype).to(device)
     h = torch.empty((M, Kd), dtype=dtype, device=device)
     K.rms_norm(h, x.contiguous(), norm, 1e-5)
-    assert K.rms_norm_linear_takes(x, weight)
+    assert K.rms_norm_linear_takes(x, norm, weight)
     before = wide.clone()
     for _ in range(2):
         assert torch.equal(K.rms_norm_linear(x, norm, 1e-5, weight), K.linear(h, weight))
@@ -354,7 +354,8 @@ def test_rms_norm_linear_refusals(device):
     x = torch.zeros((5, 4096), dtype=torch.bfloat16, device=device)
     w = torch.zeros((64, 4096), dtype=torch.bfloat16, device=device)
     norm = torch.ones((4096,), dtype=torch.bfloat16, device=device)
-    assert not K.rms_norm_linear_takes(x, w)
+    assert not K.rms_norm_linear_takes(x, norm, w)
+    assert not K.rms_norm_linear_takes(x[:4], torch.ones((4097,), dtype=torch.bfloat16, device=device)[1:], w)
     with pytest.raises(HipAttnError, match="at most 4 rows"):
         K.rms_norm_linear(x, norm, 1e-5, w)
     with pytest.raises(HipAttnError, match="at most 4 rows"):  # 3 rows of 8192: more than 40 KB with the norm's weight
