@@ -94,6 +94,7 @@ _ERR_FUNCS = {
     "hipattn_rotary_embedding_and_cache": [TP, TP, TP, TP, c_int, TP, c_bool, TP, TP, TP, c_void_p],
     "hipattn_rms_norm": [TP, TP, TP, c_float, c_void_p],
     "hipattn_fused_add_rms_norm": [TP, TP, TP, c_float, c_void_p],
+    "hipattn_add_rms_norm": [TP, TP, TP, TP, c_float, c_void_p],
     "hipattn_linear": [TP, TP, TP, TP, TP, TP, c_void_p],
     "hipattn_linear_silu_and_mul": [TP, TP, TP, TP, c_void_p],
     "hipattn_rms_norm_linear": [TP, TP, TP, c_float, TP, c_bool, c_void_p],

@@ -349,6 +349,7 @@ PyMethodDef g_methods[] = {
                                      "slot_mapping"),
     BIND(rms_norm, "out,input,weight,epsilon"),
     BIND(fused_add_rms_norm, "input,residual,weight,epsilon"),
+    BIND(add_rms_norm, "out,input,residual,weight,epsilon"),
     BIND(linear, "out,x,weight,bias,residual,workspace"),
     BIND(linear_silu_and_mul, "out,x,weight,workspace"),
     BIND(linear_rms_norm, "out,norm_out,x,weight,bias,residual,norm_weight,epsilon,workspace"),

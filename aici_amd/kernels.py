@@ -242,6 +242,20 @@ def fused_add_rms_norm(input: torch.Tensor, residual: torch.Tensor, weight: torc
     _native.fused_add_rms_norm(input, residual, weight, epsilon)
 
 
+def add_rms_norm_takes(input: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether `add_rms_norm` accepts these operands (else a caller makes the two calls)."""
+    return (input.dtype in (torch.float16, torch.bfloat16) and input.size(1) % 8 == 0 and input.size(1) <= 8192
+            and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (input, residual, weight)))
+
+
+def add_rms_norm(input: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, epsilon: float) -> torch.Tensor:
+    """input += residual and rms_norm of the sum, in one launch with the bits of the two calls (llama.rs:166 + 169, 173 + 165): returns
+    the norm; input [rows, hidden] holds the sum."""
+    out = torch.empty_like(input)
+    _native.add_rms_norm(out, input, residual, weight, epsilon)
+    return out
+
+
 LINEAR_MAX_ROWS = 128
 
 

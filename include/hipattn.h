@@ -303,6 +303,15 @@ char *hipattn_fused_add_rms_norm(hipattn_tensor *input,
                                  const hipattn_tensor *weight, float epsilon,
                                  void *stream);
 
+/* The residual addition and the norm behind it (llama.rs:166 + 169, 173 + 165) as the two calls round them: input = T(input + residual),
+ * out = rms_norm(input) * weight, the variance that of the rounded sum (hipattn_fused_add_rms_norm takes the unrounded one).
+ * [rows, hidden] f16 or bf16, contiguous, on 16-byte boundaries, hidden a multiple of 8, at most 8192; input must not share memory with
+ * the others. */
+char *hipattn_add_rms_norm(hipattn_tensor *out, hipattn_tensor *input,
+                           const hipattn_tensor *residual,
+                           const hipattn_tensor *weight, float epsilon,
+                           void *stream);
+
 /* A linear layer applied to at most 128 rows: out = x . weight^T (+ bias)
  * (+ residual), the projections of a generation step.  Replaces the
  * `nn::Linear::forward` calls that rLLM makes through `linear_no_bias` /

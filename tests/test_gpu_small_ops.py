@@ -318,6 +318,34 @@ def test_bias_sample_counts_equal_logits_to_the_same_tokens(device, dtype, V, sh
     assert torch.equal(got, want), torch.nonzero(got != want).flatten().tolist()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,hidden", [(1, 8), (3, 4096), (742, 512), (130, 8192), (17, 2568)])
+def test_add_rms_norm_gives_the_bits_of_the_two_calls(device, dtype, rows, hidden):
+    g = torch.Generator().manual_seed(rows + hidden)
+    x, res = ((torch.randn((rows, hidden), generator=g) * 3).to(dtype).to(device) for _ in range(2))
+    weight = (1 + 0.3 * torch.randn((hidden,), generator=g)).to(dtype).to(device)
+    total = x + res
+    want = torch.empty_like(total)
+    K.rms_norm(want, total, weight, 1e-5)
+    before = res.clone()
+    assert K.add_rms_norm_takes(x, res, weight)
+    got = K.add_rms_norm(x, res, weight, 1e-5)
+    assert torch.equal(x, total) and torch.equal(got, want) and torch.equal(res, before)
+
+
+def test_add_rms_norm_refusals(device):
+    x = torch.zeros((4, 4096), dtype=torch.bfloat16, device=device)
+    w = torch.ones((4096,), dtype=torch.bfloat16, device=device)
+    odd = torch.ones((4097,), dtype=torch.bfloat16, device=device)[1:]
+    for bad in ((x.float(), x.float(), w.float()), (x, x.clone(), odd), (x[:, ::2], x[:, ::2].clone(), w[:2048])):
+        assert not K.add_rms_norm_takes(*bad)
+    for bad in ((x.float(), x.float(), w.float()), (x, x[:3].clone(), w), (x, x.clone(), w[:8]), (x, x.clone(), odd),
+                (x[:, ::2], x[:, ::2].clone(), w[:2048]),
+                (x[:, :4].contiguous(), x[:, :4].contiguous(), w[:4])):
+        with pytest.raises(HipAttnError, match="add_rms_norm|contiguous"):
+            K.add_rms_norm(bad[0], bad[1], bad[2], 1e-5)
+
+
 @pytest.mark.parametrize("V", [24575, 24576, 32768, 32776, 128256, 262144, 262152])
 def test_bias_sample_in_pieces_gives_the_same_tokens(device, V):
     """bf16 rows of 24576 to 262144 tokens are counted by a workgroup per 16384 of them.  The same values in float32 take the
