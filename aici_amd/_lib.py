@@ -98,6 +98,7 @@ _ERR_FUNCS = {
     "hipattn_linear": [TP, TP, TP, TP, TP, TP, c_void_p],
     "hipattn_linear_silu_and_mul": [TP, TP, TP, TP, c_void_p],
     "hipattn_rms_norm_linear": [TP, TP, TP, c_float, TP, c_bool, c_void_p],
+    "hipattn_qkv_linear": [TP, TP, TP, c_float, TP, TP, TP, TP, TP, TP, c_void_p],
     "hipattn_linear_workspace_size": [TP, TP, POINTER(c_int64)],
     "hipattn_linear_rms_norm": [TP, TP, TP, TP, TP, TP, TP, c_float, TP, c_void_p],
     "hipattn_linear_rms_norm_workspace_size": [TP, TP, POINTER(c_int64)],

@@ -354,6 +354,7 @@ PyMethodDef g_methods[] = {
     BIND(linear_silu_and_mul, "out,x,weight,workspace"),
     BIND(linear_rms_norm, "out,norm_out,x,weight,bias,residual,norm_weight,epsilon,workspace"),
     BIND(rms_norm_linear, "out,x,norm_weight,epsilon,weight,silu_and_mul"),
+    BIND(qkv_linear, "out,x,norm_weight,epsilon,weight,positions,cos_sin_cache,key_cache,value_cache,slot_mapping"),
     BIND(silu_and_mul, "out,input"),
     BIND(gelu_new, "out,input"),
     BIND(gelu_fast, "out,input"),

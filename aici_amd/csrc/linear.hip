@@ -36,6 +36,7 @@
 //
 // Rounding points: fp32 accumulation over k, + bias in fp32, rounded to T -- what a library GEMM with a bias epilogue
 // does; then, if a residual is given, T(y + residual): the separate addition of llama.rs:166, 173, rounded again.
+#include "cache_geom.h"
 #include "common.h"
 #include "device_types.h"
 #include "workspace.h"
@@ -57,6 +58,16 @@ constexpr int kLinHeldBytes = 40 * 1024;  // of x and the norm's weight: two wor
 constexpr int kHeldStages = 4;
 constexpr int kLinMaxRanges = 8;  // ranges of k that the library itself chooses
 
+// Behind the projection of q, k and v: the rotation of the query and key heads and the writes of keys and values to the cache.
+struct QkvParams {
+  const void *positions, *slots, *cos_sin;  // cos_sin: rows of head_size values, cosines first
+  bool pos64, slot64;
+  int64_t max_pos;
+  int q_heads;
+  void *key_cache, *value_cache;
+  CacheGeom g;
+};
+
 struct LinearParams {
   const void *x, *w, *bias, *residual;
   void *out;
@@ -77,6 +88,7 @@ struct LinearParams {
   int64_t ldn;
   float eps;
   int norm_in;  // the norm is that of the rows of x, in front of the layer
+  QkvParams qkv;
 };
 
 template <typename T>
@@ -124,6 +136,97 @@ __device__ __forceinline__ void linear_finish_gated(const LinearParams &p, f32x4
 #pragma unroll
   for (int r = 0; r < 4; r++) o[r] = mul_t<T>(silu_t<T>(from_float<T>(gate[r])), from_float<T>(up[r]));
   *reinterpret_cast<vec4 *>(static_cast<T *>(p.out) + (int64_t)m * p.ldo + n) = o;
+}
+
+// Rows of W of tile `tile` (16 of them): of a head that is rotated eight rows from its first half and the eight that they are rotated
+// with, so that a wavefront's sums hold both; else sixteen in order.
+struct QkvRows {
+  int first, second;  // of eight rows each
+  int head;
+  bool rotated;
+};
+__device__ __forceinline__ QkvRows qkv_rows(const QkvParams &q, int tile) {
+  const int hd = q.g.head_size, n = tile * 16, head = n / hd, r = (n - head * hd) / 2;
+  QkvRows t;
+  t.head = head;
+  t.rotated = head < q.q_heads + q.g.num_heads;
+  t.first = t.rotated ? head * hd + r : n;
+  t.second = t.first + (t.rotated ? hd / 2 : 8);
+  return t;
+}
+
+// Position and slot of row m: asked for in front of the weight's copies, needed behind them.
+struct QkvToken {
+  int64_t pos, slot;
+};
+__device__ __forceinline__ QkvToken qkv_token(const QkvParams &q, int m) {
+  QkvToken t;
+  t.pos = q.pos64 ? static_cast<const int64_t *>(q.positions)[m] : (int64_t)static_cast<const int32_t *>(q.positions)[m];
+  t.slot = q.slot64 ? static_cast<const int64_t *>(q.slots)[m] : (int64_t)static_cast<const int32_t *>(q.slots)[m];
+  return t;
+}
+template <typename T>
+struct QkvTurn {  // cosines and sines of a lane's four elements
+  typedef T vec4 __attribute__((ext_vector_type(4)));
+  vec4 c, s;
+  bool rotate;
+};
+template <typename T>
+__device__ __forceinline__ QkvTurn<T> qkv_turn(const QkvParams &q, const QkvRows &rows, const QkvToken &tok, int kg) {
+  using vec4 = typename QkvTurn<T>::vec4;
+  const int hd = q.g.head_size;
+  QkvTurn<T> t;
+  t.rotate = rows.rotated && tok.pos >= 0 && tok.pos < q.max_pos;
+  t.c = t.s = vec4{(T)0.f, (T)0.f, (T)0.f, (T)0.f};
+  if (t.rotate) {
+    const T *at = static_cast<const T *>(q.cos_sin) + tok.pos * hd + (rows.first - rows.head * hd) + 4 * (kg & 1);
+    t.c = *reinterpret_cast<const vec4 *>(at);
+    t.s = *reinterpret_cast<const vec4 *>(at + hd / 2);
+  }
+  return t;
+}
+
+// linear_finish for such a tile, with the arithmetic of rotary_cache_kernel on the rounded products, so its bits.  A launch of a few
+// kilobytes less, for one more dependent load (the table's row) at the end of this one.  us, the projection and the launch behind it /
+// together, weights cold: 6144 x 4096 (32 / 8 heads of 128) 1 row 15.3 / 11.6, 16 17.4 / 13.8, 32 19.7 / 16.4, 128 26.2 / 23.2; 7680 x
+// 2560 (32 / 32 of 80) 14.0 / 9.5, 16.1 / 11.6, 19.9 / 15.7, 25.0 / 22.6; 12288 x 4096 27.7 / 22.4, 31.0 / 25.8, 32.5 / 28.4, 40.4 / 40.0.
+// From 16384 rows of weight on the sums of more than 16 rows of x are finished in the tile kernel: not built for it.
+template <typename T>
+__device__ __forceinline__ void linear_finish_qkv(const LinearParams &p, f32x4_t v, int m, int kg, const QkvRows &rows, const QkvToken &tok,
+                                                  const QkvTurn<T> &turn) {
+  using vec4 = typename QkvTurn<T>::vec4;
+  const QkvParams &q = p.qkv;
+  const int hd = q.g.head_size;
+  vec4 mine, o;
+#pragma unroll
+  for (int r = 0; r < 4; r++) mine[r] = from_float<T>(v[r]);
+  const uint2 raw = bit_cast<uint2>(mine);
+  const vec4 other = bit_cast<vec4>(make_uint2((uint32_t)__shfl_xor((int)raw.x, 32), (uint32_t)__shfl_xor((int)raw.y, 32)));
+  const bool high = kg >= 2;
+  o = mine;
+  if (turn.rotate) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const T here = mul_t<T>(mine[r], turn.c[r]), there = mul_t<T>(other[r], turn.s[r]);
+      o[r] = high ? add_t<T>(here, there) : sub_t<T>(here, there);
+    }
+  }
+  const int n = (high ? rows.second : rows.first) + 4 * (kg & 1);
+  if (m >= p.M || n >= p.N) return;
+  *reinterpret_cast<vec4 *>(static_cast<T *>(p.out) + (int64_t)m * p.ldo + n) = o;
+  if (rows.head < q.q_heads) return;
+  int off;
+  const int64_t blk = slot_block(tok.slot, q.g, off);
+  if (blk < 0) return;
+  const int i = n - rows.head * hd;  // element of the head
+  if (rows.rotated) {
+    T *kc = static_cast<T *>(q.key_cache) + blk * q.g.k_block_stride + (rows.head - q.q_heads) * q.g.k_head_stride;
+    *reinterpret_cast<vec4 *>(kc + ((int64_t)(i / 8) * q.g.block_size + off) * 8 + (i & 7)) = o;
+  } else {
+    T *vc = static_cast<T *>(q.value_cache) + blk * q.g.v_block_stride + (rows.head - q.q_heads - q.g.num_heads) * q.g.v_head_stride;
+#pragma unroll
+    for (int r = 0; r < 4; r++) vc[(int64_t)(i + r) * q.g.block_size + off] = o[r];
+  }
 }
 
 template <int N>
@@ -193,14 +296,14 @@ __device__ __forceinline__ f32x4_t add_ranges(const f32x4_t *src, int splits) {
 }
 
 // Up to 16 rows of x.  WAVES wavefronts; each owns 16 NT rows of W.  GATED: odd wavefronts take the up rows that
-// belong to the gate rows of the wavefront before them.
-template <typename T, int NT, int S, int WAVES, bool GATED>
+// belong to the gate rows of the wavefront before them.  QKV: rotation and cache writes behind it.
+template <typename T, int NT, int S, int WAVES, bool GATED, bool QKV = false>
 __global__ __launch_bounds__(WAVES * 64) void linear_stream_kernel(const LinearParams p) {
   using vec8 = typename Vec8<T>::type;
   constexpr int kParts = GATED ? 2 : 1;
   constexpr int kCopiesW = 2 * NT, kCopiesX = 2, kCopies = kCopiesW + kCopiesX;  // of 1 KB: eight rows each
   constexpr int kStageBytes = kCopies * 1024;
-  static_assert(NT == 1 || !GATED, "gated: one tile per wavefront");
+  static_assert(NT == 1 || !(GATED || QKV), "gated, q k v: one tile per wavefront");
   __shared__ __align__(1024) char ring[WAVES * S * kStageBytes];
   // NT > 1 is for weights of so many rows that k is not cut
   __shared__ f32x4_t sums[NT == 1 ? kParts * kLinMaxRanges * 64 : 1];
@@ -218,10 +321,17 @@ __global__ __launch_bounds__(WAVES * 64) void linear_stream_kernel(const LinearP
   const int stage0 = first_range * p.stages_per_split;
   const int nst = max(0, min(ranges * p.stages_per_split, p.total_stages - stage0));
 
+  QkvRows rows = {};
+  QkvToken token = {};
+  if constexpr (QKV) {
+    rows = qkv_rows(p.qkv, blockIdx.x * tiles + tile);
+    token = qkv_token(p.qkv, min(col, p.M - 1));
+  }
   CopySource<false> wsrc[kCopiesW], xsrc[kCopiesX];
 #pragma unroll
   for (int i = 0; i < kCopiesW; i++)
-    wsrc[i] = copy_source<T, false>(p.w, p.ldw, part * p.half + n_tile + i * 8, part * p.half + n_end - 1, stage0);
+    wsrc[i] = copy_source<T, false>(p.w, p.ldw, QKV ? (i ? rows.second : rows.first) : part * p.half + n_tile + i * 8,
+                                    part * p.half + n_end - 1, stage0);
 #pragma unroll
   for (int i = 0; i < kCopiesX; i++) xsrc[i] = copy_source<T, false>(p.x, p.ldx, i * 8, p.M - 1, stage0);
   const char *mine = ring + wave * S * kStageBytes;
@@ -276,6 +386,16 @@ __global__ __launch_bounds__(WAVES * 64) void linear_stream_kernel(const LinearP
       }
     }
   }
+  QkvTurn<T> turn = {};
+  // (a wavefront that finishes a tile finishes the workgroup's `wave`th, whichever it worked on)
+  if constexpr (QKV) {
+    if (meet) rows = qkv_rows(p.qkv, blockIdx.x * tiles + wave);
+    if (!meet || wave < tiles) turn = qkv_turn<T>(p.qkv, rows, token, kg);
+    if (!meet) {
+      linear_finish_qkv<T>(p, acc[0], col, kg, rows, token, turn);
+      return;
+    }
+  }
   if (!meet) {
 #pragma unroll
     for (int t = 0; t < NT; t++) linear_finish<T>(p, acc[t], col, n_tile + t * 16 + 4 * kg);
@@ -294,6 +414,8 @@ __global__ __launch_bounds__(WAVES * 64) void linear_stream_kernel(const LinearP
       for (int q = 0; q < kParts; q++) total[q] = add_ranges(sums + (wave * kParts + q) * p.splits * 64 + lane, p.splits);
       if constexpr (GATED)
         linear_finish_gated<T>(p, total[0], total[1], col, n);
+      else if constexpr (QKV)
+        linear_finish_qkv<T>(p, total[0], col, kg, rows, token, turn);
       else
         linear_finish<T>(p, total[0], col, n);
     }
@@ -305,7 +427,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_stream_kernel(const LinearP
 // rms_norm less, whose time is all latency.  The rows' part repeats in every workgroup and costs about 1 us per row, so it ends at few
 // rows.  LDS: ring | sums of ranges | rows of x | the norm's weight.
 __host__ __device__ constexpr int held_pitch(int K) { return (K * 2 + 1023) / 1024 * 1024; }
-template <typename T, int S, int ROWS, bool GATED>
+template <typename T, int S, int ROWS, bool GATED, bool QKV>
 __global__ __launch_bounds__(256) void norm_linear_kernel(const LinearParams p) {
   using vec8 = typename Vec8<T>::type;
   constexpr int WAVES = 4, kParts = GATED ? 2 : 1;
@@ -340,10 +462,17 @@ __global__ __launch_bounds__(256) void norm_linear_kernel(const LinearParams p) 
       copy_1k<false, false>(at + i * 1024, src, 0);
     }
   }
+  QkvRows rows = {};
+  QkvToken token = {};
+  if constexpr (QKV) {
+    rows = qkv_rows(p.qkv, blockIdx.x * tiles + tile);
+    token = qkv_token(p.qkv, min(col, p.M - 1));
+  }
   CopySource<false> wsrc[2];
 #pragma unroll
   for (int i = 0; i < 2; i++)
-    wsrc[i] = copy_source<T, false>(p.w, p.ldw, part * p.half + n_tile + i * 8, part * p.half + n_end - 1, stage0);
+    wsrc[i] = copy_source<T, false>(p.w, p.ldw, QKV ? (i ? rows.second : rows.first) : part * p.half + n_tile + i * 8,
+                                    part * p.half + n_end - 1, stage0);
   const char *mine = lds + wave * S * kStageBytes;
   const uint32_t mine_lds = lds_address(lds) + wave * S * kStageBytes;
   auto ask = [&](int slot, int st) {
@@ -436,6 +565,15 @@ __global__ __launch_bounds__(256) void norm_linear_kernel(const LinearParams p) 
       }
     }
   }
+  QkvTurn<T> turn = {};
+  if constexpr (QKV) {
+    if (p.splits > 1) rows = qkv_rows(p.qkv, blockIdx.x * tiles + wave);
+    if (p.splits == 1 || wave < tiles) turn = qkv_turn<T>(p.qkv, rows, token, kg);
+    if (p.splits == 1) {
+      linear_finish_qkv<T>(p, acc, col, kg, rows, token, turn);
+      return;
+    }
+  }
   if (!GATED && p.splits == 1) {
     linear_finish<T>(p, acc, col, n_tile + 4 * kg);
     return;
@@ -452,6 +590,8 @@ __global__ __launch_bounds__(256) void norm_linear_kernel(const LinearParams p) 
     for (int q = 0; q < kParts; q++) total[q] = add_ranges(sums + (wave * kParts + q) * p.splits * 64 + lane, p.splits);
     if constexpr (GATED)
       linear_finish_gated<T>(p, total[0], total[1], col, n);
+    else if constexpr (QKV)
+      linear_finish_qkv<T>(p, total[0], col, kg, rows, token, turn);
     else
       linear_finish<T>(p, total[0], col, n);
   }
@@ -574,7 +714,8 @@ __global__ __launch_bounds__(WAVES * 64) void linear_tile_kernel(const LinearPar
 }
 
 // Adds up the ranges' sums, the first range first, and finishes the tile: one thread per (16 rows of W, row tile, lane).
-template <typename T, bool GATED>
+// QKV: a lane's sums are those of the rows that linear_finish_qkv wants there, from two tiles.
+template <typename T, bool GATED, bool QKV>
 __global__ __launch_bounds__(256) void linear_reduce_kernel(const LinearParams p) {
   const int ntiles = p.N / 16;
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -583,8 +724,8 @@ __global__ __launch_bounds__(256) void linear_reduce_kernel(const LinearParams p
   const int64_t nt = (idx >> 6) / p.mtiles;
   if (nt >= (GATED ? p.half / 16 : ntiles)) return;
   const int64_t stride = (int64_t)ntiles * kLinMT * 64;
-  auto add_up = [&](int64_t tile) {
-    const f32x4_t *src = reinterpret_cast<const f32x4_t *>(p.partial) + (tile * kLinMT + mt) * 64 + lane;
+  auto add_up = [&](int64_t tile, int from) {
+    const f32x4_t *src = reinterpret_cast<const f32x4_t *>(p.partial) + (tile * kLinMT + mt) * 64 + from;
     f32x4_t s = src[0];
     for (int i = 1; i < p.splits; i++) {
       const f32x4_t v = src[i * stride];
@@ -594,10 +735,17 @@ __global__ __launch_bounds__(256) void linear_reduce_kernel(const LinearParams p
     return s;
   };
   const int m = mt * 16 + (lane & 15), n = (int)nt * 16 + 4 * (lane >> 4);
-  if constexpr (GATED)
-    linear_finish_gated<T>(p, add_up(nt), add_up(nt + p.half / 16), m, n);
+  if constexpr (QKV) {
+    const int kg = lane >> 4;
+    const QkvRows rows = qkv_rows(p.qkv, (int)nt);
+    const QkvToken token = qkv_token(p.qkv, min(m, p.M - 1));
+    const int at = (kg < 2 ? rows.first : rows.second) + 4 * (kg & 1);
+    const f32x4_t sum = add_up(at / 16, (lane & 15) + (at & 15) / 4 * 16);
+    linear_finish_qkv<T>(p, sum, m, kg, rows, token, qkv_turn<T>(p.qkv, rows, token, kg));
+  } else if constexpr (GATED)
+    linear_finish_gated<T>(p, add_up(nt, lane), add_up(nt + p.half / 16, lane), m, n);
   else
-    linear_finish<T>(p, add_up(nt), m, n);
+    linear_finish<T>(p, add_up(nt, lane), m, n);
 }
 
 // Adds up the ranges' sums of one row of y, finishes the row (bias, rounding, residual: as linear_finish) and
@@ -674,7 +822,7 @@ struct LinearPlan {
 // The ranges of k depend on the weight alone (see above).  As far as eight ranges allow: 1024 wavefronts' worth of (16 rows, range)
 // pairs, four per compute unit, and no range longer than 2048 once k is cut at all -- 4096 x 4096 and 6144 x 4096 four, 4096 x
 // 14336 eight, weights of 16384 rows and more none.
-LinearPlan plan_linear(int M, int N, int K, bool norm_in) {
+LinearPlan plan_linear(int M, int N, int K, bool few_only) {
   const Tuning &tn = tuning();
   LinearPlan pl;
   const int stages = K / kLinStageK;
@@ -683,8 +831,8 @@ LinearPlan plan_linear(int M, int N, int K, bool norm_in) {
   while (splits > 1 && splits < kLinMaxRanges && K / splits > 2048) splits *= 2;
   while (splits > stages) splits /= 2;
   pl.stream = M <= kLinStreamRows;
-  if (tn.linear_splits > 0 && !norm_in) splits = tn.linear_splits < stages ? tn.linear_splits : stages;
-  if ((tn.linear_splits > 0 || tn.linear_waves > 0 || tn.linear_tiles > 0) && !norm_in) pl.stream = false;
+  if (tn.linear_splits > 0 && !few_only) splits = tn.linear_splits < stages ? tn.linear_splits : stages;
+  if ((tn.linear_splits > 0 || tn.linear_waves > 0 || tn.linear_tiles > 0) && !few_only) pl.stream = false;
   pl.splits = splits;
   pl.stages_per_split = (stages + splits - 1) / splits;
   // Workgroups of 64 rows while the device holds all of them at once, one per compute unit, or where 32 rows of x leave the copies of x
@@ -720,11 +868,11 @@ void launch_tile(const LinearParams &p, const LinearPlan &pl, hipStream_t stream
   hipLaunchKernelGGL((linear_tile_kernel<T, MT, ring_stages<MT, 8>(), 8, GATED, WIDE>), grid, block, 0, stream, p);
 }
 
-template <typename T, int ROWS, bool GATED>
+template <typename T, int ROWS, bool GATED, bool QKV>
 void launch_norm_linear(const LinearParams &p, hipStream_t stream) {
   constexpr int S = kHeldStages;
   static bool attr_set = false;  // benign race: setting twice is harmless
-  auto kernel = norm_linear_kernel<T, S, ROWS, GATED>;
+  auto kernel = norm_linear_kernel<T, S, ROWS, GATED, QKV>;
   if (!attr_set) {
     HA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                4 * S * 2048 + 16 * 1024 + kLinHeldBytes));
@@ -738,19 +886,19 @@ void launch_norm_linear(const LinearParams &p, hipStream_t stream) {
   check_launch("rms_norm_linear");
 }
 
-template <typename T, bool GATED>
+template <typename T, bool GATED, bool QKV = false>
 void launch_linear(const LinearParams &p, const LinearPlan &pl, hipStream_t stream) {
   if (p.norm_in) {
     if (p.M == 1)
-      launch_norm_linear<T, 1, GATED>(p, stream);
+      launch_norm_linear<T, 1, GATED, QKV>(p, stream);
     else if (p.M == 2)
-      launch_norm_linear<T, 2, GATED>(p, stream);
+      launch_norm_linear<T, 2, GATED, QKV>(p, stream);
     else
-      launch_norm_linear<T, kLinHeldRows, GATED>(p, stream);
+      launch_norm_linear<T, kLinHeldRows, GATED, QKV>(p, stream);
     return;
   }
   if (pl.stream) {
-    if (!GATED && p.splits == 1 && p.N >= 65536) {
+    if (!GATED && !QKV && p.splits == 1 && p.N >= 65536) {
       // A vocabulary's rows: 512 per workgroup, so that one round of workgroups covers the device (128256 x 4096, 16 rows: 161
       // us against 182 with 64 rows per workgroup).
       if constexpr (!GATED)
@@ -759,7 +907,7 @@ void launch_linear(const LinearParams &p, const LinearPlan &pl, hipStream_t stre
       const int parts = GATED ? 2 : 1, n = GATED ? p.half : p.N;
       const int per_tile = p.splits < 4 / parts ? p.splits : 4 / parts;
       const int rows = 16 * (4 / parts / per_tile);
-      hipLaunchKernelGGL((linear_stream_kernel<T, 1, 3, 4, GATED>), dim3((n + rows - 1) / rows), dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((linear_stream_kernel<T, 1, 3, 4, GATED, QKV>), dim3((n + rows - 1) / rows), dim3(256), 0, stream, p);
     }
     check_launch("linear (few rows)");
     return;
@@ -782,7 +930,7 @@ void launch_linear(const LinearParams &p, const LinearPlan &pl, hipStream_t stre
     check_launch("linear (sum of the ranges + rms_norm)");
   } else if (p.tile_sums) {
     const int64_t threads = (int64_t)((GATED ? p.half : p.N) / 16) * p.mtiles * 64;
-    hipLaunchKernelGGL((linear_reduce_kernel<T, GATED>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((linear_reduce_kernel<T, GATED, QKV>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, p);
     check_launch("linear (sum of the ranges)");
   }
 }
@@ -806,12 +954,47 @@ bool rows_overlap(const hipattn_tensor *a, const hipattn_tensor *b) {
   return within < a->sizes[1] * 2 || within + b->sizes[1] * 2 > ld;
 }
 
+struct QkvOperands {
+  const hipattn_tensor *positions, *cos_sin, *key_cache, *value_cache, *slot_mapping;
+};
+
+QkvParams qkv_params(const QkvOperands &o, int64_t M, int64_t N, int dt) {
+  const char *op = "qkv_linear";
+  QkvParams q{};
+  q.g = cache_geometry(o.key_cache, o.value_cache, op);
+  check_index_tensor(o.positions, "positions", 1);
+  check_index_tensor(o.slot_mapping, "slot_mapping", 1);
+  check_tensor(o.cos_sin, "cos_sin_cache", 2);
+  const int hd = q.g.head_size;
+  HA_CHECK(o.key_cache->dtype == dt && o.cos_sin->dtype == dt, "%s: cos_sin_cache and the caches must be %s", op, dtype_name(dt));
+  HA_CHECK(o.positions->sizes[0] == M && o.slot_mapping->sizes[0] == M, "%s: %lld positions and %lld slots for %lld rows", op,
+           (long long)o.positions->sizes[0], (long long)o.slot_mapping->sizes[0], (long long)M);
+  HA_CHECK(hd > 0 && hd % 16 == 0 && o.cos_sin->sizes[1] == hd, "%s: heads of %d, rotated over %lld; both must be the same multiple of 16", op, hd,
+           (long long)o.cos_sin->sizes[1]);
+  HA_CHECK(N % hd == 0 && N / hd > 2 * (int64_t)q.g.num_heads && q.g.num_heads > 0,
+           "%s: %lld rows of weight are not query heads and %d key and value heads of %d", op, (long long)N, q.g.num_heads, hd);
+  HA_CHECK(is_contiguous(o.cos_sin) && aligned16(o.cos_sin->data) && aligned16(o.key_cache->data) && q.g.k_block_stride % 8 == 0 &&
+               q.g.k_head_stride % 8 == 0,
+           "%s: rows of cos_sin_cache and of key_cache's heads must start on 16-byte boundaries", op);
+  check_data(o.cos_sin, "cos_sin_cache");
+  q.positions = o.positions->data;
+  q.slots = o.slot_mapping->data;
+  q.cos_sin = o.cos_sin->data;
+  q.pos64 = o.positions->dtype == HIPATTN_I64;
+  q.slot64 = o.slot_mapping->dtype == HIPATTN_I64;
+  q.max_pos = o.cos_sin->sizes[0];
+  q.q_heads = (int)(N / hd) - 2 * q.g.num_heads;
+  q.key_cache = o.key_cache->data;
+  q.value_cache = o.value_cache->data;
+  return q;
+}
+
 // With `norm_out` the RMS norm of the finished rows (weight `norm_weight`, `eps`) is written there by the launch
 // that adds up the ranges' sums; the workspace is then needed whatever the number of ranges.
 void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_tensor *weight, const hipattn_tensor *bias,
                  const hipattn_tensor *residual, const hipattn_tensor *workspace, void *stream_arg, int64_t *ws_query,
                  hipattn_tensor *norm_out = nullptr, const hipattn_tensor *norm_weight = nullptr, float eps = 0.f,
-                 bool ws_query_with_norm = false, bool gated = false, bool norm_in = false) {
+                 bool ws_query_with_norm = false, bool gated = false, bool norm_in = false, const QkvOperands *qkv = nullptr) {
   check_tensor(x, "x", 2);
   check_tensor(weight, "weight", 2);
   const int dt = x->dtype;
@@ -825,7 +1008,7 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
   HA_CHECK(N % 16 == 0, "linear: the number of rows of weight (%lld) must be a multiple of 16", (long long)N);
   HA_CHECK(N < (1 << 24) && K < (1 << 24), "linear: sizes out of range");
   HA_CHECK(!gated || N % 32 == 0, "linear_silu_and_mul: gate and up rows (%lld together) must be multiples of 16 each", (long long)N);
-  LinearPlan pl = plan_linear((int)M, (int)N, (int)K, norm_in);
+  LinearPlan pl = plan_linear((int)M, (int)N, (int)K, norm_in || qkv != nullptr);
   const int64_t outputs = gated ? N / 2 : N;
   const bool with_norm = norm_out != nullptr || ws_query_with_norm;
   // the norm's launch takes rows of sums, however few the ranges
@@ -953,6 +1136,14 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
       p.partial = static_cast<float *>(library_workspace(WS_LINEAR, pl.partial_bytes, stream));
     }
   }
+  if (qkv != nullptr) {
+    HA_CHECK(N < 65536 && (pl.stream || p.tile_sums),
+             "qkv_linear: %lld rows of x and a weight of %lld rows; fewer than 65536 of weight, and than 16384 with more than %d rows of x", (long long)M,
+             (long long)N, kLinStreamRows);
+    p.qkv = qkv_params(*qkv, M, N, dt);
+    dt == HIPATTN_BF16 ? launch_linear<bf16_t, false, true>(p, pl, stream) : launch_linear<half_t, false, true>(p, pl, stream);
+    return;
+  }
   if (dt == HIPATTN_BF16)
     gated ? launch_linear<bf16_t, true>(p, pl, stream) : launch_linear<bf16_t, false>(p, pl, stream);
   else
@@ -987,6 +1178,17 @@ extern "C" char *hipattn_rms_norm_linear(hipattn_tensor *out, const hipattn_tens
                                          float epsilon, const hipattn_tensor *weight, bool silu_and_mul, void *stream) {
   HA_PROTECT(linear_impl(out, x, weight, nullptr, nullptr, nullptr, stream, nullptr, nullptr, norm_weight, epsilon, false, silu_and_mul,
                          true));
+}
+
+extern "C" char *hipattn_qkv_linear(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_tensor *norm_weight, float epsilon,
+                                    const hipattn_tensor *weight, const hipattn_tensor *positions,
+                                    const hipattn_tensor *cos_sin_cache, hipattn_tensor *key_cache, hipattn_tensor *value_cache,
+                                    const hipattn_tensor *slot_mapping, void *stream) {
+  HA_PROTECT({
+    const QkvOperands qkv{positions, cos_sin_cache, key_cache, value_cache, slot_mapping};
+    linear_impl(out, x, weight, nullptr, nullptr, nullptr, stream, nullptr, nullptr, norm_weight, epsilon, false, false,
+                norm_weight != nullptr, &qkv);
+  });
 }
 
 extern "C" char *hipattn_linear_workspace_size(const hipattn_tensor *x, const hipattn_tensor *weight, int64_t *bytes) {

@@ -315,6 +315,29 @@ def rms_norm_linear(x: torch.Tensor, norm_weight: torch.Tensor, epsilon: float, 
     return out
 
 
+def qkv_linear_takes(x: torch.Tensor, weight: torch.Tensor, cos_sin_cache: torch.Tensor, key_cache: torch.Tensor,
+                     value_cache: torch.Tensor) -> bool:
+    """Whether `qkv_linear` accepts these operands without a norm (else a caller makes the two calls)."""
+    d = cos_sin_cache.size(1)
+    return (linear_takes(x, weight) and weight.size(0) < (65536 if x.size(0) <= 16 else 16384) and d % 16 == 0
+            and key_cache.dim() == 5 and key_cache.size(2) * key_cache.size(4) == d and weight.size(0) % d == 0
+            and weight.size(0) // d > 2 * key_cache.size(1) > 0 and weight.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0
+            and 0 < weight.stride(0) < 1 << 28 and (x.size(0) == 1 or 0 <= x.stride(0) < 1 << 28)
+            and cos_sin_cache.dtype == key_cache.dtype == value_cache.dtype == x.dtype and cos_sin_cache.is_contiguous()
+            and cos_sin_cache.data_ptr() % 16 == 0 and key_cache.data_ptr() % 16 == 0 and key_cache.stride(0) % 8 == 0
+            and key_cache.stride(1) % 8 == 0)
+
+
+def qkv_linear(x: torch.Tensor, norm_weight: Optional[torch.Tensor], epsilon: float, weight: torch.Tensor, positions: torch.Tensor,
+               cos_sin_cache: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor,
+               slot_mapping: torch.Tensor) -> torch.Tensor:
+    """x @ weight.T, behind rms_norm of the rows where norm_weight is given, and rotary_embedding_and_cache of its heads (llama.rs:81-85 +
+    mod.rs:147-164) in the projection's own launches: returns [M, (Hq + 2 Hkv) d] with the bits of the calls."""
+    out = torch.empty((x.size(0), weight.size(0)), dtype=x.dtype, device=x.device)
+    _native.qkv_linear(out, x, norm_weight, epsilon, weight, positions, cos_sin_cache, key_cache, value_cache, slot_mapping)
+    return out
+
+
 def linear_rms_norm_workspace_size(x: torch.Tensor, weight: torch.Tensor) -> int:
     n = ctypes.c_int64(0)
     call("hipattn_linear_rms_norm_workspace_size", _desc(x, "x"), _desc(weight, "weight"), ctypes.byref(n))

@@ -172,14 +172,21 @@ class Llama:
         first = self.layers[0]
         h = None if self._norm_in_proj(x, first["rms_1"], first["qkv"]) else self._rms(x, first["rms_1"])  # :165
         for li, (layer, (kc, vc)) in enumerate(zip(self.layers, caches)):
-            if h is None:
+            # few rows: rotary and the cache writes happen in the projection's launch too (:85 + mod.rs:147-164)
+            rotated = (fused and self.skinny_linear
+                       and kernels.qkv_linear_takes(x if h is None else h, layer["qkv"], self.rotary.cos_sin, kc, vc))
+            if rotated:
+                qkv = kernels.qkv_linear(*((x, layer["rms_1"]) if h is None else (h, None)), cfg.rms_norm_eps, layer["qkv"],
+                                         batch_info.positions, self.rotary.cos_sin, kc, vc, batch_info.slot_mapping)
+            elif h is None:
                 qkv = kernels.rms_norm_linear(x, layer["rms_1"], cfg.rms_norm_eps, layer["qkv"])
             else:
                 qkv = self._proj(h, layer["qkv"])                               # :81-83
             if fused:
                 q, k, v = qkv.split([Hq * d, Hkv * d, Hkv * d], dim=1)
                 v = v.view(T, Hkv, d)
-                self.rotary.forward_and_cache(batch_info.positions, q, k, v, kc, vc, batch_info.slot_mapping)  # :85 + mod.rs:147-164
+                if not rotated:
+                    self.rotary.forward_and_cache(batch_info.positions, q, k, v, kc, vc, batch_info.slot_mapping)
                 y = varlen_attn(q.view(T, Hq, d), k.view(T, Hkv, d), v, batch_info, kc, vc,
                                 paged_prefill=paged_prefill, cached=True)      # :93
             else:

@@ -386,6 +386,19 @@ char *hipattn_rms_norm_linear(hipattn_tensor *out, const hipattn_tensor *x,
                               const hipattn_tensor *weight, bool silu_and_mul,
                               void *stream);
 
+/* The projection of q, k and v with hipattn_rotary_embedding_and_cache (NeoX) behind it (llama.rs:81-85 + mod.rs:147-164), for the
+ * rows of a small step: out [M, (Hq + 2 Hkv) d] = x . weight^T, query and key heads rotated, the keys and values written to the cache;
+ * the bits of the calls.  With norm_weight not NULL hipattn_rms_norm of the rows of x comes first, as in hipattn_rms_norm_linear and
+ * within its limits.  d and Hkv are the cache's; d a multiple of 16, cos_sin_cache [positions, d]; fewer than 65536 rows of weight, and
+ * than 16384 with more than 16 rows of x; operands else, and scratch, as for hipattn_linear and hipattn_rotary_embedding_and_cache. */
+char *hipattn_qkv_linear(hipattn_tensor *out, const hipattn_tensor *x,
+                         const hipattn_tensor *norm_weight, float epsilon,
+                         const hipattn_tensor *weight,
+                         const hipattn_tensor *positions,
+                         const hipattn_tensor *cos_sin_cache,
+                         hipattn_tensor *key_cache, hipattn_tensor *value_cache,
+                         const hipattn_tensor *slot_mapping, void *stream);
+
 /* Replace silu_and_mul_C / gelu_new_C / gelu_fast_C (lib.rs:162-166;
  * activation_kernels.cu:15-115). */
 char *hipattn_silu_and_mul(hipattn_tensor *out, const hipattn_tensor *input,

@@ -366,3 +366,52 @@ def test_rms_norm_linear_refusals(device):
     square = torch.zeros((4096, 4096), dtype=torch.bfloat16, device=device)
     with pytest.raises(HipAttnError, match="over x"):
         _native.rms_norm_linear(x[:2], x[:2], norm, 1e-5, square, False)
+
+
+@pytest.mark.parametrize("dtype,index", [(torch.bfloat16, torch.int64), (torch.float16, torch.int32)])
+@pytest.mark.parametrize("heads,Kd", [((32, 8, 128), 4096), ((3, 1, 80), 512), ((5, 5, 64), 1024), ((2, 1, 256), 256), ((1, 3, 48), 2560)])
+@pytest.mark.parametrize("M", [1, 2, 4, 5, 16, 17, 33, 128])
+def test_qkv_linear_gives_the_bits_of_the_calls(device, dtype, index, heads, Kd, M):
+    """With and without the norm in front, for tokens in and out of the rotary table and of the cache, blocks of 8, 16 and 32 tokens."""
+    Hq, Hkv, d = heads
+    g = torch.Generator().manual_seed(M + Kd)
+    x = torch.randn((M, Kd), generator=g).to(dtype).to(device)
+    norm = (1 + 0.2 * torch.randn((Kd,), generator=g)).to(dtype).to(device)
+    weight = (torch.randn(((Hq + 2 * Hkv) * d, Kd), generator=g) / Kd ** 0.5).to(dtype).to(device)
+    table = torch.randn((300, d), generator=g).to(dtype).to(device)
+    h = torch.empty_like(x)
+    K.rms_norm(h, x, norm, 1e-5)
+    for bs in (8, 16, 32):
+        blocks = 5 + M // bs
+        kc = torch.randn((blocks, Hkv, d // 8, bs, 8), generator=g).to(dtype).to(device)
+        vc = torch.randn((blocks, Hkv, d, bs), generator=g).to(dtype).to(device)
+        pos = torch.randint(0, 300, (M,), generator=g)
+        slots = torch.randperm(blocks * bs, generator=g)[:M]
+        if M > 4:
+            pos[2], pos[3] = 300, -1
+            slots[0], slots[1] = -1, blocks * bs
+        pos, slots = pos.to(index).to(device), slots.to(index).to(device)
+        assert K.qkv_linear_takes(x, weight, table, kc, vc)
+        want, wkc, wvc = K.linear(h, weight), kc.clone(), vc.clone()
+        q, k, v = want.split([Hq * d, Hkv * d, Hkv * d], dim=1)
+        K.rotary_embedding_and_cache(pos, q, k, v.view(M, Hkv, d), d, table, True, wkc, wvc, slots)
+        for rows, nw in ((h, None), (x, norm)):
+            if nw is not None and not K.rms_norm_linear_takes(x, norm, weight):
+                continue
+            got_k, got_v = kc.clone(), vc.clone()
+            got = K.qkv_linear(rows, nw, 1e-5, weight, pos, table, got_k, got_v, slots)
+            assert torch.equal(got, want) and torch.equal(got_k, wkc) and torch.equal(got_v, wvc)
+
+
+def test_qkv_linear_refusals(device):
+    z = lambda *s: torch.zeros(s, dtype=torch.bfloat16, device=device)
+    x, w, table, kc, vc = z(4, 256), z(6 * 64, 256), z(32, 64), z(2, 1, 8, 16, 8), z(2, 1, 64, 16)
+    at = torch.zeros((4,), dtype=torch.int64, device=device)
+    for bad, msg in (((z(17, 256), z(256 * 64, 256), table, kc, vc), "more than 16 rows"), ((x, z(2 * 64, 256), table, kc, vc), "query heads"),
+                     ((x, w, z(32, 32), kc, vc), "heads of 64"), ((x, w, table.half(), kc, vc), "must be")):
+        assert not K.qkv_linear_takes(*bad)
+        idx = torch.zeros((bad[0].size(0),), dtype=torch.int64, device=device)
+        with pytest.raises(HipAttnError, match=msg):
+            K.qkv_linear(bad[0], None, 0.0, bad[1], idx, bad[2], bad[3], bad[4], idx)
+    with pytest.raises(HipAttnError, match="3 positions"):
+        K.qkv_linear(x, None, 0.0, w, at[:3], table, kc, vc, at)
