@@ -163,7 +163,8 @@ class Llama:
         """batch_info on the device; caches[layer] = (key_cache, value_cache), updated in place.
         paged_prefill: multi-token rows read their context through block tables (no gather copy).
         fused: q, k, v stay views of the fused projection's output (the kernels honour the row stride) and
-        rotary + cache scatter are one launch -- four launches fewer per layer, the same bits."""
+        rotary + cache scatter are one launch, or part of the projection's -- four or five launches fewer per layer, the same
+        bits."""
         cfg = self.cfg
         Hq, Hkv, d = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
         x = self.wte.index_select(0, batch_info.tokens.long())                   # llama.rs:203
@@ -220,7 +221,7 @@ def aici_sample(logits: torch.Tensor, allow_masks: torch.Tensor, temperature: to
     allow-masks: rows with temperature < 1e-5 are greedy, the others are drawn with one uniform number per
     row in [0, 1) -- the caller's, or drawn here from `generator` (a seeded torch.Generator on the CPU stands
     in for the reference's per-sequence `StdRng`: the same seed gives the same tokens).  All rows in one
-    launch, no host round trip.  Returns int32 [S]."""
+    call, no host round trip.  Returns int32 [S]."""
     if uniforms is None:
         uniforms = torch.rand((logits.size(0),), generator=generator, dtype=torch.float32).to(logits.device)
     return kernels.bias_sample(logits, temperature, top_p, uniforms, mask=allow_masks)
