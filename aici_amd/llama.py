@@ -174,7 +174,7 @@ class Llama:
         h = None if self._norm_in_proj(x, first["rms_1"], first["qkv"]) else self._rms(x, first["rms_1"])  # :165
         for li, (layer, (kc, vc)) in enumerate(zip(self.layers, caches)):
             # few rows: rotary and the cache writes happen in the projection's launch too (:85 + mod.rs:147-164)
-            rotated = (fused and self.skinny_linear
+            rotated = (fused and self.skinny_linear and kc.dim() == 5 and kc.size(1) == Hkv
                        and kernels.qkv_linear_takes(x if h is None else h, layer["qkv"], self.rotary.cos_sin, kc, vc))
             if rotated:
                 qkv = kernels.qkv_linear(*((x, layer["rms_1"]) if h is None else (h, None)), cfg.rms_norm_eps, layer["qkv"],
