@@ -450,17 +450,18 @@ __global__ __launch_bounds__(256) void prefill_varlen_kernel(PrefillParams p) {
 //     (read with ds_read_b64_tr_b16) or, from the cache, as the [d][16 tokens] images that ds_read_b128 takes;
 //   staged (paged cache, head sizes below 32 or on request): tiles through registers into three padded stages
 //     (TileW8 below: K rows and V^T rows), one software-pipelined loop per wavefront.
-// NW = 4: workgroups of four wavefronts and three stages, three to a compute unit, so that every SIMD has a wavefront of each.
-// The alternation of the two pipes is left to chance; what it gains is that a workgroup's set-up and wind-down (block ids, Q, the
-// first tile; the output) pass while the other two work.  Head sizes up to 64 always, larger ones, with tiles of 32 keys to fit the
-// registers and the LDS of a third of a compute unit, where contexts are short (four_wavefronts_pay).
+// NW = 4: workgroups of four wavefronts, three to a compute unit (two at head sizes above 96, by their registers), so that every SIMD has
+// a wavefront of each.  The alternation of the two pipes is left to chance; what it gains is that a workgroup's set-up and wind-down (block
+// ids, Q, the first tile; the output) pass while the others work.  Same tiles, same order of the same operations: a row has the same bits
+// in either form, so the form may follow the sizes of the whole batch (four_wavefronts_pay).  Tiles of 32 keys, which let three
+// workgroups on a compute unit at head size 128 too (64 x 30..300 tokens 71 -> 59 us, 32 / 8 heads), give other last bits: not kept.
 // ---------------------------------------------------------------------------
 // Where the eight-wavefront kernel takes its K/V tiles from.
 enum { W8_ROWS = 0, W8_PAGED = 1, W8_PAGED_DMA = 2, W8_PAGED_DMA_PART = 3 };
 
-// Keys per tile and wavefronts per SIMD of the forms with eight and four wavefronts.
-constexpr int w8_tile_keys(int hdp, int nw) { return nw == 4 && hdp > 64 ? 32 : 64; }
-constexpr int w8_wavefronts(int hdp, int nw) { return nw == 4 ? 3 : 2; }
+// Wavefronts per SIMD and places for tiles in LDS of the forms with eight and four wavefronts.
+constexpr int w8_wavefronts(int hdp, int nw) { return nw == 4 && hdp <= 96 ? 3 : 2; }
+constexpr int w8_stages(int hdp, int nw) { return nw == 8 ? 5 : hdp <= 64 ? 3 : 2; }
 
 // LDS geometry of the staged form.
 template <int HDP>
@@ -477,7 +478,6 @@ template <typename T, int HDP, int MODE, int NW = 8>
 __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varlen_w8_kernel(PrefillParams p) {
   typedef typename Vec8<T>::type vec8;
   typedef TileW8<HDP> TL;
-  constexpr int BN = w8_tile_keys(HDP, NW), NKT = BN / 32;  // keys per tile, halves of 32
   constexpr bool PAGED = MODE != W8_ROWS;
   constexpr bool ROWS = MODE == W8_ROWS;
   constexpr bool DMA = MODE == W8_PAGED_DMA || MODE == W8_PAGED_DMA_PART;
@@ -492,10 +492,11 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
   // first d / HDP of its place in LDS; the rest is cleared once, so the contraction steps and output rows past d
   // work on zeros.
   constexpr bool DMA_PART = MODE == W8_PAGED_DMA_PART;
-  // W8_PAGED_DMA keeps a tile as the four block images of the cache, unpadded, in four stages.
-  // Block images and rows: five stages (all of the 160 KB at head size 128) and one barrier per tile; staged:
-  // three.  No tile is padded; where reads would collide, runs change places within their row (see v_rows_dma).
-  constexpr int NST = NW == 4 ? 3 : PINGPONG ? 5 : 3;
+  // W8_PAGED_DMA keeps a tile as the four block images of the cache, unpadded.
+  // Block images and rows: five stages (all of the 160 KB at head size 128) and one barrier per tile, with four wavefronts three or two
+  // (48 KB, 64 at head sizes above 96); staged: three.  No tile is padded; where reads would collide, runs change places within their
+  // row (see v_rows_dma).
+  constexpr int NST = PINGPONG ? w8_stages(HDP, NW) : 3;
   constexpr int K_ELEMS = KIMG ? BN * HDP : TL::K_ELEMS;
   constexpr int STAGE_ELEMS = PINGPONG ? 2 * BN * HDP : K_ELEMS + TL::V_ELEMS;
   constexpr int KSTEPS = HDP / 16;
@@ -559,7 +560,8 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
   // Q operands: lane (g, c) holds q[row c][16 ks + 8 g .. + 8] for every contraction step ks.  Read in
   // that shape an instruction touches 32 bytes of 32 rows; instead the rows are read whole (16 lanes x
   // 16 bytes per row, 4 rows per instruction) and turned through a private piece of LDS buffers 1 and 2,
-  // which no tile reaches before the first barrier.
+  // which no tile reaches before the first barrier.  (With four wavefronts no such piece is left beside tiles 0 and 1: they do read
+  // it in that shape, while other workgroups work.)
   constexpr int QSTR = HDP + 8;  // row pitch of the turned Q tile, elements
   // The alternating-block forms turn Q through stages 2.., so that tiles 0 and 1 can be on their way meanwhile.
   constexpr int Q_STAGE0 = PINGPONG ? 2 : 1;
@@ -693,8 +695,7 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
   constexpr int BLK_ELEMS = HDP * 16;
   constexpr int NDMA = HDP / 32;  // instructions per wavefront and tile
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)smem_raw;
-  constexpr int BPT = BN / 16, TPG = 64 / BPT;  // blocks per tile, tiles per 64 table columns
-  constexpr int IMG = 2 * BPT / NW;  // images per wavefront: one, or K and V of block w
+  constexpr int IMG = 8 / NW;  // images per wavefront: one, or K and V of block w
   auto dma_v = [&](int im) { return IMG == 1 ? wave_u & 1 : im; };
   const int dma_r = IMG == 1 ? wave_u >> 1 : wave_u;
   unsigned dma_lane[IMG];
@@ -713,13 +714,12 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
     dma_last_ok[im] = !DMA_PART || (dma_v(im) ? c < dma_tail : lane < 2 * dma_tail);
     tbl_off[im] = 0;
   }
-  auto ids_to_offsets = [&](int blk) {
+  auto id_to_offset = [&](int blk, int im) -> int64_t {
     const int64_t bid = blk < 0 ? 0 : (blk >= p.num_blocks ? p.num_blocks - 1 : (int64_t)blk);
-#pragma unroll
-    for (int im = 0; im < IMG; im++) tbl_off[im] = bid * dma_blk_bytes[im];
+    return bid * dma_blk_bytes[im];
   };
   auto dma_piece = [&](int tile, int i, int im) {
-    const int idx = (tile % TPG) * BPT + dma_r;
+    const int idx = (tile & 15) * 4 + dma_r;
     const unsigned lo = __builtin_amdgcn_readlane((int)(uint32_t)tbl_off[im], idx);
     const unsigned hi = __builtin_amdgcn_readlane((int)(uint32_t)(tbl_off[im] >> 32), idx);
     // (an "s" operand is not made a scalar for the asm when the compiler holds the value in vector registers)
@@ -744,23 +744,32 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
       }
     }
 #undef HA_DMA_PIECE
-    if (i == NDMA - 1 && im == IMG - 1) {
-      if (tile % TPG == TPG - 2) tbl_nxt = load_ids(tile / TPG + 1);
-      if (tile % TPG == TPG - 1) ids_to_offsets(tbl_nxt);
+    if (NST == 2 && i == NDMA - 1) {
+      // (K's image is one tile ahead of V's: the ids that are asked for with the one are still there when the other turns to them)
+      if (im == 0 && (tile & 15) == 14) tbl_nxt = load_ids((tile >> 4) + 1);
+      if ((tile & 15) == 15) tbl_off[im] = id_to_offset(tbl_nxt, im);
+    } else if (NST > 2 && i == NDMA - 1 && im == IMG - 1) {
+      if ((tile & 15) == 14) tbl_nxt = load_ids((tile >> 4) + 1);
+      if ((tile & 15) == 15) {
+#pragma unroll
+        for (int m = 0; m < IMG; m++) tbl_off[m] = id_to_offset(tbl_nxt, m);
+      }
     }
+  };
+  auto dma_image = [&](int tile, int im) {
+#pragma unroll
+    for (int i = 0; i < NDMA; i++) dma_piece(tile, i, im);
   };
   auto dma_tile = [&](int tile) {
 #pragma unroll
-    for (int im = 0; im < IMG; im++)
-#pragma unroll
-      for (int i = 0; i < NDMA; i++) dma_piece(tile, i, im);
+    for (int im = 0; im < IMG; im++) dma_image(tile, im);
   };
   // W8_PAGED_DMA_PART: clears what the images leave untouched in stages first..last: per block the K runs of
   // head elements d..HDP and, in the last V piece, the rows d..HDP of both 8-token halves.
   auto clear_image_tails = [&](int first, int last) {
     if constexpr (DMA_PART) {
       const int R = HDP - p.d;       // a multiple of 8 below 32
-      const int per_stage = 4 * BPT * R;  // 16-byte runs: per block 2 R of K + 2 R of V
+      const int per_stage = 16 * R;  // 16-byte runs: 4 blocks x (2 R of K + 2 R of V)
       for (int st = first; st <= last; st++)
         for (int idx = tid; idx < per_stage; idx += NW * 64) {
           const int r = idx / (4 * R), rem = idx % (4 * R);
@@ -807,7 +816,7 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
   // l % 16.  On a full tile the lane's offset is the same for every piece (the piece's own part is added to
   // the scalar base); only the last piece of a block clamps runs past d, and the last tile keys past Lk.
   constexpr int KPB = HDP / 32;   // pieces per block
-  constexpr int KNP = BPT * KPB;  // pieces per tile
+  constexpr int KNP = 4 * KPB;    // pieces per tile
   const int kd_tok = lane & 15, kd_run = lane >> 4;
   const uint32_t kd_off = (uint32_t)(((int64_t)kd_tok * p.k_row + kd_run * 8) * (int64_t)sizeof(T));
   const uint32_t kd_off_last =
@@ -843,8 +852,15 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
         uint32_t off = k_off0[i] + tile_off;
         if (k0 + BN > Lk) {
           const int r = q / KPB, pi = q % KPB;
-          const int key = min(k0 + 16 * r + kd_tok, Lk - 1);
-          off = (uint32_t)(((int64_t)key * p.k_row + min(4 * pi + kd_run, d_chunks - 1) * 8) * (int64_t)sizeof(T));
+          int tok = kd_tok, run = kd_run;
+          if constexpr (NW == 4 && HDP == 96) {  // (168 registers: the lane number through an opaque copy, as for the values below)
+            int l2 = lane;
+            asm volatile("" : "+v"(l2));
+            tok = l2 & 15;
+            run = l2 >> 4;
+          }
+          const int key = min(k0 + 16 * r + tok, Lk - 1);
+          off = (uint32_t)(((int64_t)key * p.k_row + min(4 * pi + run, d_chunks - 1) * 8) * (int64_t)sizeof(T));
         }
         const unsigned dst = dst0 + (unsigned)i * (NW * 1024u);
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
@@ -945,12 +961,18 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
   if constexpr (PINGPONG) q_issue();
   if (PAGED && n_tiles > 0) tbl_cur = load_ids(0);
   if constexpr (DMA) {
-    ids_to_offsets(tbl_cur);
+#pragma unroll
+    for (int im = 0; im < IMG; im++) tbl_off[im] = id_to_offset(tbl_cur, im);
     if (n_tiles > 0) dma_tile(0);
-    if (n_tiles > 1) dma_tile(1);
+    if (n_tiles > 1) {
+      if constexpr (NST == 2)
+        dma_image(1, 0);
+      else
+        dma_tile(1);
+    }
     clear_image_tails(0, 1);
     q_finish();
-    if (n_tiles > 0) dma_wait(0, n_tiles > 1);
+    if (n_tiles > 0) dma_wait(0, NST > 2 && n_tiles > 1);
     __syncthreads();
     if (NST > 3 && n_tiles > 2) dma_tile(2);
     clear_image_tails(2, NST - 1);  // seen by all after the barrier in front of the loop
@@ -961,7 +983,7 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
     }
     if (n_tiles > 1) {
       k_rows_dma(1);
-      v_rows_dma(1);
+      if (NST > 2) v_rows_dma(1);
     }
     q_finish();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1005,27 +1027,41 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
 
   // S^T = K . Q^T of one tile on its own (used for tile 0): both 32-key halves,
   // LDS reads two contraction steps ahead of the MFMAs that consume them.
-  auto phase_qk = [&](int buf, f32x16_t(&s)[NKT]) {
+  auto phase_qk = [&](int buf, f32x16_t(&s)[2]) {
     const T *ks_base = smem + buf * STAGE_ELEMS;
     auto rd = [&](int kt, int ks) -> vec8 {
       return *reinterpret_cast<const vec8 *>(ks_base + k_lane_off + kt * K_HALF + ks * K_STEP);
     };
-    vec8 ka[3][NKT];
+    if constexpr (NW == 4 && HDP == 96) {
+      // (168 registers: three operands ahead, one at a time, are what fits)
+      vec8 kb[4];
 #pragma unroll
-    for (int kt = 0; kt < NKT; kt++) ka[0][kt] = rd(kt, 0);
+      for (int n = 0; n < 3; n++) kb[n] = rd(n & 1, n >> 1);
+#pragma unroll
+      for (int n = 0; n < 2 * KSTEPS; n++) {
+        if (n + 3 < 2 * KSTEPS) kb[(n + 3) % 4] = rd((n + 3) & 1, (n + 3) >> 1);
+        __builtin_amdgcn_sched_barrier(0);
+        s[n & 1] = Mfma32<T>::run(kb[n % 4], qreg[n >> 1], n < 2 ? zero : s[n & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      return;
+    }
+    vec8 ka[3][2];
+    ka[0][0] = rd(0, 0);
+    ka[0][1] = rd(1, 0);
     if (KSTEPS > 1) {
-#pragma unroll
-      for (int kt = 0; kt < NKT; kt++) ka[1][kt] = rd(kt, 1);
+      ka[1][0] = rd(0, 1);
+      ka[1][1] = rd(1, 1);
     }
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ks++) {
       if (ks + 2 < KSTEPS) {
-#pragma unroll
-        for (int kt = 0; kt < NKT; kt++) ka[(ks + 2) % 3][kt] = rd(kt, ks + 2);
+        ka[(ks + 2) % 3][0] = rd(0, ks + 2);
+        ka[(ks + 2) % 3][1] = rd(1, ks + 2);
       }
       __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int kt = 0; kt < NKT; kt++) s[kt] = Mfma32<T>::run(ka[ks % 3][kt], qreg[ks], ks == 0 ? zero : s[kt]);
+      s[0] = Mfma32<T>::run(ka[ks % 3][0], qreg[ks], ks == 0 ? zero : s[0]);
+      s[1] = Mfma32<T>::run(ka[ks % 3][1], qreg[ks], ks == 0 ? zero : s[1]);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -1039,15 +1075,14 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
   // runs with the staging of tile j+2 (registers -> LDS) and the loads of tile
   // j+3 in its shadow.  Three LDS buffers: iteration j reads K of (j+1)%3 and V
   // of j%3 and writes (j+2)%3; one barrier per iteration.
-  constexpr int NQ = 2 * KSTEPS;   // MFMAs of one S tile of 64 keys: step n = (contraction step n/2, key half n%2)
+  constexpr int NQ = 2 * KSTEPS;   // MFMAs of one S tile: step n = (contraction step n/2, key half n%2)
   constexpr int MAXS = NQ / 4;     // of which the first MAXS shadow the row maximum,
   constexpr int EXPS = NQ - MAXS;  // the rest the exponentials
   constexpr int QK_DEPTH = 3;      // K operands read ahead of their MFMA
 
   // DO_QK: S(j+1) is wanted (written to sn); the softmax of S(j) (in s) always runs.
-  auto qk_softmax = [&](auto do_qk, int j, f32x16_t(&s)[NKT], f32x16_t(&sn)[NKT], vec8(&pk)[NKT][2]) {
+  auto qk_softmax = [&](auto do_qk, int j, f32x16_t(&s)[2], f32x16_t(&sn)[2], vec8(&pk)[2][2]) {
     constexpr bool DO_QK = decltype(do_qk)::value;
-    static_assert(!DO_QK || NKT == 2, "tiles of 64 keys");
     const int k0 = j * BN;
     const T *ks_base = smem + ((j + 1) % NST) * STAGE_ELEMS;
     auto rd = [&](int n) -> vec8 {
@@ -1059,7 +1094,7 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
       for (int n = 0; n < QK_DEPTH && n < NQ; n++) ka[n] = rd(n);
     }
     auto qk_step = [&](int n) {
-      if constexpr (DO_QK) {
+      if (DO_QK) {
         if (n + QK_DEPTH < NQ) ka[(n + QK_DEPTH) % (QK_DEPTH + 1)] = rd(n + QK_DEPTH);
         __builtin_amdgcn_sched_barrier(0);
         sn[n & 1] = Mfma32<T>::run(ka[n % (QK_DEPTH + 1)], qreg[n >> 1], (n >> 1) == 0 ? zero : sn[n & 1]);
@@ -1073,7 +1108,7 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
       int limit = p.causal ? row + off : Lk - 1;
       limit = min(limit, Lk - 1);
 #pragma unroll
-      for (int kt = 0; kt < NKT; kt++)
+      for (int kt = 0; kt < 2; kt++)
 #pragma unroll
         for (int i = 0; i < 16; i++) {
           const int key = KIMG ? k0 + kt * 32 + ((i >> 3) & 1) * 16 + g * 8 + ((i >> 2) & 1) * 4 + (i & 3)
@@ -1082,18 +1117,16 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
         }
     }
     // row maximum in the shadow of the first MAXS MFMAs
-    float mx = fmaxf(s[0][0], s[NKT - 1][NKT == 2 ? 0 : 1]);
+    float mx = fmaxf(s[0][0], s[1][0]);
 #pragma unroll
     for (int n = 0; n < MAXS; n++) {
       qk_step(n);
 #pragma unroll
       for (int i = 16 * n / MAXS; i < 16 * (n + 1) / MAXS; i++)
-        if (NKT == 2 ? i > 0 : (i > 0 && i % 2 == 0)) mx = max3(mx, s[0][i], s[NKT - 1][NKT == 2 ? i : i + 1]);
+        if (i > 0) mx = max3(mx, s[0][i], s[1][i]);
     }
     mx = max_across_halves(mx) * p.scale_log2;
-    // (tiles of 32 keys: behind the second one the reference is the largest of 64 keys, as with tiles of 64 behind the first, so that this
-    // one's probability is exactly 1 in either; without, the output is 2 to 5 % further from float64)
-    const bool grow = mx > m_run + (NKT == 1 && j == 1 ? 0.f : p.rescale_thr);
+    const bool grow = mx > m_run + p.rescale_thr;
     if (__builtin_expect(__any(grow), 0)) {
       const float m_new = grow ? mx : m_run;
       const float alpha = grow ? fast_exp2(m_run - m_new) : 1.0f;
@@ -1110,7 +1143,7 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
     for (int n = 0; n < EXPS; n++) {
       qk_step(MAXS + n);
 #pragma unroll
-      for (int v = 16 * NKT * n / EXPS; v < 16 * NKT * (n + 1) / EXPS; v++) {
+      for (int v = 32 * n / EXPS; v < 32 * (n + 1) / EXPS; v++) {
         const float e = fast_exp2(s[v / 16][v % 16] * p.scale_log2 - msub);
         psum += e;
         pk[v / 16][(v % 16) / 8][v % 8] = from_float<T>(e);
@@ -1119,8 +1152,8 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
     l_run += psum;
   };
 
-  constexpr int PV_STEPS = NDT * 2 * NKT;
-  f32x16_t s_a[NKT], s_b[NKT];
+  constexpr int PV_STEPS = NDT * 4;
+  f32x16_t s_a[2], s_b[2];
   if constexpr (PINGPONG) {
     // ---- block images and rows: the two wavefronts of a SIMD alternate between the matrix pipe and the vector ALU ----
     // A wavefront that issues MFMAs and vector instructions in turn has its vector instructions held up
@@ -1137,7 +1170,7 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
     // M(t), and swap in the middle.
     // Measured on 8 x 4096 tokens from the paged cache: 1.118 -> 1.058 ms with four stages and a barrier per
     // half period, 1.091 -> 1.075 ms from there to five stages and one barrier.
-    vec8 pk[NKT][2];
+    vec8 pk[2][2];
     auto pv_images = [&](int j) {
       const T *vs_base = smem + (j % NST) * STAGE_ELEMS + K_ELEMS;
       // Step n = (contraction step n / NDT, output tile n % NDT): consecutive MFMAs go to different
@@ -1190,13 +1223,17 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
         }
       }
     };
-    auto send_tile = [&](int t) {
-      if constexpr (DMA) {
-        dma_tile(t);
-      } else {
+    auto send_keys = [&](int t) {
+      if constexpr (DMA)
+        dma_image(t, 0);
+      else
         k_rows_dma(t);
+    };
+    auto send_values = [&](int t) {
+      if constexpr (DMA)
+        dma_image(t, IMG - 1);
+      else
         v_rows_dma(t);
-      }
     };
     auto m_block = [&](int t) {
       if (t >= 1 && !skip_tile(t - 1)) pv_images(t - 1);
@@ -1218,53 +1255,59 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
       }
     };
     if constexpr (NW == 4) {
-      // Four wavefronts, one per SIMD, with two more workgroups on the compute unit to fill the pipes: three stages.  A period sends tile
-      // t + 2 into the place of tile t - 1 first of all and ends when it is there.
+      // Four wavefronts, one per SIMD, with other workgroups on the compute unit to fill the pipes.  A period sends a tile first of all
+      // and ends when it is there.  Three places: tile j + 2 goes to that of tile j - 1.  Two: in period j the keys of tile j and the
+      // values of tile j - 1 have been read for the last time, so the keys of tile j + 2 and the values of tile j + 1 take their places.
+      constexpr int V_AHEAD = NST - 1;
       m_block(0);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      if (DMA && n_tiles > 1) dma_wait(1, false);
+      if (DMA && NST > 2 && n_tiles > 1) dma_wait(1, false);
       lds_barrier();
       asm volatile(".p2align 6");
       for (int j = 0; j < n_tiles; j++) {
-        if (j + 2 < n_tiles) send_tile(j + 2);
+        if (j + 2 < n_tiles) {
+          send_keys(j + 2);
+          if (V_AHEAD == 2) send_values(j + 2);
+        }
+        if (V_AHEAD == 1 && j + 1 < n_tiles) send_values(j + 1);
         if (!skip_tile(j)) qk_softmax(std::false_type{}, j, s_a, s_b, pk);
         m_block(j + 1);
-        if (DMA && j + 2 < n_tiles) dma_wait(j + 2, false);
+        if (DMA && j + V_AHEAD < n_tiles) dma_wait(j + V_AHEAD, false);
         if (ROWS) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         lds_barrier();
       }
     } else {
-    // The prologue has sent tiles 0, 1 and 2; tiles 0 and 1 have to be complete before the first period.
-    const bool second_group = wave_u >= 4;  // (none with four wavefronts: its SIMD mates are another workgroup's)
-    if constexpr (DMA) {
-      if (!second_group) m_block(0);
-      if (n_tiles > 1) dma_wait(1, n_tiles > 2);
-    } else {
-      if (!second_group) m_block(0);
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // tiles 1 and 2
-    }
-    lds_barrier();
-    if (!second_group) {
-      // The loop starts on a 64-byte boundary: where it happens to fall otherwise moves the time of this
-      // kernel by several per cent from one build to the next (1.09 against 1.03 ms on 8 x 4096 tokens for
-      // the same instructions at another address).
-      asm volatile(".p2align 6");
-      for (int j = 0; j < n_tiles; j++) {
-        v_block(j);
-        m_block(j + 1);
-        lds_barrier();
+      // The prologue has sent tiles 0, 1 and 2; tiles 0 and 1 have to be complete before the first period.
+      const bool second_group = wave_u >= 4;
+      if constexpr (DMA) {
+        if (!second_group) m_block(0);
+        if (n_tiles > 1) dma_wait(1, n_tiles > 2);
+      } else {
+        if (!second_group) m_block(0);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // tiles 1 and 2
       }
-      lds_barrier();  // the other group's last product still reads its tile
-    } else {
-      asm volatile(".p2align 6");
-      for (int j = 0; j < n_tiles; j++) {
-        m_block(j);
-        v_block(j);
-        lds_barrier();
-      }
-      m_block(n_tiles);
       lds_barrier();
-    }
+      if (!second_group) {
+        // The loop starts on a 64-byte boundary: where it happens to fall otherwise moves the time of this
+        // kernel by several per cent from one build to the next (1.09 against 1.03 ms on 8 x 4096 tokens for
+        // the same instructions at another address).
+        asm volatile(".p2align 6");
+        for (int j = 0; j < n_tiles; j++) {
+          v_block(j);
+          m_block(j + 1);
+          lds_barrier();
+        }
+        lds_barrier();  // the other group's last product still reads its tile
+      } else {
+        asm volatile(".p2align 6");
+        for (int j = 0; j < n_tiles; j++) {
+          m_block(j);
+          v_block(j);
+          lds_barrier();
+        }
+        m_block(n_tiles);
+        lds_barrier();
+      }
     }
   } else {
     // ---- staged tiles: one software-pipelined loop per wavefront ----
@@ -1398,7 +1441,7 @@ template <typename T, int HDP, int MODE, int NW>
 void launch_prefill_nw(PrefillParams p, int hl, hipStream_t stream) {
   static bool attr_set = false;  // benign race: setting twice is harmless
   auto kernel = prefill_varlen_w8_kernel<T, HDP, MODE, NW>;
-  constexpr size_t lds_bytes = MODE == W8_PAGED ? TileW8<HDP>::LDS_BYTES : (size_t)(NW == 4 ? 3 : 5) * 2 * w8_tile_keys(HDP, NW) * HDP * 2;
+  constexpr size_t lds_bytes = MODE == W8_PAGED ? TileW8<HDP>::LDS_BYTES : (size_t)w8_stages(HDP, NW) * 2 * BN * HDP * 2;
   if (!attr_set) {
     HA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)lds_bytes));
@@ -1413,22 +1456,35 @@ void launch_prefill_nw(PrefillParams p, int hl, hipStream_t stream) {
   check_launch("mha_varlen_fwd");
 }
 
-// Whether a launch of head sizes above 64 takes workgroups of four wavefronts.  They hide a workgroup's set-up and wind-down behind the
-// two others on the compute unit (about 8 us per workgroup of eight, which has the compute unit to itself), but their tiles of 32
-// keys cost more per key.  So: more workgroups of eight than compute units, and contexts short enough that those 8 us count.  us,
-// eight / four wavefronts (32 q / 8 kv x 128; 32 / 32 x 80; 32 / 32 x 128), by sequences and lengths:
-//   64 x 30..300     70 / 52      94 / 57      93 / 67       16 x 20..256     22 / 19      27 / 19      29 / 21
-//   32 x 512        130 / 114    125 / 106    140 / 142      16 x 100..1000   98 / 88     100 / 86     110 / 97
-//   32 x 1024       346 / 353    335 / 319    393 / 387      16 x 2048       591 / 624    537 / 570    628 / 662
-//   8 x 512          39 / 40      38 / 37      40 / 41       8 x 384             -         29 / 23      30 / 25
-//   4 x 512          20 / 22      22 / 25      24 / 27       1 x 1024         29 / 32      28 / 32      30 / 33
-// (8 x 512 is two full rounds of 256 workgroups of eight, and one and a third of 768 of four: between one round and two the
-// contexts have to be shorter.)  With keys cached in front of the queries only the longest context is known here.
-bool four_wavefronts_pay(const PrefillParams &p, int heads) {
-  const int bm = 256 / heads;
-  const int64_t wgs = (p.total_q / bm + p.batch / 2) * (p.Hq / heads);
-  const int64_t keys = p.block_tables == nullptr ? p.total_k / p.batch : p.max_k > p.max_q ? p.max_k : p.total_q / p.batch;
-  return wgs > 300 && keys <= (wgs < 600 ? 400 : 640);
+// Whether a launch takes workgroups of four wavefronts: a matter of time alone, the bits are those of eight.  The sizes are those that both
+// entry points know -- workgroups of eight (wgs) and keys of a sequence, about -- so that rows and paged cache choose alike.  Two or three
+// workgroups of four on a compute unit hide their set-up and wind-down behind one another (about 8 us of a workgroup of eight, which has its
+// compute unit to itself); two wavefronts of one workgroup that alternate between the pipes need less time per key.  us, eight / four, rows
+// of k / v (the paged cache within 5 % of the same ratios), by sequences x lengths:
+//                     32 / 32 x 80    32 / 8 x 128    32 / 32 x 128
+//   64 x 30..300       114 / 65         84 / 71         122 / 96
+//   24 x 40..700       96 / 72         87 / 81         104 / 93
+//   32 x 512           127 / 99        132 / 119        142 / 149
+//   32 x 1024          346 / 329       361 / 382        410 / 424
+//   16 x 2048          533 / 526       593 / 638        645 / 679
+//   4 x 512            20.2 / 20.2     18.7 / 21.3      21.2 / 22.1
+//   2 x 2048           65 / 76
+//   2 x 4096           222 / 231       259 / 284        278 / 296
+//   1 x 300            11.3 / 11.0     14.0 / 12.5      12.5 / 11.9
+//   32 x 20..100 + 500 69 / 55         43 / 46          79 / 63
+//   8 x 512 + 2048     131 / 148
+// Over 190 such sizes of each of nine kinds of heads these lines cost 0.8 % on average against the better form of each, all four 1.3 % (2.7 % at
+// head sizes above 96), all eight 10 % (5 %).
+bool four_wavefronts_pay(const PrefillParams &p, int hdp, int heads) {
+  const int64_t wgs = (p.total_q / (256 / heads) + p.batch / 2) * (p.Hq / heads);
+  const int64_t keys = p.max_k > p.max_q ? p.max_k : p.total_q / p.batch;
+  // Three workgroups to a compute unit.  Long contexts whose workgroups of eight are one round over 256 compute units (with two or three
+  // sequences up to two rounds: a sequence's heavy row blocks then meet the next one's on the same compute units) stay with eight.
+  if (hdp <= 64) return true;  // (at every size measured but for a few long contexts)
+  if (hdp <= 96) return !(p.batch > 1 && keys >= 1000 && wgs > 250 && wgs <= (p.batch <= 3 ? 560 : 320));
+  // Two: where eight leave many compute units without work, and where there is more than a round of them and contexts are short.
+  if (wgs <= 220) return wgs <= 160 && keys <= 1900;
+  return keys <= (wgs < 400 ? 500 : 640);
 }
 
 template <typename T, int HDP, int MODE = W8_ROWS>
@@ -1445,15 +1501,10 @@ void launch_prefill_w8(const PrefillParams &p, hipStream_t stream) {
   while (hl < 3 && p.G % (2 << hl) == 0 && (2 << hl) <= limit) hl++;
   if constexpr (MODE == W8_PAGED) {
     launch_prefill_nw<T, HDP, MODE, 8>(p, hl, stream);
-  } else if constexpr (HDP <= 64) {
-    // One wavefront's chain of a tile (scores, softmax, products) is as long as the work of two on a SIMD: a third one is free.  us,
-    // eight wavefronts per workgroup / four, 16 q / 2 kv heads x 64: 32 x 1..2048 213 / 190, 64 x 30..300 28 / 21, 64 x 2048 855 / 731,
-    // 8 x 8000 1264 / 1190, 1 x 300 10.0 / 9.1, 1 x 8000 160 / 163.
-    launch_prefill_nw<T, HDP, MODE, 4>(p, hl < 2 ? hl : 2, stream);
   } else {
-    const int force = tuning().prefill_kernel;
-    if (force == 5 || (force != 1 && four_wavefronts_pay(p, 1 << (hl < 2 ? hl : 2))))
-      launch_prefill_nw<T, HDP, MODE, 4>(p, hl < 2 ? hl : 2, stream);
+    const int force = tuning().prefill_kernel, hl4 = hl < 2 ? hl : 2;
+    if (force == 5 || ((HDP <= 64 || force != 1) && four_wavefronts_pay(p, HDP, 1 << hl4)))
+      launch_prefill_nw<T, HDP, MODE, 4>(p, hl4, stream);
     else
       launch_prefill_nw<T, HDP, MODE, 8>(p, hl, stream);
   }

@@ -388,3 +388,62 @@ def test_workgroups_of_four_wavefronts(device, tuning, kernel_choice, dtype, hea
         tuning("prefill_kernel", 1)
         eight = run(p, device)
         assert (eight.float() - got.float()).abs().max().item() <= TOL[dtype]
+
+
+@pytest.mark.parametrize("heads", [(32, 8, 128), (32, 32, 80), (16, 2, 64)])
+@pytest.mark.parametrize("seqs,least,most,prior", [(64, 30, 300, 0), (20, 100, 380, 0), (64, 600, 700, 0), (48, 20, 100, 500), (9, 20, 90, 900)])
+def test_a_prompt_has_the_same_bits_in_any_company(device, tuning, kernel_choice, heads, seqs, least, most, prior):
+    """The library chooses the form of the launch by the sizes of the whole batch; a sequence's output and its log-sum-exp are the same bits
+    in a batch, alone, from rows of k / v, from the paged cache and with either form of the workgroups forced, on batches of many
+    and few workgroups, of short and longer contexts, behind cached keys and not."""
+    if kernel_choice != "auto":
+        pytest.skip("forces its own kernels")
+    Hq, Hkv, d = heads
+    lens_q = np.random.default_rng(seqs + prior).integers(least, most + 1, size=seqs).tolist()
+    lens_k = [n + prior * (i % 2) for i, n in enumerate(lens_q)]
+    g = torch.Generator(device=device).manual_seed(seqs)
+    q = torch.randn((sum(lens_q), Hq, d), generator=g, device=device).to(torch.bfloat16)
+    k, v = (torch.randn((sum(lens_k), Hkv, d), generator=g, device=device).to(torch.bfloat16) for _ in range(2))
+    scale = 1.0 / math.sqrt(d)
+    blocks = [(n + 15) // 16 for n in lens_k]
+    order = torch.randperm(sum(blocks), generator=torch.Generator().manual_seed(7)).split(blocks)
+    tables = torch.zeros((seqs, max(blocks)), dtype=torch.int32)
+    for i, mine in enumerate(order):
+        tables[i, :blocks[i]] = mine
+    slots = torch.cat([(mine[:, None] * 16 + torch.arange(16)).flatten()[:n] for mine, n in zip(order, lens_k)]).to(device)
+    kc = torch.full((sum(blocks), Hkv, d // 8, 16, 8), float("nan"), dtype=q.dtype, device=device)
+    vc = torch.full((sum(blocks), Hkv, d, 16), float("nan"), dtype=q.dtype, device=device)
+    K.reshape_and_cache(k, v, kc, vc, slots)
+    at_q, at_k = W.offsets(lens_q).tolist(), W.offsets(lens_k).tolist()
+
+    def rows(i, j):
+        """Sequences i .. j - 1 as a batch of their own."""
+        return K.flash_attn_varlen(q[at_q[i]:at_q[j]], k[at_k[i]:at_k[j]], v[at_k[i]:at_k[j]], W.offsets(lens_q[i:j]).to(device),
+                                   W.offsets(lens_k[i:j]).to(device), max(lens_q[i:j]), max(lens_k[i:j]), scale, True, return_lse=True)
+
+    def paged(i, j):
+        return K.flash_attn_varlen_paged(q[at_q[i]:at_q[j]], kc, vc, tables[i:j].to(device), W.offsets(lens_q[i:j]).to(device),
+                                         torch.tensor(lens_k[i:j], dtype=torch.int32, device=device), max(lens_q[i:j]), max(lens_k[i:j]),
+                                         scale, True, return_lse=True)
+
+    def same(got, i, j):
+        assert torch.equal(got[0], out[at_q[i]:at_q[j]])
+        for b in range(i, j):
+            assert torch.equal(got[1][b - i, :, :lens_q[b]], lse[b, :, :lens_q[b]])
+
+    out, lse = rows(0, seqs)
+    assert not torch.isnan(out).any()
+    same(paged(0, seqs), 0, seqs)
+    longest, shortest = lens_k.index(max(lens_k)), lens_k.index(min(lens_k))
+    for i in {0, seqs - 1, longest, shortest}:
+        same(rows(i, i + 1), i, i + 1)
+        same(paged(i, i + 1), i, i + 1)
+    same(paged(0, 5), 0, 5)
+    for form in (1, 5):
+        tuning("prefill_kernel", form)
+        same(rows(0, seqs), 0, seqs)
+        same(paged(0, seqs), 0, seqs)
+    i = longest
+    want = ref.varlen_attn_fp64(*(t.cpu().float() for t in (q[at_q[i]:at_q[i + 1]], k[at_k[i]:at_k[i + 1]], v[at_k[i]:at_k[i + 1]])),
+                                W.offsets(lens_q[i:i + 1]), W.offsets(lens_k[i:i + 1]), scale, True)
+    assert (out[at_q[i]:at_q[i + 1]].cpu().double() - want).abs().max().item() <= TOL[torch.bfloat16]
