@@ -1461,18 +1461,18 @@ void launch_prefill_nw(PrefillParams p, int hl, hipStream_t stream) {
 // workgroups of four on a compute unit hide their set-up and wind-down behind one another (about 8 us of a workgroup of eight, which has its
 // compute unit to itself); two wavefronts of one workgroup that alternate between the pipes need less time per key.  us, eight / four, rows
 // of k / v (the paged cache within 5 % of the same ratios), by sequences x lengths:
-//                     32 / 32 x 80    32 / 8 x 128    32 / 32 x 128
-//   64 x 30..300       114 / 65         84 / 71         122 / 96
-//   24 x 40..700       96 / 72         87 / 81         104 / 93
-//   32 x 512           127 / 99        132 / 119        142 / 149
-//   32 x 1024          346 / 329       361 / 382        410 / 424
-//   16 x 2048          533 / 526       593 / 638        645 / 679
-//   4 x 512            20.2 / 20.2     18.7 / 21.3      21.2 / 22.1
-//   2 x 2048           65 / 76
-//   2 x 4096           222 / 231       259 / 284        278 / 296
-//   1 x 300            11.3 / 11.0     14.0 / 12.5      12.5 / 11.9
-//   32 x 20..100 + 500 69 / 55         43 / 46          79 / 63
-//   8 x 512 + 2048     131 / 148
+//                     16 q / 2 kv x 64   32 / 32 x 80    32 / 8 x 128    32 / 32 x 128
+//   64 x 30..300        33 / 25           114 / 65         84 / 71         122 / 96
+//   24 x 40..700        37 / 31            96 / 72         87 / 81         104 / 93
+//   32 x 512            54 / 42           127 / 99        132 / 119        142 / 149
+//   32 x 1024          144 / 114          346 / 329       361 / 382        410 / 424
+//   16 x 2048          214 / 196          533 / 526       593 / 638        645 / 679
+//   4 x 512           13.8 / 12.3        20.2 / 20.2     18.7 / 21.3      21.2 / 22.1
+//   2 x 2048            39 / 44            65 / 76
+//   2 x 4096            91 / 109          222 / 231       259 / 284        278 / 296
+//   1 x 300           10.0 / 9.1         11.3 / 11.0     14.0 / 12.5      12.5 / 11.9
+//   32 x 20..100 + 500 17.0 / 17.7         69 / 55         43 / 46          79 / 63
+//   8 x 512 + 2048      53 / 59           131 / 148
 // Over 190 such sizes of each of nine kinds of heads these lines cost 0.8 % on average against the better form of each, all four 1.3 % (2.7 % at
 // head sizes above 96), all eight 10 % (5 %).
 bool four_wavefronts_pay(const PrefillParams &p, int hdp, int heads) {
@@ -1480,7 +1480,6 @@ bool four_wavefronts_pay(const PrefillParams &p, int hdp, int heads) {
   const int64_t keys = p.max_k > p.max_q ? p.max_k : p.total_q / p.batch;
   // Three workgroups to a compute unit.  Long contexts whose workgroups of eight are one round over 256 compute units (with two or three
   // sequences up to two rounds: a sequence's heavy row blocks then meet the next one's on the same compute units) stay with eight.
-  if (hdp <= 64) return true;  // (at every size measured but for a few long contexts)
   if (hdp <= 96) return !(p.batch > 1 && keys >= 1000 && wgs > 250 && wgs <= (p.batch <= 3 ? 560 : 320));
   // Two: where eight leave many compute units without work, and where there is more than a round of them and contexts are short.
   if (wgs <= 220) return wgs <= 160 && keys <= 1900;
@@ -1503,7 +1502,7 @@ void launch_prefill_w8(const PrefillParams &p, hipStream_t stream) {
     launch_prefill_nw<T, HDP, MODE, 8>(p, hl, stream);
   } else {
     const int force = tuning().prefill_kernel, hl4 = hl < 2 ? hl : 2;
-    if (force == 5 || ((HDP <= 64 || force != 1) && four_wavefronts_pay(p, HDP, 1 << hl4)))
+    if (force == 5 || (force != 1 && four_wavefronts_pay(p, HDP, 1 << hl4)))
       launch_prefill_nw<T, HDP, MODE, 4>(p, hl4, stream);
     else
       launch_prefill_nw<T, HDP, MODE, 8>(p, hl, stream);

@@ -31,10 +31,10 @@ struct Tuning {
   int decode_flat;         // -1: the library chooses; 0 / 1: partitioned / flat-split launch
   int decode_flat_wgs;     // 0: what the device holds at once; else workgroups of the flat launch
   int decode_part_blocks;  // 0: chosen per call; else KV blocks per partition (2..64)
-  int prefill_kernel;      // 0: the library chooses; 1: eight wavefronts; 2 / 3: four wavefronts, 2 / 1 row tiles each; 4: three groups of four; 5: as 1, in workgroups of four wavefronts
+  int prefill_kernel;      // 0: the library chooses; 1: workgroups of eight wavefronts, 5: the same kernel in workgroups of four; 2 / 3: another of four, 2 / 1 row tiles each; 4: three groups of four
   int paged_prefill_dma;   // -1: the library chooses; 0: staged tiles; 1: block images where possible
   int cache_move_lds;      // -1: the library chooses; 0: never the LDS-transposing kernels
-  int prefill_wg_heads;      // eight-wavefront prefill: query heads of one kv group per workgroup, at most (0: the library chooses -- up to four; 1: one)
+  int prefill_wg_heads;      // prefill_kernel 1 and (up to four) 5: query heads of one kv group per workgroup, at most (0: the library chooses -- up to four; 1: one)
   int prefill_rescale_log2;  // prefill: a row's reference maximum moves when outgrown by more than 2^this (0..16, default 8)
   int linear_tiles;          // linear: 64-row tiles of the weight per workgroup (0: the library chooses; 1 or 2)
   int linear_waves;          // linear: wavefronts per workgroup, 16 rows of the weight each (0: the library chooses; 4 or 8)

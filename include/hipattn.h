@@ -542,12 +542,14 @@ char *hipattn_shutdown(void);
  * name in capitals); ops never read the environment.  Names: decode_flat
  * (-1 library's choice, 0 partitioned launch, 1 flat split), decode_flat_wgs
  * (0 = what the device holds at once), decode_part_blocks (0 = chosen per
- * call, else 2..64), prefill_kernel (0 library's choice, 1 eight wavefronts,
- * 2 / 3 four wavefronts with 2 / 1 row tiles, 4 three groups of four
- * wavefronts, 5 as 1 in workgroups of four), paged_prefill_dma (-1 library's
+ * call, else 2..64), prefill_kernel (0 library's choice, 1 workgroups of eight
+ * wavefronts, 5 the same kernel in workgroups of four -- the bits of 1 -- 2 / 3
+ * another of four wavefronts with 2 / 1 row tiles, 4 three groups of four
+ * wavefronts; what a kernel does not cover, the one that does takes),
+ * paged_prefill_dma (-1 library's
  * choice, 0 staged tiles), cache_move_lds (-1 library's choice, 0 never the
  * LDS-transposing kernels), prefill_wg_heads (query heads of one kv group per
- * workgroup of the eight-wavefront prefill kernel, at most; 0 library's
+ * workgroup of prefill_kernel 1 and, up to four, 5, at most; 0 library's
  * choice -- up to four -- 1: one),
  * prefill_rescale_log2 (0..16, default 8: the prefill
  * kernels move a row's reference maximum only when the row outgrows it by
@@ -555,8 +557,8 @@ char *hipattn_shutdown(void);
  * does), linear_tiles (0 library's choice, 1 / 2: workgroups of 64 /
  * 128 rows of the weight in hipattn_linear), linear_splits (0 library's choice, else
  * the number of ranges the inner dimension is cut into, at most 32).  Every
- * setting computes the same results -- prefill_rescale_log2 and linear_splits
- * up to rounding.  Not
+ * setting computes the same results -- prefill_kernel 2 to 4,
+ * prefill_rescale_log2 and linear_splits up to rounding.  Not
  * synchronised with running calls: set them between calls. */
 char *hipattn_tuning_set(const char *name, int value);
 char *hipattn_tuning_get(const char *name, int *value);

@@ -1,6 +1,7 @@
 """Varlen flash-attention forward through the C ABI against the oracle.  Gates: max-abs error
 <= 2e-2 (bf16), <= 5e-3 (fp16) against the fp32/fp64 oracle on the same rounded inputs."""
 import math
+import re
 
 import numpy as np
 import pytest
@@ -17,8 +18,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.fixture(autouse=True, params=["auto", "eight_wavefronts", "four_wavefronts", "three_groups"])
 def kernel_choice(request, tuning):
-    """The forward pass has three kernels (256-row workgroups of eight wavefronts and 96- or 384-row
-    workgroups of three groups of four wavefronts for head sizes up to 128, 128-row workgroups of four
+    """The forward pass has three kernels (256-row workgroups of eight wavefronts, or 128-row ones of four, and 96- or
+    384-row workgroups of three groups of four wavefronts for head sizes up to 128, 128-row workgroups of four
     for the rest) and picks by shape; every test runs under the library's own choice and with each one
     forced (what a forced kernel does not cover falls through to the one that does)."""
     tuning("prefill_kernel", {"auto": 0, "eight_wavefronts": 1, "four_wavefronts": 3, "three_groups": 4}[request.param])
@@ -330,7 +331,7 @@ def test_several_heads_of_a_kv_group_per_workgroup(device, tuning, limit):
     rows of each) instead of 256 rows of one head: same results, to the bit, as one head per workgroup -- the
     arithmetic of a row does not depend on which wavefront runs it -- for GQA ratios 4 and 8, ragged chunks with
     prior context, the log-sum-exp and the fp32 output."""
-    for seed, (Hq, Hkv, d, dtype) in [(51, (32, 8, 128, torch.bfloat16)), (52, (16, 2, 64, torch.float16))]:
+    for seed, (Hq, Hkv, d, dtype) in [(51, (32, 8, 128, torch.bfloat16)), (52, (16, 2, 64, torch.float16)), (53, (16, 2, 96, torch.bfloat16))]:
         p = general_inputs(seed, [300, 1, 70, 513], [300, 40, 517, 513], Hq, Hkv, d, dtype)
         dv = p.to(device)
         args = (dv.q, dv.k, dv.v, dv.cu_q, dv.cu_k, p.max_q, p.max_k, p.scale, True)
@@ -447,3 +448,48 @@ def test_a_prompt_has_the_same_bits_in_any_company(device, tuning, kernel_choice
     want = ref.varlen_attn_fp64(*(t.cpu().float() for t in (q[at_q[i]:at_q[i + 1]], k[at_k[i]:at_k[i + 1]], v[at_k[i]:at_k[i + 1]])),
                                 W.offsets(lens_q[i:i + 1]), W.offsets(lens_k[i:i + 1]), scale, True)
     assert (out[at_q[i]:at_q[i + 1]].cpu().double() - want).abs().max().item() <= TOL[torch.bfloat16]
+
+
+@pytest.mark.filterwarnings("ignore:Profiler clears events")
+def test_the_form_of_the_workgroups(device, tuning, kernel_choice):
+    """Which kernel a launch takes, by its name: what prefill_kernel asks for at every head size, and the library's own choice on either
+    side of its limits, the same from rows of k / v and from the paged cache."""
+    if kernel_choice != "auto":
+        pytest.skip("forces its own kernels")
+
+    def wavefronts(Hq, Hkv, d, seqs, lq, prior, paged):
+        q = torch.zeros((seqs * lq, Hq, d), dtype=torch.bfloat16, device=device)
+        lk, cu_q = lq + prior, W.offsets([lq] * seqs).to(device)
+        if paged:
+            blocks = (lk + 15) // 16
+            kc = torch.zeros((seqs * blocks, Hkv, d // 8, 16, 8), dtype=q.dtype, device=device)
+            vc = torch.zeros((seqs * blocks, Hkv, d, 16), dtype=q.dtype, device=device)
+            tables = torch.arange(seqs * blocks, dtype=torch.int32, device=device).view(seqs, blocks)
+            ctx = torch.full((seqs,), lk, dtype=torch.int32, device=device)
+            call = lambda: K.flash_attn_varlen_paged(q, kc, vc, tables, cu_q, ctx, lq, lk, 0.1, True)
+        else:
+            k = torch.zeros((seqs * lk, Hkv, d), dtype=q.dtype, device=device)
+            cu_k = W.offsets([lk] * seqs).to(device)
+            call = lambda: K.flash_attn_varlen(q, k, k, cu_q, cu_k, lq, lk, 0.1, True)
+        call()
+        torch.cuda.synchronize()
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+            call()
+            torch.cuda.synchronize()
+        names = [e.key for e in prof.key_averages() if "prefill_varlen_w8_kernel" in e.key]
+        assert len(names) == 1, [e.key for e in prof.key_averages()]
+        return int((re.search(r", (\d+)>\(", names[0]) or re.search(r"Li(\d+)EEEv", names[0])).group(1))
+
+    for paged in (False, True):
+        for heads in ((16, 2, 32), (16, 2, 64), (32, 32, 80), (32, 8, 128)):
+            for form, n in ((1, 8), (5, 4)):
+                tuning("prefill_kernel", form)
+                assert wavefronts(*heads, 3, 200, 50, paged) == n
+        tuning("prefill_kernel", 0)
+        for heads, seqs, lq, prior, n in (((16, 2, 64), 32, 300, 0, 4), ((16, 2, 64), 2, 4096, 0, 8), ((16, 2, 64), 1, 4096, 0, 4),
+                                          ((16, 2, 64), 2, 1000, 0, 4), ((16, 2, 64), 4, 4096, 0, 4), ((16, 2, 64), 8, 512, 2048, 8),
+                                          ((32, 32, 80), 32, 1024, 0, 4), ((32, 32, 80), 2, 2048, 0, 8),
+                                          ((32, 8, 128), 32, 512, 0, 4), ((32, 8, 128), 32, 1024, 0, 8), ((32, 8, 128), 4, 512, 0, 8),
+                                          ((32, 8, 128), 1, 1024, 0, 4), ((32, 8, 128), 1, 128, 2048, 8), ((32, 8, 128), 48, 64, 500, 4),
+                                          ((32, 8, 128), 48, 64, 700, 8)):
+            assert wavefronts(*heads, seqs, lq, prior, paged) == n, (heads, seqs, lq, prior, paged)
