@@ -46,6 +46,7 @@ struct ScratchKey {
 struct ScratchBuffer {
   void *ptr = nullptr;
   size_t bytes = 0;
+  std::mutex holder;  // of a buffer that several launches of a call share
 };
 std::map<ScratchKey, ScratchBuffer> g_scratch;
 std::vector<std::pair<int, void *>> g_retired;  // (device, pointer)
@@ -100,13 +101,14 @@ hipStream_t resolve_stream(void *stream) {
   return tl_current_stream;
 }
 
-void *library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream) {
+// The buffer of (user, current device, stream), at least `bytes` large; where it has to be allocated, `spare` more.
+static ScratchBuffer &scratch_buffer(WorkspaceUser user, size_t bytes, size_t spare, hipStream_t stream) {
   int dev = 0;
   HA_HIP(hipGetDevice(&dev));
   HA_CHECK(dev >= 0 && dev < kMaxDevices, "device index %d out of range", dev);
   std::lock_guard<std::mutex> lock(g_mutex);
   ScratchBuffer &ws = g_scratch[ScratchKey{(int)user, dev, stream}];
-  if (ws.bytes >= bytes && ws.ptr != nullptr) return ws.ptr;
+  if (ws.bytes >= bytes && ws.ptr != nullptr) return ws;
   // Allocating is not something a capture can record, and the graph would keep the old pointer.
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   const hipError_t asked = hipStreamIsCapturing(stream, &capturing);
@@ -119,8 +121,7 @@ void *library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream) {
            "the library's scratch buffer for this stream must grow to %zu bytes, which cannot happen while the stream is "
            "being captured: run the call once outside the capture first, or use the entry point that takes a workspace",
            bytes);
-  size_t want = bytes + bytes / 2;
-  want = (want + 255) & ~(size_t)255;
+  const size_t want = (bytes + spare + 255) & ~(size_t)255;
   void *fresh = nullptr;
   HA_HIP(hipMalloc(&fresh, want));
   // Counters kept in the buffer start at zero.  The fill goes onto the stream that the buffer belongs to (which is
@@ -134,25 +135,31 @@ void *library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream) {
   g_lib_allocated[dev] += (int64_t)want;
   ws.ptr = fresh;
   ws.bytes = want;
-  return ws.ptr;
+  return ws;
 }
 
-void *try_library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream) {
+void *library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream) {
+  return scratch_buffer(user, bytes, bytes / 2, stream).ptr;
+}
+
+HeldWorkspace try_library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream) {
+  HeldWorkspace ws;
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) {
     (void)hipGetLastError();
-    return nullptr;
+    return ws;
   }
-  if (capturing != hipStreamCaptureStatusNone) return nullptr;
+  if (capturing != hipStreamCaptureStatusNone) return ws;
   // A capture on some other stream forbids allocations, in every thread unless the thread says otherwise.
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
     (void)hipGetLastError();
-    return nullptr;
+    return ws;
   }
-  void *ws = nullptr;
   try {
-    ws = library_workspace(user, bytes, stream);
+    ScratchBuffer &buffer = scratch_buffer(user, bytes, 0, stream);
+    ws.ptr = buffer.ptr;
+    ws.held = std::unique_lock<std::mutex>(buffer.holder);
   } catch (const Error &) {
     (void)hipGetLastError();
   }

@@ -32,8 +32,6 @@
 // 128 rows of 128256 bf16 logits, 5 % allowed, top-p 0.9: any row 199 us, counting 43 us; all allowed 221 / 55, one row
 // 177 / 40; fp16 203 / 60 (the logits take 5 us to read once; a pass over one row on one compute unit takes 6 to 12).  Counted in
 // pieces, bf16: 26 and, all allowed, 29 us; one row 15.
-#include <mutex>
-
 #include "common.h"
 #include "device_types.h"
 #include "workspace.h"
@@ -553,6 +551,7 @@ constexpr int kCountThreads = 512;   // four workgroups per compute unit, by LDS
 constexpr int kLeastPieces = 24576;  // tokens
 constexpr int kMaxPieces = kWaves;   // a wavefront of the row's workgroup for each
 constexpr int kPieceListed = 1016;
+constexpr int kMostPieces = 2048;    // of all rows together
 struct PieceCounts {
   uint16_t counts[Counted<bf16_t>::kBins];
   int n_others, pad[3];
@@ -1209,20 +1208,18 @@ void bias_sample_impl(const hipattn_tensor *logits, const hipattn_tensor *bias, 
   p.uniforms = static_cast<const float *>(uniforms->data);
   p.out_tokens = static_cast<int32_t *>(out_tokens->data);
   HA_CHECK(S <= 0x7fffffff, "%s: too many sequences", op);
-  // Pieces, where there are several and workgroups for them: the scratch memory then stays below 40 MB.  Under capture the row's
+  // Pieces, where there are several and workgroups for them.  Their counts lie in a buffer of the stream's, allocated once for the
+  // largest call (kMostPieces, 38 MB: buffers that grow with the batch are all kept, some 170 MB together).  Under capture the row's
   // workgroup does it alone: the graph may be replayed beside other calls on this stream's scratch memory.
   // Two launches that share it stay next to one another where several threads use one stream; hipStreamPerThread names a stream of each
   // thread's own by one handle, so it has no scratch memory.
-  static std::mutex pair_mutex;
-  std::unique_lock<std::mutex> pair(pair_mutex, std::defer_lock);
   const int64_t n_pieces = (V + kPieceTokens - 1) / kPieceTokens;
-  PieceCounts *pieces = nullptr;
-  if (mask && logits->dtype == HIPATTN_BF16 && V >= kLeastPieces && n_pieces <= kMaxPieces && S * n_pieces <= 2048 &&
-      stream != hipStreamPerThread) {
-    pair.lock();
-    pieces = static_cast<PieceCounts *>(try_library_workspace(WS_SAMPLE, (size_t)(S * n_pieces) * sizeof(PieceCounts), stream));
-  }
-  if (pieces != nullptr) {
+  HeldWorkspace counts;
+  if (mask && logits->dtype == HIPATTN_BF16 && V >= kLeastPieces && n_pieces <= kMaxPieces && S * n_pieces <= kMostPieces &&
+      stream != hipStreamPerThread)
+    counts = try_library_workspace(WS_SAMPLE, kMostPieces * sizeof(PieceCounts), stream);
+  if (counts.ptr != nullptr) {
+    PieceCounts *pieces = static_cast<PieceCounts *>(counts.ptr);
     sample_count_kernel<bf16_t><<<dim3((unsigned)n_pieces, (unsigned)S), kCountThreads, 0, stream>>>(p, pieces);
     check_launch(op);
     bias_sample_kernel<bf16_t, 1, SAMPLE_PIECES><<<dim3((unsigned)S), kThreads, 0, stream>>>(p, pieces, (int)n_pieces);

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <mutex>
 
 namespace hipattn {
 
@@ -19,9 +20,15 @@ enum WorkspaceUser { WS_PAGED_ATTENTION = 0, WS_BIAS_ARGMAX = 1, WS_LINEAR = 2, 
 // message that says so.
 void *library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream);
 
-// The same for an op that has another way without scratch memory: null while the stream is being captured (also where the buffer is
-// there: a graph may be replayed on any stream, beside calls that use it) and where there is no memory to be had.
-void *try_library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream);
+// A buffer that several launches of a call share, for an op that has another way without: null while the stream is being captured
+// (also where the buffer is there: a graph may be replayed on any stream, beside calls that use it) and where there is no memory to be
+// had.  `bytes` is the op's constant -- the buffer has that size and never grows -- and no other call, of another thread on this stream,
+// gets the buffer while `held` lives.
+struct HeldWorkspace {
+  void *ptr = nullptr;
+  std::unique_lock<std::mutex> held;
+};
+HeldWorkspace try_library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream);
 
 // Switches for tuning and for tests that want one particular kernel; read
 // from the environment (HIPATTN_<NAME in capitals>) once, when the library is

@@ -457,7 +457,8 @@ char *hipattn_bias_argmax(const hipattn_tensor *logits,
  * out_tokens int32 [S].
  * bf16 rows of 24576 to 262144 tokens under a mask are read by several
  * workgroups each, which leave their counts in a buffer of the library's that
- * belongs to the stream (up to 58 MB, kept until hipattn_shutdown).  While the stream
+ * belongs to the stream (38 MB from the first such call on, kept until
+ * hipattn_shutdown).  While the stream
  * is being captured, or without memory for the buffer, one workgroup reads the
  * row, as for other rows: the same tokens. */
 char *hipattn_bias_sample(const hipattn_tensor *logits,

@@ -431,6 +431,23 @@ def test_bias_sample_in_pieces_from_several_threads(device):
         assert torch.equal(captured, rows[0] * 2)
 
 
+def test_bias_sample_in_pieces_keeps_one_buffer_per_stream(device):
+    """A batch that grows row by row, and one of a wider vocabulary, on a stream that is new to the library: what it holds for the stream
+    afterwards is one buffer of the largest call's size, 2048 pieces of 18432 bytes."""
+    stream = torch.cuda.Stream()
+    rows = torch.zeros((256, 128256), dtype=torch.bfloat16, device=device)
+    mask = torch.full((256, 262144 // 8), 255, dtype=torch.uint8, device=device)
+    ones = torch.ones((256,), device=device)
+    torch.cuda.synchronize()
+    before = K.cuda_get_stats_allocated_bytes(0).allocated
+    with torch.cuda.stream(stream):
+        for S in (1, 2, 3, 5, 8, 12, 18, 27, 41, 62, 93, 140, 210, 256):
+            K.bias_sample(rows[:S], ones[:S], 0.9 * ones[:S], 0.5 * ones[:S], mask=mask[:S, :128256 // 8].contiguous())
+        K.bias_sample(rows.view(-1)[:100 * 262144].view(100, 262144), ones[:100], 0.9 * ones[:100], 0.5 * ones[:100], mask=mask[:100])
+    stream.synchronize()
+    assert K.cuda_get_stats_allocated_bytes(0).allocated - before <= 2048 * 18432
+
+
 def test_bias_sample_corner_rows(device):
     """Rows outside what the reference defines still give a defined, allowed token: an infinite logit (its first
     holder), uniform numbers outside [0, 1) (the first / the last token with weight), an infinite temperature
