@@ -54,7 +54,7 @@ constexpr int kLinMT = 8;         // 16-row tiles of x
 constexpr int kLinStageK = 64;    // values of k per stage: 128 bytes of a row
 constexpr int kLinStreamRows = 16;
 constexpr int kLinHeldRows = 4;
-constexpr int kLinHeldBytes = 40 * 1024;  // of x and the norm's weight: two workgroups per compute unit
+constexpr int kLinHeldBytes = 40 * 1024;  // of x and the norm's weight: two workgroups per compute unit, where the ranges' sums take 4 KB (16 at most)
 constexpr int kHeldStages = 4;
 constexpr int kLinMaxRanges = 8;  // ranges of k that the library itself chooses
 

@@ -245,7 +245,7 @@ def fused_add_rms_norm(input: torch.Tensor, residual: torch.Tensor, weight: torc
 def add_rms_norm_takes(input: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether `add_rms_norm` accepts these operands (else a caller makes the two calls)."""
     return (input.dtype in (torch.float16, torch.bfloat16) and input.size(1) % 8 == 0 and input.size(1) <= 8192
-            and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (input, residual, weight)))
+            and all(t.dtype == input.dtype and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (input, residual, weight)))
 
 
 def add_rms_norm(input: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, epsilon: float) -> torch.Tensor:
@@ -263,7 +263,8 @@ def linear_takes(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether `linear` accepts these operands (else a caller multiplies with a library GEMM)."""
     return (x.dim() == 2 and weight.dim() == 2 and 0 < x.size(0) <= LINEAR_MAX_ROWS and x.size(1) % 256 == 0
             and weight.size(0) % 16 == 0 and x.dtype in (torch.float16, torch.bfloat16) and weight.dtype == x.dtype
-            and x.stride(1) == 1 and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0)
+            and x.stride(1) == 1 and weight.stride(1) == 1 and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
@@ -301,8 +302,10 @@ RMS_NORM_LINEAR_MAX_ROWS = 4
 
 def rms_norm_linear_takes(x: torch.Tensor, norm_weight: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether `rms_norm_linear` accepts these operands (else a caller makes the two calls)."""
-    return (linear_takes(x, weight) and norm_weight.data_ptr() % 16 == 0 and norm_weight.is_contiguous() and x.size(0) <= RMS_NORM_LINEAR_MAX_ROWS and x.size(1) <= 8192
-            and (x.size(0) + 1) * ((x.size(1) * 2 + 1023) // 1024) <= 40 and weight.size(0) < 65536 and weight.size(0) % 32 == 0
+    return (linear_takes(x, weight) and x.size(0) <= RMS_NORM_LINEAR_MAX_ROWS and x.size(1) <= 8192
+            and norm_weight.dtype == x.dtype and norm_weight.numel() == x.size(1) and norm_weight.is_contiguous()
+            and norm_weight.data_ptr() % 16 == 0 and (x.size(0) + 1) * ((x.size(1) * 2 + 1023) // 1024) <= 40
+            and weight.size(0) < 65536 and weight.size(0) % 32 == 0
             and 0 < weight.stride(0) < 1 << 28 and (x.size(0) == 1 or 0 <= x.stride(0) < 1 << 28))
 
 
@@ -321,7 +324,7 @@ def qkv_linear_takes(x: torch.Tensor, weight: torch.Tensor, cos_sin_cache: torch
     d = cos_sin_cache.size(1)
     return (linear_takes(x, weight) and weight.size(0) < (65536 if x.size(0) <= 16 else 16384) and d % 16 == 0
             and key_cache.dim() == 5 and key_cache.size(2) * key_cache.size(4) == d and weight.size(0) % d == 0
-            and weight.size(0) // d > 2 * key_cache.size(1) > 0 and weight.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0
+            and weight.size(0) // d > 2 * key_cache.size(1) > 0
             and 0 < weight.stride(0) < 1 << 28 and (x.size(0) == 1 or 0 <= x.stride(0) < 1 << 28)
             and cos_sin_cache.dtype == key_cache.dtype == value_cache.dtype == x.dtype and cos_sin_cache.is_contiguous()
             and cos_sin_cache.data_ptr() % 16 == 0 and key_cache.data_ptr() % 16 == 0 and key_cache.stride(0) % 8 == 0

@@ -1,5 +1,6 @@
 """hipattn_linear (x . weight^T + bias + residual for the rows of a generation step) through the C ABI against
 the oracle's fp64 product, on the projection shapes of the configured models and on awkward ones."""
+import numpy as np
 import pytest
 import torch
 
@@ -415,3 +416,29 @@ def test_qkv_linear_refusals(device):
             K.qkv_linear(bad[0], None, 0.0, bad[1], idx, bad[2], bad[3], bad[4], idx)
     with pytest.raises(HipAttnError, match="3 positions"):
         K.qkv_linear(x, None, 0.0, w, at[:3], table, kc, vc, at)
+
+
+def test_operands_off_16_byte_boundaries_are_not_taken(device):
+    """Whether a call is accepted is answered for rows, weights and norm weights that start anywhere: what the answer takes runs, what it does
+    not take is what the call refuses."""
+    def at(offset, *shape):
+        n = int(np.prod(shape))
+        return torch.zeros((n + 8,), dtype=torch.bfloat16, device=device)[offset:offset + n].view(shape)
+
+    table, kc, vc = at(0, 32, 64), at(0, 2, 1, 8, 16, 8), at(0, 2, 1, 64, 16)
+    index = torch.zeros((2,), dtype=torch.int64, device=device)
+    for ox, ow, on in ((0, 0, 0), (1, 0, 0), (4, 0, 0), (0, 1, 0), (0, 4, 0), (0, 0, 4)):
+        x, w, norm = at(ox, 2, 256), at(ow, 384, 256), at(on, 256)
+        assert K.linear_takes(x, w) == (ox == ow == 0)
+        assert K.rms_norm_linear_takes(x, norm, w) == (ox == ow == on == 0)
+        assert K.qkv_linear_takes(x, w, table, kc, vc) == (ox == ow == 0)
+        for taken, call in ((ox == ow == 0, lambda: K.linear(x, w)), (ox == ow == on == 0, lambda: K.rms_norm_linear(x, norm, 1e-5, w)),
+                            (ox == ow == 0, lambda: K.qkv_linear(x, None, 0.0, w, index, table, kc, vc, index))):
+            if taken:
+                call()
+            else:
+                with pytest.raises(HipAttnError, match="16-byte"):
+                    call()
+    x, w, norm = at(0, 2, 256), at(0, 384, 256), at(0, 256)
+    assert not K.rms_norm_linear_takes(x, norm.half(), w) and not K.rms_norm_linear_takes(x, norm[:128], w)
+    assert not K.add_rms_norm_takes(x, x.half(), norm) and not K.add_rms_norm_takes(x, x.clone(), norm.float())
