@@ -11,8 +11,9 @@ import numpy as np
 import pytest
 import torch
 
-from aici_amd import llama, paged
+from aici_amd import kernels, llama, paged
 from aici_amd import workloads as W
+from aici_amd._lib import HipAttnError
 from oracle import aici as oaici
 from oracle import hostkv
 from oracle import llama as ollama
@@ -239,3 +240,73 @@ def test_32_layer_step_at_llama3_8b_shape_properties(device):
         torch.cuda.synchronize()
         assert torch.equal(toks_graph, toks)
         assert torch.equal(step(), toks)          # eager work between the replays
+
+
+def decode_step(cfg, device, contexts, rows=None, seed=3):
+    """A step in which a sequence per context, or the first `rows` of them, decodes one token, and caches that hold the tokens in front
+    of it."""
+    pool = sum((n + 15) // 16 for n in contexts) + 8
+    alloc = paged.BlockAllocator(16, pool)
+    builder = paged.BatchInfoBuilder(16, cfg.max_position_embeddings, 1)
+    rng = np.random.default_rng(seed)
+    for sid, n in enumerate(contexts[:rows], start=1):
+        alloc.alloc_seq(sid, n)
+        builder.sched_out(alloc, sid, rng.integers(0, cfg.vocab_size, size=n).astype(np.int32), n - 1)
+    g = torch.Generator(device=device).manual_seed(seed)
+    d, Hkv = cfg.head_dim, cfg.num_key_value_heads
+    caches = [(torch.randn((pool, Hkv, d // 8, 16, 8), generator=g, device=device).to(cfg.dtype),
+               torch.randn((pool, Hkv, d, 16), generator=g, device=device).to(cfg.dtype)) for _ in range(cfg.num_hidden_layers)]
+    return builder.finish().to(device), caches
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [1, 3, 4, 5, 16, 17, 128, 129])
+def test_the_fused_launches_of_a_step_give_the_bits_of_the_separate_ones(device, monkeypatch, dtype, rows):
+    """Norms inside projections (up to 4 rows), rotary and cache writes inside the projection of q, k and v (up to 128), residual and norm in
+    the launch that adds a projection's ranges up (17 to 128) and behind a library GEMM (129 and more): logits and caches of a whole
+    step against the step that makes every call by itself."""
+    cfg = make_cfg(dtype)
+    model = llama.Llama(cfg, llama.random_weights(cfg, seed=7, std=0.04), device)
+    batch, caches = decode_step(cfg, device, np.random.default_rng(rows).integers(1, 200, size=rows).tolist())
+    apart = [(k.clone(), v.clone()) for k, v in caches]
+    got = model.forward(batch, caches, fused=True)
+    model.fused_norm = False
+    monkeypatch.setattr(kernels, "add_rms_norm_takes", lambda *a: False)
+    want = model.forward(batch, apart, fused=False)
+    assert not torch.isnan(got).any()
+    assert torch.equal(got, want)
+    for a, b in zip(caches, apart):
+        assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_a_row_has_the_same_logits_in_steps_of_every_route(device, dtype):
+    """The first sequences of a step of 128 alone in steps of fewer rows, which take other launches for their norms and projections: the same
+    bits.  (Contexts of one block: how paged decode cuts a longer one depends on the batch.  The step of 128 rows asks for 48 rows' logits:
+    beyond them the product with the vocabulary may be a library GEMM's.)"""
+    cfg = make_cfg(dtype)
+    cfg.vocab_size = 3008
+    model = llama.Llama(cfg, llama.random_weights(cfg, seed=8, std=0.04), device)
+    contexts = np.random.default_rng(4).integers(1, 17, size=128).tolist()
+    seen = {}
+    for rows in (1, 2, 4, 5, 16, 17, 48, 128):
+        step, caches = decode_step(cfg, device, contexts, rows)
+        if rows == 128:
+            step.logit_idxs = step.logit_idxs[:48].contiguous()
+        seen[rows] = model.forward(step, caches, fused=True)
+    assert not torch.isnan(seen[48]).any()
+    for rows, got in seen.items():
+        n = min(rows, 48)
+        assert torch.equal(got[:n], seen[48][:n]), rows
+
+
+@pytest.mark.parametrize("heads", [1, 4])
+def test_a_step_over_caches_with_another_number_of_heads_is_refused(device, heads):
+    cfg = make_cfg(torch.bfloat16)
+    model = llama.Llama(cfg, llama.random_weights(cfg, seed=9, std=0.04), device)
+    batch, caches = decode_step(cfg, device, [20, 5, 33])
+    bad = [(torch.zeros((k.size(0), heads, *k.shape[2:]), dtype=k.dtype, device=device),
+            torch.zeros((v.size(0), heads, *v.shape[2:]), dtype=v.dtype, device=device)) for k, v in caches]
+    with pytest.raises(HipAttnError):
+        model.forward(batch, bad, fused=True)
+    assert not any(t.any() for kv in bad for t in kv)
