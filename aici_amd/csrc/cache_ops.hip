@@ -526,7 +526,7 @@ __global__ __launch_bounds__(256) void rotary_cache_group_kernel(const Pos *__re
                                                                  T *__restrict__ key_cache, T *__restrict__ value_cache,
                                                                  const Slot *__restrict__ slot_mapping, CacheGeom g,
                                                                  int64_t tokens) {
-  __shared__ uint16_t rows[kGroupTokens * (kGroupHead + 2)];
+  __shared__ __align__(16) uint16_t rows[kGroupTokens * (kGroupHead + 2)];  // (written two at a time)
   const int tid = threadIdx.x;
   const int64_t t0 = (int64_t)blockIdx.x * kGroupTokens;
   const int n = (int)min((int64_t)kGroupTokens, tokens - t0);
