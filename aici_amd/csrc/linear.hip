@@ -3,7 +3,7 @@
 // `linear_no_bias`, llm/mod.rs:401-407; phi.rs:70-71, 99, 116-117 through `linear`, mod.rs:409-416), where every
 // element of W is used once per row of x and the time goes into reading W from HBM exactly once.
 //
-// Both kernels copy W and x global -> LDS (global_load_lds_dwordx4, no registers) into a ring of stages of 64 values
+// The kernels copy W and x global -> LDS (global_load_lds_dwordx4, no registers) into a ring of stages of 64 values
 // of k: an instruction brings 128 whole bytes of eight rows, its runs of 16 bytes swizzled by the row's low bits so that the
 // operands of v_mfma_f32_16x16x32 are read from LDS without bank conflicts.  What bounds them is how many whole
 // cache lines are on their way: the same loop with W loaded straight into the operands (16 rows x 64 bytes per instruction, so
@@ -13,6 +13,7 @@
 //   linear_stream_kernel, up to 16 rows of x: a wavefront owns 16 (or 64) rows of W and keeps a private ring, its own copy of
 //   the rows of x in it, so nothing waits for anything but the wavefront's own copies; wavefronts that share rows of W
 //   take different ranges of k and meet once, in LDS, at the end.
+//   norm_linear_kernel, up to 4 rows with the RMS norm in front: the rows are held in LDS whole and normalised there, the ring is W's alone.
 //   linear_tile_kernel, 17 to 128 rows: the copies of x are shared by the workgroup (one barrier per stage); ranges of k
 //   go to workgroups of their own, which leave fp32 sums for a second launch to add up.
 //
