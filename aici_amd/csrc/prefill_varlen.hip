@@ -560,14 +560,18 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
   // Q operands: lane (g, c) holds q[row c][16 ks + 8 g .. + 8] for every contraction step ks.  Read in
   // that shape an instruction touches 32 bytes of 32 rows; instead the rows are read whole (16 lanes x
   // 16 bytes per row, 4 rows per instruction) and turned through a private piece of LDS buffers 1 and 2,
-  // which no tile reaches before the first barrier.  (With four wavefronts no such piece is left beside tiles 0 and 1: they do read
-  // it in that shape, while other workgroups work.)
+  // which no tile reaches before the first barrier.  With four wavefronts, whose stages leave less room, only head sizes above 96 do so,
+  // half of the columns at a time through the place of the values of tile 1, without padding (runs change places instead).  us, operand
+  // shape / turned: 32 / 8 heads of 128, 64 x 30..300 tokens 70 / 67, 32 x 1024 395 / 373, 1 x 8000 522 / 496; at 80, where a half row is not
+  // whole lines, turned 66 -> 78, at 64 +-1 %.
   constexpr int QSTR = HDP + 8;  // row pitch of the turned Q tile, elements
   // The alternating-block forms turn Q through stages 2.., so that tiles 0 and 1 can be on their way meanwhile.
-  constexpr int Q_STAGE0 = PINGPONG ? 2 : 1;
-  constexpr bool Q_VIA_LDS = (size_t)NW * 32 * QSTR <= (size_t)(NST - Q_STAGE0) * STAGE_ELEMS;
-  constexpr int CPRQ = HDP / 8;
-  constexpr int NQL = (32 * CPRQ + 63) / 64;
+  constexpr int Q_STAGE0 = PINGPONG && NST > 2 ? 2 : 1;
+  constexpr bool Q_VIA_LDS = NW == 4 ? HDP == 128 : (size_t)NW * 32 * QSTR <= (size_t)(NST - Q_STAGE0) * STAGE_ELEMS;
+  constexpr int Q_PARTS = NW == 4 && Q_VIA_LDS ? 2 : 1;
+  constexpr int CPRQ = HDP / 8 / Q_PARTS;          // 16-byte runs of a row in a part
+  constexpr int NQL1 = (32 * CPRQ + 63) / 64;      // loads per part
+  constexpr int NQL = Q_PARTS * NQL1;
   vec8 qreg[KSTEPS];
   u32x4_t qraw[Q_VIA_LDS ? NQL : 1];
   // The loads of Q (the workgroup's longest wait: nothing else has touched these rows) ...
@@ -575,15 +579,18 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
     if constexpr (Q_VIA_LDS) {
 #pragma unroll
       for (int it = 0; it < NQL; it++) {
-        const int idx = min(it * 64 + lane, 32 * CPRQ - 1);
-        const int r = idx / CPRQ, ch = idx % CPRQ;
+        const int idx = min(it % NQL1 * 64 + lane, 32 * CPRQ - 1);
+        const int r = idx / CPRQ, ch = idx % CPRQ + it / NQL1 * CPRQ;
         const int row = min(wave_row0 + r, Lq - 1);
         qraw[it] = u32x4_t{0u, 0u, 0u, 0u};
         // (Q is read once and the output written once: with the non-temporal hint they do not displace the
         // K / V tiles that the other row blocks of the sequence are about to fetch from L2 -- 8 x 4096 tokens
-        // 1.066 -> 1.051 ms from rows, 1.040 -> 1.019 ms from the paged cache; 16 x 1024 tokens 193 -> 188 us)
-        if (ch < d_chunks)
-          qraw[it] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(qp + (int64_t)row * p.q_row + ch * 8));
+        // 1.066 -> 1.051 ms from rows, 1.040 -> 1.019 ms from the paged cache; 16 x 1024 tokens 193 -> 188 us.  Not
+        // with four wavefronts: 64 x 30..300 tokens 67 -> 73 us, 128 x 256 188 -> 178)
+        if (ch < d_chunks) {
+          const u32x4_t *run = reinterpret_cast<const u32x4_t *>(qp + (int64_t)row * p.q_row + ch * 8);
+          qraw[it] = NW == 4 ? *run : __builtin_nontemporal_load(run);
+        }
       }
     } else {
       const int row = min(wave_row0 + c, Lq - 1);
@@ -598,7 +605,20 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
   };
   // ... and their way through LDS into the operand registers.
   auto q_finish = [&]() {
-    if constexpr (Q_VIA_LDS) {
+    if constexpr (NW == 4 && Q_VIA_LDS) {
+      T *qst = smem + Q_STAGE0 * STAGE_ELEMS + K_ELEMS + wave * (32 * CPRQ * 8);
+#pragma unroll
+      for (int part = 0; part < Q_PARTS; part++) {
+#pragma unroll
+        for (int it = 0; it < NQL1; it++) {
+          const int idx = it * 64 + lane, r = idx / CPRQ, ch = idx % CPRQ;
+          *reinterpret_cast<u32x4_t *>(qst + (r * CPRQ + (ch ^ (r & 7))) * 8) = qraw[part * NQL1 + it];
+        }
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS / Q_PARTS; ks++)
+          qreg[part * (KSTEPS / Q_PARTS) + ks] = *reinterpret_cast<const vec8 *>(qst + (c * CPRQ + ((2 * ks + g) ^ (c & 7))) * 8);
+      }
+    } else if constexpr (Q_VIA_LDS) {
       T *qst = smem + Q_STAGE0 * STAGE_ELEMS + wave * (32 * QSTR);
 #pragma unroll
       for (int it = 0; it < NQL; it++) {
@@ -970,12 +990,12 @@ __global__ __launch_bounds__(NW * 64, w8_wavefronts(HDP, NW)) void prefill_varle
       else
         dma_tile(1);
     }
-    clear_image_tails(0, 1);
+    clear_image_tails(0, Q_STAGE0 - 1);
     q_finish();
     if (n_tiles > 0) dma_wait(0, NST > 2 && n_tiles > 1);
     __syncthreads();
     if (NST > 3 && n_tiles > 2) dma_tile(2);
-    clear_image_tails(2, NST - 1);  // seen by all after the barrier in front of the loop
+    clear_image_tails(Q_STAGE0, NST - 1);  // seen by all after the barrier in front of the loop
   } else if constexpr (ROWS) {
     if (n_tiles > 0) {
       k_rows_dma(0);
@@ -1462,28 +1482,27 @@ void launch_prefill_nw(PrefillParams p, int hl, hipStream_t stream) {
 // compute unit to itself); two wavefronts of one workgroup that alternate between the pipes need less time per key.  us, eight / four, rows
 // of k / v (the paged cache within 5 % of the same ratios), by sequences x lengths:
 //                     16 q / 2 kv x 64   32 / 32 x 80    32 / 8 x 128    32 / 32 x 128
-//   64 x 30..300        33 / 25           114 / 65         84 / 71         122 / 96
-//   24 x 40..700        37 / 31            96 / 72         87 / 81         104 / 93
-//   32 x 512            54 / 42           127 / 99        132 / 119        142 / 149
-//   32 x 1024          144 / 114          346 / 329       361 / 382        410 / 424
-//   16 x 2048          214 / 196          533 / 526       593 / 638        645 / 679
-//   4 x 512           13.8 / 12.3        20.2 / 20.2     18.7 / 21.3      21.2 / 22.1
+//   64 x 30..300        33 / 25           114 / 65         84 / 67         121 / 93
+//   24 x 40..700        37 / 31            96 / 72         88 / 79         104 / 92
+//   32 x 512            54 / 42           127 / 99        132 / 117        139 / 147
+//   32 x 1024          144 / 114          346 / 329       365 / 373        417 / 419
+//   16 x 2048          214 / 196          533 / 526       583 / 621        653 / 683
+//   4 x 512           13.8 / 12.3        20.2 / 20.2     18.8 / 19.9      21.3 / 22.2
 //   2 x 2048            39 / 44            65 / 76
-//   2 x 4096            91 / 109          222 / 231       259 / 284        278 / 296
-//   1 x 300           10.0 / 9.1         11.3 / 11.0     14.0 / 12.5      12.5 / 11.9
-//   32 x 20..100 + 500 17.0 / 17.7         69 / 55         43 / 46          79 / 63
+//   2 x 4096            91 / 109          222 / 231       266 / 277        277 / 289
+//   1 x 300           10.0 / 9.1         11.3 / 11.0     14.0 / 12.2      12.5 / 12.0
+//   32 x 20..100 + 500 17.0 / 17.7         69 / 55         43 / 44          79 / 62
 //   8 x 512 + 2048      53 / 59           131 / 148
-// Over 190 such sizes of each of nine kinds of heads these lines cost 0.8 % on average against the better form of each, all four 1.3 % (2.7 % at
-// head sizes above 96), all eight 10 % (5 %).
+// Over 170 such sizes of each of nine kinds of heads, from both places, these lines cost 0.8 % on average against the better form of each (0.5 %
+// at head sizes above 96), all four 1.2 % (1.8), all eight 11 % (7).
 bool four_wavefronts_pay(const PrefillParams &p, int hdp, int heads) {
   const int64_t wgs = (p.total_q / (256 / heads) + p.batch / 2) * (p.Hq / heads);
   const int64_t keys = p.max_k > p.max_q ? p.max_k : p.total_q / p.batch;
   // Three workgroups to a compute unit.  Long contexts whose workgroups of eight are one round over 256 compute units (with two or three
   // sequences up to two rounds: a sequence's heavy row blocks then meet the next one's on the same compute units) stay with eight.
   if (hdp <= 96) return !(p.batch > 1 && keys >= 1000 && wgs > 250 && wgs <= (p.batch <= 3 ? 560 : 320));
-  // Two: where eight leave many compute units without work, and where there is more than a round of them and contexts are short.
-  if (wgs <= 220) return wgs <= 160 && keys <= 1900;
-  return keys <= (wgs < 400 ? 500 : 640);
+  // Two: where eight leave compute units without work, and where there are more of them and contexts are short.
+  return keys <= (wgs <= 220 ? 1900 : 800);
 }
 
 template <typename T, int HDP, int MODE = W8_ROWS>

@@ -489,7 +489,7 @@ def test_the_form_of_the_workgroups(device, tuning, kernel_choice):
         for heads, seqs, lq, prior, n in (((16, 2, 64), 32, 300, 0, 4), ((16, 2, 64), 2, 4096, 0, 8), ((16, 2, 64), 1, 4096, 0, 4),
                                           ((16, 2, 64), 2, 1000, 0, 4), ((16, 2, 64), 4, 4096, 0, 4), ((16, 2, 64), 8, 512, 2048, 8),
                                           ((32, 32, 80), 32, 1024, 0, 4), ((32, 32, 80), 2, 2048, 0, 8),
-                                          ((32, 8, 128), 32, 512, 0, 4), ((32, 8, 128), 32, 1024, 0, 8), ((32, 8, 128), 4, 512, 0, 8),
+                                          ((32, 8, 128), 32, 512, 0, 4), ((32, 8, 128), 32, 1024, 0, 8), ((32, 8, 128), 4, 1024, 0, 8),
                                           ((32, 8, 128), 1, 1024, 0, 4), ((32, 8, 128), 1, 128, 2048, 8), ((32, 8, 128), 48, 64, 500, 4),
-                                          ((32, 8, 128), 48, 64, 700, 8)):
+                                          ((32, 8, 128), 48, 64, 800, 8)):
             assert wavefronts(*heads, seqs, lq, prior, paged) == n, (heads, seqs, lq, prior, paged)
