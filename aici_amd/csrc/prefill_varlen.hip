@@ -454,7 +454,8 @@ __global__ __launch_bounds__(256) void prefill_varlen_kernel(PrefillParams p) {
 // a wavefront of each.  The alternation of the two pipes is left to chance; what it gains is that a workgroup's set-up and wind-down (block
 // ids, Q, the first tile; the output) pass while the others work.  Same tiles, same order of the same operations: a row has the same bits
 // in either form, so the form may follow the sizes of the whole batch (four_wavefronts_pay).  Tiles of 32 keys, which let three
-// workgroups on a compute unit at head size 128 too (64 x 30..300 tokens 71 -> 59 us, 32 / 8 heads), give other last bits: not kept.
+// workgroups on a compute unit at head size 128 too (64 x 30..300 tokens 67 -> 60 us, 32 / 8 heads), give other last bits: not kept.  Three
+// with tiles of 64 (one place for the values, a second barrier, 168 registers) keep part of Q in scratch memory: 67 -> 86 us.
 // ---------------------------------------------------------------------------
 // Where the eight-wavefront kernel takes its K/V tiles from.
 enum { W8_ROWS = 0, W8_PAGED = 1, W8_PAGED_DMA = 2, W8_PAGED_DMA_PART = 3 };

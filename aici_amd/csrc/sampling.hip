@@ -544,7 +544,8 @@ __device__ __forceinline__ bool sample_counted(const SampleParams &p, Scratch &s
 // us, 128256 tokens, 5 % allowed, top-p 0.9, one workgroup / pieces: 1 row 38.3 / 15.4, 32 rows 42.7 / 19.8, 128 rows 44.6 / 25.9 (12 of
 // them the count, which moves 52 MB with its counters, 13 the row's part: a chain of barriers and instructions on one compute
 // unit), 256 rows 48.1 / 36.9; all allowed without a cut, 128 rows, 70.6 / 35.6.  Pieces from 24576 tokens on: 20000 tokens, 256 rows, no
-// cut 28.5 / 29.6 (with a cut 25.0 / 19.9), 32000 tokens 32.0 / 30.9 (26.4 / 21.2).  Only what is not all zero written and read of the
+// cut 28.5 / 29.6 (with a cut 25.0 / 19.9), 32000 tokens 32.0 / 30.9 (26.4 / 21.2).  A batch of greedy rows alone, which the host cannot
+// know, pays for the first launch: 128 rows 16.4 / 18.0.  Only what is not all zero written and read of the
 // counters: 0.7 us less in the count, 0.7 more in the row's part.
 constexpr int kPieceTokens = 16384;  // no counter above 16 bits
 constexpr int kCountThreads = 512;   // four workgroups per compute unit, by LDS and by wavefronts
