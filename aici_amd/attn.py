@@ -63,6 +63,17 @@ class RmsNorm:
         return out
 
 
+def _reads_through_tables(q: torch.Tensor, batch_info: BatchInfo, key_cache: torch.Tensor, value_cache: torch.Tensor) -> bool:
+    """Whether the context of the multi-token rows need not be gathered (us, gathered / through the tables, 32 heads of 80: 120 decode rows
+    of 1k..8k tokens beside 4 x 512 new ones over up to 3072 1012 / 920, 15 rows of 253 beside 4 x 65..263 103 / 39)."""
+    tables = batch_info.multi_block_tables
+    return (batch_info.q_multi > 0 and tables is not None and tables.size(1) * 16 >= batch_info.max_seqlen_k and q.size(2) in (64, 80, 96, 112, 128)
+            and q.dtype in (torch.float16, torch.bfloat16) and key_cache.dtype == q.dtype and value_cache.dtype == q.dtype
+            and key_cache.dim() == 5 and value_cache.dim() == 4 and key_cache.size(3) == 16 and value_cache.size(3) == 16
+            and key_cache.is_contiguous() and value_cache.is_contiguous()
+            and key_cache.data_ptr() % 16 == 0 and value_cache.data_ptr() % 16 == 0)
+
+
 def varlen_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, batch_info: BatchInfo, key_cache: torch.Tensor,
                 value_cache: torch.Tensor, softmax_scale: Optional[float] = None,
                 paged_prefill: bool = False, cached: bool = False) -> torch.Tensor:
@@ -70,16 +81,16 @@ def varlen_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, batch_info: B
     already (kernels.rotary_embedding_and_cache) and the scatter is skipped.
 
     batch_info must already live on the GPU.  The whole composition (scatter,
-    gather, varlen prefill rows, paged decode rows) is one C-ABI call.  With
-    `paged_prefill` the multi-token rows read their context from the cache
-    through block tables instead of a gathered copy (needs the builder's
-    multi_block_tables)."""
+    varlen prefill rows, paged decode rows) is one C-ABI call.  The multi-token
+    rows read their context from the cache through block tables, or, where the
+    caches are not what that takes, from a gathered copy; with `paged_prefill`
+    always through the tables (needs the builder's multi_block_tables)."""
     T, Hq, d = q.shape
     Hkv = k.size(1)
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(d)
     y = torch.empty((T, Hq, d), dtype=q.dtype, device=q.device)
-    if paged_prefill:
+    if paged_prefill or _reads_through_tables(q, batch_info, key_cache, value_cache):
         if batch_info.multi_block_tables is None:
             raise ValueError("paged_prefill needs batch_info.multi_block_tables (slots must follow the blocks in order)")
         has_m, has_p = batch_info.q_multi > 0, batch_info.q_multi < T

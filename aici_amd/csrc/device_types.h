@@ -134,4 +134,9 @@ __device__ __forceinline__ float block_sum(float v, float *smem /* >= 17 floats 
   return smem[16];
 }
 
+constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kLn2 = 0.6931471805599453f;
+
+__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+
 }  // namespace hipattn

@@ -11,9 +11,6 @@
 
 namespace hipattn {
 
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kLn2 = 0.6931471805599453f;
-
 struct PrefillParams {
   const void *q, *k, *v;
   void *out;
@@ -66,8 +63,6 @@ struct Mfma32<bf16_t> {
   }
 };
 
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-
 // A pointer that is the same in every lane, as the scalar it is: an "s" operand of inline asm is not made one
 // when the compiler holds the value in vector registers.
 template <typename P>
@@ -100,6 +95,26 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
   asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
+
+// log2 of the query heads per workgroup, at most `most`: the largest power of two up to four (or up to the tuning switch prefill_wg_heads,
+// when that is set) that divides the GQA ratio.
+inline int prefill_heads_log2(const PrefillParams &p, int most) {
+  int hl = 0;
+  const int limit = tuning().prefill_wg_heads > 0 ? tuning().prefill_wg_heads : 4;
+  while (hl < most && p.G % (2 << hl) == 0 && (2 << hl) <= limit) hl++;
+  return hl;
+}
+
+// What hipattn_mha_varlen_fwd_paged checks of its arguments and makes of them; false: nothing to do.
+struct PagedPrefillCall {
+  const hipattn_tensor *q, *key_cache, *value_cache, *block_tables, *cu_q, *context_lens;
+  int max_q, max_k;
+  float scale;
+  bool causal;
+};
+bool paged_prefill_params(const PagedPrefillCall &c, hipattn_tensor *out, hipattn_tensor *lse, PrefillParams &p);
+// Whether the blocks of the caches can go into LDS as they are (16-token blocks, 16-byte aligned images, and no switch against it).
+bool paged_prefill_copies_images(const PrefillParams &p);
 
 // Launches the kernel that rotates three groups of wavefronts through the matrix pipe (prefill_r3.hip) when it
 // covers the shapes in p; returns false, having done nothing, when it does not.

@@ -9,7 +9,7 @@
 namespace hipattn {
 
 // Which op a library-owned scratch buffer belongs to: ops never share one.
-enum WorkspaceUser { WS_PAGED_ATTENTION = 0, WS_BIAS_ARGMAX = 1, WS_LINEAR = 2, WS_SAMPLE = 3 };
+enum WorkspaceUser { WS_PAGED_ATTENTION = 0, WS_BIAS_ARGMAX = 1, WS_LINEAR = 2, WS_SAMPLE = 3, WS_STEP_ATTENTION = 4 };
 
 // Returns at least `bytes` of device memory on the current device for `user`,
 // private to `stream`: calls on different streams never share a buffer, so

@@ -851,7 +851,12 @@ char *hipattn_varlen_attn(
  * context from the cache through multi_block_tables int32 [num_multi, cols] and
  * multi_context_lens int32 [num_multi] (hipattn_mha_varlen_fwd_paged).  No
  * counterpart in the reference, which always gathers (mod.rs:181-197).  Head
- * sizes up to 256. */
+ * sizes up to 256.  Steps of f16 / bf16 over 16-token blocks with head sizes
+ * 64, 80, 96, 112 or 128 take one launch for both kinds of rows and one that
+ * merges partial results, where that is faster: its 64 MiB of scratch memory
+ * are allocated once per stream.  Under capture, on hipStreamPerThread and
+ * where there is no such memory the two go by themselves, as
+ * hipattn_mha_varlen_fwd_paged and hipattn_paged_attention_v1 would. */
 char *hipattn_varlen_attn_paged(
     const hipattn_tensor *q, const hipattn_tensor *k, const hipattn_tensor *v,
     hipattn_tensor *key_cache, hipattn_tensor *value_cache,

@@ -2,6 +2,7 @@
 builder: a mixed continuous-batching step with prefill chunks that have prior context in the
 paged cache plus single-token decode rows, against the oracle pipeline that rLLM's CPU build
 runs (scatter -> gather -> repeat_kv -> varlen SDPA for every row)."""
+import dataclasses
 import math
 
 import numpy as np
@@ -204,3 +205,100 @@ def test_config4_full_size_sampled(device, layout, paged_prefill):
         want = torch.einsum("ht,thd->hd", w, vv.double())
         worst = max(worst, (y[row].cpu().double() - want).abs().max().item())
     assert worst <= TOL[dtype], worst
+
+
+STEPS = {  # heads, type, cached tokens in front of each chunk, tokens per chunk, decode rows and their contexts; whether it is one launch
+    "gqa": ((32, 8, 128), torch.bfloat16, [0, 640, 1000, 2048], 33, 9, 1, 600, True),                 # pieces; a row block and a row
+    "mha": ((32, 32, 80), torch.float16, [255, 0, 256, 257, 1500], 129, 5, 16, 300, True),            # one head a workgroup
+    "tile_edges": ((16, 2, 64), torch.float16, [64 * 15 - 32, 64 * 15 - 31, 64 * 15 - 33], 32, 3, 31, 33, True),
+    "ratio_2": ((16, 8, 96), torch.bfloat16, [1300, 40], 2, 40, 1, 2000, True),                       # decode shares end inside contexts
+    "ratio_3": ((12, 4, 112), torch.float16, [900, 0, 450], 70, 17, 500, 900, True),
+    "two_column_groups": ((20, 1, 64), torch.bfloat16, [700, 1], 50, 6, 1, 1500, True),
+    "many_chunks": ((8, 2, 128), torch.bfloat16, [300 + i for i in range(70)], 2, 2, 10, 50, True),   # more than a wavefront finds at once
+    "chunks_alone": ((32, 8, 128), torch.float16, [3000, 100, 0], 20, 0, 1, 1, True),
+    "short": ((32, 8, 128), torch.bfloat16, [0, 100], 20, 4, 10, 200, False),
+    "block_8": ((32, 8, 128), torch.bfloat16, [0, 1000], 20, 4, 10, 200, False),
+}
+
+
+def launched(call):
+    call()
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        out = call()
+        torch.cuda.synchronize()
+    return out, [e.key for e in prof.key_averages()]
+
+
+@pytest.mark.filterwarnings("ignore:Profiler clears events")
+@pytest.mark.parametrize("name", STEPS)
+def test_chunks_and_decode_rows_in_one_launch(device, monkeypatch, tuning, name):
+    """The launch that holds both kinds of rows against the oracle, against the launches by themselves (a switch that asks for one of
+    their kernels), and under an understated bound on the keys."""
+    (Hq, Hkv, d), dtype, priors, new, rows, lo, hi, together = STEPS[name]
+    bs = 8 if name == "block_8" else 16
+    pool = sum(p + new + 2 * bs for p in priors) // bs + rows * (hi // bs + 2) + 8
+    routes = {}
+
+    def run(q, k, v, batch, kc, vc, **kw):
+        def call():
+            return attn_call(q, k, v, batch, kc, vc, **kw)
+
+        y, kernels = launched(call)
+        routes["one"] = (y, any("step_merge_kernel" in n for n in kernels))
+        short = batch.max_seqlen_k
+        batch.max_seqlen_k = max(short - 200, 0)
+        routes["understated"] = call()
+        batch.max_seqlen_k = short
+        tuning("decode_flat", 0)
+        y, kernels = launched(call)
+        routes["apart"] = (y, any("step_merge_kernel" in n for n in kernels))
+        return routes["one"][0]
+
+    attn_call = attn.varlen_attn
+    monkeypatch.setattr(attn, "varlen_attn", run)
+    y, want, _, _ = mixed_step(40, priors, new, rows, lo, hi, Hq, Hkv, d, dtype, pool, False, device, paged_prefill=bs == 8, bs=bs)
+    assert routes["one"][1] == together and not routes["apart"][1]
+    for got in (y, *(r.cpu().reshape(y.shape) for r in (routes["understated"], routes["apart"][0]))):
+        assert not torch.isnan(got.float()).any()
+        assert (got.float() - want).abs().max().item() <= TOL[dtype]
+
+
+def test_a_captured_step_takes_the_launches_by_themselves(device):
+    """A graph holds no pointer into the buffer of the combined launch: replays, with eager steps between them, against the eager result."""
+    (Hq, Hkv, d), dtype, priors, new, rows, lo, hi, _ = STEPS["gqa"]
+    got = {}
+
+    def run(q, k, v, batch, kc, vc, **kw):
+        def call():
+            return attn_call(q, k, v, batch, kc, vc, **kw)
+
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            got["eager"] = call()
+            attn_call(q[batch.q_multi:], k[batch.q_multi:], v[batch.q_multi:], decode_rows(batch), kc, vc)  # decode's own scratch memory
+            side.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                out = call()
+            for _ in range(3):
+                out.zero_()
+                graph.replay()
+                assert (out - got["eager"]).abs().max().item() <= TOL[dtype]
+                assert torch.equal(call(), got["eager"])
+        torch.cuda.current_stream().wait_stream(side)
+        return got["eager"]
+
+    def decode_rows(batch):
+        alone = dataclasses.replace(batch, q_multi=0, seqlen_multi=0, slot_mapping=batch.slot_mapping[batch.q_multi:].contiguous())
+        return alone
+
+    attn_call = attn.varlen_attn
+    mp = pytest.MonkeyPatch()
+    mp.setattr(attn, "varlen_attn", run)
+    try:
+        y, want, _, _ = mixed_step(41, priors, new, rows, lo, hi, Hq, Hkv, d, dtype, 2000, False, device)
+    finally:
+        mp.undo()
+    assert (y.float() - want).abs().max().item() <= TOL[dtype]
