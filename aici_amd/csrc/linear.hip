@@ -10,26 +10,26 @@
 // every line asked for twice, and both copies of it held in the 32 KB L1) reached 5.1 TB/s on a 28672 x 4096 weight and one row of x,
 // 4.0 with sixteen; this form 5.9 and 5.4 (library GEMM: 4.0 / 3.9).
 //
-//   linear_stream_kernel, up to 16 rows of x: a wavefront owns 16 (or 64) rows of W and keeps a private ring, its own copy of
-//   the rows of x in it, so nothing waits for anything but the wavefront's own copies; wavefronts that share rows of W
-//   take different ranges of k and meet once, in LDS, at the end.
+//   linear_stream_kernel, up to 16 rows of x and a weight whose k is cut into ranges: a wavefront owns 16 rows of W and keeps a private
+//   ring, its own copy of the rows of x in it, so nothing waits for anything but the wavefront's own copies; wavefronts that share
+//   rows of W take different ranges of k and meet once, in LDS, at the end.
 //   norm_linear_kernel, up to 4 rows with the RMS norm in front: the rows are held in LDS whole and normalised there, the ring is W's alone.
-//   linear_tile_kernel, 17 to 128 rows: the copies of x are shared by the workgroup (one barrier per stage); ranges of k
+//   linear_tile_kernel, 17 to 128 rows, fewer where k is not cut: the copies of x are shared by the workgroup (one barrier per stage); ranges of k
 //   go to workgroups of their own, which leave fp32 sums for a second launch to add up.
 //
 // The ranges of k are a function of the weight's shape alone, every range is summed front to back and the ranges are
 // added up first to last: a row gets the same bits whichever kernel, launch shape and company it is computed in, and
-// on every run (no atomics).
+// on every run (no atomics).  Front to back: from a stage of the range on that follows from the row of W, and round (StageOrder).
 //
 // Microseconds (bf16, copies of W in turns so that no cache holds it; library GEMM -> here):
 //                       1 row          16 rows        32 rows        64 rows        128 rows
 //   4096 x 4096         22.8 -> 7.7    20.8 -> 8.2    21.1 -> 11.3   21.1 -> 12.2   24.2 -> 16.1
 //   6144 x 4096         20.8 -> 10.9   19.8 -> 12.7   19.8 -> 14.5   19.6 -> 16.6   25.3 -> 21.3
 //   4096 x 14336        25.6 -> 19.2   25.8 -> 22.7   30.8 -> 24.9   38.9 -> 27.0   75.3 -> 31.4
-//   28672 x 4096        58.8 -> 40.1   59.8 -> 43.7   51.2 -> 43.0   51.4 -> 47.2   53.9 -> 53.1
-//     + silu_and_mul    62.9 -> 41.7   64.2 -> 44.0   56.8 -> 43.1   57.9 -> 49.7   61.0 -> 54.8
-//   128256 x 4096       183 -> 166     186 -> 166     196 -> 186     208 -> 211     232 -> 248
-// (one row of 28672 x 4096 is 5.9 TB/s, 128 rows are 4.4.  At that end every workgroup copies as many bytes of x into LDS as of W and
+//   28672 x 4096        58.8 -> 36.4   59.8 -> 36.8   51.2 -> 38.4   51.4 -> 39.2   53.9 -> 49.3
+//     + silu_and_mul    62.9 -> 36.5   64.2 -> 36.5   56.8 -> 38.5   57.9 -> 39.4   61.0 -> 50.3
+//   128256 x 4096       183 -> 152     186 -> 154     197 -> 161     209 -> 176     233 -> 219
+// (one row of 28672 x 4096 is 6.5 TB/s, 128 rows are 4.8.  At that end every workgroup copies as many bytes of x into LDS as of W and
 // has the compute unit to itself, its start and end open; the reads of x from LDS, eight times the bytes of W, are not what bounds it:
 // a third fewer of them changed nothing.)
 // Narrower weights keep these kernels' lead: 1024 x 4096 13.6 -> 6.4 with one row and 18.3 -> 12.7 with 128 against a kernel that cut them
@@ -82,6 +82,7 @@ struct LinearParams {
   // with an RMS norm behind the layer: the sums go to the workspace as rows ([range][128 rows][N] fp32), and the
   // launch that adds them up also normalises the finished row
   int row_sums;
+  int turned;     // ranges of k begin inside (StageOrder), the order that of a row's place in this many; 0: they do not
   int wide;       // rows of x or W more than 2^28 elements apart
   int tile_sums;  // the sums go to the workspace as tiles, and a second launch finishes them
   const void *norm_w;
@@ -230,6 +231,32 @@ __device__ __forceinline__ void linear_finish_qkv(const LinearParams &p, f32x4_t
   }
 }
 
+// The order in which a wavefront takes the stages of its ranges, one after the other: a range begins at a stage that follows from the
+// rows of W, and wraps round.  Wavefronts that all walk their rows front to back ask for the same bytes of every row at a time, and
+// where rows lie 8 KB apart those are a few of the memory's channels (see LinearPlan::turned).  kTurnRows rows of W share a place, and the
+// two halves of the weight have the same ones (gate and up rows of an output share their copies of x): the order is that of the row,
+// whatever the kernel and the launch.
+constexpr int kTurnRows = 128;
+struct StageOrder {
+  int per_range, stages, turn;
+  int at = 0, end = 0, left = 0, start;
+  // n: a row of the tile
+  __device__ __forceinline__ StageOrder(const LinearParams &p, int n, int stages_)
+      : per_range(p.stages_per_split), stages(stages_), turn(p.turned ? n % p.turned / kTurnRows * 21 : 0), start(-p.stages_per_split) {}
+  __device__ __forceinline__ int next() {
+    if (left == 0) {
+      start += per_range;
+      left = min(per_range, stages - start);
+      at = start + (int)((unsigned)turn % (unsigned)left);
+      end = start + left;
+    }
+    const int st = at;
+    at = at + 1 == end ? start : at + 1;
+    left--;
+    return st;
+  }
+};
+
 template <int N>
 __device__ __forceinline__ void wait_copies() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -296,28 +323,26 @@ __device__ __forceinline__ f32x4_t add_ranges(const f32x4_t *src, int splits) {
   return total;
 }
 
-// Up to 16 rows of x.  WAVES wavefronts; each owns 16 NT rows of W.  GATED: odd wavefronts take the up rows that
+// Up to 16 rows of x.  WAVES wavefronts; each owns 16 rows of W.  GATED: odd wavefronts take the up rows that
 // belong to the gate rows of the wavefront before them.  QKV: rotation and cache writes behind it.
-template <typename T, int NT, int S, int WAVES, bool GATED, bool QKV = false>
+template <typename T, int S, int WAVES, bool GATED, bool QKV = false>
 __global__ __launch_bounds__(WAVES * 64) void linear_stream_kernel(const LinearParams p) {
   using vec8 = typename Vec8<T>::type;
   constexpr int kParts = GATED ? 2 : 1;
-  constexpr int kCopiesW = 2 * NT, kCopiesX = 2, kCopies = kCopiesW + kCopiesX;  // of 1 KB: eight rows each
+  constexpr int kCopiesW = 2, kCopiesX = 2, kCopies = kCopiesW + kCopiesX;  // of 1 KB: eight rows each
   constexpr int kStageBytes = kCopies * 1024;
-  static_assert(NT == 1 || !(GATED || QKV), "gated, q k v: one tile per wavefront");
   __shared__ __align__(1024) char ring[WAVES * S * kStageBytes];
-  // NT > 1 is for weights of so many rows that k is not cut
-  __shared__ f32x4_t sums[NT == 1 ? kParts * kLinMaxRanges * 64 : 1];
+  __shared__ f32x4_t sums[kParts * kLinMaxRanges * 64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, kg = lane >> 4;
-  // wavefronts per tile of 16 NT rows, and the ranges of k each of them takes, one after the other
+  // wavefronts per tile of 16 rows, and the ranges of k each of them takes, one after the other
   const int per_tile = min(p.splits, WAVES / kParts);
   const int ranges = p.splits / per_tile;
   const int part = GATED ? wave & 1 : 0;
   const int tile = (wave / kParts) / per_tile, first_range = ((wave / kParts) % per_tile) * ranges;
   const int tiles = WAVES / kParts / per_tile;
-  const int n_tile = (blockIdx.x * tiles + tile) * 16 * NT;
+  const int n_tile = (blockIdx.x * tiles + tile) * 16;
   const int n_end = GATED ? p.half : p.N;
   const int stage0 = first_range * p.stages_per_split;
   const int nst = max(0, min(ranges * p.stages_per_split, p.total_stages - stage0));
@@ -337,23 +362,23 @@ __global__ __launch_bounds__(WAVES * 64) void linear_stream_kernel(const LinearP
   for (int i = 0; i < kCopiesX; i++) xsrc[i] = copy_source<T, false>(p.x, p.ldx, i * 8, p.M - 1, stage0);
   const char *mine = ring + wave * S * kStageBytes;
   const uint32_t mine_lds = lds_address(ring) + wave * S * kStageBytes;
-  auto ask = [&](int slot, int st) {
+  StageOrder order(p, n_tile, nst);
+  auto ask = [&](int slot) {
+    const int st = order.next();
     const uint32_t at = mine_lds + slot * kStageBytes;
 #pragma unroll
     for (int i = 0; i < kCopiesX; i++) copy_1k<false, false>(at + (kCopiesW + i) * 1024, xsrc[i], st);
 #pragma unroll
     for (int i = 0; i < kCopiesW; i++) copy_1k<true, false>(at + i * 1024, wsrc[i], st);
   };
-  f32x4_t acc[NT];
-#pragma unroll
-  for (int t = 0; t < NT; t++) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const bool meet = GATED || p.splits > 1;
+  f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const bool meet = !QKV || p.splits > 1;
   f32x4_t *range_sums = sums + ((tile * kParts + part) * p.splits + first_range) * 64 + lane;
   int left = p.stages_per_split, range = 0;  // of the range in hand
 
 #pragma unroll
   for (int j = 0; j < S; j++)
-    if (j < nst) ask(j, j);
+    if (j < nst) ask(j);
   for (int base = 0; base < nst; base += S) {
 #pragma unroll
     for (int j = 0; j < S; j++) {
@@ -365,23 +390,19 @@ __global__ __launch_bounds__(WAVES * 64) void linear_stream_kernel(const LinearP
         else
           wait_copies<0>();
         const char *stage = mine + j * kStageBytes;
-        uint4 wf[2][NT], xf[2];
+        uint4 wf[2], xf[2];
 #pragma unroll
         for (int s = 0; s < 2; s++) {
-#pragma unroll
-          for (int t = 0; t < NT; t++) wf[s][t] = *staged_run(stage, t * 16 + col, 4 * s + kg);
+          wf[s] = *staged_run(stage, col, 4 * s + kg);
           xf[s] = *staged_run(stage + kCopiesW * 1024, col, 4 * s + kg);
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage is in registers: its place can be filled again
-        if (st + S < nst) ask(j, st + S);
+        if (st + S < nst) ask(j);
 #pragma unroll
-        for (int s = 0; s < 2; s++)
-#pragma unroll
-          for (int t = 0; t < NT; t++)
-            acc[t] = LinMfma<T>::run(bit_cast<vec8>(wf[s][t]), bit_cast<vec8>(xf[s]), acc[t]);
-        if (NT == 1 && ranges > 1 && --left == 0) {
-          range_sums[range++ * 64] = acc[0];
-          acc[0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < 2; s++) acc = LinMfma<T>::run(bit_cast<vec8>(wf[s]), bit_cast<vec8>(xf[s]), acc);
+        if (ranges > 1 && --left == 0) {
+          range_sums[range++ * 64] = acc;
+          acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
           left = p.stages_per_split;
         }
       }
@@ -393,33 +414,26 @@ __global__ __launch_bounds__(WAVES * 64) void linear_stream_kernel(const LinearP
     if (meet) rows = qkv_rows(p.qkv, blockIdx.x * tiles + wave);
     if (!meet || wave < tiles) turn = qkv_turn<T>(p.qkv, rows, token, kg);
     if (!meet) {
-      linear_finish_qkv<T>(p, acc[0], col, kg, rows, token, turn);
+      linear_finish_qkv<T>(p, acc, col, kg, rows, token, turn);
       return;
     }
   }
-  if (!meet) {
-#pragma unroll
-    for (int t = 0; t < NT; t++) linear_finish<T>(p, acc[t], col, n_tile + t * 16 + 4 * kg);
-    return;
+  for (; range < ranges; range++) {  // what is left of the last range; ranges past the end of k are zero
+    range_sums[range * 64] = acc;
+    acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
-  if constexpr (NT == 1) {
-    for (; range < ranges; range++) {  // what is left of the last range; ranges past the end of k are zero
-      range_sums[range * 64] = acc[0];
-      acc[0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
-    __syncthreads();
-    if (wave < tiles) {
-      const int n = (blockIdx.x * tiles + wave) * 16 + 4 * kg;
-      f32x4_t total[kParts];
+  __syncthreads();
+  if (wave < tiles) {
+    const int n = (blockIdx.x * tiles + wave) * 16 + 4 * kg;
+    f32x4_t total[kParts];
 #pragma unroll
-      for (int q = 0; q < kParts; q++) total[q] = add_ranges(sums + (wave * kParts + q) * p.splits * 64 + lane, p.splits);
-      if constexpr (GATED)
-        linear_finish_gated<T>(p, total[0], total[1], col, n);
-      else if constexpr (QKV)
-        linear_finish_qkv<T>(p, total[0], col, kg, rows, token, turn);
-      else
-        linear_finish<T>(p, total[0], col, n);
-    }
+    for (int q = 0; q < kParts; q++) total[q] = add_ranges(sums + (wave * kParts + q) * p.splits * 64 + lane, p.splits);
+    if constexpr (GATED)
+      linear_finish_gated<T>(p, total[0], total[1], col, n);
+    else if constexpr (QKV)
+      linear_finish_qkv<T>(p, total[0], col, kg, rows, token, turn);
+    else
+      linear_finish<T>(p, total[0], col, n);
   }
 }
 
@@ -476,13 +490,15 @@ __global__ __launch_bounds__(256) void norm_linear_kernel(const LinearParams p) 
                                     part * p.half + n_end - 1, stage0);
   const char *mine = lds + wave * S * kStageBytes;
   const uint32_t mine_lds = lds_address(lds) + wave * S * kStageBytes;
-  auto ask = [&](int slot, int st) {
+  StageOrder order(p, n_tile, nst);
+  auto ask = [&](int slot) {
+    const int st = order.next();
 #pragma unroll
     for (int i = 0; i < 2; i++) copy_1k<true, false>(mine_lds + slot * kStageBytes + i * 1024, wsrc[i], st);
   };
 #pragma unroll
   for (int j = 0; j < S; j++)
-    if (j < nst) ask(j, j);
+    if (j < nst) ask(j);
   if (nst >= S)
     wait_copies<2 * S>();
   else
@@ -535,6 +551,7 @@ __global__ __launch_bounds__(256) void norm_linear_kernel(const LinearParams p) 
   }
   const int xr = min(col, p.M - 1);
   const char *xrow = xrows + xr * pitch + stage0 * (kLinStageK * 2);
+  StageOrder held(p, n_tile, nst);  // the stages as they come out of the ring
   f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
   f32x4_t *range_sums = sums + ((tile * kParts + part) * p.splits + first_range) * 64 + lane;
   int left = p.stages_per_split, range = 0;  // of the range in hand
@@ -548,14 +565,15 @@ __global__ __launch_bounds__(256) void norm_linear_kernel(const LinearParams p) 
         else
           wait_copies<0>();
         const char *stage = mine + j * kStageBytes;
+        const char *xstage = xrow + held.next() * (kLinStageK * 2);
         uint4 wf[2], xf[2];
 #pragma unroll
         for (int s = 0; s < 2; s++) {
           wf[s] = *staged_run(stage, col, 4 * s + kg);
-          xf[s] = *reinterpret_cast<const uint4 *>(xrow + st * (kLinStageK * 2) + ((4 * s + kg) ^ (xr & 7)) * 16);
+          xf[s] = *reinterpret_cast<const uint4 *>(xstage + ((4 * s + kg) ^ (xr & 7)) * 16);
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage is in registers: its place can be filled again
-        if (st + S < nst) ask(j, st + S);
+        if (st + S < nst) ask(j);
 #pragma unroll
         for (int s = 0; s < 2; s++) acc = LinMfma<T>::run(bit_cast<vec8>(wf[s]), bit_cast<vec8>(xf[s]), acc);
         if (ranges > 1 && --left == 0) {
@@ -605,7 +623,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_tile_kernel(const LinearPar
   using vec8 = typename Vec8<T>::type;
   // The read-once hint on W (stream kernel: always) measured 3 to 8 % faster here as well, except on the short ranges that the
   // 64-row workgroups serve with many rows of x (4096 x 4096, 128 rows: 15.6 us without, 17.0 with).
-  constexpr bool kOnce = MT == 2 || WAVES == 8;
+  constexpr bool kOnce = MT <= 2 || WAVES == 8;
   constexpr int kCopiesW = 2;                           // of 1 KB per stage: this wavefront's rows of W
   constexpr int kAllX = 2 * MT, kCopiesX = (kAllX + WAVES - 1) / WAVES;  // all copies of x, this wavefront's share
   constexpr int kCopies = kCopiesW + kCopiesX;
@@ -634,7 +652,9 @@ __global__ __launch_bounds__(WAVES * 64) void linear_tile_kernel(const LinearPar
 #pragma unroll
   for (int i = 0; i < kCopiesX; i++) xsrc[i] = copy_source<T, WIDE>(p.x, p.ldx, ((wave + i * WAVES) % kAllX) * 8, p.M - 1, stage0);
   const uint32_t ring_lds = lds_address(ring);
-  auto ask = [&](int slot, int st) {
+  StageOrder order(p, n_group, nst);
+  auto ask = [&](int slot) {
+    const int st = order.next();
     const uint32_t at = ring_lds + slot * kStageBytes;
 #pragma unroll
     for (int i = 0; i < kCopiesX; i++)
@@ -647,7 +667,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_tile_kernel(const LinearPar
   for (int mt = 0; mt < MT; mt++) acc[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int j = 0; j < S - 1; j++)
-    if (j < nst) ask(j, j);
+    if (j < nst) ask(j);
   for (int base = 0; base < nst; base += S) {
 #pragma unroll
     for (int j = 0; j < S; j++) {
@@ -660,7 +680,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_tile_kernel(const LinearPar
         else
           wait_copies<0>();
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (st + S - 1 < nst) ask((j + S - 1) % S, st + S - 1);
+        if (st + S - 1 < nst) ask((j + S - 1) % S);
         const char *stage = ring + j * kStageBytes;
         const char *wrows = stage + wave * kCopiesW * 1024, *xrows = stage + kCopiesW * WAVES * 1024;
 #pragma unroll
@@ -817,6 +837,7 @@ struct LinearPlan {
   int waves;    // tile kernel: wavefronts per workgroup
   int splits;   // ranges of k
   int stages_per_split;
+  bool turned;  // ranges begin inside (StageOrder)
   size_t partial_bytes;  // fp32 sums of every range, [range][128 rows][N]; not used by the few-rows kernel
 };
 
@@ -831,11 +852,22 @@ LinearPlan plan_linear(int M, int N, int K, bool few_only) {
   while (splits < kLinMaxRanges && (int64_t)N * splits < 16384) splits *= 2;
   while (splits > 1 && splits < kLinMaxRanges && K / splits > 2048) splits *= 2;
   while (splits > stages) splits /= 2;
-  pl.stream = M <= kLinStreamRows;
+  // Where k is not cut, a workgroup's one copy of x: 28672 x 4096 gated, us, stream / tile kernel 1 row 38.4 / 36.4, 16 41.7 / 36.8; 51200 x 2560
+  // 45.4 / 44.9, 52.7 / 48.3; 128256 x 4096 154.8 / 151.5, 156.2 / 153.4.  With ranges the tile kernel needs its second launch: 12288 x
+  // 4096 19.3 / 21.1, 22.5 / 20.6.
+  pl.stream = M <= kLinStreamRows && (few_only || splits > 1);
   if (tn.linear_splits > 0 && !few_only) splits = tn.linear_splits < stages ? tn.linear_splits : stages;
   if ((tn.linear_splits > 0 || tn.linear_waves > 0 || tn.linear_tiles > 0) && !few_only) pl.stream = false;
   pl.splits = splits;
   pl.stages_per_split = (stages + splits - 1) / splits;
+  // Turned ranges, us (21 stages further per 128 rows of W: odd, so that consecutive places differ and all are used): 28672 x 4096
+  // gated 1 / 32 / 128 rows 40.8 -> 38.0 (here 36.5 in the tile kernel), 42.9 -> 38.5, 53.9 -> 50.3, with the norm in front 42.5 -> 38.5;
+  // 128256 x 4096 1 / 32 / 128 rows 162 -> 154, 189 -> 161, 250 -> 219; 16384 x 2048, 6144, 8192, 11008, 14336 15.0 -> 12.8, 40.4 ->
+  // 32.1, 58.5 -> 39.3, 63.8 -> 54.7, 86.9 -> 68.7; in ranges 12288 x 4096 (2) 22.2 -> 19.4, 8192 x 8192 (4) 27.8 -> 21.9.  Nothing to gain where
+  // rows are not so far apart or not by such powers of two (16384 x 1024, 3072, 5120, 20480 x 2560: +-1 %), where shorter ranges already
+  // spread the wavefronts (4096 x 4096, 6144 x 4096, 4096 x 14336: +-1 %, with 128 rows 6144 x 4096 21.0 -> 21.6; 8192 x 28672, eight ranges,
+  // 106 -> 108).
+  pl.turned = N >= 8192 && N % (2 * kTurnRows) == 0 && splits <= 4 && (K % 2048 == 0 || K >= 6144);
   // Workgroups of 64 rows while the device holds all of them at once, one per compute unit, or where 32 rows of x leave the copies of x
   // cheap (28672 x 4096, 32 rows: 43.5 us against 46.3; 64 rows: 49.5 against 47.3); else of 128 rows.
   pl.waves = ((int64_t)((N + 63) / 64) * splits <= 256 || (splits == 1 && M <= 32)) ? 4 : 8;
@@ -899,22 +931,17 @@ void launch_linear(const LinearParams &p, const LinearPlan &pl, hipStream_t stre
     return;
   }
   if (pl.stream) {
-    if (!GATED && !QKV && p.splits == 1 && p.N >= 65536) {
-      // A vocabulary's rows: 512 per workgroup, so that one round of workgroups covers the device (128256 x 4096, 16 rows: 161
-      // us against 182 with 64 rows per workgroup).
-      if constexpr (!GATED)
-        hipLaunchKernelGGL((linear_stream_kernel<T, 4, 2, 8, false>), dim3((p.N + 511) / 512), dim3(512), 0, stream, p);
-    } else {
-      const int parts = GATED ? 2 : 1, n = GATED ? p.half : p.N;
-      const int per_tile = p.splits < 4 / parts ? p.splits : 4 / parts;
-      const int rows = 16 * (4 / parts / per_tile);
-      hipLaunchKernelGGL((linear_stream_kernel<T, 1, 3, 4, GATED, QKV>), dim3((n + rows - 1) / rows), dim3(256), 0, stream, p);
-    }
+    const int parts = GATED ? 2 : 1, n = GATED ? p.half : p.N;
+    const int per_tile = p.splits < 4 / parts ? p.splits : 4 / parts;
+    const int rows = 16 * (4 / parts / per_tile);
+    hipLaunchKernelGGL((linear_stream_kernel<T, 3, 4, GATED, QKV>), dim3((n + rows - 1) / rows), dim3(256), 0, stream, p);
     check_launch("linear (few rows)");
     return;
   }
   if (p.wide)
     launch_tile<T, 8, GATED, true>(p, pl, stream);
+  else if (p.M <= 16)
+    launch_tile<T, 1, GATED>(p, pl, stream);
   else if (p.M <= 32)
     launch_tile<T, 2, GATED>(p, pl, stream);
   else if (p.M <= 64)
@@ -1120,6 +1147,7 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
   }
   p.tile_sums = !pl.stream && !p.row_sums && (pl.splits > 1 || overlap);
   p.splits = pl.splits;
+  p.turned = pl.turned ? (int)(N / 2) : 0;
   p.stages_per_split = pl.stages_per_split;
   p.total_stages = (int)(K / kLinStageK);
   p.half = gated ? (int)(N / 2) : 0;
@@ -1142,6 +1170,8 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
              "qkv_linear: %lld rows of x and a weight of %lld rows; fewer than 65536 of weight, and than 16384 with more than %d rows of x", (long long)M,
              (long long)N, kLinStreamRows);
     p.qkv = qkv_params(*qkv, M, N, dt);
+    // the halves of a head have to share an order (heads of 80, 96, 256, ...: the order without turns, in every form of this call)
+    if (kTurnRows % p.qkv.g.head_size != 0) p.turned = 0;
     dt == HIPATTN_BF16 ? launch_linear<bf16_t, false, true>(p, pl, stream) : launch_linear<half_t, false, true>(p, pl, stream);
     return;
   }

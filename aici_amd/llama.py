@@ -124,9 +124,9 @@ class Llama:
                 and kernels.rms_norm_linear_takes(x, norm_weight, weight))
 
     def _proj(self, x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-        """x @ weight.T (llama.rs:81-83, 210).  A vocabulary's rows with more than 48 sequences stay with the library
-        (128256 x 4096, us, library / C ABI: 48 rows 206 / 203, 64 rows 208 / 211, 128 rows 232 / 248)."""
-        if self.skinny_linear and kernels.linear_takes(x, weight) and (x.size(0) <= 48 or weight.size(0) < 65536):
+        """x @ weight.T (llama.rs:81-83, 210).  (A vocabulary's rows, 128256 x 4096, us, library / C ABI: 32 rows 197 / 161, 64 rows
+        209 / 176, 128 rows 233 / 219.)"""
+        if self.skinny_linear and kernels.linear_takes(x, weight):
             return kernels.linear(x, weight)
         return x @ weight.t()
 

@@ -442,3 +442,62 @@ def test_operands_off_16_byte_boundaries_are_not_taken(device):
     x, w, norm = at(0, 2, 256), at(0, 384, 256), at(0, 256)
     assert not K.rms_norm_linear_takes(x, norm.half(), w) and not K.rms_norm_linear_takes(x, norm[:128], w)
     assert not K.add_rms_norm_takes(x, x.half(), norm) and not K.add_rms_norm_takes(x, x.clone(), norm.float())
+
+
+# Weights whose ranges of k begin inside: 2, 4 and 1 ranges, halves of 33, 32, 65 and 64 groups of rows, ranges of 25 stages; and one that is left.
+TURNED = [(8448, 2048), (8192, 6400), (16640, 2048), (16384, 6400), (16400, 2048)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N,Kd", TURNED)
+def test_ranges_that_begin_inside_give_a_row_the_same_bits_in_every_kernel(device, dtype, N, Kd):
+    x, w, g = operands(128, N, Kd, dtype, seed=N + Kd)
+    xd, wd = x.to(device), w.to(device)
+    whole = K.linear(xd, wd)
+    check(whole[:40], x[:40], w)
+    norm = (1 + 0.2 * torch.randn((Kd,), generator=g)).to(dtype).to(device)
+    h = torch.empty_like(xd)
+    K.rms_norm(h, xd, norm, 1e-5)
+    normed, gated = K.linear(h, wd), K.linear_silu_and_mul(xd, wd) if N % 32 == 0 else None
+    if gated is not None:
+        act = torch.empty_like(gated)
+        K.silu_and_mul(act, whole)
+        assert torch.equal(gated, act)
+    for m in (1, 2, 4, 5, 16, 17, 33, 65, 97):
+        assert torch.equal(K.linear(xd[:m], wd), whole[:m])
+        if gated is not None:
+            assert torch.equal(K.linear_silu_and_mul(xd[:m], wd), gated[:m])
+        if K.rms_norm_linear_takes(xd[:m], norm, wd):
+            assert torch.equal(K.rms_norm_linear(xd[:m], norm, 1e-5, wd), normed[:m])
+    # ranges of uneven lengths
+    for splits in (3, 7):
+        K.tuning_set("linear_splits", splits)
+        check(K.linear(xd[:17], wd), x[:17], w)
+
+
+@pytest.mark.parametrize("heads,same", [((48, 8, 128), True), ((120, 4, 64), True), ((32, 2, 256), False), ((88, 4, 96), False)])
+def test_qkv_linear_of_many_heads(device, heads, same):
+    """Heads that divide the 128 rows that share an order of k: the bits of the calls; others: their own order, the same in every form."""
+    Hq, Hkv, d = heads
+    Kd, M, N = 2048, 40, (Hq + 2 * Hkv) * d
+    x, w, g = operands(M, N, Kd, torch.bfloat16, seed=d)
+    xd, wd = x.to(device), w.to(device)
+    table = torch.randn((64, d), generator=g).to(torch.bfloat16).to(device)
+    caches = [torch.zeros((4, Hkv, d // 8, 16, 8), dtype=torch.bfloat16, device=device),
+              torch.zeros((4, Hkv, d, 16), dtype=torch.bfloat16, device=device)]
+    pos = torch.randint(0, 64, (M,), generator=g).to(device)
+    slots = torch.randperm(64, generator=g)[:M].to(device)
+    assert K.qkv_linear_takes(xd, wd, table, *caches) and N >= 8192
+    first = [c.clone() for c in caches]
+    got = K.qkv_linear(xd, None, 0.0, wd, pos, table, *first, slots)
+    for m in (5, 16, 17):
+        few = [c.clone() for c in caches]
+        assert torch.equal(K.qkv_linear(xd[:m], None, 0.0, wd, pos[:m], table, *few, slots[:m]), got[:m])
+    want, wkc, wvc = K.linear(xd, wd), caches[0].clone(), caches[1].clone()
+    q, k, v = want.split([Hq * d, Hkv * d, Hkv * d], dim=1)
+    K.rotary_embedding_and_cache(pos, q, k, v.view(M, Hkv, d), d, table, True, wkc, wvc, slots)
+    if same:
+        assert torch.equal(got, want) and torch.equal(first[0], wkc) and torch.equal(first[1], wvc)
+    else:
+        check(got[:, (Hq + Hkv) * d:], x, w[(Hq + Hkv) * d:])  # values are not rotated
+        assert ((got - want).float().norm() / want.float().norm()).item() <= 2.0 ** -8
