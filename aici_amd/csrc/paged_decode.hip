@@ -442,21 +442,31 @@ struct DecodePlan {
   size_t bytes = 0;          // scratch memory in all
 };
 
-// Partition length used by v1, in KV blocks: a multiple of 8 (one block pair
-// per wavefront and round).  Measured on MI355X, long partitions win as long
-// as the launch still has a couple of thousand workgroups (fewer fp32
-// partials, fewer start-up bubbles per byte); short contexts or small batches
-// get shorter partitions so that all CUs have work, never below 8 blocks.
+// Partition length used by v1, in KV blocks: a multiple of 8 (one block pair per wavefront and round).  Long steps have some 2048
+// workgroups: fewer fp32 partial results and start-ups per byte, and contexts of different lengths still even out.  With up to 128 (sequence,
+// kv head) pairs partitions are longer: a workgroup's start-up and its partial result cost about what one more round does, so as long as
+// leaves some 320 workgroups, one and a bit per compute unit, up to 32 blocks, and 64 where there are that many several times over.  A
+// whole context of up to 64 blocks where that leaves as many: nothing to merge then (but where a few of them would be left for a
+// last round, 17 x 630 at 32 kv heads 33.0 / 34.7).  Work is counted in blocks of 128 head elements.
+// us, 2048 workgroups wanted / this rule, contexts of that length (uniform from a tenth of it), 32 / 8 heads of 128: 4 x 4096 19.0 / 16.4
+// (18.9 / 14.9), 8 x 2048 18.5 / 16.4 (16.7 / 14.1), 8 x 4096 29.7 / 26.0 (25.9 / 22.0), 16 x 1600 25.0 / 22.7 (19.7 / 19.2), 16 x
+// 2048 29.0 / 25.9 (23.5 / 20.3), 96 x 700 51.7 / 44.2 (36.7 / 31.5); 32 / 32 of 80: 2 x 4096 19.7 / 18.1 (18.7 / 16.5), 16 x 700 23.7 /
+// 20.6 (19.1 / 16.3).  With more pairs: 24 x 1600 31.0 / 31.8 (22.9 / 24.5), 48 x 2048 from 204 on 45.0 / 47.8, 53 x 385..1541 42.6 / 44.6.
 // The tuning switch decode_part_blocks overrides the choice.
-int choose_part_blocks(int64_t S, int Hkv, int col_groups, int max_ctx) {
+int choose_part_blocks(int64_t S, int Hkv, int col_groups, int head_size, int max_ctx) {
   const int forced = tuning().decode_part_blocks;
   if (forced >= 2 && forced <= 64) return forced + (forced & 1);
   const int64_t max_blocks = (max_ctx + kBlockSize - 1) / kBlockSize;
   const int64_t items = S * Hkv * col_groups;  // workgroups per partition index
+  const int64_t work = items * max_blocks * (head_size < 64 ? 64 : head_size) / 128;
   const int64_t want_wgs = 2048;
   int64_t parts = (want_wgs + items - 1) / (items > 0 ? items : 1);
   if (parts < 1) parts = 1;
   int64_t pb = (max_blocks + parts - 1) / parts;
+  if (max_blocks <= 64 && work > 32 * 320 && (items <= 512 || items % 512 == 0 || items % 512 >= 256))
+    pb = 64;
+  else if (items <= 128)
+    pb = std::max(pb, work >= 65536 ? (int64_t)64 : std::min<int64_t>(32, (work + 319) / 320));
   pb = ((pb + 7) / 8) * 8;
   if (pb < 8) pb = 8;
   if (pb > 64) pb = 64;
@@ -489,7 +499,7 @@ DecodePlan plan_decode(int64_t S, int Hq, int Hkv, int head_size, int block_size
       pl.bytes = pl.flat_scratch.bytes;
       return pl;
     } else {
-      pl.part_blocks = choose_part_blocks(S, Hkv, col_groups, max_context_len);
+      pl.part_blocks = choose_part_blocks(S, Hkv, col_groups, head_size, max_context_len);
       const int64_t max_blocks = ((int64_t)max_context_len + kBlockSize - 1) / kBlockSize;
       // A whole context per workgroup of eight wavefronts instead of partitions and their merge.  The merge costs about 3 us;
       // each block pair a wavefront takes after its first costs 2.4 us where only a few compute units run (head size 128; 1.5
@@ -511,7 +521,8 @@ DecodePlan plan_decode(int64_t S, int Hq, int Hkv, int head_size, int block_size
       const int64_t most_wgs = small || partials > kStaticScratchBytes ? 1023 : 512;
       if (tuning().decode_part_blocks <= 0 && head_size <= 128 && max_blocks > pl.part_blocks && wgs <= most_wgs && one_wg) {
         pl.part_blocks = 64;
-        pl.waves = 8;
+        // (beyond one such workgroup per compute unit the usual four wavefronts do: 64 x 700 34.5 / 31.9, 96 x 700 51.7 / 44.2)
+        if (small || wgs <= 256) pl.waves = 8;
       }
       int64_t P = (max_blocks + pl.part_blocks - 1) / pl.part_blocks;
       if (P < 1) P = 1;

@@ -113,6 +113,14 @@ def test_whole_contexts_per_workgroup_and_merges_of_few_partitions(device, tunin
     assert torch.all(got[~live] == 0)
 
 
+@pytest.mark.parametrize("S,heads,longest", [
+    (2, (32, 8, 128), 4000), (16, (32, 8, 128), 1025), (8, (32, 8, 128), 2033),   # 16 blocks, 32 and one more, 32
+    (32, (2, 2, 128), 16500),                                                      # 64
+    (33, (32, 8, 128), 1024), (65, (32, 8, 128), 700), (97, (32, 8, 128), 641)])   # whole contexts, four wavefronts each; not; again
+def test_partitions_of_16_to_64_blocks(device, tuning, S, heads, longest):
+    test_whole_contexts_per_workgroup_and_merges_of_few_partitions(device, tuning, S, heads, longest, 0)
+
+
 def test_single_partition_path_and_many_partitions_agree_with_oracle(device):
     # S large -> one partition per sequence; S = 1 -> the context is split many ways.
     big = W.decode_inputs(13, 300, 100, 400, 8, 2, 128, torch.float16, 8000)
