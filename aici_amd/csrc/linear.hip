@@ -442,10 +442,10 @@ __global__ __launch_bounds__(WAVES * 64) void linear_stream_kernel(const LinearP
 // rms_norm less, whose time is all latency.  The rows' part repeats in every workgroup and costs about 1 us per row, so it ends at few
 // rows.  LDS: ring | sums of ranges | rows of x | the norm's weight.
 __host__ __device__ constexpr int held_pitch(int K) { return (K * 2 + 1023) / 1024 * 1024; }
-template <typename T, int S, int ROWS, bool GATED, bool QKV>
-__global__ __launch_bounds__(256) void norm_linear_kernel(const LinearParams p) {
+template <typename T, int S, int ROWS, int WAVES, bool GATED, bool QKV>
+__global__ __launch_bounds__(WAVES * 64) void norm_linear_kernel(const LinearParams p) {
   using vec8 = typename Vec8<T>::type;
-  constexpr int WAVES = 4, kParts = GATED ? 2 : 1;
+  constexpr int kParts = GATED ? 2 : 1;
   constexpr int kStageBytes = 2048;
   extern __shared__ __align__(1024) char lds[];
   __shared__ float part_sums[ROWS * 16];
@@ -844,6 +844,14 @@ struct LinearPlan {
 // The ranges of k depend on the weight alone (see above).  As far as eight ranges allow: 1024 wavefronts' worth of (16 rows, range)
 // pairs, four per compute unit, and no range longer than 2048 once k is cut at all -- 4096 x 4096 and 6144 x 4096 four, 4096 x
 // 14336 eight, weights of 16384 rows and more none.
+// Weights that are not cut and whose workgroups of 64 rows are more than one to a compute unit, but not two, while those of 128 rows are at most
+// one: then every unit with work has the same.  us, 64 / 128 rows, 16 rows of x: 16384 x 4096 21.7 / 28.9; 18432 x 4096 33.7 / 29.2; 22016 x 4096
+// gated 34.6 / 30.8; 28672 x 4096 gated 36.5 / 36.1, 32 rows 38.4 / 36.7; 32000 x 4096 40.4 / 40.5; 37888 x 3584 gated 46.4 / 56.0; 51200 x 2560
+// 48.3 / 47.6.  With the norm in front, whose work on the
+// rows of x repeats in every workgroup, 1 row: 28672 x 4096 gated 38.3 / 37.5, 22016 x 4096 33.6 / 30.7, 20480 x 2560 23.3 / 22.1; its ring of four
+// stages for six: 37.5 / 38.8.
+bool wide_workgroups(int N) { return N > 64 * 256 && N <= 128 * 256; }
+
 LinearPlan plan_linear(int M, int N, int K, bool few_only) {
   const Tuning &tn = tuning();
   LinearPlan pl;
@@ -869,8 +877,9 @@ LinearPlan plan_linear(int M, int N, int K, bool few_only) {
   // 106 -> 108).
   pl.turned = N >= 8192 && N % (2 * kTurnRows) == 0 && splits <= 4 && (K % 2048 == 0 || K >= 6144);
   // Workgroups of 64 rows while the device holds all of them at once, one per compute unit, or where 32 rows of x leave the copies of x
-  // cheap (28672 x 4096, 32 rows: 43.5 us against 46.3; 64 rows: 49.5 against 47.3); else of 128 rows.
-  pl.waves = ((int64_t)((N + 63) / 64) * splits <= 256 || (splits == 1 && M <= 32)) ? 4 : 8;
+  // cheap (37888 x 3584, 32 rows: 49.8 us against 60.2; 28672 x 4096, 64 rows: 49.2 against 40.0) and 128 rows are not one per unit; else of
+  // 128 rows.
+  pl.waves = ((int64_t)((N + 63) / 64) * splits <= 256 || (splits == 1 && M <= 32 && !wide_workgroups(N))) ? 4 : 8;
   if (tn.linear_tiles > 0) pl.waves = 4 * tn.linear_tiles;
   if (tn.linear_waves > 0) pl.waves = tn.linear_waves;
   pl.partial_bytes = (size_t)pl.splits * kLinMaxRows * N * sizeof(float);
@@ -901,22 +910,30 @@ void launch_tile(const LinearParams &p, const LinearPlan &pl, hipStream_t stream
   hipLaunchKernelGGL((linear_tile_kernel<T, MT, ring_stages<MT, 8>(), 8, GATED, WIDE>), grid, block, 0, stream, p);
 }
 
-template <typename T, int ROWS, bool GATED, bool QKV>
-void launch_norm_linear(const LinearParams &p, hipStream_t stream) {
+template <typename T, int ROWS, int WAVES, bool GATED, bool QKV>
+void launch_norm_linear_waves(const LinearParams &p, hipStream_t stream) {
   constexpr int S = kHeldStages;
   static bool attr_set = false;  // benign race: setting twice is harmless
-  auto kernel = norm_linear_kernel<T, S, ROWS, GATED, QKV>;
+  auto kernel = norm_linear_kernel<T, S, ROWS, WAVES, GATED, QKV>;
   if (!attr_set) {
     HA_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               4 * S * 2048 + 16 * 1024 + kLinHeldBytes));
+                               WAVES * S * 2048 + 16 * 1024 + kLinHeldBytes));
     attr_set = true;
   }
   const int parts = GATED ? 2 : 1, n = GATED ? p.half : p.N;
-  const int per_tile = p.splits < 4 / parts ? p.splits : 4 / parts, tiles = 4 / parts / per_tile;
+  const int per_tile = p.splits < WAVES / parts ? p.splits : WAVES / parts, tiles = WAVES / parts / per_tile;
   const int rows = 16 * tiles;
-  const size_t bytes = 4 * S * 2048 + tiles * parts * p.splits * 1024 + (size_t)(p.M + 1) * held_pitch(p.K);
-  hipLaunchKernelGGL(kernel, dim3((n + rows - 1) / rows), dim3(256), bytes, stream, p);
+  const size_t bytes = WAVES * S * 2048 + tiles * parts * p.splits * 1024 + (size_t)(p.M + 1) * held_pitch(p.K);
+  hipLaunchKernelGGL(kernel, dim3((n + rows - 1) / rows), dim3(WAVES * 64), bytes, stream, p);
   check_launch("rms_norm_linear");
+}
+
+template <typename T, int ROWS, bool GATED, bool QKV>
+void launch_norm_linear(const LinearParams &p, hipStream_t stream) {
+  if (p.splits == 1 && wide_workgroups(p.N))
+    launch_norm_linear_waves<T, ROWS, 8, GATED, QKV>(p, stream);
+  else
+    launch_norm_linear_waves<T, ROWS, 4, GATED, QKV>(p, stream);
 }
 
 template <typename T, bool GATED, bool QKV = false>

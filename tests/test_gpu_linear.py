@@ -501,3 +501,28 @@ def test_qkv_linear_of_many_heads(device, heads, same):
     else:
         check(got[:, (Hq + Hkv) * d:], x, w[(Hq + Hkv) * d:])  # values are not rotated
         assert ((got - want).float().norm() / want.float().norm()).item() <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("d,M", [(128, 1), (128, 4), (64, 3), (128, 16)])
+def test_qkv_linear_in_workgroups_of_128_rows(device, d, M):
+    Hkv, Kd = 8, 2048
+    Hq = 18432 // d - 2 * Hkv
+    x, w, g = operands(M, 18432, Kd, torch.bfloat16, seed=d + M)
+    xd, wd = x.to(device), w.to(device)
+    norm = (1 + 0.2 * torch.randn((Kd,), generator=g)).to(torch.bfloat16).to(device)
+    h = torch.empty_like(xd)
+    K.rms_norm(h, xd, norm, 1e-5)
+    table = torch.randn((64, d), generator=g).to(torch.bfloat16).to(device)
+    pos, slots = torch.arange(M, device=device) + 3, torch.arange(M, device=device) * 3
+    caches = [torch.zeros((4, Hkv, d // 8, 16, 8), dtype=torch.bfloat16, device=device),
+              torch.zeros((4, Hkv, d, 16), dtype=torch.bfloat16, device=device)]
+    want, wkc, wvc = K.linear(h, wd), caches[0].clone(), caches[1].clone()
+    check(want, h.cpu(), w)
+    q, k, v = want.split([Hq * d, Hkv * d, Hkv * d], dim=1)
+    K.rotary_embedding_and_cache(pos, q, k, v.view(M, Hkv, d), d, table, True, wkc, wvc, slots)
+    for rows, nw in ((h, None), (xd, norm)):
+        if nw is not None and not K.rms_norm_linear_takes(xd, norm, wd):
+            continue
+        kc, vc = caches[0].clone(), caches[1].clone()
+        got = K.qkv_linear(rows, nw, 1e-5, wd, pos, table, kc, vc, slots)
+        assert torch.equal(got, want) and torch.equal(kc, wkc) and torch.equal(vc, wvc)
