@@ -167,7 +167,7 @@ class Llama:
         bits."""
         cfg = self.cfg
         Hq, Hkv, d = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
-        x = self.wte.index_select(0, batch_info.tokens.long())                   # llama.rs:203
+        x = self.wte.index_select(0, batch_info.tokens)                          # llama.rs:203
         T = x.size(0)
         # h: the normalised rows, None where the projection that takes them does it
         first = self.layers[0]
@@ -203,7 +203,7 @@ class Llama:
             behind = self.layers[li + 1] if li + 1 < len(self.layers) else {"rms_1": self.ln_f, "qkv": None}
             x, h = self._proj_add_norm(act, layer["down"], x, behind["rms_1"], behind["qkv"])  # :143, :173
         x0 = h
-        sel = x0.index_select(0, batch_info.logit_idxs.long())                  # :209 extract_positions
+        sel = x0.index_select(0, batch_info.logit_idxs)                         # :209 extract_positions
         return self._proj(sel, self.lm_head)                                    # :210
 
 
