@@ -886,12 +886,13 @@ LinearPlan plan_linear(int M, int N, int K, bool few_only) {
   return pl;
 }
 
-// Stages of the ring: what fits half of the 160 KB of LDS (two workgroups per compute unit), or all of it where a stage takes more
-// than 24 KB.
+// Stages of the ring: what fits half of the 160 KB of LDS (two workgroups per compute unit), or four where a stage takes more than 24 KB
+// (us, five / four, 96 and 128 rows: 6144 x 4096 19.8 / 19.5, 20.9 / 20.2; 4096 x 14336 31.7 / 31.3, 34.0 / 33.6; 128256 x 4096 207.2 / 206.0,
+// 217.8 / 217.1; three: 4096 x 4096 17.4 / 18.1).
 template <int MT, int WAVES>
 constexpr int ring_stages() {
   constexpr int kb = 2 * WAVES + 2 * MT;
-  constexpr int s = (kb <= 24 ? 80 : 160) / kb;
+  constexpr int s = kb <= 24 ? 80 / kb : 4;
   return s > 6 ? 6 : s;
 }
 
@@ -904,6 +905,14 @@ void launch_tile(const LinearParams &p, const LinearPlan &pl, hipStream_t stream
   if constexpr (!WIDE) {
     if (waves == 4) {
       hipLaunchKernelGGL((linear_tile_kernel<T, MT, ring_stages<MT, 4>(), 4, GATED, false>), grid, block, 0, stream, p);
+      return;
+    }
+  }
+  if constexpr (MT == 4 && !WIDE) {
+    // one workgroup to a compute unit: five stages for three (28672 x 4096 gated, us, 33 / 64 rows of x 40.5 / 39.8 -> 39.1 / 38.8; 128256 x 4096, 64
+    // rows 177 -> 182)
+    if (p.splits == 1 && wide_workgroups(p.N)) {
+      hipLaunchKernelGGL((linear_tile_kernel<T, MT, 5, 8, GATED, false>), grid, block, 0, stream, p);
       return;
     }
   }
