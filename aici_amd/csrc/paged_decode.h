@@ -54,6 +54,8 @@ struct DecodeCall {
   const char *op;
 };
 bool decode_params(const DecodeCall &c, hipattn_tensor *out, DecodeParams &p);
+// Bytes of the library's scratch memory that hipattn_paged_attention_v1 takes for a call that decode_params has accepted.
+size_t decode_scratch_bytes(const DecodeCall &c);
 
 // Scratch memory of the flat split over `workgroups` workgroups: the prefix table of the block pairs, and behind it the partial results.
 struct FlatScratch {

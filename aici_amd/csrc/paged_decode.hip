@@ -749,6 +749,12 @@ bool decode_params(const DecodeCall &c, hipattn_tensor *out, DecodeParams &p) {
   return true;
 }
 
+size_t decode_scratch_bytes(const DecodeCall &c) {
+  return plan_decode(c.query->sizes[0], (int)c.query->sizes[1], c.num_kv_heads, (int)c.query->sizes[2], c.block_size, c.query->dtype,
+                     c.max_context_len)
+      .bytes;
+}
+
 FlatScratch flat_scratch(int64_t S, int G, int head_size, int workgroups) {
   FlatScratch f;
   f.cols = G < 16 ? G : 16;

@@ -142,29 +142,41 @@ void *library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream) {
   return scratch_buffer(user, bytes, bytes / 2, stream).ptr;
 }
 
-HeldWorkspace try_library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream) {
-  HeldWorkspace ws;
+// scratch_buffer, or null where it throws and while the stream is being captured.
+static ScratchBuffer *try_scratch_buffer(WorkspaceUser user, size_t bytes, size_t spare, hipStream_t stream) {
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) {
     (void)hipGetLastError();
-    return ws;
+    return nullptr;
   }
-  if (capturing != hipStreamCaptureStatusNone) return ws;
+  if (capturing != hipStreamCaptureStatusNone) return nullptr;
   // A capture on some other stream forbids allocations, in every thread unless the thread says otherwise.
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
     (void)hipGetLastError();
-    return ws;
+    return nullptr;
   }
+  ScratchBuffer *buffer = nullptr;
   try {
-    ScratchBuffer &buffer = scratch_buffer(user, bytes, 0, stream);
-    ws.ptr = buffer.ptr;
-    ws.held = std::unique_lock<std::mutex>(buffer.holder);
+    buffer = &scratch_buffer(user, bytes, spare, stream);
   } catch (const Error &) {
     (void)hipGetLastError();
   }
   (void)hipThreadExchangeStreamCaptureMode(&mode);
+  return buffer;
+}
+
+HeldWorkspace try_library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream) {
+  HeldWorkspace ws;
+  if (ScratchBuffer *buffer = try_scratch_buffer(user, bytes, 0, stream)) {
+    ws.ptr = buffer->ptr;
+    ws.held = std::unique_lock<std::mutex>(buffer->holder);
+  }
   return ws;
+}
+
+void reserve_library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream) {
+  if (bytes > 0) (void)try_scratch_buffer(user, bytes, bytes / 2, stream);
 }
 
 }  // namespace hipattn

@@ -245,6 +245,8 @@ bool step_attention(const PagedPrefillCall &chunks, hipattn_tensor *chunks_out, 
   // The two launches here stay next to one another where several threads use one stream.
   hipStream_t stream = resolve_stream(stream_arg);
   if (stream == hipStreamPerThread) return false;
+  // A capture of this step will run them, and cannot allocate the decode rows' scratch memory: this call is the one made ahead of it.
+  if (rows != nullptr) reserve_library_workspace(WS_PAGED_ATTENTION, decode_scratch_bytes(*rows), stream);
   const HeldWorkspace ws = try_library_workspace(WS_STEP_ATTENTION, kStepScratchBytes, stream);
   if (ws.ptr == nullptr) return false;
   return dtype == HIPATTN_BF16 ? dispatch_step<bf16_t>(pp, dp, pl, hd, static_cast<char *>(ws.ptr), stream)

@@ -30,6 +30,10 @@ struct HeldWorkspace {
 };
 HeldWorkspace try_library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream);
 
+// library_workspace ahead of need: what a later call of the same shapes asks for while the stream is being captured.  Does nothing where
+// that cannot be had now (a capture of this stream, no memory); the later call says so itself.
+void reserve_library_workspace(WorkspaceUser user, size_t bytes, hipStream_t stream);
+
 // Switches for tuning and for tests that want one particular kernel; read
 // from the environment (HIPATTN_<NAME in capitals>) once, when the library is
 // loaded, and changed afterwards only through hipattn_tuning_set.  Ops read

@@ -856,7 +856,11 @@ char *hipattn_varlen_attn(
  * merges partial results, where that is faster: its 64 MiB of scratch memory
  * are allocated once per stream.  Under capture, on hipStreamPerThread and
  * where there is no such memory the two go by themselves, as
- * hipattn_mha_varlen_fwd_paged and hipattn_paged_attention_v1 would. */
+ * hipattn_mha_varlen_fwd_paged and hipattn_paged_attention_v1 would, with the
+ * latter's scratch memory, which an eager call on the stream allocates
+ * whichever way it goes: one is all that a capture of the same shapes needs.
+ * A replay's last bits may differ from the eager call's, whose keys are added
+ * up in other pieces. */
 char *hipattn_varlen_attn_paged(
     const hipattn_tensor *q, const hipattn_tensor *k, const hipattn_tensor *v,
     hipattn_tensor *key_cache, hipattn_tensor *value_cache,

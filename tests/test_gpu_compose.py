@@ -302,3 +302,49 @@ def test_a_captured_step_takes_the_launches_by_themselves(device):
     finally:
         mp.undo()
     assert (y.float() - want).abs().max().item() <= TOL[dtype]
+
+
+def random_step(device, heads, dtype, priors, new, contexts, seed=50):
+    """A mixed step over caches of random values: (q, k, v, batch on the device, key cache, value cache)."""
+    Hq, Hkv, d = heads
+    pool = sum(p // 16 + new // 16 + 2 for p in priors) + sum(c // 16 + 1 for c in contexts)
+    alloc, builder = paged.BlockAllocator(16, pool), paged.BatchInfoBuilder(16, 1 << 20, 1)
+    for sid, (total, computed) in enumerate([(p + new, p) for p in priors] + [(c, c - 1) for c in contexts], 1):
+        alloc.alloc_seq(sid, total)
+        builder.sched_out(alloc, sid, [1] * total, computed)
+    batch = builder.finish().to(device)
+    g = torch.Generator(device=device).manual_seed(seed)
+
+    def normal(*shape):
+        return torch.randn(shape, generator=g, device=device).to(dtype)
+
+    T = batch.tokens.numel()
+    return normal(T, Hq, d), normal(T, Hkv, d), normal(T, Hkv, d), batch, normal(pool, Hkv, d // 8, 16, 8), normal(pool, Hkv, d, 16)
+
+
+@pytest.mark.parametrize("rows,context", [(9, 600), (70, 3000)])  # partitions, flat split
+def test_one_eager_step_is_all_that_a_capture_of_it_needs(device, tuning, rows, context):
+    """The eager step takes the combined launch, its capture the launches by themselves, on the stream's scratch memory for decode rows."""
+    q, k, v, batch, kc, vc = random_step(device, (32, 8, 128), torch.bfloat16, [0, 640, 1000, 2048], 33,
+                                         [context - 7 * i for i in range(rows)])
+
+    def call():
+        return attn.varlen_attn(q, k, v, batch, kc, vc)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        eager, kernels = launched(call)
+        assert any("step_merge_kernel" in n for n in kernels)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            out = call()
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            assert (out - eager).abs().max().item() <= TOL[torch.bfloat16]
+            assert torch.equal(call(), eager)
+        if context < 1024:
+            tuning("decode_flat", 0)  # the launches by themselves
+            assert torch.equal(call(), out)
+    torch.cuda.current_stream().wait_stream(side)
