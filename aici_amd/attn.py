@@ -63,14 +63,17 @@ class RmsNorm:
         return out
 
 
-def _reads_through_tables(q: torch.Tensor, batch_info: BatchInfo, key_cache: torch.Tensor, value_cache: torch.Tensor) -> bool:
+def _reads_through_tables(q: torch.Tensor, k: torch.Tensor, batch_info: BatchInfo, key_cache: torch.Tensor, value_cache: torch.Tensor) -> bool:
     """Whether the context of the multi-token rows need not be gathered (us, gathered / through the tables, 32 heads of 80: 120 decode rows
-    of 1k..8k tokens beside 4 x 512 new ones over up to 3072 1012 / 920, 15 rows of 253 beside 4 x 65..263 103 / 39)."""
-    tables = batch_info.multi_block_tables
-    return (batch_info.q_multi > 0 and tables is not None and tables.size(1) * 16 >= batch_info.max_seqlen_k and q.size(2) in (64, 80, 96, 112, 128)
+    of 1k..8k tokens beside 4 x 512 new ones over up to 3072 1012 / 920, 15 rows of 253 beside 4 x 65..263 103 / 39).  What the tables' route
+    would not take, or would not refuse as the gather does (caches with other heads than k), is gathered."""
+    tables, lens = batch_info.multi_block_tables, batch_info.multi_context_lens
+    return (batch_info.q_multi > 0 and tables is not None and lens is not None and tables.size(1) * 16 >= batch_info.max_seqlen_k
+            and tables.dtype == lens.dtype == torch.int32 and tables.size(0) == lens.size(0) == batch_info.seqlens_q.size(0) - 1
+            and (tables.size(1) <= 1 or tables.stride(1) == 1) and lens.is_contiguous() and q.size(2) in (64, 80, 96, 112, 128)
             and q.dtype in (torch.float16, torch.bfloat16) and key_cache.dtype == q.dtype and value_cache.dtype == q.dtype
             and key_cache.dim() == 5 and value_cache.dim() == 4 and key_cache.size(3) == 16 and value_cache.size(3) == 16
-            and key_cache.is_contiguous() and value_cache.is_contiguous()
+            and key_cache.size(1) == k.size(1) and key_cache.is_contiguous() and value_cache.is_contiguous()
             and key_cache.data_ptr() % 16 == 0 and value_cache.data_ptr() % 16 == 0)
 
 
@@ -90,7 +93,7 @@ def varlen_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, batch_info: B
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(d)
     y = torch.empty((T, Hq, d), dtype=q.dtype, device=q.device)
-    if paged_prefill or _reads_through_tables(q, batch_info, key_cache, value_cache):
+    if paged_prefill or _reads_through_tables(q, k, batch_info, key_cache, value_cache):
         if batch_info.multi_block_tables is None:
             raise ValueError("paged_prefill needs batch_info.multi_block_tables (slots must follow the blocks in order)")
         has_m, has_p = batch_info.q_multi > 0, batch_info.q_multi < T

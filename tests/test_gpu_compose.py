@@ -11,6 +11,7 @@ import torch
 
 from aici_amd import attn, paged
 from aici_amd import workloads as W
+from aici_amd._lib import HipAttnError
 from oracle import refkernels as ref
 from tests.common import TOL, make_cache
 
@@ -348,3 +349,25 @@ def test_one_eager_step_is_all_that_a_capture_of_it_needs(device, tuning, rows, 
             tuning("decode_flat", 0)  # the launches by themselves
             assert torch.equal(call(), out)
     torch.cuda.current_stream().wait_stream(side)
+
+
+@pytest.mark.parametrize("heads", [1, 4, 16])
+@pytest.mark.parametrize("contexts", [[], [5, 40]])
+def test_caches_with_other_heads_than_the_keys_are_refused(device, heads, contexts):
+    q, k, v, batch, kc, vc = random_step(device, (32, 8, 128), torch.bfloat16, [0, 100], 20, contexts)
+    other = k[:, :1].expand(-1, heads, -1)
+    with pytest.raises(HipAttnError):
+        attn.varlen_attn(q, other, other, batch, kc, vc, cached=True)
+
+
+def test_a_batch_whose_tables_are_not_those_of_its_rows_is_gathered(device):
+    """The first chunk of a batch of two, cut out by hand: the tables still have the rows of both, and may lack their context lengths."""
+    q, k, v, batch, kc, vc = random_step(device, (32, 8, 128), torch.bfloat16, [30, 100], 20, [])
+    both = attn.varlen_attn(q, k, v, batch, kc, vc)
+    n, m = int(batch.seqlens_q[1]), int(batch.seqlens_k[1])
+    cut = dict(tokens=batch.tokens[:n], positions=batch.positions[:n], slot_mapping=batch.slot_mapping[:n], q_multi=n, seqlen_multi=1,
+               seqlens_q=batch.seqlens_q[:2].contiguous(), seqlens_k=batch.seqlens_k[:2].contiguous(),
+               gather_mapping=batch.gather_mapping[:m].contiguous())
+    for more in ({}, {"multi_context_lens": None}):
+        got = attn.varlen_attn(q[:n], k[:n], v[:n], dataclasses.replace(batch, **cut, **more), kc, vc)
+        assert (got - both[:n]).abs().max().item() <= TOL[torch.bfloat16]
