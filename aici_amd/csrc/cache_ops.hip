@@ -706,13 +706,6 @@ void cache_move(const hipattn_tensor *key, const hipattn_tensor *value,
   }
 }
 
-void take_error(char *err) {
-  if (err == nullptr) return;
-  const std::string msg(err);
-  free(err);
-  fail("%s", msg.c_str());
-}
-
 void rotary_and_cache(const hipattn_tensor *positions, hipattn_tensor *query, hipattn_tensor *key,
                       const hipattn_tensor *value, int head_size, const hipattn_tensor *cos_sin, bool is_neox,
                       hipattn_tensor *key_cache, hipattn_tensor *value_cache,
@@ -749,8 +742,8 @@ void rotary_and_cache(const hipattn_tensor *positions, hipattn_tensor *query, hi
       g.k_block_stride % 8 == 0 && g.k_head_stride % 8 == 0 && aligned16(query->data) && aligned16(key->data) &&
       aligned16(value->data) && aligned16(cos_sin->data) && aligned16(key_cache->data) && T > 0 && T <= 0x7fffffff;
   if (!fused) {  // every other case: the two calls, with their own checks
-    take_error(hipattn_rotary_embedding(positions, query, key, head_size, cos_sin, is_neox, stream));
-    take_error(hipattn_reshape_and_cache(&key3, value, key_cache, value_cache, slot_mapping, stream));
+    raise(hipattn_rotary_embedding(positions, query, key, head_size, cos_sin, is_neox, stream));
+    raise(hipattn_reshape_and_cache(&key3, value, key_cache, value_cache, slot_mapping, stream));
     return;
   }
   check_data(query, "query");

@@ -31,6 +31,14 @@ struct Error : std::runtime_error {
   throw Error(buf);
 }
 
+// Throws what another entry point of the library has returned, if that is an error.
+inline void raise(char *err) {
+  if (err == nullptr) return;
+  const std::string msg(err);
+  free(err);
+  fail("%s", msg.c_str());
+}
+
 #define HA_CHECK(cond, ...)                 \
   do {                                      \
     if (!(cond)) ::hipattn::fail(__VA_ARGS__); \

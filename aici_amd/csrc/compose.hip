@@ -15,13 +15,6 @@ hipattn_tensor rows(const hipattn_tensor *t, int64_t begin, int64_t end) {
   return r;
 }
 
-void raise(char *err) {
-  if (err == nullptr) return;
-  std::string msg(err);
-  free(err);
-  fail("%s", msg.c_str());
-}
-
 }  // namespace
 }  // namespace hipattn
 

@@ -1009,7 +1009,9 @@ bool rows_overlap(const hipattn_tensor *a, const hipattn_tensor *b) {
 }
 
 struct QkvOperands {
-  const hipattn_tensor *positions, *cos_sin, *key_cache, *value_cache, *slot_mapping;
+  const hipattn_tensor *positions, *cos_sin;
+  hipattn_tensor *key_cache, *value_cache;
+  const hipattn_tensor *slot_mapping;
 };
 
 QkvParams qkv_params(const QkvOperands &o, int64_t M, int64_t N, int dt) {
@@ -1196,8 +1198,28 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
              "qkv_linear: %lld rows of x and a weight of %lld rows; fewer than 65536 of weight, and than 16384 with more than %d rows of x", (long long)M,
              (long long)N, kLinStreamRows);
     p.qkv = qkv_params(*qkv, M, N, dt);
-    // the halves of a head have to share an order (heads of 80, 96, 256, ...: the order without turns, in every form of this call)
-    if (kTurnRows % p.qkv.g.head_size != 0) p.turned = 0;
+    if (p.turned != 0 && kTurnRows % p.qkv.g.head_size != 0) {
+      // A row and the one that it is rotated with would have to share an order of k, and here they may have different ones (heads of 80, 96,
+      // 256, ...): the calls themselves, with their bits.  us, an order without turns in one launch / the calls: 9216 x 2048 16 rows 12.5 /
+      // 16.4, 12288 x 4096 16 and 64 rows 25.0 / 27.3, 29.6 / 31.2, 15360 x 8192 64 rows 64.7 / 57.0, 21504 x 8192 16 rows 80.5 / 63.4.
+      linear_impl(out, x, weight, nullptr, nullptr, nullptr, stream_arg, nullptr, nullptr, norm_weight, eps, false, false, norm_in);
+      const int hd = p.qkv.g.head_size, Hkv = p.qkv.g.num_heads;
+      auto columns = [&](int64_t first, int64_t heads) {
+        hipattn_tensor t = *out;
+        t.data = static_cast<char *>(out->data) + first * hd * 2;
+        t.sizes[1] = heads * hd;
+        return t;
+      };
+      hipattn_tensor q = columns(0, p.qkv.q_heads), k = columns(p.qkv.q_heads, Hkv), v = columns(p.qkv.q_heads + Hkv, Hkv);
+      v.ndim = 3;
+      v.sizes[1] = Hkv;
+      v.sizes[2] = hd;
+      v.strides[1] = hd;
+      v.strides[2] = 1;
+      raise(hipattn_rotary_embedding_and_cache(qkv->positions, &q, &k, &v, hd, qkv->cos_sin, true, qkv->key_cache, qkv->value_cache,
+                                               qkv->slot_mapping, stream_arg));
+      return;
+    }
     dt == HIPATTN_BF16 ? launch_linear<bf16_t, false, true>(p, pl, stream) : launch_linear<half_t, false, true>(p, pl, stream);
     return;
   }
@@ -1205,14 +1227,7 @@ void linear_impl(hipattn_tensor *out, const hipattn_tensor *x, const hipattn_ten
     gated ? launch_linear<bf16_t, true>(p, pl, stream) : launch_linear<bf16_t, false>(p, pl, stream);
   else
     gated ? launch_linear<half_t, true>(p, pl, stream) : launch_linear<half_t, false>(p, pl, stream);
-  if (norm_out != nullptr && pl.stream) {
-    char *err = hipattn_rms_norm(norm_out, out, norm_weight, eps, stream_arg);
-    if (err != nullptr) {
-      const std::string msg(err);
-      free(err);
-      fail("%s", msg.c_str());
-    }
-  }
+  if (norm_out != nullptr && pl.stream) raise(hipattn_rms_norm(norm_out, out, norm_weight, eps, stream_arg));
 }
 
 }  // namespace

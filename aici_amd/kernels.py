@@ -335,8 +335,8 @@ def qkv_linear(x: torch.Tensor, norm_weight: Optional[torch.Tensor], epsilon: fl
                cos_sin_cache: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor,
                slot_mapping: torch.Tensor) -> torch.Tensor:
     """x @ weight.T, behind rms_norm of the rows where norm_weight is given, and rotary_embedding_and_cache of its heads (llama.rs:81-85 +
-    mod.rs:147-164) in the projection's own launches: returns [M, (Hq + 2 Hkv) d] with the bits of the calls (where the head size
-    divides 128 or the weight has fewer than 8192 rows; else but for last bits)."""
+    mod.rs:147-164) in the projection's own launches (wide weights and heads that do not divide 128: one more): returns [M, (Hq + 2 Hkv) d]
+    with the bits of the calls."""
     out = torch.empty((x.size(0), weight.size(0)), dtype=x.dtype, device=x.device)
     _native.qkv_linear(out, x, norm_weight, epsilon, weight, positions, cos_sin_cache, key_cache, value_cache, slot_mapping)
     return out

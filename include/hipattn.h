@@ -388,7 +388,7 @@ char *hipattn_rms_norm_linear(hipattn_tensor *out, const hipattn_tensor *x,
 
 /* The projection of q, k and v with hipattn_rotary_embedding_and_cache (NeoX) behind it (llama.rs:81-85 + mod.rs:147-164), for the
  * rows of a small step: out [M, (Hq + 2 Hkv) d] = x . weight^T, query and key heads rotated, the keys and values written to the cache;
- * the bits of the calls (last bits may differ where d does not divide 128 and weight has 8192 rows or more).  With norm_weight not NULL hipattn_rms_norm of the rows of x comes first, as in hipattn_rms_norm_linear and
+ * the bits of the calls, and the calls themselves where d does not divide 128 and hipattn_linear turns the weight's ranges.  With norm_weight not NULL hipattn_rms_norm of the rows of x comes first, as in hipattn_rms_norm_linear and
  * within its limits.  d and Hkv are the cache's; d a multiple of 16, cos_sin_cache [positions, d]; fewer than 65536 rows of weight, and
  * than 16384 with more than 16 rows of x; operands else, and scratch, as for hipattn_linear and hipattn_rotary_embedding_and_cache. */
 char *hipattn_qkv_linear(hipattn_tensor *out, const hipattn_tensor *x,

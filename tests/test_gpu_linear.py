@@ -526,3 +526,31 @@ def test_qkv_linear_in_workgroups_of_128_rows(device, d, M):
         kc, vc = caches[0].clone(), caches[1].clone()
         got = K.qkv_linear(rows, nw, 1e-5, wd, pos, table, kc, vc, slots)
         assert torch.equal(got, want) and torch.equal(kc, wkc) and torch.equal(vc, wvc)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads,Kd", [((32, 2, 256), 2048), ((88, 4, 96), 2048), ((64, 32, 80), 4096), ((64, 16, 112), 6144),
+                                      ((70, 5, 208), 2048)])
+def test_qkv_linear_of_heads_that_do_not_divide_128_has_the_bits_of_the_calls(device, dtype, heads, Kd):
+    """Weights whose ranges of k begin inside, up to 16 rows also uncut ones; also through rows of out on 8-byte boundaries."""
+    Hq, Hkv, d = heads
+    M, N = 40, (Hq + 2 * Hkv) * d
+    x, w, g = operands(M, N, Kd, dtype, seed=d)
+    xd, wd = x.to(device), w.to(device)
+    norm = (1 + 0.2 * torch.randn((Kd,), generator=g)).to(dtype).to(device)
+    table = torch.randn((64, d), generator=g).to(dtype).to(device)
+    empty = [torch.zeros((4, Hkv, d // 8, 16, 8), dtype=dtype, device=device), torch.zeros((4, Hkv, d, 16), dtype=dtype, device=device)]
+    pos, slots = torch.randint(0, 64, (M,), generator=g).to(device), torch.randperm(64, generator=g)[:M].to(device)
+    for m in (1, 4, 5, 16, 17, 40):
+        if not K.qkv_linear_takes(xd[:m], wd, table, *empty):
+            assert N >= 16384 and m > 16
+            continue
+        for nw in (None, norm) if K.rms_norm_linear_takes(xd[:m], norm, wd) else (None,):
+            want = K.linear(xd[:m], wd) if nw is None else K.rms_norm_linear(xd[:m], nw, 1e-5, wd)
+            q, k, v = want.split([Hq * d, Hkv * d, Hkv * d], dim=1)
+            caches = [c.clone() for c in empty]
+            K.rotary_embedding_and_cache(pos[:m], q, k, v.view(m, Hkv, d), d, table, True, *caches, slots[:m])
+            for out in (torch.empty((m, N), dtype=dtype, device=device), torch.empty((m, N + 8), dtype=dtype, device=device)[:, 4:-4]):
+                mine = [c.clone() for c in empty]
+                _native.qkv_linear(out, xd[:m], nw, 1e-5, wd, pos[:m], table, *mine, slots[:m])
+                assert torch.equal(out, want) and torch.equal(mine[0], caches[0]) and torch.equal(mine[1], caches[1])
