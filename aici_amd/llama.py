@@ -85,6 +85,11 @@ def random_weights(cfg: LlamaConfig, seed: int, device=None, std: float = 0.02) 
     return ws
 
 
+def _rows(t: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
+    """t[idx]: index_select takes 32- and 64-bit indices as they are, others are converted."""
+    return t.index_select(0, idx if idx.dtype in (torch.int32, torch.int64) else idx.long())
+
+
 class Llama:
     """llama.rs:194-213.  `forward` returns the logits of every sequence's last token."""
 
@@ -168,7 +173,7 @@ class Llama:
         bits."""
         cfg = self.cfg
         Hq, Hkv, d = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
-        x = self.wte.index_select(0, batch_info.tokens)                          # llama.rs:203
+        x = _rows(self.wte, batch_info.tokens)                                   # llama.rs:203
         T = x.size(0)
         # h: the normalised rows, None where the projection that takes them does it
         first = self.layers[0]
@@ -204,7 +209,7 @@ class Llama:
             behind = self.layers[li + 1] if li + 1 < len(self.layers) else {"rms_1": self.ln_f, "qkv": None}
             x, h = self._proj_add_norm(act, layer["down"], x, behind["rms_1"], behind["qkv"])  # :143, :173
         x0 = h
-        sel = x0.index_select(0, batch_info.logit_idxs)                         # :209 extract_positions
+        sel = _rows(x0, batch_info.logit_idxs)                                  # :209 extract_positions
         return self._proj(sel, self.lm_head)                                    # :210
 
 

@@ -310,3 +310,13 @@ def test_a_step_over_caches_with_another_number_of_heads_is_refused(device, head
     with pytest.raises(HipAttnError):
         model.forward(batch, bad, fused=True)
     assert not any(t.any() for kv in bad for t in kv)
+
+
+@pytest.mark.parametrize("dtype", [torch.int16, torch.int64])
+def test_a_step_takes_indices_of_any_integer_type(device, dtype):
+    cfg = make_cfg(torch.bfloat16)
+    model = llama.Llama(cfg, llama.random_weights(cfg, seed=9, std=0.04), device)
+    batch, caches = decode_step(cfg, device, [20, 5, 33])
+    want = model.forward(batch, caches, fused=True)
+    batch.tokens, batch.logit_idxs = batch.tokens.to(dtype), batch.logit_idxs.to(dtype)
+    assert torch.equal(model.forward(batch, caches, fused=True), want)
