@@ -15,8 +15,8 @@
 //   18 of 489..1957 + 6 x 36 over 0..3000, 32 / 8 x 128                                  110 / 94 / 44
 //   15 of 253 + 4 x 65..263 over 0..3000, 32 / 32 x 80                                   103 / 79 / 39
 //   20 of 100..2000 + 3 x 50..300 over 0..2000, 16 / 2 x 64                               49 / 46 / 31
-// Geometric mean over 167 batches (seven kinds of heads, 0..120 rows of 16..8192 tokens, 1..8 chunks of 2..3000 over up to 12000): 1.9 times the
-// separate launches' speed, 2.35 times the gathered copy's; none slower than the noise.
+// Geometric mean over 3825 batches (nine kinds of heads; 0..120 rows of up to 3000 tokens beside 17 sets of 1..8 chunks of 3..4096 over
+// up to 12000): 1.37 times the separate launches' speed; 2.5 % of them more than 3 % slower than those, at most 14 %.
 #include <algorithm>
 
 #include "paged_decode.h"
@@ -140,17 +140,26 @@ bool plan_step(const PrefillParams &pp, const DecodeParams &dp, int hd, StepPlan
   const int tiles = std::max((pp.max_k + BN - 1) / BN, 1), bm = 128 >> pl.heads_log2;
   const int64_t wgs = (pp.total_q / bm + (pp.batch + 1) / 2) * (pp.Hq >> pl.heads_log2);  // of prefill with whole row blocks, about
   // Pieces: as many as make the longest row block's tiles, or the decode rows behind which they pass, cheaper by more than writing and
-  // merging the pieces costs, all in us.  A tile: measured beside decode rows and without.  A piece: 8 bytes per element there and back at
-  // 5 TB/s, of which about 60 % of the rows have one.  The merge's launch is there for the decode rows anyway; without them it costs 7.
-  // Pieces of fewer than three tiles are all set-up, and two and a half workgroups per compute unit need no more.
+  // merging the pieces costs, all in us.  A tile: measured beside decode rows and without.  A piece: 8 bytes per element there and back, of
+  // which about 60 % of the rows have one, and twice that with what a workgroup's start costs.  The merge's launch is there for the
+  // decode rows anyway; without them it costs 7.  Pieces of fewer than three tiles are all set-up.  Two workgroups of a compute unit have a tile
+  // in little less than twice the time of one, so pieces pay while there are compute units without work, up to seven workgroups on four
+  // of them, and two where the rows alone (padding aside) leave some idle and the chain is long.  us, apart / whole / 2 / 3 / 4 / 6 pieces: 1 x 300
+  // over 6000, 32 / 8 x 128 (80 workgroups) 110 / 97 / 65 / 52 / 48 / 55; 1 x 1000 over 1000 (256) 46 / 45 / 52 / 54 / 54 / 54, over 6000
+  // 136 / 128 / 112 / 126 / 125 / 126; 8 x 500 over 1000, 12 / 4 x 112 (420) 49 / 44 / 68 / 64 / 64 / 64; 8 x 50 over 3000, 40 / 8 x 112 (280,
+  // 125 of them rows) 91 / 91 / 65 / 64 / 58 / 62.  Three also where long chains are some more workgroups than there are places, so that a last round
+  // would run nearly alone (16 / 2 x 64, 8 x 600 over 12000, 616 of 512: 304 / 272 / 293 / 256).
   const double per_tile = hd > 96 ? (decode ? 1.6 : 1.2) : (decode ? 1.2 : 0.9);
-  const double per_part = (double)pp.total_q * pp.Hq * (hd + 2) * 1e-6;
+  const double per_part = (double)pp.total_q * pp.Hq * (hd + 2) * 2e-6;
   const double decode_us = units * hd * 128 * 1e-7;  // contexts of 0.65 of the longest at 6.5 TB/s
   const size_t part_bytes = (size_t)pp.total_q * pp.Hq * (hd + 2) * sizeof(float);
+  int most = (int)std::min<int64_t>(std::max<int64_t>(7 * (int64_t)cus / 4 / std::max<int64_t>(wgs, 1), 1), kMostParts);
+  if (most == 1 && pp.total_q * pp.Hq / 128 <= cus && tiles >= 30) most = 2;
+  if (most == 1 && tiles >= 128 && wgs > 2 * cus && 2 * wgs < 5 * (int64_t)cus) most = 3;
   double best = 0;
   int parts = 1;
-  for (int n = 1; n <= kMostParts; n++) {
-    if (n > 1 && (n * 3 > tiles || 2 * wgs >= 5 * (int64_t)cus || pl.flat_bytes + n * part_bytes > kStepScratchBytes)) break;
+  for (int n = 1; n <= most; n++) {
+    if (n > 1 && (n * 3 > tiles || pl.flat_bytes + n * part_bytes > kStepScratchBytes)) break;
     const double t = std::max(per_tile * ((tiles + n - 1) / n), decode_us) + (n > 1 ? (decode ? 2 : 7) + n * per_part : 0);
     if (n == 1 || t < best) {
       best = t;
@@ -162,11 +171,16 @@ bool plan_step(const PrefillParams &pp, const DecodeParams &dp, int hd, StepPlan
   const double prefill_us = std::max(per_tile * ((tiles + parts - 1) / parts), 2.8 * 0.5 * tiles * wgs / (2.0 * cus));
   if (parts == 1) {
     // Apart where what passes behind the decode rows is not worth what the flat split costs them, if they would not take it alone (70 rows of
-    // 77..778 tokens, 32 heads x 80, beside 3 x 2..14: 59 us apart, 66 here), or where narrow heads, which have a third workgroup on a
-    // compute unit or alternate in eight wavefronts by themselves, lose more than the decode rows are worth (16 / 2 x 64, 8 x 512 over
-    // 1000: beside 30 rows of up to 2048 tokens 42 / 45, 60 of up to 4096 53 / 53; 2 x 1500 over 500 47 / 51 and 59 / 50).
+    // 77..778 tokens, 32 heads x 80, beside 3 x 2..14: 59 us apart, 66 here), or where the chunks by themselves run in a form that is faster by
+    // more than the decode rows are worth: narrow heads with a third workgroup on a compute unit or eight alternating wavefronts
+    // (16 / 2 x 64, 8 x 512 over 1000: beside 30 rows of up to 2048 tokens 42 / 45, 60 of up to 4096 53 / 53; 2 x 1500 over 500 47 / 51 and 59 /
+    // 50; with fewer workgroups, or some more and contexts of 12000, 304 / 272), heads of 128 with eight wavefronts once there are several
+    // workgroups per compute unit (32 / 8 x 128, one row beside 1 x 4096 over 4096: 373 / 405; 64 / 8 x 128, 8 rows beside 4 x 1024 over 4000
+    // 436 / 458; 120 rows of up to 3000 beside 8 x 600 over 12000: 768 / 697).
     if (!use_flat_split(dp.num_seqs, heads, dp.max_ctx) && prefill_us < 0.3 * decode_us) return false;
-    if (hd <= 96 && decode_us < 0.3 * prefill_us) return false;
+    const bool many = 2 * wgs >= 7 * (int64_t)cus;
+    if (hd <= 96 && 2 * wgs >= 3 * (int64_t)cus && (many || tiles <= 128) && decode_us < 0.3 * prefill_us) return false;
+    if (hd > 112 && many && decode_us < 0.25 * prefill_us) return false;
   }
   // The decode rows behind the chunks where they pass in the shadow of the last of them, else in front, where the chunks pass in theirs
   // (32 / 8 x 128, 8 x 512 over 1000, front / behind: 30 rows of up to 2048 tokens 92 / 85, 60 of up to 4096 139 / 169).

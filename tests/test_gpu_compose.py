@@ -371,3 +371,19 @@ def test_a_batch_whose_tables_are_not_those_of_its_rows_is_gathered(device):
     for more in ({}, {"multi_context_lens": None}):
         got = attn.varlen_attn(q[:n], k[:n], v[:n], dataclasses.replace(batch, **cut, **more), kc, vc)
         assert (got - both[:n]).abs().max().item() <= TOL[torch.bfloat16]
+
+
+@pytest.mark.filterwarnings("ignore:Profiler clears events")
+@pytest.mark.parametrize("heads,priors,new,contexts,together", [
+    ((40, 8, 112), [900], 1000, [], False),            # 320 workgroups: pieces of their keys would only wait for one another
+    ((32, 8, 96), [0], 2000, [60, 300], False),        # 504 of narrow heads beside next to nothing
+    ((32, 8, 128), [2000], 4096, [100], False),        # 1032: faster in eight wavefronts, by more than the row is worth
+    ((32, 8, 128), [2000], 4096, [3000] * 60, True),   # not by more than these are
+    ((12, 4, 112), [800], 300, [], True)])             # 36: seven pieces find compute units without work
+def test_which_steps_are_one_launch(device, tuning, heads, priors, new, contexts, together):
+    q, k, v, batch, kc, vc = random_step(device, heads, torch.bfloat16, priors, new, contexts)
+    got, kernels = launched(lambda: attn.varlen_attn(q, k, v, batch, kc, vc, cached=True))
+    assert any("step_merge_kernel" in n for n in kernels) == together
+    tuning("decode_flat", 0)  # the launches by themselves
+    want = attn.varlen_attn(q, k, v, batch, kc, vc, cached=True)
+    assert (got - want).abs().max().item() <= TOL[torch.bfloat16]
