@@ -445,13 +445,18 @@ struct DecodePlan {
 // Partition length used by v1, in KV blocks: a multiple of 8 (one block pair per wavefront and round).  Long steps have some 2048
 // workgroups: fewer fp32 partial results and start-ups per byte, and contexts of different lengths still even out.  With up to 128 (sequence,
 // kv head) pairs partitions are longer: a workgroup's start-up and its partial result cost about what one more round does, so as long as
-// leaves some 320 workgroups, one and a bit per compute unit, up to 32 blocks, and 64 where there are that many several times over.  A
+// leaves some 320 workgroups, one and a bit per compute unit, up to 32 blocks, and 64 where there are that many several times over (but 8
+// where those are at most one to a compute unit, of 17 to 1023 blocks: heads of 256, us, 8 / 16 blocks, 8 / 2: 24 x 500 12.2 / 14.8, 8 x 1300 11.7 /
+// 14.1, 12 x 1600 19.5 / 15.4; 8 / 1: 128 x 256 14.7 / 12.4, 2 x 16384 19.1 / 18.1).  A
 // whole context of up to 64 blocks where that leaves as many: nothing to merge then (but where a few of them would be left for a
 // last round, 17 x 630 at 32 kv heads 33.0 / 34.7).  Work is counted in blocks of 128 head elements.
 // us, 2048 workgroups wanted / this rule, contexts of that length (uniform from a tenth of it), 32 / 8 heads of 128: 4 x 4096 19.0 / 16.4
 // (18.9 / 14.9), 8 x 2048 18.5 / 16.4 (16.7 / 14.1), 8 x 4096 29.7 / 26.0 (25.9 / 22.0), 16 x 1600 25.0 / 22.7 (19.7 / 19.2), 16 x
 // 2048 29.0 / 25.9 (23.5 / 20.3), 96 x 700 51.7 / 44.2 (36.7 / 31.5); 32 / 32 of 80: 2 x 4096 19.7 / 18.1 (18.7 / 16.5), 16 x 700 23.7 /
 // 20.6 (19.1 / 16.3).  With more pairs: 24 x 1600 31.0 / 31.8 (22.9 / 24.5), 48 x 2048 from 204 on 45.0 / 47.8, 53 x 385..1541 42.6 / 44.6.
+// 4528 calls (eight kinds of heads, 1 to 508 sequences of up to 256..131072 tokens): 0.966 of the time of the 2048; 2.5 % of them are more than
+// 5 % slower, most of them 64 to 120 pairs of 500 to 1100 tokens that differ in length (12 x 70..700 12.6 / 11.6, 11 x 102..1024 13.7 / 12.3) -- what
+// gains there (partitions rounded down) loses as much where lengths are alike.
 // The tuning switch decode_part_blocks overrides the choice.
 int choose_part_blocks(int64_t S, int Hkv, int col_groups, int head_size, int max_ctx) {
   const int forced = tuning().decode_part_blocks;
@@ -465,7 +470,7 @@ int choose_part_blocks(int64_t S, int Hkv, int col_groups, int head_size, int ma
   int64_t pb = (max_blocks + parts - 1) / parts;
   if (max_blocks <= 64 && work > 32 * 320 && (items <= 512 || items % 512 == 0 || items % 512 >= 256))
     pb = 64;
-  else if (items <= 128)
+  else if (items <= 128 && (items * ((max_blocks + 7) / 8) > 256 || max_blocks <= 16 || max_blocks >= 1024))
     pb = std::max(pb, work >= 65536 ? (int64_t)64 : std::min<int64_t>(32, (work + 319) / 320));
   pb = ((pb + 7) / 8) * 8;
   if (pb < 8) pb = 8;
@@ -523,6 +528,12 @@ DecodePlan plan_decode(int64_t S, int Hq, int Hkv, int head_size, int block_size
         pl.part_blocks = 64;
         // (beyond one such workgroup per compute unit the usual four wavefronts do: 64 x 700 34.5 / 31.9, 96 x 700 51.7 / 44.2)
         if (small || wgs <= 256) pl.waves = 8;
+      } else if (tuning().decode_part_blocks <= 0 && head_size > 64 && head_size < 128 && max_blocks > 32 && max_blocks <= pl.part_blocks &&
+                 wgs <= 256 && one_wg) {
+        // Contexts that are whole already.  With heads of 128 four wavefronts do there too (32 x 1024 24.9 / 24.1), with smaller ones they lose
+        // where lengths differ: us, eight / four, 12 / 4 x 112, 48 x 102..1024 16.3 / 18.1 (all 1024: 19.0 / 19.8), 32 / 4 x 96, 64 x 102..1024
+        // 15.4 / 16.8 (20.4 / 19.9).
+        pl.waves = 8;
       }
       int64_t P = (max_blocks + pl.part_blocks - 1) / pl.part_blocks;
       if (P < 1) P = 1;

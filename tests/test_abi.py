@@ -42,6 +42,14 @@ def test_version_and_error_convention_on_host_only_calls():
         _lib.call("hipattn_reshape_and_cache", None, None, None, None, None, None)
 
 
+@pytest.mark.parametrize("S,context", [(24, 500), (8, 1300), (2, 8192), (1, 16000)])
+def test_partitions_of_wide_heads_leave_no_compute_unit_idle(S, context):
+    """(sequence, kv head) pairs x partitions of 8 blocks are at most one workgroup to a compute unit: longer ones only take longer."""
+    need = ctypes.c_int64(0)
+    _lib.call("hipattn_paged_attention_workspace_size", S, 8, 2, 256, 16, context, 2, ctypes.byref(need))
+    assert need.value == S * 8 * ((context + 127) // 128) * (256 + 2) * 4
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "_lib", None)
     monkeypatch.setattr(_lib, "LIB_PATH", tmp_path / "libhipattn.so")

@@ -121,6 +121,19 @@ def test_partitions_of_16_to_64_blocks(device, tuning, S, heads, longest):
     test_whole_contexts_per_workgroup_and_merges_of_few_partitions(device, tuning, S, heads, longest, 0)
 
 
+@pytest.mark.parametrize("S,heads,longest", [
+    (48, (12, 4, 112), 1024), (47, (4, 4, 112), 1024), (64, (32, 4, 96), 1009), (65, (8, 4, 96), 1009), (64, (4, 4, 112), 736)])
+def test_uncut_contexts_of_narrower_heads(device, tuning, S, heads, longest):
+    """Contexts of 46 to 64 blocks that the partition length covers whole: on both sides of what takes eight wavefronts."""
+    test_whole_contexts_per_workgroup_and_merges_of_few_partitions(device, tuning, S, heads, longest, 0)
+
+
+@pytest.mark.parametrize("S,longest", [(24, 500), (16, 1024), (16, 1040), (8, 2049)])
+def test_partitions_of_wide_heads(device, tuning, S, longest):
+    """128 to 256 workgroups of 8 blocks, and partitions of 16 where those would be some more."""
+    test_whole_contexts_per_workgroup_and_merges_of_few_partitions(device, tuning, S, (8, 2, 256), longest, 0)
+
+
 def test_single_partition_path_and_many_partitions_agree_with_oracle(device):
     # S large -> one partition per sequence; S = 1 -> the context is split many ways.
     big = W.decode_inputs(13, 300, 100, 400, 8, 2, 128, torch.float16, 8000)
