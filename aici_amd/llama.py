@@ -130,9 +130,14 @@ class Llama:
                 and kernels.rms_norm_linear_takes(x, norm_weight, weight))
 
     def _proj(self, x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-        """x @ weight.T (llama.rs:81-83, 210).  (A vocabulary's rows, 128256 x 4096, us, library / C ABI: 32 rows 197 / 161, 64 rows
-        209 / 176, 128 rows 233 / 219.)"""
-        if self.skinny_linear and kernels.linear_takes(x, weight):
+        """x @ weight.T (llama.rs:81-83, 210).  A vocabulary's rows with more than 64 sequences stay with the library where the kernel reads
+        them front to back (columns no multiple of 2048, rows none of 256), and with long rows from 97 sequences on.  us, library / C ABI:
+        128256 x 4096 32 rows 197 / 161, 64 rows 209 / 176, 128 rows 233 / 219; 64 / 96 / 128 rows 65536 x 5120 118 / 115, 122 / 140, 126 / 150,
+        65536 x 3072 77 / 70, 81 / 85, 84 / 91, 151936 x 4096 260 / 253, 268 / 287, 278 / 296, 131072 x 8192 0.91, 0.95, 1.05 of the library's.
+        49 to 64 rows: 0.65 to 1.06 of it, 0.87 on average."""
+        rows, (n, k) = x.size(0), weight.shape
+        if self.skinny_linear and kernels.linear_takes(x, weight) and (
+                rows <= 64 or n < 65536 or (n % 256 == 0 and k % 2048 == 0 and (k <= 4096 or (k <= 8192 and rows <= 96)))):
             return kernels.linear(x, weight)
         return x @ weight.t()
 
