@@ -387,3 +387,45 @@ def test_which_steps_are_one_launch(device, tuning, heads, priors, new, contexts
     tuning("decode_flat", 0)  # the launches by themselves
     want = attn.varlen_attn(q, k, v, batch, kc, vc, cached=True)
     assert (got - want).abs().max().item() <= TOL[torch.bfloat16]
+
+
+def gathered(monkeypatch):
+    """attn.varlen_attn on batches without block tables for their chunks: hipattn_varlen_attn, whose gather is counted."""
+    calls, inner = [], attn.varlen_attn
+
+    def run(q, k, v, batch, kc, vc, **kw):
+        def call():
+            return inner(q, k, v, dataclasses.replace(batch, multi_block_tables=None), kc, vc, **kw)
+
+        out, kernels = launched(call)
+        calls.append(sum("cache_move" in n for n in kernels))
+        return out
+
+    monkeypatch.setattr(attn, "varlen_attn", run)
+    return calls
+
+
+@pytest.mark.filterwarnings("ignore:Profiler clears events")
+@pytest.mark.parametrize("name", ["phi2", "phi2_fused", "gqa", "all_prefill", "ratio_2", "ratio_3", "narrow"])
+def test_gathered_route_of_16_token_blocks(device, monkeypatch, name):
+    args = {"phi2": (31, [0, 100, 200, 300], 64, 20, 30, 500, 32, 32, 80, torch.float16, 1024, False),
+            "phi2_fused": (31, [0, 100, 200, 300], 64, 20, 30, 500, 32, 32, 80, torch.float16, 1024, True),
+            "gqa": (32, [0, 17, 640], 200, 33, 1, 900, 32, 8, 128, torch.bfloat16, 2048, False),
+            "all_prefill": (33, [0, 0, 0], 150, 0, 1, 2, 8, 8, 64, torch.float16, 256, False),
+            "ratio_2": (36, [1300, 40], 2, 40, 1, 2000, 16, 8, 96, torch.float16, 3000, False),
+            "ratio_3": (37, [900, 0, 450], 70, 17, 500, 900, 12, 4, 112, torch.bfloat16, 1500, False),
+            "narrow": (38, [480, 479], 33, 3, 31, 33, 16, 2, 64, torch.bfloat16, 200, False)}[name]
+    calls = gathered(monkeypatch)
+    y, want, (kc, vc, kc_ref, vc_ref), _ = mixed_step(*args, device)
+    assert calls == [2]  # the scatter and the gather
+    assert not torch.isnan(y.float()).any()
+    assert (y.float() - want).abs().max().item() <= TOL[args[9]]
+    assert torch.equal(kc.view(torch.int16), kc_ref.view(torch.int16)) and torch.equal(vc.view(torch.int16), vc_ref.view(torch.int16))
+
+
+@pytest.mark.filterwarnings("ignore:Profiler clears events")
+@pytest.mark.parametrize("layout", ["contiguous", "fused_qkv"])
+def test_config4_full_size_gathered(device, monkeypatch, layout):
+    calls = gathered(monkeypatch)
+    test_config4_full_size_sampled(device, layout, False)
+    assert calls == [2]
