@@ -382,7 +382,9 @@ def mixed_step_leg(dev, stream, steps: int) -> dict:
     """One layer's attention for a mixed continuous-batching step in the Phi-2 shape (32 MHA heads, d 80,
     fp16): four 512-token chunks with 0/1k/2k/3k tokens already cached plus 120 single-token rows with
     contexts U[1k,8k] (seed 4) -- `llm::varlen_attn` as one C-ABI call, by the reference's route (scatter,
-    gather, varlen prefill, paged decode) and with the multi-token rows reading the cache through block tables."""
+    gather, varlen prefill, paged decode: a batch without block tables for its chunks) and with the multi-token rows
+    reading the cache through block tables."""
+    import dataclasses
     import math
 
     import numpy as np
@@ -418,8 +420,8 @@ def mixed_step_leg(dev, stream, steps: int) -> dict:
     out = {"config": {"workload": "mixed step: 4 x 512 new tokens after 0/1k/2k/3k cached + 120 decode rows ctx "
                                   "U[1k,8k] (seed 4), 32 MHA heads, d 80, fp16", "tokens": T,
                       "prefill_flops": flops, "decode_kv_bytes": kv_bytes}}
-    for name, paged_prefill in (("reference_route", False), ("paged_prefill_route", True)):
-        fn = lambda: attn.varlen_attn(q, k, v, bi, kc, vc, 1.0 / math.sqrt(d), paged_prefill=paged_prefill)
+    for name, batch in (("reference_route", dataclasses.replace(bi, multi_block_tables=None)), ("paged_prefill_route", bi)):
+        fn = lambda: attn.varlen_attn(q, k, v, batch, kc, vc, 1.0 / math.sqrt(d), paged_prefill=name == "paged_prefill_route")
         for _ in range(10):
             fn()
         torch.cuda.synchronize()
