@@ -8,7 +8,7 @@
 // operands of v_mfma_f32_16x16x32 are read from LDS without bank conflicts.  What bounds them is how many whole
 // cache lines are on their way: the same loop with W loaded straight into the operands (16 rows x 64 bytes per instruction, so
 // every line asked for twice, and both copies of it held in the 32 KB L1) reached 5.1 TB/s on a 28672 x 4096 weight and one row of x,
-// 4.0 with sixteen; this form 5.9 and 5.4 (library GEMM: 4.0 / 3.9).
+// 4.0 with sixteen; this form 5.9 and 5.4, and with ranges of k that begin inside (StageOrder) 6.5 and 6.4 (library GEMM: 4.0 / 3.9).
 //
 //   linear_stream_kernel, up to 16 rows of x and a weight whose k is cut into ranges: a wavefront owns 16 rows of W and keeps a private
 //   ring, its own copy of the rows of x in it, so nothing waits for anything but the wavefront's own copies; wavefronts that share
@@ -55,7 +55,9 @@ constexpr int kLinMT = 8;         // 16-row tiles of x
 constexpr int kLinStageK = 64;    // values of k per stage: 128 bytes of a row
 constexpr int kLinStreamRows = 16;
 constexpr int kLinHeldRows = 4;
-constexpr int kLinHeldBytes = 40 * 1024;  // of x and the norm's weight: two workgroups per compute unit, where the ranges' sums take 4 KB (16 at most)
+// Of x and the norm's weight: two workgroups of four wavefronts per compute unit, where the ranges' sums take 4 KB (16 at most); one of eight
+// (64 KB of ring, 8 of sums), which has the unit to itself (wide_workgroups).
+constexpr int kLinHeldBytes = 40 * 1024;
 constexpr int kHeldStages = 4;
 constexpr int kLinMaxRanges = 8;  // ranges of k that the library itself chooses
 
@@ -841,9 +843,6 @@ struct LinearPlan {
   size_t partial_bytes;  // fp32 sums of every range, [range][128 rows][N]; not used by the few-rows kernel
 };
 
-// The ranges of k depend on the weight alone (see above).  As far as eight ranges allow: 1024 wavefronts' worth of (16 rows, range)
-// pairs, four per compute unit, and no range longer than 2048 once k is cut at all -- 4096 x 4096 and 6144 x 4096 four, 4096 x
-// 14336 eight, weights of 16384 rows and more none.
 // Weights that are not cut and whose workgroups of 64 rows are more than one to a compute unit, but not two, while those of 128 rows are at most
 // one: then every unit with work has the same.  us, 64 / 128 rows, 16 rows of x: 16384 x 4096 21.7 / 28.9; 18432 x 4096 33.7 / 29.2; 22016 x 4096
 // gated 34.6 / 30.8; 28672 x 4096 gated 36.5 / 36.1, 32 rows 38.4 / 36.7; 32000 x 4096 40.4 / 40.5; 37888 x 3584 gated 46.4 / 56.0; 51200 x 2560
@@ -852,6 +851,9 @@ struct LinearPlan {
 // stages for six: 37.5 / 38.8.
 bool wide_workgroups(int N) { return N > 64 * 256 && N <= 128 * 256; }
 
+// The ranges of k depend on the weight alone (see above).  As far as eight ranges allow: 1024 wavefronts' worth of (16 rows, range)
+// pairs, four per compute unit, and no range longer than 2048 once k is cut at all -- 4096 x 4096 and 6144 x 4096 four, 4096 x
+// 14336 eight, weights of 16384 rows and more none.
 LinearPlan plan_linear(int M, int N, int K, bool few_only) {
   const Tuning &tn = tuning();
   LinearPlan pl;
